@@ -259,6 +259,11 @@ struct Ctrl {
 
 struct Unet;  // learned warm start (tl_unet.hip)
 
+// field copies between the host and the pitched device layout go through
+// pinned slots of at most this size, this many of them
+constexpr int STAGE_SLOTS = 8;
+constexpr size_t STAGE_BYTES = (size_t)4 << 20;
+
 }  // namespace tl
 
 struct tl_ctx {
@@ -301,6 +306,11 @@ struct tl_ctx {
     tl_state *states_d = nullptr;
     std::string err;
     hipEvent_t ev[2] = {nullptr, nullptr};   // batch pipeline
+    // pinned host staging of the field copies: up to STAGE_SLOTS slots of
+    // stage_slot bytes, one event per slot (allocated on the first copy)
+    char *stage = nullptr;
+    size_t stage_slot = 0;
+    hipEvent_t stage_ev[tl::STAGE_SLOTS] = {};
     // per-launch event timing of selected kernels (tl_profile_begin)
     unsigned prof_mask = 0;
     unsigned prof_period = 1;   // bracket every prof_period-th launch of a kernel
@@ -340,6 +350,9 @@ hipError_t launch_set_state(tl_ctx *c, const tl_state *states_d, int nstates);
 hipError_t launch_copy_full(tl_ctx *c, const double *a, double *b);
 hipError_t launch_copy_vec(tl_ctx *c, const double *a, double *b);
 hipError_t launch_copy_energy(tl_ctx *c);
+// rows j0 .. j0+rows-1 of a field to / from packed rows of X doubles
+hipError_t launch_pack_rows(tl_ctx *c, const double *field, double *packed, int j0, int rows);
+hipError_t launch_unpack_rows(tl_ctx *c, double *field, const double *packed, int j0, int rows);
 // what k_init_coef writes besides kx, ky
 enum { INIT_CG = 0, INIT_JACOBI = 1, INIT_COEF_ONLY = 2 };
 hipError_t launch_init_coef(tl_ctx *c, double rx, double ry, int coefficient, int what);

@@ -538,6 +538,24 @@ __global__ __launch_bounds__(TB) void k_copy_full(Geo g, const double *__restric
     b[i] = a[i];
 }
 
+// Rows of a field between the pitched layout and packed rows of X doubles in
+// pinned host memory (grid: 256-column strips x rows), one double per lane.
+// The kernel itself is the transfer: its packed side goes over the host link.
+// A strided hipMemcpy2D to or from pageable memory costs 7-9 us per row
+// (2048^2: 17.2 ms, 1.95 GB/s), whatever the row length; through the slots
+// 2048^2 takes 1.4 ms, 512^2 0.13 instead of 3.7, 4096^2 4.7 instead of 42.
+__global__ __launch_bounds__(TB) void k_pack_rows(Geo g, const double *__restrict__ a, double *__restrict__ p, int j0)
+{
+    const int k = blockIdx.x * TB + threadIdx.x;
+    if (k < g.X) p[(size_t)blockIdx.y * g.X + k] = a[(long)(j0 + (int)blockIdx.y) * g.pitch + k + (XCOL - g.hd)];
+}
+
+__global__ __launch_bounds__(TB) void k_unpack_rows(Geo g, double *__restrict__ a, const double *__restrict__ p, int j0)
+{
+    const int k = blockIdx.x * TB + threadIdx.x;
+    if (k < g.X) a[(long)(j0 + (int)blockIdx.y) * g.pitch + k + (XCOL - g.hd)] = p[(size_t)blockIdx.y * g.X + k];
+}
+
 // plain 16-byte-per-lane copy of n2 double pairs (bandwidth calibration)
 __global__ __launch_bounds__(TB) void k_copy_vec(const double2 *__restrict__ a, double2 *__restrict__ b, size_t n2)
 {
@@ -3404,6 +3422,18 @@ hipError_t launch_copy_vec(tl_ctx *c, const double *a, double *b)
 {
     const size_t n2 = c->g.elems / 2;
     k_copy_vec<<<(unsigned)((n2 + TB - 1) / TB), TB, 0, c->stream>>>((const double2 *)a, (double2 *)b, n2);
+    return hipGetLastError();
+}
+
+hipError_t launch_pack_rows(tl_ctx *c, const double *field, double *packed, int j0, int rows)
+{
+    k_pack_rows<<<dim3((c->g.X + TB - 1) / TB, rows), TB, 0, c->stream>>>(c->g, field, packed, j0);
+    return hipGetLastError();
+}
+
+hipError_t launch_unpack_rows(tl_ctx *c, double *field, const double *packed, int j0, int rows)
+{
+    k_unpack_rows<<<dim3((c->g.X + TB - 1) / TB, rows), TB, 0, c->stream>>>(c->g, field, packed, j0);
     return hipGetLastError();
 }
 
