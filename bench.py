@@ -39,10 +39,9 @@ from tealeaf_hip import _lib, decks  # noqa: E402
 PEAK_HBM_GBS = 8000.0
 PROFILE_PERIOD = 15  # odd: both parities of the alternating FP32 UR kernel are sampled
 # algorithmic bytes per interior cell per launch (arrays read once + written once).
-# A CG iteration is two kernels.
-#   FP64:  PW = [p = r + beta p; w = A p] reads p, r, Kx, Ky, writes p', w  (48 B)
-#          UR = [u += alpha p; r -= alpha w] reads u, p, r, w, writes u, r   (48 B)
-#   FP32 inner CG (operator from one 16-bit cell-coefficient array gc: half with a
+#   FP64:  an iteration is one sweep; reads r, p, the cell coefficient, writes r, p (40 B)
+#          and at even iterations also reads and writes u                  (+16 B)
+#   FP32 inner CG as two kernels per iteration (operator from one 16-bit cell-coefficient array gc: half with a
 #   power-of-two scale, or bfloat16 when the range does not fit; w not stored):
 #          PW reads p, r (4 B each), gc (2 B), writes p'                    (14 B)
 #          UR = [r -= alpha A p] reads p, r, gc, writes r                   (14 B)
@@ -57,9 +56,9 @@ PROFILE_PERIOD = 15  # odd: both parities of the alternating FP32 UR kernel are 
 #          first sweep reads r(t-1), p(t-1), gc                           (10 B)
 #          second sweep reads r(t-1), p(t-1), gc, x, writes r(t+1), p(t+1), x (26 B)
 #          i.e. 18 B per iteration
-# P64 is only the final p update of an FP64 solve.
+# P64 is the p update of PPCG's outer iterations.
 KERNEL_BYTES = {
-    _lib.TL_K_CG_W64: 48, _lib.TL_K_CG_UR64: 48, _lib.TL_K_CG_P64: 24,
+    _lib.TL_K_CG_W64: 40, _lib.TL_K_CG_UR64: 56, _lib.TL_K_CG_P64: 24,
     _lib.TL_K_CG_W32: 14, _lib.TL_K_CG_UR32: 20, _lib.TL_K_CG_P32: 0, _lib.TL_K_CGF32: 22,
     _lib.TL_K_CGP_G32: 10, _lib.TL_K_CGP_U32: 26,
 }

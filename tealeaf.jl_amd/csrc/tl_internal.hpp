@@ -50,20 +50,6 @@ constexpr int TBV = TL_TBV;
 #ifndef TL_PIPE_UR32
 #define TL_PIPE_UR32 1
 #endif
-// the same for the FP64 CG kernels (measured: PW 4 rows pipelined 2.6%
-// faster than plain; the streaming UR gains nothing from it)
-#ifndef TL_RV_PW64
-#define TL_RV_PW64 TL_RV
-#endif
-#ifndef TL_RV_UR64
-#define TL_RV_UR64 TL_RV
-#endif
-#ifndef TL_PIPE_PW64
-#define TL_PIPE_PW64 1
-#endif
-#ifndef TL_PIPE_UR64
-#define TL_PIPE_UR64 0
-#endif
 #ifndef TL_VEC_BLOCKS32
 #define TL_VEC_BLOCKS32 2048
 #endif
@@ -118,6 +104,19 @@ constexpr int TBV = TL_TBV;
 #ifndef TL_VEC_BLOCKS_PPCG2
 #define TL_VEC_BLOCKS_PPCG2 768
 #endif
+// the single-sweep FP64 CG kernel: columns per wave, waves on large grids (one
+// round at 2 waves per SIMD) and least rows per band.  Measured in one box, us
+// per iteration at 3072^2 / 1501x1103: 120 columns (60 lanes, 64-byte aligned
+// stores) 88.2 / 21.9, 124 (62 lanes) 92.3 / 22.0, 112 (whole cache lines) 87.8 /
+// 22.1; 3 waves per SIMD (168 VGPRs, 32 spilled) 102 / 28; 4096 waves in two
+// rounds 98.6 / 29.6; two rows requested ahead 96.8 / 21.7
+#define TL_S64_COLS 120
+#define TL_S64_WAVES 2048
+#define TL_S64_ROWS 4
+// sweeps over more bytes than this (the Infinity Cache) use streaming access.
+// Measured with the FP64 CG sweep: 453 MB of arrays (3072^2) 92.6 us per
+// iteration streaming, 102.2 cached; 83 MB (1501x1103) 25.1 and 21.9.
+constexpr size_t TL_CACHE_BYTES = (size_t)256 << 20;
 #ifndef TL_CGF_DEPTH
 #define TL_CGF_DEPTH 0
 #endif
@@ -205,6 +204,15 @@ enum GcFmt : int { GC_BF16 = 0, GC_F16 = 1 };
 #define TL_NT_2STEP_ST 0
 #endif
 
+// Waves of a sweep with overlapped tiles: a wave owns a strip of columns (lanes
+// beside them hold the neighbouring tiles' columns) and a band of ty rows; 4
+// waves per block.  See wave_tile for the order.
+struct Tiles {
+    int strips, ty, bands, blocks;
+};
+// neighbouring tiles dealt to one XCD in a run (4 and 64: 1-2% slower)
+constexpr int TILE_CHUNK = 16;
+
 struct Geo {
     int nx, ny, hd;
     int X, Y;                  // nx + 2hd, ny + 2hd
@@ -216,6 +224,7 @@ struct Geo {
     int gx2, gy2, ty2;         // FP64 vector kernels: blocks of 2*TB columns x ty2 rows
     int gyf, tyf;              // fused FP32 kernel: gx4*gyf blocks of 4*TB columns x tyf rows
     int gyq, tyq;              // two-step PPCG kernel: gx2*gyq blocks of 2*TB columns x tyq rows
+    Tiles s64;                 // single-sweep FP64 CG
     int nbmax;                 // stride of the partial-sum arrays (max block count)
     size_t elems;              // elements per allocation
 };
@@ -274,7 +283,9 @@ struct tl_ctx {
     // FP64 fields (reference Chunk fields; u and sd have ping-pong twins)
     double *f[TL_NFIELDS] = {};
     double *u_alt = nullptr, *sd_alt = nullptr, *guess = nullptr;
-    double *r_alt1 = nullptr, *r_alt2 = nullptr;  // PPCG: r between two-step sweeps
+    double *r_alt1 = nullptr, *r_alt2 = nullptr;  // r's second buffer (CG sweeps) / between PPCG's two-step sweeps
+    double *g64 = nullptr;    // FP64 cell coefficient 1/w of the CG sweeps (see k_init_coef)
+    double hx64 = 0, hy64 = 0;  // its face scales rx/2, ry/2
     // FP32 fields of the mixed-precision solve
     // FP32 inner CG: cell coefficient gc = 1/w (tl_gc_t) and its face scale
     // (rx/2, ry/2), search direction, residual, correction
@@ -288,8 +299,8 @@ struct tl_ctx {
     double *partials = nullptr;
     size_t partials_len = 0;
     unsigned nb_w = 0, nb_r[2] = {0, 0}, nb_m = 0;  // block counts of the last producer of each partial array
-    double *p_alt = nullptr;   // ping-pong twin of p for the fused CG kernels (FP64)
-    double *cg_u = nullptr;    // the vector the fused FP64 UR adds alpha p to: u, or (relative stop
+    double *p_alt = nullptr;   // ping-pong twin of p for the CG sweeps (FP64)
+    double *cg_u = nullptr;    // the vector the FP64 CG adds alpha p to: u, or (relative stop
                                // rule) a correction added to u at every true-residual check
     float *p32b = nullptr;     // same for FP32
     // fused FP32 inner CG: second residual buffer (r ping-pongs, being read
@@ -353,8 +364,9 @@ hipError_t launch_copy_energy(tl_ctx *c);
 // rows j0 .. j0+rows-1 of a field to / from packed rows of X doubles
 hipError_t launch_pack_rows(tl_ctx *c, const double *field, double *packed, int j0, int rows);
 hipError_t launch_unpack_rows(tl_ctx *c, double *field, const double *packed, int j0, int rows);
-// what k_init_coef writes besides kx, ky
-enum { INIT_CG = 0, INIT_JACOBI = 1, INIT_COEF_ONLY = 2 };
+// what k_init_coef writes besides kx, ky (INIT_CG64: also what the single-sweep
+// FP64 CG needs, the cell coefficient and cleared second buffers)
+enum { INIT_CG = 0, INIT_JACOBI = 1, INIT_COEF_ONLY = 2, INIT_CG64 = 3 };
 hipError_t launch_init_coef(tl_ctx *c, double rx, double ry, int coefficient, int what);
 hipError_t launch_halo(tl_ctx *c, unsigned mask, int depth, double *const *extra, int nextra);
 hipError_t launch_cg_init_resid(tl_ctx *c, const double *guess);
@@ -362,9 +374,10 @@ hipError_t launch_resid_norm_slot(tl_ctx *c, const double *b, const double *x, i
 // tref > 0: the launch is being captured into a hipGraph batch whose first
 // iteration is tref (t only selects the buffers; the kernel takes its
 // iteration number from Ctrl::tg)
-hipError_t launch_cg_pw64(tl_ctx *c, int t, int tref = 0);
-hipError_t launch_cg_urv64(tl_ctx *c, int t, int tref = 0);
-hipError_t launch_cg_pfinal64(tl_ctx *c, int t);
+hipError_t launch_cgs64(tl_ctx *c, int t, int tref = 0);
+hipError_t launch_cgs_dots(tl_ctx *c, int T);
+hipError_t launch_cgs_pending(tl_ctx *c, int T);
+hipError_t launch_cgs_final(tl_ctx *c, int T);
 hipError_t launch_cg_w64(tl_ctx *c, int t);
 hipError_t launch_cg_ur64(tl_ctx *c, int t);
 hipError_t launch_cg_p64(tl_ctx *c, int t);

@@ -8,7 +8,7 @@
 // fetched from HBM once per sweep.  Left/right neighbours are re-read through
 // L1/L2.
 //
-// The CG iteration kernels (k_cg_pwv, k_cg_urv, k_cgg) are vectorised: a
+// The iteration kernels are vectorised: a
 // thread owns V = 4 (FP32) or 2 (FP64) consecutive columns loaded as one
 // 16-byte vector, left/right neighbours come from the adjacent lanes (lanes
 // 0 and 63 load the column outside the wave together with the row loads),
@@ -40,6 +40,20 @@
 #include "tl_internal.hpp"
 
 namespace tl {
+
+// Tiles of `cols` columns for at most about `waves` waves (one round of them on
+// the chip), bands of at least `min_rows` rows.
+static Tiles make_tiles(int nx, int ny, int cols, int waves, int min_rows)
+{
+    Tiles t{};
+    t.strips = (nx + cols - 1) / cols;
+    const int bands = std::min(std::max(waves / t.strips, 1), (ny + min_rows - 1) / min_rows);
+    t.ty = (ny + bands - 1) / bands;
+    t.bands = (ny + t.ty - 1) / t.ty;
+    const int chunks = (t.strips * t.bands + TILE_CHUNK - 1) / TILE_CHUNK;
+    t.blocks = 8 * ((chunks + 7) / 8 * TILE_CHUNK / 4);
+    return t;
+}
 
 Geo make_geo(int nx, int ny, int hd)
 {
@@ -104,6 +118,8 @@ Geo make_geo(int nx, int ny, int hd)
     }
     g.nbmax = std::max(std::max(g.gx * g.gy, g.gx4 * g.gyp4), std::max(g.gx4 * g.gy4, g.gx2 * g.gy2));
     g.nbmax = std::max(g.nbmax, g.gx4 * g.gyf);
+    g.s64 = make_tiles(nx, ny, TL_S64_COLS, TL_S64_WAVES, TL_S64_ROWS);
+    g.nbmax = std::max(g.nbmax, g.s64.blocks);
     return g;
 }
 
@@ -566,12 +582,19 @@ __global__ __launch_bounds__(TB) void k_copy_vec(const double2 *__restrict__ a, 
 // CG.init! lines 51-68 (CG.jl) / Jacobi.init! lines 38-55 (Jacobi.jl):
 // u = energy*density on every cell; p = r = 0 (CG) or u0 = u (Jacobi); the
 // face coefficients kx, ky over the reference's range k, j in hd+1 : X-1.
+// INIT_CG64 also clears the second buffers of p and r and writes the cell
+// coefficient g64 = 1/w over the interior and its negative, mirrored, into the
+// ring of cells around it: the face coefficient hx (g + g') of a domain face is
+// then exactly zero, which is the zero flux of the reflective halo
+// (kernels.jl:191-210), so the sweeps need no special case at the domain's
+// edges as long as what the ring holds of p and r is finite (it is cleared).
 __global__ __launch_bounds__(TB) void k_init_coef(Geo g, const double *__restrict__ rho,
                                                   const double *__restrict__ e, double *__restrict__ u,
                                                   double *__restrict__ p, double *__restrict__ r,
                                                   double *__restrict__ u0, double *__restrict__ kx,
-                                                  double *__restrict__ ky, double rx, double ry, int recip,
-                                                  int what)
+                                                  double *__restrict__ ky, double *__restrict__ p2,
+                                                  double *__restrict__ r2, double *__restrict__ g64, double rx,
+                                                  double ry, int recip, int what)
 {
     const int k = blockIdx.x * TB + threadIdx.x;
     const int j = blockIdx.y;
@@ -585,6 +608,15 @@ __global__ __launch_bounds__(TB) void k_init_coef(Geo g, const double *__restric
         } else {
             p[i] = 0.0;
             r[i] = 0.0;
+        }
+        if (what == INIT_CG64) {
+            p2[i] = 0.0;
+            r2[i] = 0.0;
+            const int x = k - g.hd, y = j - g.hd;
+            const int xc = min(max(x, 0), g.nx - 1), yc = min(max(y, 0), g.ny - 1);
+            const double w = rho[at(g, xc, yc)];
+            const double gv = recip ? w : 1.0 / w;
+            g64[i] = xc == x && yc == y ? gv : -gv;
         }
     }
     if (k >= g.hd && k <= g.X - 2 && j >= g.hd && j <= g.Y - 2) {
@@ -1011,216 +1043,282 @@ __device__ __forceinline__ void row_batches(int y0, int y1, Load &&load, Compute
     }
 }
 
-// Iteration t of the fused CG: for t >= 2, first the end of iteration t-1 --
-// beta = rr(t-1)/rr(t-2) and the stop test (CG.jl:39-42, 24) -- then
-// p = r + beta p (CG.p!, written to pout; p is ping-ponged because every
-// thread reads its neighbours' old p), then w = A p and the partial sums of
-// p.w (CG.w!).  For t = 1, p comes from CG.init!.
-template <typename T, int V, int RB, bool PIPE>
-__global__ __launch_bounds__(TBV) void k_cg_pwv(Geo g, int ty, int t, const T *__restrict__ pin, T *__restrict__ pout,
-                                               const T *__restrict__ r, const T *__restrict__ kx,
-                                               const T *__restrict__ ky, T *__restrict__ w, Ctrl *__restrict__ ctrl,
-                                               double *__restrict__ pw, const double *__restrict__ prcur, unsigned nbc,
-                                               double *__restrict__ hist_b)
+// -------------------------------- FP64 CG, one sweep over the grid per iteration
+//
+// Overlapped wave tiles.  A lane owns V = 2 consecutive columns (16 bytes);
+// lanes 1-60 of a wave own its tile's 120 columns and the lanes beside them hold
+// the columns to either side, so every value a lane needs two columns away
+// comes from its neighbour lane and no lane has a special role: the outer lanes
+// compute along and store nothing.  6% of the loads and arithmetic are done
+// twice (the loads hit the caches); the alternative, edge lanes that load and
+// compute the columns outside the wave, costs registers and selects in every
+// row.  120 columns keep the stores 64-byte aligned.  A wave walks its band from
+// two rows below to two rows above it.
+//
+// Tile of this wave (false: none).  Tiles are numbered strip by strip, band by
+// band.  Blocks go round-robin to the 8 XCDs, each with its own L2, so runs of
+// TILE_CHUNK neighbouring tiles are dealt to the XCDs in turn: neighbours share
+// an L2 and every XCD gets the same number of tiles.
+__device__ __forceinline__ bool wave_tile(const Tiles &o, int &strip, int &band)
 {
-    t = iter_of(t, ctrl);
-    if (t > ctrl->stop_iter) return;
-    T beta = (T)0;
-    const bool fuse = t >= 2;
-    if (fuse) {
-        // rr(t-1) from the partials of UR(t-1); rr(t-2) as this kernel's
-        // previous launch summed it
-        double a1[1];
-        sum_partials<1, TBV>(prcur, nbc, g.nbmax, a1);
-        const double rrn = a1[0], rro = ctrl->rrs[(t - 2) & 1];
-        const double b = rrn / rro;
-        const int why = decide_why(ctrl, t - 1, rrn);
-        if (block_id() == 0 && threadIdx.x == 0) {
-            ctrl->rrs[(t - 1) & 1] = rrn;
-            ctrl->beta = b;
-            ctrl->rro = rrn;
-            ctrl->err = rrn;
-            ctrl->iters = t - 1;
-            if (hist_b) hist_b[t - 2] = b;
-            record_stop(ctrl, t - 1, why);
-        }
-        if (why != WHY_NONE) return;  // every block derives the same decision
-        beta = (T)b;
-    }
-    const VCol<V> cl = vcolumn<V>(g, ty);
-    const T *pp = fuse ? pin : pout;
-#if !TL_EDGE_PF
-    // p after the update at column x of row element index i
-    auto pnew = [&](long i) -> T { return fuse ? r[i] + beta * pp[i] : pp[i]; };
-#endif
-    double acc[1] = {0.0};
-    if (cl.y0 < g.ny) {
-        T dn[V], cur[V], kyd[V];
-        {
-            const long i0 = at(g, cl.xl, cl.y0), id = at(g, cl.xl, max(cl.y0 - 1, 0));
-            T a[V], b2[V];
-            vload<T, V>(a, pp + i0);
-            if (fuse) {
-                vload<T, V>(b2, r + i0);
-#pragma unroll
-                for (int j = 0; j < V; ++j) cur[j] = b2[j] + beta * a[j];
-                vload<T, V>(a, pp + id);
-                vload<T, V>(b2, r + id);
-#pragma unroll
-                for (int j = 0; j < V; ++j) dn[j] = b2[j] + beta * a[j];
-            } else {
-#pragma unroll
-                for (int j = 0; j < V; ++j) cur[j] = a[j];
-                vload<T, V>(dn, pp + id);
-            }
-            vload<T, V>(kyd, ky + i0);
-        }
-#if TL_EDGE_PF
-        // lanes 0 / 63 of a wave read the column left / right of the wave's
-        // columns (and lane 63 the face coefficient right of it) together
-        // with the row loads below, not when the row is used
-        const bool eneed = (cl.lane == 0 && cl.xl > 0) || (cl.lane == 63 && cl.xl + V < g.nx);
-        const long eoff = cl.lane == 0 ? -1 : V;
-        T ecur = (T)0;
-        if (eneed) {
-            const long ie = at(g, cl.xl, cl.y0) + eoff;
-            ecur = fuse ? r[ie] + beta * pp[ie] : pp[ie];
-        }
-#endif
-        // the loads of RB rows, issued together
-        struct Batch {
-            T up[RB][V], kxv[RB][V], kyu[RB][V], rup[RB][V];
-#if TL_EDGE_PF
-            T eup_p[RB], eup_r[RB], ekx[RB];
-#endif
-        };
-        auto load_batch = [&](Batch &B, int yb) {
-#pragma unroll
-            for (int q = 0; q < RB; ++q) {
-                const int y = yb + q;
-                const long ic = atc(g, cl.xl, y), iu = atc(g, cl.xl, y + 1);
-                vload<T, V>(B.up[q], pp + iu);
-                if (fuse) vload<T, V>(B.rup[q], r + iu);
-                vload<T, V>(B.kxv[q], kx + ic);
-                vload<T, V>(B.kyu[q], ky + at(g, cl.xl, min(y + 1, g.ny)));
-#if TL_EDGE_PF
-                B.eup_p[q] = B.eup_r[q] = B.ekx[q] = (T)0;
-                if (eneed) {
-                    B.eup_p[q] = pp[iu + eoff];
-                    if (fuse) B.eup_r[q] = r[iu + eoff];
-                }
-                if (cl.lane == 63) B.ekx[q] = kx[ic + V];
-#endif
-            }
-        };
-        auto compute_batch = [&](const Batch &B, int yb) {
-#pragma unroll
-            for (int q = 0; q < RB; ++q) {
-                const int y = yb + q;
-                const long ic = atc(g, cl.xl, y);
-                T u2[V];
-#pragma unroll
-                for (int j = 0; j < V; ++j) u2[j] = fuse ? B.rup[q][j] + beta * B.up[q][j] : B.up[q][j];
-                // clamp the row above at the top edge (reflection: the row itself)
-                if (y + 1 >= g.ny) {
-#pragma unroll
-                    for (int j = 0; j < V; ++j) u2[j] = cur[j];
-                }
-                T lv, rv;
-#if TL_EDGE_PF
-                auto col_val = [&](int) -> T { return ecur; };
-#else
-                auto col_val = [&](int x) -> T { return pnew(ic + (x - cl.xl)); };
-#endif
-                vneigh<T, V>(g, cl, cur, col_val, lv, rv);
-                // kx of the face right of the last column: next lane's first kx
-                T kxn = lane_down1<false>(B.kxv[q][0]);
-#if TL_EDGE_PF
-                if (cl.lane == 63) kxn = B.ekx[q];
-#else
-                if (cl.lane == 63) kxn = kx[ic + V];
-#endif
-                T wv[V];
-#pragma unroll
-                for (int j = 0; j < V; ++j) {
-                    const T kxr = j < V - 1 ? B.kxv[q][j + 1] : kxn;
-                    wv[j] = vsmvp<T, V>(g, cl.xl, j, cur, lv, rv, dn[j], u2[j], B.kxv[q][j], kxr, kyd[j],
-                                        B.kyu[q][j]);
-                }
-                if (y < cl.y1 && cl.active) {
-                    vstore_n<T, V>(w + ic, wv, g.nx - cl.x0);
-                    if (fuse) vstore_n<T, V>(pout + ic, cur, g.nx - cl.x0);
-#pragma unroll
-                    for (int j = 0; j < V; ++j)
-                        if (cl.x0 + j < g.nx) acc[0] += (double)wv[j] * (double)cur[j];
-                }
-#pragma unroll
-                for (int j = 0; j < V; ++j) {
-                    dn[j] = cur[j];
-                    cur[j] = u2[j];
-                    kyd[j] = B.kyu[q][j];
-                }
-#if TL_EDGE_PF
-                // the row above becomes the current row (at the top edge the
-                // clamped load read the current row itself)
-                ecur = fuse ? B.eup_r[q] + beta * B.eup_p[q] : B.eup_p[q];
-#endif
-            }
-        };
-        row_batches<PIPE, RB, Batch>(cl.y0, cl.y1, load_batch, compute_batch);
-    }
-    write_partials<1, TBV>(acc, pw, g.nbmax);
+    const int i = (int)(blockIdx.x >> 3) * 4 + (int)(threadIdx.x >> 6);
+    const int n = (i / TILE_CHUNK * 8 + (int)(blockIdx.x & 7)) * TILE_CHUNK + i % TILE_CHUNK;
+    strip = n % o.strips;
+    band = n / o.strips;
+    return band < o.bands;
 }
 
-// CG.ur!, CG.jl:93-98 on V-vectors: alpha = rro/pw from the partials, then
-// u += alpha p; r -= alpha w; partial sums of r^2
-template <typename T, int V, int RB, bool PIPE>
-__global__ __launch_bounds__(TBV) void k_cg_urv(Geo g, int ty, int t, T *__restrict__ u, const T *__restrict__ p,
-                                               T *__restrict__ r, const T *__restrict__ w, Ctrl *__restrict__ ctrl,
-                                               const double *__restrict__ pw, unsigned nbw,
-                                               double *__restrict__ prcur, double *__restrict__ hist_a)
+// Single-reduction CG.  Sweep t receives from sweep t-1 (or from k_cgs_dots
+// after a start or a new true residual) four sums of r = r(t-1), p' = p(t-1):
+//   gamma = (r, r), delta = (r, A r), eps = (r, A p'), pi = (p', A p')
+// and derives, identically in every block,
+//   beta = gamma / gamma(t-2)   (0 at t = 1), the stop test of iteration t-1,
+//   (p, A p) = delta + 2 beta eps + beta^2 pi,   alpha = gamma / (p, A p),
+// the expansion of (r + beta p', A (r + beta p')), which assumes nothing of
+// r and p'.  It then applies the iteration (CG.p!, CG.w!, CG.ur!, CG.jl:82-104):
+// p = r + beta p', q = A p, r(t) = r - alpha q, and at even t the updates of
+// iterations t-1 and t, u += alpha(t-1) p' + alpha p, each rounded as if
+// stored; and it accumulates the four sums of iteration t+1.
+// The operator is c + sum k (c - neighbour) with k = hx (g + g') from one cell
+// coefficient g = 1/w per cell instead of the face arrays (8 bytes per cell
+// instead of 16; equal to CG.jl:61-68 up to rounding); the difference across a
+// face serves the cells on both sides.
+// Bytes per cell: reads r, p', g, writes r, p: 40; at even t also reads and
+// writes u: 56, 48 on average, against 96 for an iteration as two kernels with
+// w stored (p update + operator, then u and r updates), which it replaced.
+// Bound by HBM on large grids (8192^2: 0.68 ms per iteration, 4.8 TB/s of
+// these bytes, against 1.16 ms for the two kernels; 3072^2: 88 us, 5.1 TB/s,
+// against 231), by launch and latency below about 1500^2 (22 us at 1501x1103,
+// against 42).  NT: streaming access (TL_CACHE_BYTES).
+template <bool XUPD, bool NT>
+__global__ __launch_bounds__(TBV) __attribute__((amdgpu_waves_per_eu(2))) void k_cgs(
+    Geo g, int t, const double *__restrict__ rin, double *__restrict__ rout, const double *__restrict__ pin,
+    double *__restrict__ pout, double *__restrict__ u, const double *__restrict__ gc, double hx, double hy,
+    Ctrl *__restrict__ ctrl, const double *__restrict__ sin, unsigned nbin, double *__restrict__ sout, double *__restrict__ hist_a, double *__restrict__ hist_b)
 {
+    constexpr int V = 2;
+    struct Row {
+        double r[V], p[V], g[V], u[V];
+    };
     t = iter_of(t, ctrl);
     if (t > ctrl->stop_iter) return;
-    double ad;
-    if (!cg_alpha_slot<TBV>(g, t, ctrl, pw, nbw, hist_a, &ad)) return;
-    const T alpha = (T)ad;
-    const VCol<V> cl = vcolumn<V>(g, ty);
-    double acc[1] = {0.0};
-    if (cl.active && cl.y0 < g.ny) {
-        struct Batch {
-            T uv[RB][V], pv[RB][V], rv[RB][V], wv[RB][V];
-        };
-        auto load_batch = [&](Batch &B, int yb) {
+    int strip, band;
+    const bool tile = wave_tile(g.s64, strip, band);
+    const int lane = threadIdx.x & 63;
+    const int x = strip * TL_S64_COLS + (lane - 1) * V;
+    const bool act = tile && lane >= 1 && lane <= TL_S64_COLS / V && x < g.nx;
+    const int y0 = band * g.s64.ty, y1 = min(y0 + g.s64.ty, g.ny);
+    // lanes past the ring's column nx + 1 read it again (never used)
+    const long ix = at(g, min(x, (g.nx + 1) / V * V), 0);
+    auto load_row = [&](Row &B, int L) {
+        const long i = ix + L * g.pitch;
+        vload<double, V, NT>(B.r, rin + i);
+        vload<double, V, NT>(B.p, pin + i);
+        vload<double, V, false>(B.g, gc + i);  // streaming: 13% slower at 3072^2
+        if constexpr (XUPD) vload<double, V, NT>(B.u, u + i);
+    };
+    // the band's first row is requested before the block sums the previous
+    // sweep's partials
+    Row Bs[2];
+    if (tile) load_row(Bs[0], y0 - 2);
+
+    double s4[4];
+    sum_partials<4, TBV>(sin, nbin, g.nbmax, s4);
+    const double gam = s4[0];
+    const int why = t >= 2 ? decide_why(ctrl, t - 1, gam) : (int)WHY_NONE;
+    const double bd = t >= 2 ? gam / ctrl->rrs[(t - 2) & 1] : 0.0;
+    const double pap = s4[1] + bd * (2.0 * s4[2] + bd * s4[3]);
+    const double alpha = gam / pap;
+    const bool ok = pap > 0.0 && isfinite(alpha);
+    if (block_id() == 0 && threadIdx.x == 0) {
+        ctrl->rrs[(t - 1) & 1] = gam;
+        ctrl->rro = gam;
+        if (t >= 2) {
+            ctrl->err = gam;
+            ctrl->beta = bd;
+            ctrl->iters = t - 1;
+            hist_b[t - 2] = bd;
+            record_stop(ctrl, t - 1, why);
+        }
+        if (why == WHY_NONE) {
+            ctrl->pw = pap;
+            ctrl->alpha = alpha;
+            ctrl->alphas[t & 1] = alpha;
+            hist_a[t - 1] = alpha;
+            if (!ok) {  // non-positive curvature: stop before this iteration's update
+                ctrl->status = TL_E_BREAKDOWN;
+                ctrl->why = WHY_BREAKDOWN;
+                ctrl->stop_iter = t - 1;
+            }
+        }
+    }
+    if (why != WHY_NONE || !ok) return;  // every block derives the same decision
+    const double alpha_prev = XUPD ? ctrl->alphas[(t - 1) & 1] : 0.0;
+    double acc[4] = {0.0, 0.0, 0.0, 0.0};  // gamma, delta, eps, pi of iteration t+1
+    if (tile) {
+        // Row windows indexed by row, L - (y0 - 2) modulo 3 or 2, in a walk
+        // unrolled six rows at a time: every index is a constant and no value
+        // moves between registers.
+        double P[3][V], N[3][V];   // p(t) at rows L-2..L; r(t) at L-3..L-1
+        double R[2][V], G[2][V];   // r(t-1), g at L-1, L
+        double KX[2][V + 1];       // face coefficients of rows L-2, L-1 (left of column 0 .. right of V-1)
+        double KY[3][V];           // of the faces L-3|L-2, L-2|L-1, L-1|L
 #pragma unroll
-            for (int q = 0; q < RB; ++q) {
-                const long i = atc(g, cl.xl, yb + q);
-                vload<T, V>(B.uv[q], u + i);
-                vload<T, V>(B.pv[q], p + i);
-                vload<T, V>(B.rv[q], r + i);
-                vload<T, V>(B.wv[q], w + i);
+        for (int j = 0; j < V; ++j) {
+#pragma unroll
+            for (int w = 0; w < 3; ++w) P[w][j] = N[w][j] = KY[w][j] = 0.0;
+#pragma unroll
+            for (int w = 0; w < 2; ++w) R[w][j] = G[w][j] = KX[w][j] = KX[w][j + 1] = 0.0;
+        }
+        // A applied to row c (rows dn below, up above)
+        auto apply = [&](double (&q)[V], const double (&c)[V], const double (&dn)[V], const double (&up)[V],
+                         const double (&kxr)[V + 1], const double (&kyd)[V], const double (&kyu)[V]) {
+            double D[V + 1];  // differences c[j] - c[j-1] across the V+1 vertical faces
+            D[0] = c[0] - lane_up1<true>(c[V - 1]);
+#pragma unroll
+            for (int j = 1; j < V; ++j) D[j] = c[j] - c[j - 1];
+            D[V] = lane_down1<true>(D[0]);
+#pragma unroll
+            for (int j = 0; j < V; ++j) {
+                double s = kxr[j] * D[j];
+                s = __builtin_fma(-kxr[j + 1], D[j + 1], s);
+                s = __builtin_fma(kyd[j], c[j] - dn[j], s);
+                s = __builtin_fma(kyu[j], c[j] - up[j], s);
+                q[j] = c[j] + s;
             }
         };
-        auto compute_batch = [&](const Batch &B, int yb) {
+        auto step = [&](auto kc, int L) -> bool {
+            constexpr int K = decltype(kc)::value;
+            // slots: rows L, L-1, L-2 (and L-3 = L) of the three-row windows, L
+            // and L-1 of the two-row ones
+            constexpr int a = K % 3, b = (K + 2) % 3, c = (K + 1) % 3, e = K % 2, f = (K + 1) % 2;
+            if (L > y1 + 1) return false;
+            if (L + 1 <= y1 + 1) load_row(Bs[f], L + 1);
+            const Row &B = Bs[e];
+            const long i = ix + L * g.pitch;
+            KX[f][0] = hx * (lane_up1<true>(G[f][V - 1]) + G[f][0]);
 #pragma unroll
-            for (int q = 0; q < RB; ++q) {
-                if (yb + q < cl.y1) {
-                    const long i = at(g, cl.xl, yb + q);
-                    T un[V], rn[V];
+            for (int j = 1; j < V; ++j) KX[f][j] = hx * (G[f][j - 1] + G[f][j]);
+            KX[f][V] = lane_down1<true>(KX[f][0]);
 #pragma unroll
-                    for (int j = 0; j < V; ++j) {
-                        un[j] = B.uv[q][j] + alpha * B.pv[q][j];
-                        rn[j] = B.rv[q][j] - alpha * B.wv[q][j];
-                        if (cl.x0 + j < g.nx) acc[0] += (double)rn[j] * (double)rn[j];
-                    }
-                    vstore_n<T, V>(u + i, un, g.nx - cl.x0);
-                    vstore_n<T, V>(r + i, rn, g.nx - cl.x0);
+            for (int j = 0; j < V; ++j) {
+                KY[a][j] = hy * (G[f][j] + B.g[j]);
+                G[e][j] = B.g[j];
+                R[e][j] = B.r[j];
+                P[a][j] = __builtin_fma(bd, B.p[j], B.r[j]);
+            }
+            if (act && L >= y0 && L < y1) {
+                vstore<double, V, NT>(pout + i, P[a]);
+                if constexpr (XUPD) {
+                    double un[V];
+#pragma unroll
+                    for (int j = 0; j < V; ++j)
+                        un[j] = __builtin_fma(alpha, P[a][j], __builtin_fma(alpha_prev, B.p[j], B.u[j]));
+                    vstore<double, V, NT>(u + i, un);
                 }
             }
+            if (L < y0) return true;
+            // q = A p(t) and r(t) on row L-1
+            double q[V];
+            apply(q, P[b], P[c], P[a], KX[f], KY[b], KY[a]);
+#pragma unroll
+            for (int j = 0; j < V; ++j) N[b][j] = __builtin_fma(-alpha, q[j], R[f][j]);
+            if (act && L - 1 >= y0 && L - 1 < y1) {
+                vstore<double, V, NT>(rout + i - g.pitch, N[b]);
+#pragma unroll
+                for (int j = 0; j < V; ++j) {
+                    acc[2] = __builtin_fma(N[b][j], q[j], acc[2]);
+                    acc[3] = __builtin_fma(P[b][j], q[j], acc[3]);
+                }
+            }
+            if (L < y0 + 2) return true;
+            // A r(t) on row L-2
+            double ar[V];
+            apply(ar, N[c], N[a], N[b], KX[e], KY[c], KY[b]);
+            if (act) {
+#pragma unroll
+                for (int j = 0; j < V; ++j) {
+                    acc[0] = __builtin_fma(N[c][j], N[c][j], acc[0]);
+                    acc[1] = __builtin_fma(N[c][j], ar[j], acc[1]);
+                }
+            }
+            return true;
         };
-        row_batches<PIPE, RB, Batch>(cl.y0, cl.y1, load_batch, compute_batch);
+        for (int L = y0 - 2; L <= y1 + 1; L += 6) {
+            if (!step(std::integral_constant<int, 0>{}, L)) break;
+            if (!step(std::integral_constant<int, 1>{}, L + 1)) break;
+            if (!step(std::integral_constant<int, 2>{}, L + 2)) break;
+            if (!step(std::integral_constant<int, 3>{}, L + 3)) break;
+            if (!step(std::integral_constant<int, 4>{}, L + 4)) break;
+            if (!step(std::integral_constant<int, 5>{}, L + 5)) break;
+        }
     }
-    write_partials<1, TBV>(acc, prcur, g.nbmax);
+    write_partials<4, TBV>(acc, sout, g.nbmax);
+}
+
+// The four sums k_cgs needs at its first iteration and after a new true
+// residual, for r and the kept direction p, with its operator.  One thread per
+// cell of a column band; runs once per start or new residual.
+__global__ __launch_bounds__(TB) void k_cgs_dots(Geo g, const double *__restrict__ r, const double *__restrict__ p,
+                                                 const double *__restrict__ gc, double hx, double hy,
+                                                 double *__restrict__ part)
+{
+    const Col c = column(g);
+    double acc[4] = {0.0, 0.0, 0.0, 0.0};
+    if (c.active) {
+        for (int y = c.y0; y < c.y1; ++y) {
+            const long i = at(g, c.x, y);
+            const double gm = gc[i];
+            const double kxl = hx * (gc[i - 1] + gm), kxr = hx * (gm + gc[i + 1]);
+            const double kyd = hy * (gc[i - g.pitch] + gm), kyu = hy * (gm + gc[i + g.pitch]);
+            auto apply = [&](const double *__restrict__ v) {
+                const double vc = v[i];
+                double s = kxl * (vc - v[i - 1]);
+                s = __builtin_fma(kxr, vc - v[i + 1], s);
+                s = __builtin_fma(kyd, vc - v[i - g.pitch], s);
+                s = __builtin_fma(kyu, vc - v[i + g.pitch], s);
+                return vc + s;
+            };
+            const double rc = r[i], ar = apply(r), ap = apply(p);
+            acc[0] += rc * rc;
+            acc[1] += rc * ar;
+            acc[2] += rc * ap;
+            acc[3] += p[i] * ap;
+        }
+    }
+    write_partials<4>(acc, part, g.nbmax);
+}
+
+// What the sweeps leave open when a CG stops after iteration T.  u: for odd T
+// the update alpha(T) p(T) (the sweeps add two iterations' at even t).  fin:
+// CG.p! of iteration T, p = beta p + r with beta = rr(T) / rr(T-1) (CG.jl:39,
+// 101-104), recorded like the sweeps record it.
+__global__ __launch_bounds__(TB) void k_cgs_end(Geo g, int T, double *__restrict__ u, double *__restrict__ p,
+                                                const double *__restrict__ r, int fin, Ctrl *__restrict__ ctrl,
+                                                double *__restrict__ hist_b)
+{
+    const Col c = column(g);
+    const double al = ctrl->alphas[T & 1];
+    const double beta = ctrl->rrs[T & 1] / ctrl->rrs[(T - 1) & 1];
+    if (fin && block_id() == 0 && threadIdx.x == 0) {
+        ctrl->beta = beta;
+        hist_b[T - 1] = beta;
+    }
+    if (!c.active) return;
+    for (int yb = c.y0; yb < c.y1; yb += R) {
+        double uv[R], pv[R], rv[R];
+        load_rows(pv, g, c, yb, p);
+        if (u) load_rows(uv, g, c, yb, u);
+        if (fin) load_rows(rv, g, c, yb, r);
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+            if (yb + q < c.y1) {
+                const long i = at(g, c.x, yb + q);
+                if (u) u[i] = uv[q] + al * pv[q];
+                if (fin) p[i] = beta * pv[q] + rv[q];
+            }
+        }
+    }
 }
 
 // Cell coefficients.  A coefficient is held in a 32-bit register as loaded
@@ -2700,7 +2798,7 @@ __global__ __launch_bounds__(TB) void k_ppcg_ur_sd(Geo g, int t, double *__restr
 // ------------------------------- vectorised FP64 Chebyshev / PPCG / Jacobi
 //
 // The three stencil-update kernels of the other FP64 solvers on 16-byte
-// vectors (2 doubles per lane), in the row-batch scheme of k_cg_pwv: a lane
+// vectors (2 doubles per lane), in the row-batch scheme of k_cgg: a lane
 // walks its column pair up a band keeping the rows below / at the current
 // row in registers, takes the columns left / right of its pair from the
 // adjacent lanes (lanes 0 and 63 load them with the row loads), and the next
@@ -3353,8 +3451,7 @@ static inline double *part_w(tl_ctx *c) { return c->partials; }
 static inline double *part_r(tl_ctx *c, int t) { return c->partials + (size_t)(1 + (t & 1)) * stride(c); }
 static inline double *part_m(tl_ctx *c) { return c->partials + (size_t)3 * stride(c); }
 static inline unsigned &nbr(tl_ctx *c, int t) { return c->nb_r[t & 1]; }
-// p of iteration t >= 1 of the fused CG lives in buffer (t-1) & 1
-static inline double *p64(tl_ctx *c, int t) { return ((t - 1) & 1) ? c->p_alt : c->f[TL_F_P]; }
+// p of iteration t >= 1 of the two-kernel FP32 CG lives in buffer (t-1) & 1
 static inline float *p32(tl_ctx *c, int t) { return ((t - 1) & 1) ? c->p32b : c->p32; }
 
 // kernel argument for iteration t: t itself, or, in a launch captured into a
@@ -3443,7 +3540,10 @@ hipError_t launch_init_coef(tl_ctx *c, double rx, double ry, int coefficient, in
 {
     k_init_coef<<<fgrid(c->g), TB, 0, c->stream>>>(c->g, c->f[TL_F_DENSITY], c->f[TL_F_ENERGY], c->f[TL_F_U],
                                                    c->f[TL_F_P], c->f[TL_F_R], c->f[TL_F_U0], c->f[TL_F_KX],
-                                                   c->f[TL_F_KY], rx, ry, coefficient == 2 ? 1 : 0, what);
+                                                   c->f[TL_F_KY], c->p_alt, c->r_alt1, c->g64, rx, ry,
+                                                   coefficient == 2 ? 1 : 0, what);
+    c->hx64 = 0.5 * rx;
+    c->hy64 = 0.5 * ry;
     return hipGetLastError();
 }
 
@@ -3477,12 +3577,10 @@ hipError_t launch_cg_w64(tl_ctx *c, int t)
 
 hipError_t launch_cg_ur64(tl_ctx *c, int t)
 {
-    const bool prof = prof_start(c, TL_K_CG_UR64);
     k_cg_ur<double><<<sgrid(c->g), TB, 0, c->stream>>>(c->g, t, c->f[TL_F_U], c->f[TL_F_P], c->f[TL_F_R],
                                                         c->f[TL_F_W], c->ctrl, part_w(c), c->nb_w, part_r(c, t - 1),
                                                         nbr(c, t - 1), part_r(c, t), c->hist_a);
     nbr(c, t) = nbh(c);
-    if (prof) prof_stop(c);
     return hipGetLastError();
 }
 
@@ -3496,37 +3594,59 @@ hipError_t launch_cg_p64(tl_ctx *c, int t)
     return hipGetLastError();
 }
 
-// fused CG, FP64: PW(t) then UR(t)
-hipError_t launch_cg_pw64(tl_ctx *c, int t, int tref)
+// FP64 CG sweeps: r(t) and p(t) in buffer t & 1, the four per-block sums for
+// iteration t+1 in set t & 1
+static inline double *cgs_r(tl_ctx *c, int t) { return (t & 1) ? c->r_alt1 : c->f[TL_F_R]; }
+static inline double *cgs_p(tl_ctx *c, int t) { return (t & 1) ? c->p_alt : c->f[TL_F_P]; }
+static inline double *cgs_u(tl_ctx *c) { return c->cg_u ? c->cg_u : c->f[TL_F_U]; }
+static inline double *part_f(tl_ctx *c, int t) { return c->part_f + (size_t)4 * (t & 1) * stride(c); }
+
+hipError_t launch_cgs64(tl_ctx *c, int t, int tref)
 {
-    const bool prof = prof_start(c, TL_K_CG_W64);
-    k_cg_pwv<double, 2, TL_RV_PW64, TL_PIPE_PW64 != 0><<<nb2(c), TBV, 0, c->stream>>>(
-        c->g, c->g.ty2, targ(t, tref), t >= 2 ? p64(c, t - 1) : nullptr, p64(c, t), c->f[TL_F_R], c->f[TL_F_KX], c->f[TL_F_KY],
-        c->f[TL_F_W], c->ctrl, part_w(c), t >= 2 ? part_r(c, t - 1) : nullptr, t >= 2 ? nbr(c, t - 1) : 0,
-        c->hist_b);
-    c->nb_w = nb2(c);
+    const bool even = (t & 1) == 0;
+    const bool prof = prof_start(c, even ? TL_K_CG_UR64 : TL_K_CG_W64);
+    // r, r', p, p', g and u
+    const bool nt = (size_t)6 * c->g.elems * sizeof(double) > TL_CACHE_BYTES;
+    auto kern = even ? (nt ? k_cgs<true, true> : k_cgs<true, false>) : (nt ? k_cgs<false, true> : k_cgs<false, false>);
+    kern<<<c->g.s64.blocks, TBV, 0, c->stream>>>(c->g, targ(t, tref), cgs_r(c, t - 1), cgs_r(c, t), cgs_p(c, t - 1),
+                                                cgs_p(c, t), cgs_u(c), c->g64, c->hx64, c->hy64, c->ctrl,
+                                                part_f(c, t - 1), c->nb_f[(t - 1) & 1], part_f(c, t), c->hist_a,
+                                                c->hist_b);
+    c->nb_f[t & 1] = (unsigned)c->g.s64.blocks;
     if (prof) prof_stop(c);
     return hipGetLastError();
 }
 
-hipError_t launch_cg_urv64(tl_ctx *c, int t, int tref)
+// the four sums of r(T) and p(T) for iteration T+1 (after a start or a new
+// true residual)
+hipError_t launch_cgs_dots(tl_ctx *c, int T)
 {
-    const bool prof = prof_start(c, TL_K_CG_UR64);
-    k_cg_urv<double, 2, TL_RV_UR64, TL_PIPE_UR64 != 0><<<nb2(c), TBV, 0, c->stream>>>(
-        c->g, c->g.ty2, targ(t, tref), c->cg_u ? c->cg_u : c->f[TL_F_U], p64(c, t), c->f[TL_F_R], c->f[TL_F_W], c->ctrl,
-        part_w(c), c->nb_w,
-        part_r(c, t), c->hist_a);
-    nbr(c, t) = nb2(c);
-    if (prof) prof_stop(c);
+    k_cgs_dots<<<sgrid(c->g), TB, 0, c->stream>>>(c->g, cgs_r(c, T), cgs_p(c, T), c->g64, c->hx64, c->hy64,
+                                                  part_f(c, T));
+    c->nb_f[T & 1] = nbh(c);
     return hipGetLastError();
 }
 
-// the CG.p! of the last iteration T of a fused FP64 CG solve (p_{T+1} in the
-// buffer of p_T, as the unfused solver leaves it); returns that buffer
-hipError_t launch_cg_pfinal64(tl_ctx *c, int T)
+// the update of an odd last iteration T that the sweeps have not applied yet
+hipError_t launch_cgs_pending(tl_ctx *c, int T)
 {
-    k_cg_p<double><<<sgrid(c->g), TB, 0, c->stream>>>(c->g, T, p64(c, T), c->f[TL_F_R], c->ctrl, part_r(c, T - 1),
-                                                       nbr(c, T - 1), part_r(c, T), nbr(c, T), c->hist_b);
+    if (!(T & 1)) return hipSuccess;
+    k_cgs_end<<<sgrid(c->g), TB, 0, c->stream>>>(c->g, T, cgs_u(c), cgs_p(c, T), cgs_r(c, T), 0, c->ctrl, c->hist_b);
+    return hipGetLastError();
+}
+
+// after the last iteration T >= 1 (its pending update applied): w = A p(T) and
+// the CG.p! of iteration T, so that p, r and w end as the reference leaves
+// them, in the context's fields
+hipError_t launch_cgs_final(tl_ctx *c, int T)
+{
+    if (T & 1) {
+        std::swap(c->f[TL_F_P], c->p_alt);
+        std::swap(c->f[TL_F_R], c->r_alt1);
+    }
+    hipError_t e = launch_apply(c, c->f[TL_F_P], c->f[TL_F_W]);
+    if (e != hipSuccess) return e;
+    k_cgs_end<<<sgrid(c->g), TB, 0, c->stream>>>(c->g, T, nullptr, c->f[TL_F_P], c->f[TL_F_R], 1, c->ctrl, c->hist_b);
     return hipGetLastError();
 }
 
@@ -3574,7 +3694,7 @@ hipError_t launch_graph_seed(tl_ctx *c, int t0)
 hipError_t launch_cg64_true_residual(tl_ctx *c, int T)
 {
     k_residual<<<sgrid(c->g), TB, 0, c->stream>>>(c->g, 0, c->f[TL_F_U0], c->f[TL_F_U], c->f[TL_F_KX],
-                                                  c->f[TL_F_KY], c->f[TL_F_R], nullptr, nullptr, c->ctrl,
+                                                  c->f[TL_F_KY], cgs_r(c, T), nullptr, nullptr, c->ctrl,
                                                   part_r(c, T));
     nbr(c, T) = nbh(c);
     hipError_t e = hipGetLastError();
@@ -3817,7 +3937,6 @@ hipError_t launch_ir_accumulate(tl_ctx *c, int T, const float *pT)
 // per-block sums for iteration t+1 in set t & 1
 float *cgf_r(tl_ctx *c, int t) { return (t & 1) ? c->r32b : c->r32; }
 float *cgf_p(tl_ctx *c, int t) { return (t & 1) ? c->p32b : c->p32; }
-static inline double *part_f(tl_ctx *c, int t) { return c->part_f + (size_t)4 * (t & 1) * stride(c); }
 static inline unsigned nbf(const tl_ctx *c) { return (unsigned)(c->g.gx4 * c->g.gyf); }
 
 hipError_t launch_cgf(tl_ctx *c, int t, int tref)

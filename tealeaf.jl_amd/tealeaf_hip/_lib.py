@@ -45,7 +45,7 @@ TL_FP32_KERNELS_AUTO, TL_FP32_KERNELS_TWO, TL_FP32_KERNELS_FUSED, TL_FP32_KERNEL
 TL_WARM_POLICY_BACKOFF, TL_WARM_POLICY_EVERY = 0, 1
 TL_PPCG_PAIRS_AUTO, TL_PPCG_PAIRS_OFF = 0, 1
 TL_CHEBY_PAIRS_AUTO, TL_CHEBY_PAIRS_OFF = 0, 1
-KERNEL_NAMES = {0: "k_cg_pwv<double, 2, 4, true>", 1: "k_cg_urv<double, 2, 4, false>", 2: "k_cg_p<double>",
+KERNEL_NAMES = {0: "k_cgs<false, true>", 1: "k_cgs<true, true>", 2: "k_cg_p<double>",
                 3: "k_cgg<4, false, 2, true, 1>", 4: "k_cgg<4, true, 4, true, 1>",
                 5: "(fused into k_cgg<4, false, 2, true, 1>)",
                 6: "k_vs64<0, 4, true>", 7: "k_vs64<1, 4, true>", 8: "k_vs64<2, 4, true>", 9: "k_residual",
