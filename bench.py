@@ -367,6 +367,7 @@ TABLE_BYTES = dict(KERNEL_BYTES)
 TABLE_BYTES.update({_lib.TL_K_CHEBY64: 56, _lib.TL_K_PPCG64: 64, _lib.TL_K_JACOBI64: 40, _lib.TL_K_RESID64: 40,
                     _lib.TL_K_PPCG2_64: 64,   # two PPCG inner steps: 64 B/cell per launch
                     _lib.TL_K_CHEBY2_64: 56})  # two Chebyshev iterations: 56 B/cell per launch
+# (TL_K_JACOBI64: eight Jacobi iterations, 40 B/cell per launch)
 
 
 def kernel_table(n, seed, reps):

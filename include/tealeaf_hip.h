@@ -123,13 +123,13 @@ typedef struct {
 #define TL_WARM_POLICY_EVERY 1   /* every solve */
 
 /* tl_solve_params.ppcg_pairs: PPCG's inner Chebyshev steps (PPCG.jl:78-83)
- * two per sweep over the grid, or one.  Bit-identical results. */
-#define TL_PPCG_PAIRS_AUTO 0 /* two steps per sweep when ppcg_inner_steps >= 4 (an odd last step alone) */
+ * several per sweep over the grid, or one.  Bit-identical results. */
+#define TL_PPCG_PAIRS_AUTO 0 /* when ppcg_inner_steps >= 4: two in the last sweep, up to eight in the others */
 #define TL_PPCG_PAIRS_OFF 1  /* one step per sweep */
 
-/* tl_solve_params.cheby_pairs: Chebyshev iterations (Cheby.jl:93-107) two per
- * sweep over the grid, or one.  Bit-identical results. */
-#define TL_CHEBY_PAIRS_AUTO 0 /* two iterations per sweep where the first needs no residual norm */
+/* tl_solve_params.cheby_pairs: Chebyshev iterations (Cheby.jl:93-107) several
+ * per sweep over the grid, or one.  Bit-identical results. */
+#define TL_CHEBY_PAIRS_AUTO 0 /* up to eight iterations per sweep between those with a residual norm */
 #define TL_CHEBY_PAIRS_OFF 1  /* one iteration per sweep */
 
 /* tl_solve_params.fp32_kernels: how a TL_FP32_IR iteration is split into kernels.
@@ -309,7 +309,7 @@ int tl_get_cg_history(tl_ctx *ctx, double *alpha, double *beta, int n);
 #define TL_K_CG_P32 5  /* unused: folded into TL_K_CG_W32 */
 #define TL_K_CHEBY64 6 /* Chebyshev iteration (Cheby.mainstep!) */
 #define TL_K_PPCG64 7  /* PPCG inner Chebyshev step */
-#define TL_K_JACOBI64 8 /* Jacobi sweep (the sweeps that do not also form the residual) */
+#define TL_K_JACOBI64 8 /* up to eight Jacobi iterations in one sweep */
 #define TL_K_RESID64 9 /* residual! r = u0 - A u (also the FP64 refresh of TL_FP32_IR) */
 #define TL_K_CGF32 10  /* FP32 inner CG iteration as one kernel (TL_FP32_KERNELS_FUSED) */
 #define TL_K_PPCG2_64 11 /* two PPCG inner steps in one sweep (TL_PPCG_PAIRS_AUTO) */

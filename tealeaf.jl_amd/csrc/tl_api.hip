@@ -160,7 +160,7 @@ extern "C" void tl_destroy(tl_ctx *c)
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     unet_destroy(c);
     void *bufs[] = {c->u_alt, c->sd_alt, c->r_alt1, c->r_alt2, c->p_alt, c->p32b, c->guess, c->gcell, c->gc_range, c->p32, c->r32, c->x32,
-                    c->r32b, c->part_f, c->partials, c->ctrl, c->hist_a, c->hist_b, c->states_d};
+                    c->r32b, c->part_f, c->part_j, c->g64, c->partials, c->ctrl, c->hist_a, c->hist_b, c->states_d};
     for (int i = 0; i < TL_NFIELDS; ++i)
         if (c->f[i]) (void)hipFree(c->f[i]);
     for (void *b : bufs)
@@ -898,8 +898,8 @@ static int solve_cheby(tl_ctx *c, const tl_solve_params *p, double rx, double ry
     }
     HIPCHK(c, launch_set_mode(c, MODE_JACOBI, maxiters));
     double *ucur = c->f[TL_F_U], *unext = c->u_alt;
-    double *pcur = c->f[TL_F_P], *pnext = c->p_alt;  // p moves only in two-iteration launches
-    const bool pairs = p->cheby_pairs == TL_CHEBY_PAIRS_AUTO;
+    double *pcur = c->f[TL_F_P], *pnext = c->p_alt;  // p moves only in launches of several iterations
+    const bool pairs = p->cheby_pairs == TL_CHEBY_PAIRS_AUTO;  // several iterations per launch
     // u (and p) move between two buffers and either may end up as the
     // field: the cells no kernel writes (the outer halo) start equal in both
     HIPCHK(c, launch_copy_full(c, ucur, unext));
@@ -914,51 +914,64 @@ static int solve_cheby(tl_ctx *c, const tl_solve_params *p, double rx, double ry
     RETIF(read_ctrl(c, &k));
     const int estiter = tl_cheby_calciter(eigmin, eigmax, k.err, k.bb);
     st->est_iters = estiter;
-    if (k.stop_iter == INT_MAX) {
-        // main loop (Cheby.jl:46-53); every launch swaps the u buffers.  Two
-        // iterations per launch (TL_CHEBY_PAIRS_AUTO) unless the first needs
-        // the residual norm, so that a stop can only follow a launch's last
-        // iteration
-        while (tt < maxiters) {
-            int nb = 0;
-            int norm = 0;
-            while (tt < maxiters && nb < 64) {
-                const bool norm1 = (chebyiters + 1 >= estiter) && ((tt + 2) % 10 == 0);
-                if (pairs && !norm1 && tt + 2 <= maxiters) {
-                    norm = (chebyiters + 2 >= estiter) && ((tt + 3) % 10 == 0);
-                    HIPCHK(c, launch_cheby_iter2(c, ca[chebyiters + 2], cb[chebyiters + 2], ca[chebyiters + 3],
-                                                 cb[chebyiters + 3], ucur, unext, pcur, pnext, norm, tt + 1));
-                    std::swap(pcur, pnext);
-                    tt += 2;
-                    chebyiters += 2;
-                    nb += 2;
+    // main loop (Cheby.jl:46-53), enqueued up to `ahead` residual norms ahead of
+    // the host's check.  With TL_CHEBY_PAIRS_AUTO the iterations between two
+    // norms take up to STEPS_HALO per launch, and the last two before a norm
+    // share its launch (whose sum is the single iteration's bit for bit).
+    // Every launch swaps the u buffers, those of several iterations also p's.
+    struct Launch {
+        int tt, chebyiters;  // after it
+        double *u, *p;
+    };
+    std::vector<Launch> made;
+    int ahead = 1;
+    while (k.stop_iter == INT_MAX && tt < maxiters) {
+        made.clear();
+        for (int norms = 0; norms < ahead && tt < maxiters;) {
+            // iterations up to the next one with a norm (Cheby.jl:47-50)
+            int d = 1;
+            while (tt + d < maxiters && !(chebyiters + d >= estiter && (tt + d + 1) % 10 == 0)) ++d;
+            const int norm = chebyiters + d >= estiter && (tt + d + 1) % 10 == 0;
+            const int n = !pairs || d == 1 ? 1 : d == 2 ? 2 : std::min(STEPS_HALO, norm ? d - 2 : d);
+            const int last = norm && n == d;
+            const double *a = &ca[chebyiters + 2], *b = &cb[chebyiters + 2];
+            if (n == 1) {
+                HIPCHK(c, launch_cheby_iter(c, a[0], b[0], ucur, unext, pcur, last, tt + 1));
+            } else {
+                if (n == 2) {
+                    HIPCHK(c, launch_cheby_iter2(c, a[0], b[0], a[1], b[1], ucur, unext, pcur, pnext, last, tt + 1));
                 } else {
-                    ++tt;
-                    ++chebyiters;
-                    norm = (chebyiters >= estiter) && ((tt + 1) % 10 == 0);
-                    HIPCHK(c, launch_cheby_iter(c, ca[chebyiters + 1], cb[chebyiters + 1], ucur, unext, pcur, norm,
-                                                tt));
-                    ++nb;
+                    StepCoef co;
+                    for (int i = 0; i < n; ++i) {
+                        co.a[i] = a[i];
+                        co.b[i] = b[i];
+                    }
+                    HIPCHK(c, launch_cheby_steps(c, n, co, ucur, unext, pcur, pnext, tt + 1));
                 }
-                std::swap(ucur, unext);
-                if (norm) break;
+                std::swap(pcur, pnext);
             }
-            if (norm) {
-                RETIF(read_ctrl(c, &k));
-                if (k.stop_iter != INT_MAX) break;
-            }
+            std::swap(ucur, unext);
+            tt += n;
+            chebyiters += n;
+            norms += last;
+            made.push_back({tt, chebyiters, ucur, pcur});
+            if (made.size() >= 512) break;
         }
         RETIF(read_ctrl(c, &k));
-        if (pairs && k.stop_iter != INT_MAX && k.stop_iter != tt) {
-            // stops follow norm iterations, which end a launch
-            c->err = "Chebyshev: stop inside a two-iteration launch";
+        if (ahead < 8) ahead *= 2;
+    }
+    if (k.stop_iter != INT_MAX && k.stop_iter != tt) {
+        // launches past the stop exited at once: the state of the one that ended at it
+        size_t i = 0;
+        while (i < made.size() && made[i].tt != k.stop_iter) ++i;
+        if (i == made.size()) {
+            c->err = "Chebyshev: stop inside a launch of several iterations";
             return TL_E_STATE;
         }
-        if (k.stop_iter != INT_MAX && ((tt - k.stop_iter) & 1)) std::swap(ucur, unext);
-        if (k.stop_iter != INT_MAX) {
-            chebyiters -= tt - k.stop_iter;
-            tt = k.stop_iter;
-        }
+        tt = made[i].tt;
+        chebyiters = made[i].chebyiters;
+        ucur = made[i].u;
+        pcur = made[i].p;
     }
     if (ucur != c->f[TL_F_U]) std::swap(c->f[TL_F_U], c->u_alt);
     if (pcur != c->f[TL_F_P]) std::swap(c->f[TL_F_P], c->p_alt);
@@ -991,14 +1004,22 @@ static int solve_ppcg(tl_ctx *c, const tl_solve_params *p, double rx, double ry,
     HIPCHK(c, launch_residual(c));
     HIPCHK(c, launch_set_mode(c, MODE_PPCG, p->max_iters));
     double *sd0 = c->f[TL_F_SD], *sd1 = c->sd_alt;
-    // two inner steps per sweep (r through two spare buffers, back in r's
-    // own at the end of every outer iteration), an odd last step alone
+    // several inner steps per sweep, two in the last one, which forms rr (r
+    // through two spare buffers, back in r's own at the end of every outer
+    // iteration)
     const bool pairs = p->ppcg_pairs == TL_PPCG_PAIRS_AUTO && inner >= 4;
     if (pairs) {
         if (!c->r_alt1) RETIF(alloc_d(c, &c->r_alt1, c->g.elems));
         if (!c->r_alt2) RETIF(alloc_d(c, &c->r_alt2, c->g.elems));
     }
-    const int sd_moves = pairs ? inner / 2 + (inner & 1) : inner;  // sweeps per outer iteration
+    std::vector<int> sweeps;  // inner steps of each
+    if (pairs) {
+        int left = inner - 2;
+        for (; left > 0; left -= sweeps.back()) sweeps.push_back(std::min(STEPS_HALO, left));
+        sweeps.push_back(2);
+    } else {
+        sweeps.assign((size_t)inner, 1);
+    }
     int t = cgiters;
     RETIF(run_until_stop(c, 16, (long)p->max_iters + 16,
                          [&]() -> hipError_t {
@@ -1007,27 +1028,34 @@ static int solve_ppcg(tl_ctx *c, const tl_solve_params *p, double rx, double ry,
                              if (e == hipSuccess) e = launch_ppcg_ur_sd(c, theta, t);
                              double *a = sd0, *b = sd1;
                              int pp = 0;
-                             if (pairs) {
-                                 const int np = inner / 2;
-                                 const double *rs = c->f[TL_F_R];
-                                 for (int q = 0; q < np && e == hipSuccess; ++q, pp += 2) {
-                                     double *rd = q == np - 1 ? c->f[TL_F_R] : (q & 1) ? c->r_alt2 : c->r_alt1;
-                                     e = launch_ppcg_inner2(c, ca[pp], cb[pp], ca[pp + 1], cb[pp + 1], a, b, rs, rd,
-                                                            pp + 2 == inner, t);
-                                     std::swap(a, b);
-                                     rs = rd;
+                             const double *rs = c->f[TL_F_R];
+                             for (size_t q = 0; q < sweeps.size() && e == hipSuccess; ++q) {
+                                 const int n = sweeps[q];
+                                 const bool end = q + 1 == sweeps.size();
+                                 double *rd = !pairs || end ? c->f[TL_F_R] : (q & 1) ? c->r_alt2 : c->r_alt1;
+                                 if (!pairs) {
+                                     e = launch_ppcg_inner(c, ca[pp], cb[pp], a, b, end, t);
+                                 } else if (n == 2) {
+                                     e = launch_ppcg_inner2(c, ca[pp], cb[pp], ca[pp + 1], cb[pp + 1], a, b, rs, rd, end,
+                                                            t);
+                                 } else {
+                                     StepCoef co;
+                                     for (int i = 0; i < n; ++i) {
+                                         co.a[i] = ca[pp + i];
+                                         co.b[i] = cb[pp + i];
+                                     }
+                                     e = launch_ppcg_steps(c, n, co, a, b, rs, rd, t);
                                  }
-                             }
-                             for (; pp < inner && e == hipSuccess; ++pp) {
-                                 e = launch_ppcg_inner(c, ca[pp], cb[pp], a, b, pp == inner - 1, t);
                                  std::swap(a, b);
+                                 rs = rd;
+                                 pp += n;
                              }
                              if (inner == 0 && e == hipSuccess) e = launch_sumsq_rr(c, c->f[TL_F_R], t);
                              if (e == hipSuccess) e = launch_cg_p64(c, t);
                              return e;
                          },
                          &k));
-    if (sd_moves & 1) std::swap(c->f[TL_F_SD], c->sd_alt);
+    if (sweeps.size() & 1) std::swap(c->f[TL_F_SD], c->sd_alt);
     st->cheby_iters = k.stop_iter - cgiters;
     st->iterations = k.stop_iter;
     fill_stats(k, st);
@@ -1038,26 +1066,61 @@ static int solve_ppcg(tl_ctx *c, const tl_solve_params *p, double rx, double ry,
 // Jacobi.driver!, Jacobi.jl:7-31 (intended form)
 static int solve_jacobi(tl_ctx *c, const tl_solve_params *p, double rx, double ry, tl_solve_stats *st)
 {
+    if (!c->part_j) RETIF(alloc_d(c, &c->part_j, (size_t)2 * STEPS_HALO * c->g.nbmax));
+    if (!c->r_alt1) RETIF(alloc_d(c, &c->r_alt1, c->g.elems));
     HIPCHK(c, launch_init_coef(c, rx, ry, p->coefficient, INIT_JACOBI));
     HIPCHK(c, launch_init_ctrl(c, MODE_JACOBI, p->max_iters, p->eps, p->rel_tol, 0.0, 0, 0, p->epslim));
+    // Several iterations per launch; the iterations 50, 100, ... end a launch,
+    // which also forms the residual that joins their error (Jacobi.jl:21-24).
+    // Its r goes to two buffers in turn: a launch may have run past the stop.
+    HIPCHK(c, launch_copy_full(c, c->f[TL_F_R], c->r_alt1));
     double *ucur = c->f[TL_F_U], *unext = c->u_alt;
-    int tt = 0;
+    struct Launch {
+        int t0, n;  // iterations t0 .. t0+n-1
+        double *in, *out;
+    };
+    std::vector<Launch> made;  // the last ones enqueued
+    int tt = 0, nprev = 0, residp = 0;
     Ctrl k;
-    RETIF(run_until_stop(c, 50, (long)p->max_iters + 16,
+    RETIF(run_until_stop(c, 16, (long)p->max_iters + 16,
                          [&]() -> hipError_t {
-                             if (tt >= p->max_iters) return hipSuccess;
-                             ++tt;
-                             const int every = (tt % 50) == 0;
-                             hipError_t e = launch_jacobi(c, ucur, unext, tt, every);
-                             if (every && e == hipSuccess) e = launch_jacobi_residual(c, unext, tt);
+                             if (tt >= p->max_iters) {  // the last launch's stop test
+                                 const hipError_t e = nprev ? launch_jacobi_end(c, nprev, residp, tt + 1) : hipSuccess;
+                                 nprev = 0;
+                                 return e;
+                             }
+                             const int to50 = 50 - tt % 50;
+                             int n = std::min(to50 >= STEPS_HALO ? STEPS_HALO : to50, p->max_iters - tt);
+                             // leave the residual's launch at most STEPS_HALO - 1 steps, and one at least
+                             if (n == to50 && n == STEPS_HALO) n = STEPS_HALO / 2;
+                             const int resid = (tt + n) % 50 == 0;
+                             const hipError_t e = launch_jacobi_steps(
+                                 c, n, ucur, unext, ((tt + n) / 50) & 1 ? c->r_alt1 : c->f[TL_F_R], resid, nprev,
+                                 residp, tt + 1);
+                             if (made.size() >= 256) made.erase(made.begin(), made.begin() + 128);
+                             made.push_back({tt + 1, n, ucur, unext});
                              std::swap(ucur, unext);
+                             tt += n;
+                             nprev = n;
+                             residp = resid;
                              return e;
                          },
                          &k));
-    // tt launches were made; the last one that ran was k.stop_iter
-    if ((tt - k.stop_iter) & 1) std::swap(ucur, unext);
+    const int T = k.stop_iter;
+    // the launch that holds iteration T (the ones after it exited at once): its
+    // result if T is its last step, else its first steps again
+    for (size_t i = made.size(); i-- > 0;) {
+        const Launch &m = made[i];
+        if (T < m.t0 || T >= m.t0 + m.n) continue;
+        ucur = m.out;
+        unext = m.in;
+        if (T != m.t0 + m.n - 1)
+            HIPCHK(c, launch_jacobi_steps(c, T - m.t0 + 1, m.in, m.out, nullptr, 0, 0, 0, m.t0));
+        break;
+    }
     if (ucur != c->f[TL_F_U]) std::swap(c->f[TL_F_U], c->u_alt);
-    st->iterations = k.stop_iter;
+    if ((T / 50) & 1) std::swap(c->f[TL_F_R], c->r_alt1);
+    st->iterations = T;
     fill_stats(k, st);
     HIPCHK(c, launch_halo(c, TL_X_U, 1, nullptr, 0));
     return status_of(c, k);
@@ -1246,6 +1309,7 @@ extern "C" int tl_kernel_repeat(tl_ctx *c, int kernel_id, int reps)
         // one FP64 solver kernel, `reps` launches on the CG-initialised fields
         // (u, u0, p, r, kx, ky) with fixed coefficients; never stopped
         HIPCHK(c, launch_set_mode(c, MODE_JACOBI, 1 << 30));
+        if (!c->part_j) RETIF(alloc_d(c, &c->part_j, (size_t)2 * STEPS_HALO * c->g.nbmax));
         double *a = c->f[TL_F_U], *b = c->u_alt, *s0 = c->f[TL_F_SD], *s1 = c->sd_alt;
         double *r0 = c->f[TL_F_R], *r1 = c->r_alt1, *q0 = c->f[TL_F_P], *q1 = c->p_alt;
         for (int i = 0; i < reps; ++i) {
@@ -1266,7 +1330,10 @@ extern "C" int tl_kernel_repeat(tl_ctx *c, int kernel_id, int reps)
                 std::swap(s0, s1);
                 std::swap(r0, r1);
                 break;
-            case TL_K_JACOBI64: HIPCHK(c, launch_jacobi(c, a, b, t, 0)); std::swap(a, b); break;
+            case TL_K_JACOBI64:
+                HIPCHK(c, launch_jacobi_steps(c, STEPS_HALO, a, b, nullptr, 0, 0, 0, t));
+                std::swap(a, b);
+                break;
             default: HIPCHK(c, launch_residual(c)); break;
             }
         }

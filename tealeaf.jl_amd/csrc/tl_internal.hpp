@@ -59,11 +59,11 @@ constexpr int TBV = TL_TBV;
 #ifndef TL_VEC_BLOCKS64
 #define TL_VEC_BLOCKS64 8192
 #endif
-// rows per load batch of the vectorised FP64 Chebyshev / PPCG / Jacobi
+// rows per load batch of the vectorised FP64 Chebyshev / PPCG
 // kernels, and whether the next batch's loads are issued before the current
 // one is computed.  Measured at 8192^2 (A/B in one box): 4 rows pipelined
 // (236 VGPRs, 2 waves per SIMD) against 2 rows: Chebyshev 5.28 / 5.18 TB/s,
-// PPCG 5.18 / 5.11, Jacobi 5.39 / 5.11; 4 rows unpipelined, 3 rows, and
+// PPCG 5.18 / 5.11; 4 rows unpipelined, 3 rows, and
 // 12288 or 16384 blocks no better
 #ifndef TL_RV_VS64
 #define TL_RV_VS64 4
@@ -187,7 +187,7 @@ enum GcFmt : int { GC_BF16 = 0, GC_F16 = 1 };
 // Measured at 8192^2 (A/B in one box, loads and stores together against
 // neither): fused FP32 CG 4.68 / 4.78 -> 5.14 / 5.04 TB/s (odd / even t), FP32
 // PW 4.65 -> 5.37, FP32 UR 5.03 / 5.09 -> 6.08 / 5.98, FP64 PW 5.23 -> 5.33,
-// FP64 UR 5.17 -> 5.56, Chebyshev / PPCG / Jacobi steps +6-7%; loads alone
+// Chebyshev / PPCG steps +6-7%; loads alone
 // made the fused kernel 4% slower.  The two-step solver kernels have their
 // own switches: with both they ran 2-4% slower, with loads alone 6-8% slower,
 // with stores alone within +-2%.
@@ -210,6 +210,15 @@ enum GcFmt : int { GC_BF16 = 0, GC_F16 = 1 };
 struct Tiles {
     int strips, ty, bands, blocks;
 };
+// Multi-step sweeps (k_steps): a block holds a tile in registers, its outer
+// STEPS_HALO cells on every side shared with the neighbouring tiles; tiles are
+// dealt to the XCDs in runs of STEPS_CHUNK
+constexpr int STEPS_HALO = 8;
+constexpr int STEPS_CHUNK = 4;
+struct StepCoef {
+    double a[STEPS_HALO], b[STEPS_HALO];
+};
+
 // neighbouring tiles dealt to one XCD in a run (4 and 64: 1-2% slower)
 constexpr int TILE_CHUNK = 16;
 
@@ -308,6 +317,9 @@ struct tl_ctx {
     float *r32b = nullptr;
     double *part_f = nullptr;
     unsigned nb_f[2] = {0, 0};
+    // Jacobi: two sets of the per-block sums of a multi-step sweep, and the last written
+    double *part_j = nullptr;
+    int jset = 0;
     tl::Ctrl *ctrl = nullptr;        // device
     tl::Ctrl *ctrl_h = nullptr;      // pinned host mirror
     double *hist_a = nullptr, *hist_b = nullptr;  // device CG alpha/beta history
@@ -387,7 +399,6 @@ hipError_t launch_graph_base(tl_ctx *c, int k);
 hipError_t launch_graph_seed(tl_ctx *c, int t0);
 hipError_t launch_residual(tl_ctx *c);
 hipError_t launch_cg64_true_residual(tl_ctx *c, int T);
-hipError_t launch_jacobi_residual(tl_ctx *c, const double *u, int t);
 hipError_t launch_ir_residual(tl_ctx *c, int reset_p, int t_next, float *r_dst = nullptr);
 hipError_t launch_cgf(tl_ctx *c, int t, int tref = 0);
 hipError_t launch_cgf_dots(tl_ctx *c, int T);
@@ -410,7 +421,16 @@ hipError_t launch_ppcg_ur_sd(tl_ctx *c, double theta, int t);
 hipError_t launch_ppcg_inner(tl_ctx *c, double a, double b, const double *sd_in, double *sd_out, int last, int t);
 hipError_t launch_ppcg_inner2(tl_ctx *c, double a1, double b1, double a2, double b2, const double *sd_in,
                               double *sd_out, const double *r_in, double *r_out, int last, int t);
-hipError_t launch_jacobi(tl_ctx *c, const double *u_in, double *u_out, int t, int defer);
+// n (1 .. STEPS_HALO) solver steps in one sweep, iterations t .. t+n-1
+hipError_t launch_cheby_steps(tl_ctx *c, int n, const StepCoef &co, const double *u_in, double *u_out,
+                              const double *p_in, double *p_out, int t);
+hipError_t launch_ppcg_steps(tl_ctx *c, int n, const StepCoef &co, const double *sd_in, double *sd_out,
+                             const double *r_in, double *r_out, int t);
+// Jacobi: resid (n < STEPS_HALO): also r = u0 - A u after the last of them, into
+// r_out; nprev: steps of the previous launch (0: none), residp: its resid
+hipError_t launch_jacobi_steps(tl_ctx *c, int n, const double *u_in, double *u_out, double *r_out, int resid,
+                               int nprev, int residp, int t);
+hipError_t launch_jacobi_end(tl_ctx *c, int nprev, int residp, int t);
 hipError_t launch_ir_prepare(tl_ctx *c, double rx, double ry, int coefficient);
 hipError_t launch_ir_accumulate(tl_ctx *c, int T, const float *pT = nullptr);
 hipError_t launch_acc64(tl_ctx *c, double *u, double *d);

@@ -55,6 +55,18 @@ static Tiles make_tiles(int nx, int ny, int cols, int waves, int min_rows)
     return t;
 }
 
+// tiles of k_steps of w columns x h rows, and its blocks (a multiple of 8 runs)
+static inline int steps_tiles(int nx, int ny, int w, int h, int &gx)
+{
+    const int uw = w - 2 * STEPS_HALO, uh = h - 2 * STEPS_HALO;
+    gx = (nx + uw - 1) / uw;
+    return gx * ((ny + uh - 1) / uh);
+}
+static inline unsigned steps_blocks(int tiles)
+{
+    return (unsigned)((tiles + 8 * STEPS_CHUNK - 1) / (8 * STEPS_CHUNK) * 8 * STEPS_CHUNK);
+}
+
 Geo make_geo(int nx, int ny, int hd)
 {
     Geo g{};
@@ -120,6 +132,8 @@ Geo make_geo(int nx, int ny, int hd)
     g.nbmax = std::max(g.nbmax, g.gx4 * g.gyf);
     g.s64 = make_tiles(nx, ny, TL_S64_COLS, TL_S64_WAVES, TL_S64_ROWS);
     g.nbmax = std::max(g.nbmax, g.s64.blocks);
+    int gxs;
+    g.nbmax = std::max(g.nbmax, (int)steps_blocks(steps_tiles(nx, ny, 64, 32, gxs)));  // its smallest tiles
     return g;
 }
 
@@ -204,6 +218,98 @@ __device__ __forceinline__ void sum_partials(const double *__restrict__ part, un
 #pragma unroll
         for (int q = 1; q < NT / 64; ++q) s += sh[a][q];
         tot[a] = s;
+    }
+    __syncthreads();  // sh may be reused by the next call
+}
+
+// Several sums at once.  Summing N values over a wave one after the other is a
+// chain of 6 N dependent lane exchanges, and reading N arrays of partials one
+// after the other N memory latencies; at small grids the two made up most of a
+// CG iteration (512^2: 4 of 14 us).  Here the lanes halve the set of values
+// they carry while they exchange (N = 8: 10 exchanges instead of 48), and a
+// block's N sums lie side by side, so that one latency fetches them.
+
+// lane l gets the wave's sum of v[sum_index<N>(l)], N = 1, 2, 4 or 8
+template <int N>
+__device__ __forceinline__ int sum_index(int lane)
+{
+    return N == 1 ? 0 : N == 2 ? lane >> 5 : N == 4 ? lane >> 4 : lane >> 3;
+}
+
+template <int N, int O = 32>
+__device__ __forceinline__ double wave_sums(const double (&v)[N])
+{
+    if constexpr (N == 1) {
+        double s = v[0];
+#pragma unroll
+        for (int o = O; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+        return s;
+    } else {
+        const bool up = (threadIdx.x & O) != 0;
+        double h[N / 2];
+#pragma unroll
+        for (int i = 0; i < N / 2; ++i) {
+            const double send = up ? v[i] : v[i + N / 2], keep = up ? v[i + N / 2] : v[i];
+            h[i] = keep + __shfl_xor(send, O, 64);
+        }
+        return wave_sums<N / 2, O / 2>(h);
+    }
+}
+
+// the block's sums of v, side by side: part[block * N + a]
+template <int N, int NT = TB>
+__device__ __forceinline__ void write_block_sums(const double (&v)[N], double *__restrict__ part)
+{
+    __shared__ double sh[NT / 64][N];
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const double s = wave_sums<N>(v);
+    if ((lane & (64 / N - 1)) == 0) sh[wid][sum_index<N>(lane)] = s;
+    __syncthreads();
+    if (threadIdx.x < N) {
+        double t = sh[0][threadIdx.x];
+#pragma unroll
+        for (int q = 1; q < NT / 64; ++q) t += sh[q][threadIdx.x];
+        store_partial(&part[(size_t)block_id() * N + threadIdx.x], t);
+    }
+}
+
+// every thread of the block gets the fixed-order sums of nb blocks' partials
+template <int N, int NT = TB, bool COH = false>
+__device__ __forceinline__ void sum_block_sums(const double *__restrict__ part, unsigned nb, double (&tot)[N])
+{
+    __shared__ double sh[NT / 64][N];
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    double v[N];
+#pragma unroll
+    for (int a = 0; a < N; ++a) v[a] = 0.0;
+    for (unsigned q0 = threadIdx.x; q0 < nb; q0 += 2 * NT) {
+        double w[2][N];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const unsigned q = q0 + (unsigned)k * NT;
+            const double *p = part + (size_t)q * N;
+#pragma unroll
+            for (int a = 0; a < N; ++a) {
+                if constexpr (COH)
+                    w[k][a] = q < nb ? __hip_atomic_load(p + a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0.0;
+                else
+                    w[k][a] = q < nb ? p[a] : 0.0;
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+#pragma unroll
+            for (int a = 0; a < N; ++a) v[a] += w[k][a];
+    }
+    const double s = wave_sums<N>(v);
+    if ((lane & (64 / N - 1)) == 0) sh[wid][sum_index<N>(lane)] = s;
+    __syncthreads();
+#pragma unroll
+    for (int a = 0; a < N; ++a) {
+        double t = sh[0][a];
+#pragma unroll
+        for (int q = 1; q < NT / 64; ++q) t += sh[q][a];
+        tot[a] = t;
     }
     __syncthreads();  // sh may be reused by the next call
 }
@@ -427,12 +533,12 @@ __global__ __launch_bounds__(TB) void k_set_mode(Ctrl *c, int mode, int maxiters
 
 // Single-block finalizers: sum n partial arrays (each nb long, stride nb)
 // into ctrl->sums[slot ...] and act on them.
-enum FinKind : int { FK_SUMS = 0, FK_INIT = 1, FK_BB = 2, FK_CHEBY = 3, FK_JACOBI = 4, FK_IR = 5 };
+enum FinKind : int { FK_SUMS = 0, FK_INIT = 1, FK_BB = 2, FK_CHEBY = 3, FK_IR = 4 };
 
 __global__ __launch_bounds__(TB) void k_fin(Ctrl *__restrict__ c, const double *__restrict__ part, unsigned nb,
                                             unsigned stride, int n, int slot, int kind, int t)
 {
-    if ((kind == FK_CHEBY || kind == FK_JACOBI) && t > c->stop_iter) return;
+    if (kind == FK_CHEBY && t > c->stop_iter) return;
     double tot[2] = {0.0, 0.0};
     if (n >= 2) {
         sum_partials<2, TB, true>(part, nb, stride, tot);
@@ -473,13 +579,6 @@ __global__ __launch_bounds__(TB) void k_fin(Ctrl *__restrict__ c, const double *
             c->stop_iter = t;
         }
         break;
-    case FK_JACOBI: {  // Jacobi.jl:15-26: err = sum |u'-u| (+ sum r^2 every 50)
-        const double err = n >= 2 ? v[0] + v[1] : v[0];
-        c->err = err;
-        c->iters = t;
-        record_stop(c, t, decide_why(c, t, err));
-        break;
-    }
     case FK_IR: {  // FP64 refresh of the mixed-precision CG: converged or resume (t = last iteration)
         const double rr = v[0];
         c->rro = rr;
@@ -1061,7 +1160,7 @@ __device__ __forceinline__ void row_batches(int y0, int y1, Load &&load, Compute
 // an L2 and every XCD gets the same number of tiles.
 __device__ __forceinline__ bool wave_tile(const Tiles &o, int &strip, int &band)
 {
-    const int i = (int)(blockIdx.x >> 3) * 4 + (int)(threadIdx.x >> 6);
+    const int i = (int)(blockIdx.x >> 3) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n = (i / TILE_CHUNK * 8 + (int)(blockIdx.x & 7)) * TILE_CHUNK + i % TILE_CHUNK;
     strip = n % o.strips;
     band = n / o.strips;
@@ -1109,13 +1208,14 @@ __global__ __launch_bounds__(TBV) __attribute__((amdgpu_waves_per_eu(2))) void k
     const bool act = tile && lane >= 1 && lane <= TL_S64_COLS / V && x < g.nx;
     const int y0 = band * g.s64.ty, y1 = min(y0 + g.s64.ty, g.ny);
     // lanes past the ring's column nx + 1 read it again (never used)
-    const long ix = at(g, min(x, (g.nx + 1) / V * V), 0);
+    const unsigned xo = (unsigned)(min(x, (g.nx + 1) / V * V) + XCOL);
+    // element of row y's storage: a uniform row start and a 32-bit lane offset
+    auto row = [&](auto *p, int y) { return p + (g.off - XCOL + (long)y * g.pitch) + xo; };
     auto load_row = [&](Row &B, int L) {
-        const long i = ix + L * g.pitch;
-        vload<double, V, NT>(B.r, rin + i);
-        vload<double, V, NT>(B.p, pin + i);
-        vload<double, V, false>(B.g, gc + i);  // streaming: 13% slower at 3072^2
-        if constexpr (XUPD) vload<double, V, NT>(B.u, u + i);
+        vload<double, V, NT>(B.r, row(rin, L));
+        vload<double, V, NT>(B.p, row(pin, L));
+        vload<double, V, false>(B.g, row(gc, L));  // streaming: 13% slower at 3072^2
+        if constexpr (XUPD) vload<double, V, NT>(B.u, row(u, L));
     };
     // the band's first row is requested before the block sums the previous
     // sweep's partials
@@ -1123,7 +1223,7 @@ __global__ __launch_bounds__(TBV) __attribute__((amdgpu_waves_per_eu(2))) void k
     if (tile) load_row(Bs[0], y0 - 2);
 
     double s4[4];
-    sum_partials<4, TBV>(sin, nbin, g.nbmax, s4);
+    sum_block_sums<4, TBV>(sin, nbin, s4);
     const double gam = s4[0];
     const int why = t >= 2 ? decide_why(ctrl, t - 1, gam) : (int)WHY_NONE;
     const double bd = t >= 2 ? gam / ctrl->rrs[(t - 2) & 1] : 0.0;
@@ -1195,7 +1295,6 @@ __global__ __launch_bounds__(TBV) __attribute__((amdgpu_waves_per_eu(2))) void k
             if (L > y1 + 1) return false;
             if (L + 1 <= y1 + 1) load_row(Bs[f], L + 1);
             const Row &B = Bs[e];
-            const long i = ix + L * g.pitch;
             KX[f][0] = hx * (lane_up1<true>(G[f][V - 1]) + G[f][0]);
 #pragma unroll
             for (int j = 1; j < V; ++j) KX[f][j] = hx * (G[f][j - 1] + G[f][j]);
@@ -1208,13 +1307,13 @@ __global__ __launch_bounds__(TBV) __attribute__((amdgpu_waves_per_eu(2))) void k
                 P[a][j] = __builtin_fma(bd, B.p[j], B.r[j]);
             }
             if (act && L >= y0 && L < y1) {
-                vstore<double, V, NT>(pout + i, P[a]);
+                vstore<double, V, NT>(row(pout, L), P[a]);
                 if constexpr (XUPD) {
                     double un[V];
 #pragma unroll
                     for (int j = 0; j < V; ++j)
                         un[j] = __builtin_fma(alpha, P[a][j], __builtin_fma(alpha_prev, B.p[j], B.u[j]));
-                    vstore<double, V, NT>(u + i, un);
+                    vstore<double, V, NT>(row(u, L), un);
                 }
             }
             if (L < y0) return true;
@@ -1224,7 +1323,7 @@ __global__ __launch_bounds__(TBV) __attribute__((amdgpu_waves_per_eu(2))) void k
 #pragma unroll
             for (int j = 0; j < V; ++j) N[b][j] = __builtin_fma(-alpha, q[j], R[f][j]);
             if (act && L - 1 >= y0 && L - 1 < y1) {
-                vstore<double, V, NT>(rout + i - g.pitch, N[b]);
+                vstore<double, V, NT>(row(rout, L - 1), N[b]);
 #pragma unroll
                 for (int j = 0; j < V; ++j) {
                     acc[2] = __builtin_fma(N[b][j], q[j], acc[2]);
@@ -1253,7 +1352,7 @@ __global__ __launch_bounds__(TBV) __attribute__((amdgpu_waves_per_eu(2))) void k
             if (!step(std::integral_constant<int, 5>{}, L + 5)) break;
         }
     }
-    write_partials<4, TBV>(acc, sout, g.nbmax);
+    write_block_sums<4, TBV>(acc, sout);
 }
 
 // The four sums k_cgs needs at its first iteration and after a new true
@@ -1286,7 +1385,7 @@ __global__ __launch_bounds__(TB) void k_cgs_dots(Geo g, const double *__restrict
             acc[3] += p[i] * ap;
         }
     }
-    write_partials<4>(acc, part, g.nbmax);
+    write_block_sums<4>(acc, part);
 }
 
 // What the sweeps leave open when a CG stops after iteration T.  u: for odd T
@@ -2795,25 +2894,23 @@ __global__ __launch_bounds__(TB) void k_ppcg_ur_sd(Geo g, int t, double *__restr
     }
 }
 
-// ------------------------------- vectorised FP64 Chebyshev / PPCG / Jacobi
+// ----------------------------------- vectorised FP64 Chebyshev / PPCG steps
 //
-// The three stencil-update kernels of the other FP64 solvers on 16-byte
+// The stencil-update kernels of these solvers on 16-byte
 // vectors (2 doubles per lane), in the row-batch scheme of k_cgg: a lane
 // walks its column pair up a band keeping the rows below / at the current
 // row in registers, takes the columns left / right of its pair from the
 // adjacent lanes (lanes 0 and 63 load them with the row loads), and the next
 // batch's loads are issued before the current one is computed.  Per cell the
 // arithmetic is the reference's, operand for operand (smvp5's association;
-// Jacobi's as k_jacobi below), so results do not depend on the vector width.
+// the kernels below included), so results do not depend on the vector width.
 //   VS_CHEBY  (Cheby.mainstep!, Cheby.jl:84-106):
 //             r = u0 - A u; p = a p + b r; u' = u + p; [sum r^2 when calc2norm]
 //   VS_PPCG   (PPCG inner step, PPCG.jl:75-84 in the two-phase form: sd is
 //             ping-ponged): r -= A sd; u += sd; sd' = a sd + b r; [sum r^2 at
 //             the last inner step, PPCG.jl:88, consumed by the next CG.p!]
-//   VS_JACOBI (Jacobi.iterate!, Jacobi.jl:59-80):
-//             u' = (u0 + sum K u_nbr) / (1 + sum K); sum |u' - u|
 // `a_in` is the stencil input (u or sd), `a_out` its successor (u' or sd');
-// f1 / f2 are u0 / p (Chebyshev), r / u (PPCG), u0 / unused (Jacobi).
+// f1 / f2 are u0 / p (Chebyshev), r / u (PPCG).  (VS_JACOBI: k_steps.)
 enum VsOp : int { VS_CHEBY = 0, VS_PPCG = 1, VS_JACOBI = 2 };
 
 template <int OP, int RB, bool PIPE>
@@ -2853,7 +2950,7 @@ __global__ __launch_bounds__(TBV) void k_vs64(Geo g, int ty, int t, const double
                 vload<T, V>(B.kxv[q], kx + ic);
                 vload<T, V>(B.kyu[q], ky + at(g, cl.xl, min(y + 1, g.ny)));
                 vload<T, V>(B.e1[q], f1 + ic);
-                if (OP != VS_JACOBI) vload<T, V>(B.e2[q], f2 + ic);
+                vload<T, V>(B.e2[q], f2 + ic);
                 B.eup[q] = B.ekx[q] = (T)0;
                 if (eneed) B.eup[q] = a_in[iu + eoff];
                 if (cl.lane == 63) B.ekx[q] = kx[ic + V];
@@ -2877,33 +2974,18 @@ __global__ __launch_bounds__(TBV) void k_vs64(Geo g, int ty, int t, const double
                 for (int j = 0; j < V; ++j) {
                     const T kxl = B.kxv[q][j], kxr = j < V - 1 ? B.kxv[q][j + 1] : kxn;
                     const T kyu = B.kyu[q][j];
-                    if constexpr (OP == VS_JACOBI) {
-                        const T l = j > 0 ? cur[j - 1] : lv;
-                        T r = j < V - 1 ? cur[j + 1] : rv;
-                        if (cl.xl + j + 1 >= g.nx) r = cur[j];
-                        double num = B.e1[q][j] + kxr * r;
-                        num = num + kxl * l;
-                        num = num + kyu * u2[j];
-                        num = num + kyd[j] * dn[j];
-                        double den = 1.0 + kxl;
-                        den = den + kxr;
-                        den = den + kyd[j];
-                        den = den + kyu;
-                        o1[j] = num / den;
+                    const T w = vsmvp<T, V>(g, cl.xl, j, cur, lv, rv, dn[j], u2[j], kxl, kxr, kyd[j], kyu);
+                    if constexpr (OP == VS_CHEBY) {
+                        const T rr = B.e1[q][j] - w;        // u0 - A u
+                        const T pv = ca * B.e2[q][j] + cb * rr;
+                        o1[j] = cur[j] + pv;                // u'
+                        o2[j] = pv;                         // p
+                        o3[j] = rr;
                     } else {
-                        const T w = vsmvp<T, V>(g, cl.xl, j, cur, lv, rv, dn[j], u2[j], kxl, kxr, kyd[j], kyu);
-                        if constexpr (OP == VS_CHEBY) {
-                            const T rr = B.e1[q][j] - w;        // u0 - A u
-                            const T pv = ca * B.e2[q][j] + cb * rr;
-                            o1[j] = cur[j] + pv;                // u'
-                            o2[j] = pv;                         // p
-                            o3[j] = rr;
-                        } else {
-                            const T rr = B.e1[q][j] - w;        // r - A sd
-                            o1[j] = ca * cur[j] + cb * rr;      // sd'
-                            o2[j] = rr;                         // r
-                            o3[j] = B.e2[q][j] + cur[j];        // u + sd
-                        }
+                        const T rr = B.e1[q][j] - w;        // r - A sd
+                        o1[j] = ca * cur[j] + cb * rr;      // sd'
+                        o2[j] = rr;                         // r
+                        o3[j] = B.e2[q][j] + cur[j];        // u + sd
                     }
                 }
                 if (y < cl.y1 && cl.active) {
@@ -2914,16 +2996,12 @@ __global__ __launch_bounds__(TBV) void k_vs64(Geo g, int ty, int t, const double
 #pragma unroll
                         for (int j = 0; j < V; ++j)
                             if (j < nv) acc[0] += o3[j] * o3[j];
-                    } else if constexpr (OP == VS_PPCG) {
+                    } else {
                         vstore_n<T, V>(f1 + ic, o2, nv);
                         vstore_n<T, V>(f2 + ic, o3, nv);
 #pragma unroll
                         for (int j = 0; j < V; ++j)
                             if (j < nv) acc[0] += o2[j] * o2[j];
-                    } else {
-#pragma unroll
-                        for (int j = 0; j < V; ++j)
-                            if (j < nv) acc[0] += fabs(o1[j] - cur[j]);
                     }
                 }
 #pragma unroll
@@ -3291,47 +3369,250 @@ __global__ __launch_bounds__(TBV) void k_cheby2(Geo g, int ty, int t, const doub
     if (norm) write_partials<1, TBV>(acc, part, g.nbmax);
 }
 
-// --------------------------------------------------------------- Jacobi
+// ------------------------------------ several FP64 solver steps in one sweep
+//
+// Chebyshev iterations, PPCG inner steps and Jacobi sweeps have no scalar of the
+// iteration in their update, so a block can take up to STEPS_HALO of them on a
+// tile before it writes it back.  A block of NW waves holds 64 V columns x NW RW
+// rows in registers: a lane owns V columns of RW rows, its left and right
+// neighbours come from the adjacent lanes (DPP), the rows above and below a
+// wave's from the waves beside it through the LDS, one barrier per step.
+// Every step loses one cell of the tile's rim, so the inner tile (all but
+// STEPS_HALO cells on every side) is right after STEPS_HALO steps; the rim is
+// computed by the neighbouring blocks too.  At the domain's edges the reflected
+// neighbour is the cell itself, as elsewhere.
+// The operations and their association are the single step's (k_vs64), so each
+// step is bit-identical to a launch of it.
+//   VS_CHEBY  a: u, b: p, d: u0 (const).      Bytes per cell: 56 for up to 8 steps (56 for each)
+//   VS_PPCG   a: sd, d: r, b: u (own cells).  64 for up to 8 steps (64 for each)
+//   VS_JACOBI a: u, d: u0 (const).            40 for up to 8 steps (40 for each)
+// times the rim's re-reads (most of them cache hits).  Jacobi's error sum
+// |u' - u| of every step is one of eight sums per block; the next launch sums
+// them over the blocks, in order, and stops the solve at the first step that met
+// the rule (the host then repeats the steps up to that one from the launch's
+// input).  With resid a last stage forms r = u0 - A u and its sum of squares,
+// which Jacobi adds to the error of every 50th iteration (Jacobi.jl:21-24).
+// Bound by latency, a block per CU loading, stepping and storing in turn: eight
+// PPCG steps take 53 us at 1300x1700 (two rounds of 432 tiles; two steps as one
+// k_ppcg2 38 us), eight Chebyshev steps 97 us at 2048^2 (k_cheby2: 52 us for
+// two), eight Jacobi iterations 18 us at 200x300 with their stop tests (one with
+// its finalizer took 8.3).
 
-// Jacobi.iterate!, Jacobi.jl:59-80 (u' in a separate buffer, the reference's
-// r = copy of u): u' = (u0 + sum K u_nbr) / (1 + sum K); partials of
-// err = sum |u' - u|
-__global__ __launch_bounds__(TB) void k_jacobi(Geo g, int t, const double *__restrict__ uin,
-                                               double *__restrict__ uout, const double *__restrict__ u0,
-                                               const double *__restrict__ kx, const double *__restrict__ ky,
-                                               const Ctrl *__restrict__ ctrl, double *__restrict__ part)
+// stop test of the steps t0 .. t0+n-1 of the previous launch from its partial
+// sums, identical in every block; resid: sum r^2 joins the last step's
+template <int NT>
+__device__ __forceinline__ bool jacobi_stopped(Ctrl *__restrict__ ctrl, const double *__restrict__ part, unsigned nb,
+                                               int n, int resid, int t0)
 {
-    if (t > ctrl->stop_iter) return;
-    const Col c = column(g);
-    double acc[1] = {0.0};
-    if (c.active) {
-        Win<double> win;
-        win.start(g, c, uin, ky);
-        for (int yb = c.y0; yb < c.y1; yb += R) {
-            Stn<double> st;
-            double b[R];
-            load_stn(st, g, c, yb, uin, kx, ky);
-            load_rows(b, g, c, yb, u0);
+    double tot[STEPS_HALO];
+    sum_block_sums<STEPS_HALO, NT>(part, nb, tot);
+    bool stop = false;
 #pragma unroll
-            for (int q = 0; q < R; ++q) {
-                double num = b[q] + st.kxr[q] * st.rt[q];
-                num = num + st.kxl[q] * st.lf[q];
-                num = num + st.kyu[q] * st.up[q];
-                num = num + win.kyd * win.dn;
-                double den = 1.0 + st.kxl[q];
-                den = den + st.kxr[q];
-                den = den + win.kyd;
-                den = den + st.kyu[q];
-                const double un = num / den;
-                if (yb + q < c.y1) {
-                    uout[at(g, c.x, yb + q)] = un;
-                    acc[0] += fabs(un - win.cur);
-                }
-                win.advance(st, q);
+    for (int k = 0; k < STEPS_HALO; ++k) {
+        if (stop || k >= n) continue;
+        const double err = resid && k == n - 1 && k + 1 < STEPS_HALO ? tot[k] + tot[k + 1 < STEPS_HALO ? k + 1 : k]
+                                                                     : tot[k];
+        const int why = decide_why(ctrl, t0 + k, err);
+        if (block_id() == 0 && threadIdx.x == 0) {
+            ctrl->sums[0] = tot[k];
+            ctrl->err = err;
+            ctrl->iters = t0 + k;
+            record_stop(ctrl, t0 + k, why);
+        }
+        stop = why != WHY_NONE;
+    }
+    return stop;
+}
+
+__global__ __launch_bounds__(TB) void k_jacobi_end(Ctrl *__restrict__ ctrl, const double *__restrict__ part,
+                                                   unsigned nb, int n, int resid, int t0)
+{
+    if (t0 > ctrl->stop_iter) return;
+    (void)jacobi_stopped<TB>(ctrl, part, nb, n, resid, t0);
+}
+
+template <int OP, int V, int NW, int RW>
+__global__ __launch_bounds__(NW * 64) void k_steps(Geo g, int gx, int t, int n, const double *__restrict__ a_in,
+                                                   double *__restrict__ a_out, const double *__restrict__ d_in,
+                                                   double *__restrict__ d_out, const double *__restrict__ b_in,
+                                                   double *__restrict__ b_out, const double *__restrict__ kx,
+                                                   const double *__restrict__ ky, StepCoef co,
+                                                   Ctrl *__restrict__ ctrl, const double *__restrict__ part_in,
+                                                   double *__restrict__ part_out, int nprev, int residp, int resid)
+{
+    constexpr int W = 64 * V, H = NW * RW, HALO = STEPS_HALO, UW = W - 2 * HALO, UH = H - 2 * HALO;
+    struct vec {
+        double e[V];
+    };
+    if (t > ctrl->stop_iter) return;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // tiles dealt to the XCDs in runs, as in wave_tile
+    const int xb = (int)(blockIdx.x >> 3);
+    const int tile = (xb / STEPS_CHUNK * 8 + (int)(blockIdx.x & 7)) * STEPS_CHUNK + xb % STEPS_CHUNK;
+    const int bx = tile % gx, by = tile / gx;
+    const int x = bx * UW - HALO + lane * V;
+    const int yw = by * UH - HALO + wave * RW;  // the wave's first row
+    // left of column 0: halo and padding columns (valid memory).  Right of the
+    // grid Jacobi needs the domain face's coefficient kx(nx), which stays in its
+    // denominator; in the residual forms it cancels with the reflected neighbour
+    // and its rounding is the single step's, which reads the last vector again.
+    const int xc = min(x, (OP == VS_JACOBI ? g.nx : g.nx - 1) / V * V);
+    const bool own_x = lane >= HALO / V && lane < 64 - HALO / V && x < g.nx;
+    // element of row y's storage: a uniform row start and a 32-bit lane offset
+    const unsigned xo = (unsigned)(xc + XCOL);
+    auto row = [&](auto *p, int y) { return p + (g.off - XCOL + (long)y * g.pitch); };
+    // one array that a step touches once per cell is kept in the LDS where the
+    // registers would spill: PPCG's u, u0 of the largest tiles (PPCG's steps at
+    // 1300x1700 took 98 us with u in registers, 57 of them spilled, and 53)
+    constexpr bool PARK = OP == VS_PPCG || RW * V > 8;
+    __shared__ vec park[PARK ? RW : 1][PARK ? NW * 64 : 1];
+    double a[RW][V], b[RW][V] = {}, d[RW][V], kxl[RW][V], kyd[RW + 1][V];
+    bool own[RW];
+#pragma unroll
+    for (int q = 0; q < RW; ++q) {
+        const int y = yw + q, yc = min(max(y, 0), g.ny - 1);
+        own[q] = own_x && wave * RW + q >= HALO && wave * RW + q < H - HALO && y < g.ny;
+        vload<double, V, false>(a[q], row(a_in, yc) + xo);
+        if constexpr (PARK && OP != VS_PPCG)
+            vload<double, V, false>(park[q][threadIdx.x].e, row(d_in, yc) + xo);
+        else
+            vload<double, V, false>(d[q], row(d_in, yc) + xo);
+        if constexpr (OP == VS_CHEBY) vload<double, V, false>(b[q], row(b_in, yc) + xo);
+        if constexpr (OP == VS_PPCG)
+            if (own[q]) vload<double, V, false>(park[q][threadIdx.x].e, row(b_in, yc) + xo);
+        vload<double, V, false>(kxl[q], row(kx, yc) + xo);
+        vload<double, V, false>(kyd[q], row(ky, min(max(y, 0), g.ny)) + xo);
+    }
+    vload<double, V, false>(kyd[RW], row(ky, min(max(yw + RW, 0), g.ny)) + xo);
+    if constexpr (OP == VS_JACOBI) {
+        if (nprev && jacobi_stopped<NW * 64>(ctrl, part_in, gridDim.x, nprev, residp, t - nprev)) return;
+    }
+    __shared__ vec rows[2][NW][2][64];
+    double acc[STEPS_HALO] = {};
+    // does the tile touch the domain's edge (uniform)
+    const bool edge = bx == 0 || by == 0 || x - lane * V + W >= g.nx || by * UH - HALO + H >= g.ny;
+
+    // rows of a above and below the wave's, step k
+    auto exchange = [&](int k, double (&lo)[V], double (&hi)[V]) {
+#pragma unroll
+        for (int j = 0; j < V; ++j) {
+            rows[k & 1][wave][0][lane].e[j] = a[0][j];
+            rows[k & 1][wave][1][lane].e[j] = a[RW - 1][j];
+        }
+        __syncthreads();
+        // outside the tile: any value (its rim is lost anyway)
+        const vec l = rows[k & 1][wave > 0 ? wave - 1 : 0][1][lane];
+        const vec h = rows[k & 1][wave < NW - 1 ? wave + 1 : NW - 1][0][lane];
+#pragma unroll
+        for (int j = 0; j < V; ++j) {
+            lo[j] = l.e[j];
+            hi[j] = h.e[j];
+        }
+    };
+    // f(q, j, c, l, r, dn, up, kxl, kxr, kyd, kyu) for every cell, row by row,
+    // with the values before the step
+    auto stencil = [&](auto ec, int k, auto &&f) {
+        constexpr bool E = decltype(ec)::value;
+        double lo[V], hi[V];
+        exchange(k, lo, hi);
+#pragma unroll
+        for (int q = 0; q < RW; ++q) {
+            double c[V];
+#pragma unroll
+            for (int j = 0; j < V; ++j) c[j] = a[q][j];
+            double lv = lane_up1<true>(c[V - 1]), rv = lane_down1<true>(c[0]);
+            const double kxr = lane_down1<true>(kxl[q][0]);
+            if (E && x == 0) lv = c[0];
+            const bool ybot = E && yw + q == 0, ytop = E && yw + q == g.ny - 1;
+#pragma unroll
+            for (int j = 0; j < V; ++j) {
+                const double l = j > 0 ? c[j > 0 ? j - 1 : 0] : lv;
+                double r = j < V - 1 ? c[j < V - 1 ? j + 1 : j] : rv;
+                if (E && x + j == g.nx - 1) r = c[j];
+                const double dn = ybot ? c[j] : lo[j];
+                const double up = ytop ? c[j] : q < RW - 1 ? a[q < RW - 1 ? q + 1 : q][j] : hi[j];
+                f(q, j, c[j], l, r, dn, up, kxl[q][j], j < V - 1 ? kxl[q][j < V - 1 ? j + 1 : j] : kxr, kyd[q][j],
+                  kyd[q + 1][j]);
             }
+#pragma unroll
+            for (int j = 0; j < V; ++j) lo[j] = c[j];
+            // row by row: scheduled together, the rows' temporaries spill
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    auto u0 = [&](int q, int j) { return PARK ? park[q][threadIdx.x].e[j] : d[q][j]; };
+    auto one = [&](auto ec, int k, double ca, double cb, double &err) {
+        stencil(ec, k, [&](int q, int j, double c, double l, double r, double dn, double up, double kl, double kr,
+                           double kd, double ku) {
+            if constexpr (OP == VS_JACOBI) {
+                double num = u0(q, j) + kr * r;
+                num = num + kl * l;
+                num = num + ku * up;
+                num = num + kd * dn;
+                double den = 1.0 + kl;
+                den = den + kr;
+                den = den + kd;
+                den = den + ku;
+                const double un = num / den;
+                if (own[q] && x + j < g.nx) err += fabs(un - c);
+                a[q][j] = un;
+            } else {
+                const double w = smvp5(c, l, r, dn, up, kl, kr, kd, ku);
+                if constexpr (OP == VS_CHEBY) {
+                    const double rr = u0(q, j) - w;          // u0 - A u
+                    b[q][j] = ca * b[q][j] + cb * rr;        // p
+                    a[q][j] = c + b[q][j];                   // u
+                } else {
+                    d[q][j] = d[q][j] - w;                   // r - A sd
+                    a[q][j] = ca * c + cb * d[q][j];         // sd
+                    park[q][threadIdx.x].e[j] += c;          // u + sd
+                }
+            }
+        });
+    };
+    auto all = [&](auto ec) {
+        if constexpr (OP == VS_JACOBI) {
+#pragma unroll
+            for (int k = 0; k < HALO; ++k)
+                if (k < n) one(ec, k, 0.0, 0.0, acc[k]);
+            if (resid) {
+                // r of the last step's u; its sum in the array after the steps'
+                double r2 = 0.0;
+                stencil(ec, n, [&](int q, int j, double c, double l, double r, double dn, double up, double kl,
+                                   double kr, double kd, double ku) {
+                    b[q][j] = u0(q, j) - smvp5(c, l, r, dn, up, kl, kr, kd, ku);
+                    if (own[q] && x + j < g.nx) r2 += b[q][j] * b[q][j];
+                });
+#pragma unroll
+                for (int k = 1; k < HALO; ++k)
+                    if (k == n) acc[k] = r2;
+            }
+        } else {
+            double unused = 0.0;
+            for (int k = 0; k < n; ++k) one(ec, k, co.a[k], co.b[k], unused);
+        }
+    };
+    if (edge)
+        all(std::true_type{});
+    else
+        all(std::false_type{});
+#pragma unroll
+    for (int q = 0; q < RW; ++q) {
+        if (!own[q]) continue;
+        const int nv = g.nx - x;
+        vstore_n<double, V, false>(row(a_out, yw + q) + xo, a[q], nv);
+        if constexpr (OP == VS_PPCG) vstore_n<double, V, false>(row(d_out, yw + q) + xo, d[q], nv);
+        if constexpr (OP == VS_PPCG) {
+#pragma unroll
+            for (int j = 0; j < V; ++j) b[q][j] = park[q][threadIdx.x].e[j];
+        }
+        if constexpr (OP == VS_JACOBI) {
+            if (resid) vstore_n<double, V, false>(row(d_out, yw + q) + xo, b[q], nv);
+        } else {
+            vstore_n<double, V, false>(row(b_out, yw + q) + xo, b[q], nv);
         }
     }
-    write_partials<1>(acc, part, g.nbmax);
+    if constexpr (OP == VS_JACOBI) write_block_sums<STEPS_HALO, NW * 64>(acc, part_out);
 }
 
 // ------------------------------------------------------ mixed precision
@@ -3711,14 +3992,6 @@ hipError_t launch_residual(tl_ctx *c)
     return hipGetLastError();
 }
 
-hipError_t launch_jacobi_residual(tl_ctx *c, const double *u, int t)
-{
-    k_residual<<<sgrid(c->g), TB, 0, c->stream>>>(c->g, t, c->f[TL_F_U0], u, c->f[TL_F_KX], c->f[TL_F_KY],
-                                                  c->f[TL_F_R], nullptr, nullptr, c->ctrl, part_m(c) + stride(c));
-    hipError_t e = hipGetLastError();
-    return e == hipSuccess ? fin(c, part_m(c), nbh(c), 2, 0, FK_JACOBI, t) : e;
-}
-
 hipError_t launch_ir_residual(tl_ctx *c, int reset_p, int t_next, float *r_dst)
 {
     const bool prof = prof_start(c, TL_K_RESID64);
@@ -3850,22 +4123,80 @@ hipError_t launch_ppcg_inner2(tl_ctx *c, double a1, double b1, double a2, double
     return hipGetLastError();
 }
 
-hipError_t launch_jacobi(tl_ctx *c, const double *u_in, double *u_out, int t, int defer)
+// calls f(columns per lane, waves per block, rows per wave) for the tile: 128 x
+// 64 cells (one block per CU: 246 registers) from 128 such tiles on, half the
+// CUs, else 64 x 32.  Measured, PPCG iterations with 10 inner steps, 128x64 /
+// 64x32 / 128x32 tiles: 500x600 (65 tiles of 128x64) 36.6 / 33.3 / 33.1 us,
+// 800x700 (120) 43.4 / 42.2 / 44.9; 1000x900 (171) 48.8 and 128x32 55.1,
+// 1000x1300 (252) 62.7 and 70.3, 1600x1500 (480) 110.7 and 124.3.
+template <class F>
+static hipError_t with_steps_tile(const Geo &g, F &&f)
 {
+    int gx;
+    if (steps_tiles(g.nx, g.ny, 128, 64, gx) >= 128)
+        return f(std::integral_constant<int, 2>{}, std::integral_constant<int, 8>{}, std::integral_constant<int, 8>{});
+    return f(std::integral_constant<int, 1>{}, std::integral_constant<int, 8>{}, std::integral_constant<int, 4>{});
+}
+
+hipError_t launch_cheby_steps(tl_ctx *c, int n, const StepCoef &co, const double *u_in, double *u_out,
+                              const double *p_in, double *p_out, int t)
+{
+    return with_steps_tile(c->g, [&](auto v, auto nw, auto rw) {
+        constexpr int V = decltype(v)::value, NW = decltype(nw)::value, RW = decltype(rw)::value;
+        int gx;
+        const unsigned nb = steps_blocks(steps_tiles(c->g.nx, c->g.ny, 64 * V, NW * RW, gx));
+        k_steps<VS_CHEBY, V, NW, RW><<<nb, NW * 64, 0, c->stream>>>(c->g, gx, t, n, u_in, u_out, c->f[TL_F_U0], nullptr, p_in,
+                                                            p_out, c->f[TL_F_KX], c->f[TL_F_KY], co, c->ctrl, nullptr,
+                                                            nullptr, 0, 0, 0);
+        return hipGetLastError();
+    });
+}
+
+hipError_t launch_ppcg_steps(tl_ctx *c, int n, const StepCoef &co, const double *sd_in, double *sd_out,
+                             const double *r_in, double *r_out, int t)
+{
+    return with_steps_tile(c->g, [&](auto v, auto nw, auto rw) {
+        constexpr int V = decltype(v)::value, NW = decltype(nw)::value, RW = decltype(rw)::value;
+        int gx;
+        const unsigned nb = steps_blocks(steps_tiles(c->g.nx, c->g.ny, 64 * V, NW * RW, gx));
+        k_steps<VS_PPCG, V, NW, RW><<<nb, NW * 64, 0, c->stream>>>(c->g, gx, t, n, sd_in, sd_out, r_in, r_out, c->f[TL_F_U],
+                                                           c->f[TL_F_U], c->f[TL_F_KX], c->f[TL_F_KY], co, c->ctrl,
+                                                           nullptr, nullptr, 0, 0, 0);
+        return hipGetLastError();
+    });
+}
+
+// the error sums of a launch at iterations t .. alternate between two sets
+static inline double *part_j(tl_ctx *c, int set) { return c->part_j + (size_t)set * STEPS_HALO * stride(c); }
+
+hipError_t launch_jacobi_steps(tl_ctx *c, int n, const double *u_in, double *u_out, double *r_out, int resid,
+                               int nprev, int residp, int t)
+{
+    c->jset ^= 1;
     const bool prof = prof_start(c, TL_K_JACOBI64);
-    if (defer) {
-        // the sweep whose sum joins the residual's (every 50th): the scalar
-        // kernel, so that both partial arrays have k_residual's block count
-        k_jacobi<<<sgrid(c->g), TB, 0, c->stream>>>(c->g, t, u_in, u_out, c->f[TL_F_U0], c->f[TL_F_KX],
-                                                    c->f[TL_F_KY], c->ctrl, part_m(c));
-    } else {
-        k_vs64<VS_JACOBI, TL_RV_VS64, TL_PIPE_VS64 != 0><<<nb2(c), TBV, 0, c->stream>>>(
-            c->g, c->g.ty2, t, u_in, u_out, c->f[TL_F_KX], c->f[TL_F_KY], c->f[TL_F_U0], nullptr, 0.0, 0.0, 1,
-            c->ctrl, part_m(c));
-    }
+    const hipError_t e = with_steps_tile(c->g, [&](auto v, auto nw, auto rw) {
+        constexpr int V = decltype(v)::value, NW = decltype(nw)::value, RW = decltype(rw)::value;
+        int gx;
+        const unsigned nb = steps_blocks(steps_tiles(c->g.nx, c->g.ny, 64 * V, NW * RW, gx));
+        k_steps<VS_JACOBI, V, NW, RW><<<nb, NW * 64, 0, c->stream>>>(
+            c->g, gx, t, n, u_in, u_out, c->f[TL_F_U0], r_out, nullptr, nullptr, c->f[TL_F_KX], c->f[TL_F_KY],
+            StepCoef{}, c->ctrl, part_j(c, c->jset ^ 1), part_j(c, c->jset), nprev, residp, resid);
+        return hipGetLastError();
+    });
     if (prof) prof_stop(c);
-    hipError_t e = hipGetLastError();
-    return (e == hipSuccess && !defer) ? fin(c, part_m(c), nb2(c), 1, 0, FK_JACOBI, t) : e;
+    return e;
+}
+
+// the stop test of the last launch's steps, which ended before iteration t
+hipError_t launch_jacobi_end(tl_ctx *c, int nprev, int residp, int t)
+{
+    return with_steps_tile(c->g, [&](auto v, auto nw, auto rw) {
+        constexpr int V = decltype(v)::value, NW = decltype(nw)::value, RW = decltype(rw)::value;
+        int gx;
+        const unsigned nb = steps_blocks(steps_tiles(c->g.nx, c->g.ny, 64 * V, NW * RW, gx));
+        k_jacobi_end<<<1, TB, 0, c->stream>>>(c->ctrl, part_j(c, c->jset), nb, nprev, residp, t - nprev);
+        return hipGetLastError();
+    });
 }
 
 // u += d; d = 0 over the whole allocation (d is zero outside the interior)

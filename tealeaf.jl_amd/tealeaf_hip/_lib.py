@@ -48,7 +48,7 @@ TL_CHEBY_PAIRS_AUTO, TL_CHEBY_PAIRS_OFF = 0, 1
 KERNEL_NAMES = {0: "k_cgs<false, true>", 1: "k_cgs<true, true>", 2: "k_cg_p<double>",
                 3: "k_cgg<4, false, 2, true, 1>", 4: "k_cgg<4, true, 4, true, 1>",
                 5: "(fused into k_cgg<4, false, 2, true, 1>)",
-                6: "k_vs64<0, 4, true>", 7: "k_vs64<1, 4, true>", 8: "k_vs64<2, 4, true>", 9: "k_residual",
+                6: "k_vs64<0, 4, true>", 7: "k_vs64<1, 4, true>", 8: "k_steps<2, 2, 8, 8>", 9: "k_residual",
                 10: "k_cgf<1, 1, 0>", 11: "k_ppcg2", 12: "k_cheby2", 13: "k_cgp<1, false>", 14: "k_cgp<1, true>",
                 -1: "k_copy_full", -2: "k_copy_vec"}
 
