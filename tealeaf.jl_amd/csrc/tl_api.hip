@@ -541,7 +541,10 @@ static int ensure_history(tl_ctx *c, int n)
 static int ensure_fp32(tl_ctx *c)
 {
     const size_t n = c->g.elems;
-    if (!c->gcell && hipMalloc((void **)&c->gcell, n * sizeof(tl_gc_t)) != hipSuccess) c->gcell = nullptr;
+    if (!c->gcell) {
+        if (hipMalloc((void **)&c->gcell, n * sizeof(tl_gc_t)) != hipSuccess) c->gcell = nullptr;
+        else if (hipMemsetAsync(c->gcell, 0, n * sizeof(tl_gc_t), c->stream) != hipSuccess) return TL_E_HIP;
+    }
     if (!c->gc_range && hipMalloc((void **)&c->gc_range, 2 * TL_RANGE_BLOCKS * sizeof(float)) != hipSuccess)
         c->gc_range = nullptr;
     if (!c->gcell || !c->gc_range) {
@@ -559,7 +562,7 @@ static int ensure_fp32(tl_ctx *c)
 static int ensure_fused(tl_ctx *c)
 {
     if (!c->r32b) RETIF(alloc_f(c, &c->r32b, c->g.elems));
-    if (!c->part_f) RETIF(alloc_d(c, &c->part_f, (size_t)8 * c->g.nbmax));
+    if (!c->part_f) RETIF(alloc_d(c, &c->part_f, (size_t)9 * c->g.nbmax));
     return TL_OK;
 }
 
@@ -568,11 +571,19 @@ static int ensure_cgs(tl_ctx *c)
 {
     if (!c->r_alt1) RETIF(alloc_d(c, &c->r_alt1, c->g.elems));
     if (!c->g64) RETIF(alloc_d(c, &c->g64, c->g.elems));
-    if (!c->part_f) RETIF(alloc_d(c, &c->part_f, (size_t)8 * c->g.nbmax));
+    if (!c->part_f) RETIF(alloc_d(c, &c->part_f, (size_t)9 * c->g.nbmax));
     return TL_OK;
 }
 
 static bool fused_fits(const tl_ctx *c) { return c->g.nx % 4 == 0; }
+
+// TL_FP32_KERNELS_AUTO with stream launches: pairs of iterations, which take
+// any nx.  They are the faster form on ragged grids of every size measured
+// (milliseconds of a solve, two kernels / pairs: 63x61 2.9 / 1.9, 131x77 5.9 /
+// 3.2, 151x153 5.9 / 3.4, 201x203 10.0 / 5.6), but on small ones the two kernels
+// stay: there stream launches and hipGraph batches are held to give the same
+// bits (the pairs have no batch form), and a solve takes a few ms.
+static bool pairs_pay(const tl_ctx *c) { return fused_fits(c) || (long)c->g.nx * c->g.ny >= 16384; }
 
 static int status_of(tl_ctx *c, const Ctrl &k)
 {
@@ -1149,7 +1160,7 @@ static int solve_cg_ir(tl_ctx *c, const tl_solve_params *p, double rx, double ry
     // pairs of iterations (k_cgp) run as stream launches; with TL_LAUNCH_GRAPH
     // the automatic choice takes the fused kernel
     const bool pairs = p->fp32_kernels == TL_FP32_KERNELS_PAIRS ||
-                       (p->fp32_kernels == TL_FP32_KERNELS_AUTO && TL_CGP_AUTO && fused_fits(c) &&
+                       (p->fp32_kernels == TL_FP32_KERNELS_AUTO && TL_CGP_AUTO && pairs_pay(c) &&
                         p->launch != TL_LAUNCH_GRAPH);
     const bool fused = !pairs && (p->fp32_kernels == TL_FP32_KERNELS_FUSED ||
                                   (p->fp32_kernels == TL_FP32_KERNELS_AUTO && fused_fits(c)));

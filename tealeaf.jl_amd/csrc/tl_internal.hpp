@@ -113,6 +113,17 @@ constexpr int TBV = TL_TBV;
 #define TL_S64_COLS 120
 #define TL_S64_WAVES 2048
 #define TL_S64_ROWS 4
+// the same for the pairs of FP32 CG iterations.  Measured at 8192^2 (first /
+// second sweep, us): 3072 waves, one round at 3 per SIMD, 118 / 361; second sweep
+// in 2048 waves 118 / 387, in 4096 (4 per SIMD) 120 / 389; first sweep in 4096
+// 123; 248 columns 7% slower over a solve, 224 (whole cache lines) 119 / 362;
+// stores not streaming 177 / 381, the second
+// sweep's loads not 126 / 376, nor x's 159 / 364.  4096x3000: 50.9 us per iteration with 3072
+// waves, 51.8 with 2048, 55.4 with 4096.  Bands of 2 rows 3% slower at 1024^2,
+// of 8 rows 8%.
+#define TL_S32_COLS 240
+#define TL_S32_WAVES 3072
+#define TL_S32_ROWS 4
 // sweeps over more bytes than this (the Infinity Cache) use streaming access.
 // Measured with the FP64 CG sweep: 453 MB of arrays (3072^2) 92.6 us per
 // iteration streaming, 102.2 cached; 83 MB (1501x1103) 25.1 and 21.9.
@@ -120,16 +131,10 @@ constexpr size_t TL_CACHE_BYTES = (size_t)256 << 20;
 #ifndef TL_CGF_DEPTH
 #define TL_CGF_DEPTH 0
 #endif
-// TL_FP32_KERNELS_AUTO takes the pairs of iterations (k_cgp) where the fused
-// kernel fits and launches are stream launches (1), or the fused kernel (0).
-// Measured at 8192^2: 0.245 ms per iteration (first sweep 0.145, second
-// 0.345 per pair) against 0.287 for the fused kernel, at the same iteration
-// counts.
-// the pair's second step: A p1 by the stencil of p1 formed on three rows (1),
-// or as A r - alpha0 A^2 p + beta0 A p (0)
-#ifndef TL_CGP_AP1
-#define TL_CGP_AP1 1
-#endif
+// TL_FP32_KERNELS_AUTO takes the pairs of iterations (k_cgp) with stream launches
+// (1), or the fused kernel where it fits (0).  Measured at 8192^2: 0.240 ms per
+// iteration (first sweep 0.118, second 0.361 per pair) against 0.287 for the
+// fused kernel, at the same iteration counts.
 #ifndef TL_CGP_AUTO
 #define TL_CGP_AUTO 1
 #endif
@@ -219,7 +224,8 @@ struct StepCoef {
     double a[STEPS_HALO], b[STEPS_HALO];
 };
 
-// neighbouring tiles dealt to one XCD in a run (4 and 64: 1-2% slower)
+// neighbouring tiles dealt to one XCD in a run (FP64 CG sweep: 4 and 64 1-2%
+// slower; FP32 pairs: 4 and 8 1-2%, 36 17%)
 constexpr int TILE_CHUNK = 16;
 
 struct Geo {
@@ -234,6 +240,7 @@ struct Geo {
     int gyf, tyf;              // fused FP32 kernel: gx4*gyf blocks of 4*TB columns x tyf rows
     int gyq, tyq;              // two-step PPCG kernel: gx2*gyq blocks of 2*TB columns x tyq rows
     Tiles s64;                 // single-sweep FP64 CG
+    Tiles s32;                 // pairs of FP32 CG iterations
     int nbmax;                 // stride of the partial-sum arrays (max block count)
     size_t elems;              // elements per allocation
 };
@@ -404,7 +411,7 @@ hipError_t launch_cgf(tl_ctx *c, int t, int tref = 0);
 hipError_t launch_cgf_dots(tl_ctx *c, int T);
 float *cgf_r(tl_ctx *c, int t);
 float *cgf_p(tl_ctx *c, int t);
-hipError_t launch_cgp(tl_ctx *c, int t, bool first, int tref = 0);
+hipError_t launch_cgp(tl_ctx *c, int t, bool first);
 float *cgp_r(tl_ctx *c, int T);
 float *cgp_p(tl_ctx *c, int T);
 hipError_t launch_apply(tl_ctx *c, const double *src, double *dst);

@@ -131,7 +131,8 @@ Geo make_geo(int nx, int ny, int hd)
     g.nbmax = std::max(std::max(g.gx * g.gy, g.gx4 * g.gyp4), std::max(g.gx4 * g.gy4, g.gx2 * g.gy2));
     g.nbmax = std::max(g.nbmax, g.gx4 * g.gyf);
     g.s64 = make_tiles(nx, ny, TL_S64_COLS, TL_S64_WAVES, TL_S64_ROWS);
-    g.nbmax = std::max(g.nbmax, g.s64.blocks);
+    g.s32 = make_tiles(nx, ny, TL_S32_COLS, TL_S32_WAVES, TL_S32_ROWS);
+    g.nbmax = std::max(g.nbmax, std::max(g.s64.blocks, g.s32.blocks));
     int gxs;
     g.nbmax = std::max(g.nbmax, (int)steps_blocks(steps_tiles(nx, ny, 64, 32, gxs)));  // its smallest tiles
     return g;
@@ -2237,77 +2238,65 @@ __global__ __launch_bounds__(TBV) TL_CGF_ATTR void k_cgf(Geo g, int ty, int t, c
 // products (p, Ap), (r, Ap), (Ap, Ap), (r, Ar), (Ap, Ar), (Ap, A^2 p); it
 // stores nothing.  The second (UPD true) forms p and A p bit for bit as the
 // first did, derives the scalars from the six sums, forms p1 on three rows
-// and applies the stencil to it (TL_CGP_AP1; else A p1 from the basis as
-// above), and writes r(t+1), p(t+1) and x, with (r(t+1), r(t+1)) for the
-// next pair.  Bytes per cell for the two
+// and applies the stencil to it, and writes r(t+1), p(t+1) and x, with
+// (r(t+1), r(t+1)) for the next pair.  Bytes per cell for the two
 // iterations: 10 (r, p', 16-bit gc) + 26 (also x; writes r, p, x) = 36, or
-// 18 per iteration against 22 for k_cgf.  The walk is k_cgf's: rows L-3 .. L
-// in registers (p at L-2..L, r at L-2..L, A p at L-3..L-1, A r at L-2, L-1),
-// A p and A r at row L-1, A^2 p and the row's results at L-2; the edge lanes
-// compute A p at the column next to the wave from the two outside columns.
+// 18 per iteration against 22 for k_cgf.
+// Overlapped wave tiles as in k_cgs (lanes 1-60 of 4 columns each own 240), the
+// operator from differences across faces, zero-flux domain faces from the
+// negated coefficients around the grid (k_gcell): no lane and no edge has a case
+// of its own, and any nx fits.
 // The first sweep of pair t applies the stop and refresh tests to
 // gamma(t-1) as k_cgf does; when the pair's second step cannot be
 // taken (gamma1 or (p1, A p1) not positive, or t + 1 beyond the iteration
 // limit) the second sweep applies the first step only; when gamma1 already
 // meets the stop or refresh test, the second step is a null step and the
-// pair stops at t + 1 with p(t) kept.  Both sweeps run 3 waves per SIMD (768
-// blocks, one round): the second needs 172 VGPRs unconstrained (2 waves);
-// held to 168 it spills 4 and runs as fast as before its row windows were
-// indexed by row (the first sweep: 147 VGPRs, 4% faster).
-template <int FMT, bool UPD>
-__global__ __launch_bounds__(TBV) __attribute__((amdgpu_waves_per_eu(3))) void k_cgp(Geo g, int ty, int t, const float *__restrict__ rin,
-                                                         float *__restrict__ rout, const float *__restrict__ pin,
-                                                         float *__restrict__ pout, float *__restrict__ x,
-                                                         const tl_gc_t *__restrict__ gc, float hx, float hy,
-                                                         Ctrl *__restrict__ ctrl, const double *__restrict__ sin,
-                                                         unsigned nbin, double *__restrict__ sout)
+// pair stops at t + 1 with p(t) kept.
+// The first sweep is bound by memory latency and arithmetic (8192^2: 118 us, 5.7
+// TB/s of its 10 B; 136 with edge lanes that handled the columns beside a wave,
+// 147 registers instead of 134), the second by HBM (361 us, 4.8 TB/s of its 26
+// B; 344 with 256-column tiles, whose stores fill whole lines).  Below about
+// 2000^2 the pair is bound by latency, and more, smaller tiles and sums fetched
+// together help most: 1024^2 11.8 us per iteration against 41.9 in 32-row bands,
+// 512x400 13.1 against 34.6; 2047x1533 17.9 against 34.4 as two kernels per
+// iteration.
+template <int FMT, bool UPD, bool NT>
+__device__ __forceinline__ void cgp_sweep(const Geo &g, int t, const float *__restrict__ rin,
+                                          float *__restrict__ rout, const float *__restrict__ pin,
+                                          float *__restrict__ pout, float *__restrict__ x,
+                                          const tl_gc_t *__restrict__ gc, float hx, float hy, Ctrl *__restrict__ ctrl,
+                                          const double *__restrict__ sin, unsigned nbin, double *__restrict__ sout)
 {
-    constexpr int NS = UPD ? 1 : 6;
-    t = iter_of(t, ctrl);
-    if (t > ctrl->stop_iter) return;
-    const VCol<4> cl = vcolumn<4>(g, ty);
-    const int x0 = cl.x0, lane = cl.lane;
-    const bool eleft = lane == 0 && x0 > 0 && cl.active;
-    const bool eright = lane == 63 && x0 + 4 < g.nx && cl.active;
-    const bool eneed = eleft || eright;
-    const long eoff = lane == 0 ? -2 : 4;
-    const int hk = lane == 0 ? 1 : 0;
-    const bool at_left = x0 == 0, at_right = x0 + 4 >= g.nx;
-
-    auto load_batch = [&](FBatch<1> &B, int yb) {
-        const int yy = min(max(yb, 0), g.ny - 1);
-        const long i = at(g, cl.xl, yy);
-        vload<float, 4>(B.r[0], rin + i);
-        vload<float, 4>(B.p[0], pin + i);
-        {
-            typedef unsigned uv2 __attribute__((ext_vector_type(2)));
-            const uv2 w = *reinterpret_cast<const uv2 *>(gc + i);
-            B.g[0][0] = w[0];
-            B.g[0][1] = w[1];
-        }
-        if constexpr (UPD) {  // x of the row the sweep finishes, two rows behind
-            const int yx = min(max(yb - 2, 0), g.ny - 1);
-            vload<float, 4>(B.x[0], x + at(g, cl.xl, yx));
-        }
-        B.er[0][0] = B.er[0][1] = B.ep[0][0] = B.ep[0][1] = 0.f;
-        B.eg[0] = 0u;
-        if (eneed) {
-            typedef float fv2 __attribute__((ext_vector_type(2)));
-            const long ie = i + eoff;
-            const fv2 er = *reinterpret_cast<const fv2 *>(rin + ie);
-            const fv2 ep = *reinterpret_cast<const fv2 *>(pin + ie);
-            B.er[0][0] = er[0];
-            B.er[0][1] = er[1];
-            B.ep[0][0] = ep[0];
-            B.ep[0][1] = ep[1];
-            B.eg[0] = *reinterpret_cast<const unsigned *>(gc + ie);
-        }
+    constexpr int V = 4, NS = UPD ? 1 : 8;  // sums (the first sweep's six of eight)
+    struct Row {
+        float r[V], p[V], x[V];
+        GcRaw<V> g;
     };
-
+    if (t > ctrl->stop_iter) return;
+    int strip, band;
+    const Tiles &o = g.s32;
+    const bool tile = wave_tile(o, strip, band);
+    const int lane = threadIdx.x & 63;
+    const int xc = strip * TL_S32_COLS + (lane - 1) * V;
+    const bool act = tile && lane >= 1 && lane <= TL_S32_COLS / V && xc < g.nx;
+    const int y0 = band * o.ty, y1 = min(y0 + o.ty, g.ny);
+    // element of row y's storage: a uniform row start and a 32-bit lane offset;
+    // the lane beside the last one that owns cells reads its own columns (ring
+    // or padding, of which the next row's left padding is part), those past it
+    // the same again (never used)
+    const unsigned xo = (unsigned)(min(xc, (g.nx - 1) / V * V + V) + XCOL);
+    auto row = [&](auto *q, int y) { return q + (g.off - XCOL + (long)y * g.pitch) + xo; };
+    auto load_row = [&](Row &B, int L) {
+        vload<float, V, NT>(B.r, row(rin, L));
+        vload<float, V, NT>(B.p, row(pin, L));
+        gc_load_raw<V>(B.g, row(gc, L));
+        if constexpr (UPD)  // of the row the step finishes, inside the band only (row y0-3 may not exist)
+            if (L - 1 >= y0 && L - 1 < y1) vload<float, V, NT>(B.x, row(x, L - 1));
+    };
     // the band's first row is requested before the block sums the previous
     // sweep's partials
-    FBatch<1> Bs[2];
-    load_batch(Bs[0], cl.y0 - 2);
+    Row Bs[2];
+    if (tile) load_row(Bs[0], y0 - 2);
     // scalars of the pair, identical in every block; keep: the second step is
     // a null step that leaves p(t) as the direction
     double bd, a0 = 0.0, b0 = 0.0, a1 = 0.0;
@@ -2316,7 +2305,7 @@ __global__ __launch_bounds__(TBV) __attribute__((amdgpu_waves_per_eu(3))) void k
         double gam;
         if (sin) {
             double s1[1];
-            sum_partials<1, TBV>(sin, nbin, g.nbmax, s1);
+            sum_block_sums<1, TBV>(sin, nbin, s1);
             gam = s1[0];
         } else {
             gam = ctrl->rrs[(t - 1) & 1];  // after a start or an FP64 refresh
@@ -2333,8 +2322,8 @@ __global__ __launch_bounds__(TBV) __attribute__((amdgpu_waves_per_eu(3))) void k
         }
         if (why != WHY_NONE) return;
     } else {
-        double s6[6];
-        sum_partials<6, TBV>(sin, nbin, g.nbmax, s6);
+        double s6[8];
+        sum_block_sums<8, TBV>(sin, nbin, s6);
         const double gam = ctrl->rrs[(t - 1) & 1];
         bd = ctrl->beta;
         const double pap = s6[0], rap = s6[1], apap = s6[2], rar = s6[3], apar = s6[4], apa2p = s6[5];
@@ -2386,212 +2375,127 @@ __global__ __launch_bounds__(TBV) __attribute__((amdgpu_waves_per_eu(3))) void k
 #pragma unroll
     for (int k = 0; k < NS; ++k) acc[k] = 0.0;
 
-    {
-        const int y0 = cl.y0, y1 = cl.y1;
-        // Row windows indexed by row: row m keeps slot (m - y0 + 2) % 3 of the
-        // three-row windows and (m - y0 + 2) % 2 of the two-row ones while the
-        // walk moves on, and the walk is unrolled six rows at a time, so every
-        // index is a constant and no value moves between registers.  K = the
-        // step's row L minus (y0 - 2), modulo 6.
-        float P[3][4], Ph[3], Pf[2];     // p at L-2..L (own, hcol); fcol at L-1, L
-        float R[3][4], Rh[2];            // r at L-2..L; hcol at L-1, L
-        float N[3][4], Nh[2];            // A p at L-3..L-1; hcol at L-2, L-1
-        float AR[2][4];                  // A r at L-2, L-1
-        float Q[3][4], Qh[2];            // second sweep: p1 at L-3..L-1; hcol at L-2, L-1
-        float Gc[2][4], Gch[2], Gcf[2];  // coefficients of rows L-1, L (own, hcol, fcol)
-        unsigned Gw[2][2];               // their raw words (for the neighbour lanes)
-        float KX[2][5];                  // kx of rows L-2, L-1 (5 faces)
-        float KY[3][4], KYh[2];          // ky faces L-3|L-2, L-2|L-1, L-1|L; hcol of the last two
+    if (tile) {
+        // Row windows indexed by row, L - (y0 - 2) modulo 3 or 2, in a walk
+        // unrolled six rows at a time: every index is a constant and no value
+        // moves between registers.
+        float P[3][V];                   // p at rows L-2..L
+        float R[UPD ? 2 : 3][V];         // r at L-1, L (first sweep: L-2..L)
+        float N[UPD ? 1 : 3][V];         // first sweep: A p at L-3..L-1
+        float Q[UPD ? 3 : 1][V];         // second sweep: p1 at L-3..L-1
+        float R1[UPD ? 2 : 1][V];        // second sweep: r1 at L-2, L-1
+        float G[2][V];                   // coefficients of rows L-1, L
+        float KX[2][V + 1];              // face coefficients of rows L-2, L-1 (left of column 0 .. right of V-1)
+        float KY[3][V];                  // of the faces L-3|L-2, L-2|L-1, L-1|L
 #pragma unroll
-        for (int w = 0; w < 3; ++w) {
-            Ph[w] = 0.f;
+        for (int j = 0; j < V; ++j) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) P[w][j] = R[w][j] = N[w][j] = Q[w][j] = KY[w][j] = 0.f;
+            for (int w = 0; w < 3; ++w) {
+                P[w][j] = KY[w][j] = 0.f;
+                R[UPD ? w % 2 : w][j] = 0.f;
+                N[UPD ? 0 : w][j] = Q[UPD ? w : 0][j] = 0.f;
+            }
+#pragma unroll
+            for (int w = 0; w < 2; ++w) R1[UPD ? w : 0][j] = G[w][j] = KX[w][j] = KX[w][j + 1] = 0.f;
         }
+        // A applied to row c (rows dn below, up above): c + sum k (c - neighbour)
+        auto apply = [&](float (&q)[V], const float (&c)[V], const float (&dn)[V], const float (&up)[V],
+                         const float (&kx)[V + 1], const float (&kyd)[V], const float (&kyu)[V]) {
+            float D[V + 1];  // differences c[j] - c[j-1] across the V+1 vertical faces
+            D[0] = c[0] - dpp_up1f(c[V - 1]);
 #pragma unroll
-        for (int w = 0; w < 2; ++w) {
-            Pf[w] = Rh[w] = Nh[w] = Qh[w] = Gch[w] = Gcf[w] = KYh[w] = 0.f;
-            Gw[w][0] = Gw[w][1] = 0u;
+            for (int j = 1; j < V; ++j) D[j] = c[j] - c[j - 1];
+            D[V] = dpp_down1f(D[0]);
 #pragma unroll
-            for (int j = 0; j < 4; ++j) AR[w][j] = Gc[w][j] = 0.f;
-#pragma unroll
-            for (int j = 0; j < 5; ++j) KX[w][j] = 0.f;
-        }
-
-        auto nbr_l = [&](float src3, float c0, float hval) -> float {
-            float v = dpp_up1f(src3);
-            if (eleft) v = hval;
-            if (at_left) v = c0;
-            return v;
-        };
-        auto nbr_r = [&](float src0, float c3, float hval) -> float {
-            float v = dpp_down1f(src0);
-            if (eright) v = hval;
-            if (at_right) v = c3;
-            return v;
-        };
-
-        auto compute_row = [&](const FBatch<1> &B, int L, auto kc) {
-            constexpr int K = decltype(kc)::value;
-            // slots: three-row windows (row L: a, L-1: b, L-2: c), two-row
-            // windows (row L: e, L-1: f)
-            constexpr int a = K % 3, b = (K + 2) % 3, c = (K + 1) % 3, e = K % 2, f = (K + 1) % 2;
-            float gL[4];
-            const unsigned wL[2] = {B.g[0][0], B.g[0][1]};
-#pragma unroll
-            for (int k = 0; k < 2; ++k) {
-                gL[2 * k] = gc_word<FMT>(wL[k], 0);
-                gL[2 * k + 1] = gc_word<FMT>(wL[k], 1);
-            }
-            const float gLh = gc_word<FMT>(B.eg[0], hk), gLf = gc_word<FMT>(B.eg[0], 1 - hk);
-            float KXo;  // fcol|hcol face of row L-1
-            {
-                // faces of row L-1 (slot f) from its coefficients and row L's
-                float gl = gc_word<FMT>(dpp_up1u(Gw[f][1]), 1), gr = gc_word<FMT>(dpp_down1u(Gw[f][0]), 0);
-                if (eleft) gl = Gch[f];
-                if (eright) gr = Gch[f];
-                KX[f][0] = hx * (gl + Gc[f][0]);
-#pragma unroll
-                for (int j = 1; j < 4; ++j) KX[f][j] = hx * (Gc[f][j - 1] + Gc[f][j]);
-                KX[f][4] = hx * (Gc[f][3] + gr);
-                KXo = lane == 0 ? hx * (Gcf[f] + Gch[f]) : hx * (Gch[f] + Gcf[f]);
-#pragma unroll
-                for (int j = 0; j < 4; ++j) KY[a][j] = hy * (Gc[f][j] + gL[j]);
-                KYh[e] = hy * (Gch[f] + gLh);
-            }
-#pragma unroll
-            for (int j = 0; j < 4; ++j) Gc[e][j] = gL[j];
-            Gch[e] = gLh;
-            Gcf[e] = gLf;
-            Gw[e][0] = wL[0];
-            Gw[e][1] = wL[1];
-            // row L: r and p = r + beta p'
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                R[a][j] = B.r[0][j];
-                P[a][j] = __builtin_fmaf(beta, B.p[0][j], B.r[0][j]);
-            }
-            {
-                const float rh = B.er[0][hk], rf = B.er[0][1 - hk];
-                Ph[a] = __builtin_fmaf(beta, B.ep[0][hk], rh);
-                Pf[e] = __builtin_fmaf(beta, B.ep[0][1 - hk], rf);
-                Rh[e] = rh;
-            }
-            // A p and A r on row L-1.  The rows outside the grid were loaded
-            // clamped, so p and r there equal the edge row's, bit for bit:
-            // the zero-flux neighbours need no select here (A^2 p below, from
-            // A p of rows outside the grid, does)
-            if (L >= y0) {
-                const float pl = nbr_l(P[b][3], P[b][0], Ph[b]), pr = nbr_r(P[b][0], P[b][3], Ph[b]);
-                const float rl = nbr_l(R[b][3], R[b][0], Rh[f]), rr = nbr_r(R[b][0], R[b][3], Rh[f]);
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const float l = j > 0 ? P[b][j - 1] : pl;
-                    const float r = j < 3 ? P[b][j + 1] : pr;
-                    N[b][j] = smvp5f(P[b][j], l, r, P[c][j], P[a][j], KX[f][j], KX[f][j + 1], KY[b][j], KY[a][j]);
-                    if (!UPD || !TL_CGP_AP1) {
-                        const float lr = j > 0 ? R[b][j - 1] : rl;
-                        const float rrr = j < 3 ? R[b][j + 1] : rr;
-                        AR[f][j] =
-                            smvp5f(R[b][j], lr, rrr, R[c][j], R[a][j], KX[f][j], KX[f][j + 1], KY[b][j], KY[a][j]);
-                    }
-                }
-                {
-                    // A p at the column next to the wave (edge lanes)
-                    const float own = lane == 0 ? P[b][0] : P[b][3];
-                    const float l = lane == 0 ? Pf[f] : own, r = lane == 0 ? own : Pf[f];
-                    const float kxl = lane == 0 ? KXo : KX[f][4], kxr = lane == 0 ? KX[f][0] : KXo;
-                    Nh[f] = smvp5f(Ph[b], l, r, Ph[c], Ph[a], kxl, kxr, KYh[f], KYh[e]);
-                }
-                if constexpr (UPD && TL_CGP_AP1) {
-                    // p1 = r1 + beta0 p on row L-1 (and the next column), r1 = r - alpha0 A p
-#pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        Q[b][j] = __builtin_fmaf(fb0, P[b][j], __builtin_fmaf(-fa0, N[b][j], R[b][j]));
-                    Qh[f] = __builtin_fmaf(fb0, Ph[b], __builtin_fmaf(-fa0, Nh[f], Rh[f]));
-                }
-            }
-            // A^2 p on row L-2 and the row's sums or updates (row L-3: slot a
-            // of the three-row windows that end at L-1)
-            if (L >= y0 + 2) {
-                const int y = L - 2;
-                if (y < y1 && cl.active) {
-                    const bool ybot = y <= 0, ytop = y >= g.ny - 1;
-                    const float nl = nbr_l(N[c][3], N[c][0], Nh[e]), nr = nbr_r(N[c][0], N[c][3], Nh[e]);
-                    float ql = 0.f, qr = 0.f;
-                    if constexpr (UPD && TL_CGP_AP1) {
-                        ql = nbr_l(Q[c][3], Q[c][0], Qh[e]);
-                        qr = nbr_r(Q[c][0], Q[c][3], Qh[e]);
-                    }
-                    (void)ql;
-                    (void)qr;
-                    float o_r[4], o_p[4], o_x[4];
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        if constexpr (UPD && TL_CGP_AP1) {
-                            // the second step as the fused kernel takes a step:
-                            // A p1 by the stencil of p1
-                            const float cq = Q[c][j];
-                            const float l = j > 0 ? Q[c][j - 1] : ql;
-                            const float r = j < 3 ? Q[c][j + 1] : qr;
-                            const float d = ybot ? cq : Q[a][j];
-                            const float u = ytop ? cq : Q[b][j];
-                            const float ap1 = smvp5f(cq, l, r, d, u, KX[e][j], KX[e][j + 1], KY[c][j], KY[b][j]);
-                            const float r1 = __builtin_fmaf(-fa0, N[c][j], R[c][j]);
-                            o_x[j] = __builtin_fmaf(fa1, cq, __builtin_fmaf(fa0, P[c][j], B.x[0][j]));
-                            o_r[j] = __builtin_fmaf(-fa1, ap1, r1);
-                            o_p[j] = keep ? P[c][j] : cq;
-                            acc[0] = __builtin_fma((double)o_r[j], (double)o_r[j], acc[0]);
-                            continue;
-                        }
-                        const float cn = N[c][j];
-                        const float l = j > 0 ? N[c][j - 1] : nl;
-                        const float r = j < 3 ? N[c][j + 1] : nr;
-                        const float d = ybot ? cn : N[a][j];
-                        const float u = ytop ? cn : N[b][j];
-                        const float a2p = smvp5f(cn, l, r, d, u, KX[e][j], KX[e][j + 1], KY[c][j], KY[b][j]);
-                        const float pv = P[c][j], apv = N[c][j], rv = R[c][j], arv = AR[e][j];
-                        if constexpr (!UPD) {
-                            // a product of two FP32 values is exact in FP64, so
-                            // the fused multiply-add rounds as acc + a * b does
-                            const double ap = (double)apv, rd = (double)rv, ard = (double)arv;
-                            acc[0] = __builtin_fma((double)pv, ap, acc[0]);
-                            acc[1] = __builtin_fma(rd, ap, acc[1]);
-                            acc[2] = __builtin_fma(ap, ap, acc[2]);
-                            acc[3] = __builtin_fma(rd, ard, acc[3]);
-                            acc[4] = __builtin_fma(ap, ard, acc[4]);
-                            acc[5] = __builtin_fma(ap, (double)a2p, acc[5]);
-                            (void)o_r;
-                            (void)o_p;
-                            (void)o_x;
-                        } else {
-                            const float r1 = __builtin_fmaf(-fa0, apv, rv);
-                            const float p1 = __builtin_fmaf(fb0, pv, r1);
-                            const float ar1 = __builtin_fmaf(-fa0, a2p, arv);
-                            const float ap1 = __builtin_fmaf(fb0, apv, ar1);
-                            o_x[j] = __builtin_fmaf(fa1, p1, __builtin_fmaf(fa0, pv, B.x[0][j]));
-                            o_r[j] = __builtin_fmaf(-fa1, ap1, r1);
-                            o_p[j] = keep ? pv : p1;
-                            acc[0] = __builtin_fma((double)o_r[j], (double)o_r[j], acc[0]);
-                        }
-                    }
-                    if constexpr (UPD) {
-                        const long i = at(g, x0, y);
-                        vstore<float, 4>(rout + i, o_r);
-                        vstore<float, 4>(pout + i, o_p);
-                        vstore<float, 4>(x + i, o_x);
-                    }
-                }
+            for (int j = 0; j < V; ++j) {
+                float s = kx[j] * D[j];
+                s = __builtin_fmaf(-kx[j + 1], D[j + 1], s);
+                s = __builtin_fmaf(kyd[j], c[j] - dn[j], s);
+                s = __builtin_fmaf(kyu[j], c[j] - up[j], s);
+                q[j] = c[j] + s;
             }
         };
-        // rows y0-2 .. y1+1, the next row's loads issued before the current
-        // row is computed (the first one above; two rows ahead in the first
-        // sweep measured no faster: it is bound by its arithmetic)
         auto step = [&](auto kc, int L) -> bool {
             constexpr int K = decltype(kc)::value;
+            // slots: rows L, L-1, L-2 (and L-3 = L) of the three-row windows, L
+            // and L-1 of the two-row ones; r's windows ra, rb
+            constexpr int a = K % 3, b = (K + 2) % 3, c = (K + 1) % 3, e = K % 2, f = (K + 1) % 2;
+            constexpr int ra = UPD ? e : a, rb = UPD ? f : b;
             if (L > y1 + 1) return false;
-            if (L + 1 <= y1 + 1) load_batch(Bs[(K + 1) % 2], L + 1);
-            compute_row(Bs[K % 2], L, kc);
+            if (L + 1 <= y1 + 1) load_row(Bs[f], L + 1);
+            const Row &B = Bs[e];
+            float gL[V];
+            gc_unpack<V, FMT>(gL, B.g);
+            KX[f][0] = hx * (dpp_up1f(G[f][V - 1]) + G[f][0]);
+#pragma unroll
+            for (int j = 1; j < V; ++j) KX[f][j] = hx * (G[f][j - 1] + G[f][j]);
+            KX[f][V] = dpp_down1f(KX[f][0]);
+#pragma unroll
+            for (int j = 0; j < V; ++j) {
+                KY[a][j] = hy * (G[f][j] + gL[j]);
+                G[e][j] = gL[j];
+                R[ra][j] = B.r[j];
+                P[a][j] = __builtin_fmaf(beta, B.p[j], B.r[j]);
+            }
+            if (L < y0) return true;
+            // A p on row L-1
+            const bool own1 = act && L - 1 >= y0 && L - 1 < y1;
+            if constexpr (!UPD) {
+                float ar[V];
+                apply(N[b], P[b], P[c], P[a], KX[f], KY[b], KY[a]);
+                apply(ar, R[b], R[c], R[a], KX[f], KY[b], KY[a]);
+                if (own1) {
+                    // a product of two FP32 values is exact in FP64, so the
+                    // fused multiply-add rounds as acc + a * b does
+#pragma unroll
+                    for (int j = 0; j < V; ++j) {
+                        const double ap = (double)N[b][j], rd = (double)R[b][j], ard = (double)ar[j];
+                        acc[0] = __builtin_fma((double)P[b][j], ap, acc[0]);
+                        acc[1] = __builtin_fma(rd, ap, acc[1]);
+                        acc[2] = __builtin_fma(ap, ap, acc[2]);
+                        acc[3] = __builtin_fma(rd, ard, acc[3]);
+                        acc[4] = __builtin_fma(ap, ard, acc[4]);
+                    }
+                }
+                if (L < y0 + 2) return true;
+                // A^2 p on row L-2
+                float a2p[V];
+                apply(a2p, N[c], N[a], N[b], KX[e], KY[c], KY[b]);
+                if (act) {
+#pragma unroll
+                    for (int j = 0; j < V; ++j)
+                        acc[5] = __builtin_fma((double)N[c][j], (double)a2p[j], acc[5]);
+                }
+            } else {
+                float ap[V];
+                apply(ap, P[b], P[c], P[a], KX[f], KY[b], KY[a]);
+#pragma unroll
+                for (int j = 0; j < V; ++j) {
+                    R1[f][j] = __builtin_fmaf(-fa0, ap[j], R[rb][j]);
+                    Q[b][j] = __builtin_fmaf(fb0, P[b][j], R1[f][j]);
+                }
+                if (own1) {
+                    float o_p[V], o_x[V];
+#pragma unroll
+                    for (int j = 0; j < V; ++j) {
+                        o_x[j] = __builtin_fmaf(fa1, Q[b][j], __builtin_fmaf(fa0, P[b][j], B.x[j]));
+                        o_p[j] = keep ? P[b][j] : Q[b][j];
+                    }
+                    vstore<float, V, NT>(row(pout, L - 1), o_p);
+                    vstore<float, V, NT>(row(x, L - 1), o_x);
+                }
+                if (L < y0 + 2) return true;
+                // A p1 and r(t+1) on row L-2
+                float ap1[V], o_r[V];
+                apply(ap1, Q[c], Q[a], Q[b], KX[e], KY[c], KY[b]);
+#pragma unroll
+                for (int j = 0; j < V; ++j) o_r[j] = __builtin_fmaf(-fa1, ap1[j], R1[e][j]);
+                if (act) {
+                    vstore<float, V, NT>(row(rout, L - 2), o_r);
+#pragma unroll
+                    for (int j = 0; j < V; ++j) acc[0] = __builtin_fma((double)o_r[j], (double)o_r[j], acc[0]);
+                }
+            }
             return true;
         };
         for (int L = y0 - 2; L <= y1 + 1; L += 6) {
@@ -2603,7 +2507,25 @@ __global__ __launch_bounds__(TBV) __attribute__((amdgpu_waves_per_eu(3))) void k
             if (!step(std::integral_constant<int, 5>{}, L + 5)) break;
         }
     }
-    write_partials<NS, TBV>(acc, sout, g.nbmax);
+    write_block_sums<NS, TBV>(acc, sout);
+}
+
+#define TL_CGP_ARGS                                                                                               \
+    Geo g, int t, const float *__restrict__ rin, float *__restrict__ rout, const float *__restrict__ pin,         \
+        float *__restrict__ pout, float *__restrict__ x, const tl_gc_t *__restrict__ gc, float hx, float hy,      \
+        Ctrl *__restrict__ ctrl, const double *__restrict__ sin, unsigned nbin, double *__restrict__ sout
+
+template <int FMT, bool UPD>
+__global__ __launch_bounds__(TBV) __attribute__((amdgpu_waves_per_eu(3))) void k_cgp(TL_CGP_ARGS)
+{
+    cgp_sweep<FMT, UPD, true>(g, t, rin, rout, pin, pout, x, gc, hx, hy, ctrl, sin, nbin, sout);
+}
+
+// the same with cached access, for grids whose arrays fit the Infinity Cache
+template <int FMT, bool UPD>
+__global__ __launch_bounds__(TBV) __attribute__((amdgpu_waves_per_eu(3))) void k_cgp_cached(TL_CGP_ARGS)
+{
+    cgp_sweep<FMT, UPD, false>(g, t, rin, rout, pin, pout, x, gc, hx, hy, ctrl, sin, nbin, sout);
 }
 
 // The four sums k_cgf needs at its first iteration and after an FP64 refresh,
@@ -3617,11 +3539,10 @@ __global__ __launch_bounds__(NW * 64) void k_steps(Geo g, int gx, int t, int n, 
 
 // ------------------------------------------------------ mixed precision
 
-// cell coefficient of the inner CG over the whole allocation:
+// cell coefficient of the inner CG:
 // gc = 1/w with w = density (coefficient 1) or 1/density (CG.jl:56-58),
 // rounded to FP32, multiplied by scale (a power of two: exact) and rounded to
-// the storage format, to nearest with ties to even; cells without a density
-// (padding) get 0
+// the storage format, to nearest with ties to even
 template <int FMT>
 __device__ __forceinline__ tl_gc_t gc_store(float f)
 {
@@ -3643,13 +3564,22 @@ __device__ __forceinline__ float gc_value(double d, int coefficient)
     return coefficient == 2 ? (float)d : (d != 0.0 ? (float)(1.0 / d) : 0.0f);
 }
 
+// Like g64 (k_init_coef): 1/w over the interior, its negative, mirrored, in the
+// ring of cells around it, and 0 in the other halo and padding cells.
 template <int FMT>
-__global__ __launch_bounds__(TB) void k_gcell(const double *__restrict__ rho, tl_gc_t *__restrict__ gc, size_t n,
+__global__ __launch_bounds__(TB) void k_gcell(Geo g, const double *__restrict__ rho, tl_gc_t *__restrict__ gc,
                                               int coefficient, float scale)
 {
-    const size_t i = (size_t)blockIdx.x * TB + threadIdx.x;
-    if (i >= n) return;
-    gc[i] = gc_store<FMT>(gc_value(rho[i], coefficient) * scale);
+    const int col = blockIdx.x * TB + threadIdx.x, j = blockIdx.y;
+    if (col >= g.pitch) return;
+    const int x = col - XCOL, y = j - g.hd;
+    const int xc = min(max(x, 0), g.nx - 1), yc = min(max(y, 0), g.ny - 1);
+    float f = 0.0f;
+    if (abs(x - xc) <= 1 && abs(y - yc) <= 1) {
+        f = gc_value(rho[at(g, xc, yc)], coefficient) * scale;
+        if (x != xc || y != yc) f = -f;
+    }
+    gc[(long)j * g.pitch + col] = gc_store<FMT>(f);
 }
 
 // per-block minimum and maximum of gc over the cells with a density (grid-
@@ -4220,7 +4150,6 @@ hipError_t launch_acc64(tl_ctx *c, double *u, double *d)
 hipError_t launch_ir_prepare(tl_ctx *c, double rx, double ry, int coefficient)
 {
     const size_t n = c->g.elems;
-    const unsigned nb = (unsigned)((n + TB - 1) / TB);
     int fmt = GC_BF16;
     float scale = 1.0f;
 #if TL_GC16
@@ -4245,10 +4174,11 @@ hipError_t launch_ir_prepare(tl_ctx *c, double rx, double ry, int coefficient)
         }
     }
 #endif
+    const dim3 all((unsigned)((c->g.pitch + TB - 1) / TB), c->g.Y);
     if (fmt == GC_F16)
-        k_gcell<GC_F16><<<nb, TB, 0, c->stream>>>(c->f[TL_F_DENSITY], c->gcell, n, coefficient, scale);
+        k_gcell<GC_F16><<<all, TB, 0, c->stream>>>(c->g, c->f[TL_F_DENSITY], c->gcell, coefficient, scale);
     else
-        k_gcell<GC_BF16><<<nb, TB, 0, c->stream>>>(c->f[TL_F_DENSITY], c->gcell, n, coefficient, 1.0f);
+        k_gcell<GC_BF16><<<all, TB, 0, c->stream>>>(c->g, c->f[TL_F_DENSITY], c->gcell, coefficient, 1.0f);
     c->gc_fmt = fmt;
     c->gc_scale = scale;
     // kx = hx (gc(x-1) + gc(x)): the scale of the stored gc is divided out of hx, hy
@@ -4283,29 +4213,33 @@ hipError_t launch_cgf(tl_ctx *c, int t, int tref)
 }
 
 // pairs of FP32 inner CG iterations (k_cgp): after iteration T (even), r(T)
-// and p(T) in buffer (T / 2) & 1; the six sums of a pair's first sweep in
-// part_f[0 .. 6 stride), the residual sum of its second in part_f[6 stride ..)
+// and p(T) in buffer (T / 2) & 1; the sums of a pair's first sweep in
+// part_f[0 .. 8 blocks), the residual sum of its second behind them
 float *cgp_r(tl_ctx *c, int T) { return ((T >> 1) & 1) ? c->r32b : c->r32; }
 float *cgp_p(tl_ctx *c, int T) { return ((T >> 1) & 1) ? c->p32b : c->p32; }
 
 // the pair t, t+1 (t odd); first: the first pair after a start or an FP64
 // refresh, whose gamma(t-1) is in Ctrl::rrs
-hipError_t launch_cgp(tl_ctx *c, int t, bool first, int tref)
+hipError_t launch_cgp(tl_ctx *c, int t, bool first)
 {
-    double *const pg = c->part_f, *const pu = c->part_f + 6 * stride(c);
-    const unsigned nb = nbf(c);
+    const unsigned nb = (unsigned)c->g.s32.blocks;
+    double *const pg = c->part_f, *const pu = c->part_f + (size_t)8 * nb;
     const bool fp16 = c->gc_fmt == GC_F16;
+    // r, r', p, p', x in FP32 and the 16-bit coefficient
+    const bool nt = c->g.elems * (5 * sizeof(float) + sizeof(tl_gc_t)) > TL_CACHE_BYTES;
     bool prof = prof_start(c, TL_K_CGP_G32);
-    auto kg = fp16 ? k_cgp<GC_F16, false> : k_cgp<GC_BF16, false>;
-    kg<<<nb, TBV, 0, c->stream>>>(c->g, c->g.tyf, targ(t, tref), cgp_r(c, t - 1), nullptr, cgp_p(c, t - 1), nullptr,
-                                  nullptr, c->gcell, c->hx32, c->hy32, c->ctrl, first ? nullptr : pu, nb, pg);
+    auto kg = nt ? (fp16 ? k_cgp<GC_F16, false> : k_cgp<GC_BF16, false>)
+                 : (fp16 ? k_cgp_cached<GC_F16, false> : k_cgp_cached<GC_BF16, false>);
+    kg<<<nb, TBV, 0, c->stream>>>(c->g, t, cgp_r(c, t - 1), nullptr, cgp_p(c, t - 1), nullptr, nullptr, c->gcell,
+                                  c->hx32, c->hy32, c->ctrl, first ? nullptr : pu, nb, pg);
     if (prof) prof_stop(c);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     prof = prof_start(c, TL_K_CGP_U32);
-    auto ku = fp16 ? k_cgp<GC_F16, true> : k_cgp<GC_BF16, true>;
-    ku<<<nb, TBV, 0, c->stream>>>(c->g, c->g.tyf, targ(t, tref), cgp_r(c, t - 1), cgp_r(c, t + 1), cgp_p(c, t - 1),
-                                  cgp_p(c, t + 1), c->x32, c->gcell, c->hx32, c->hy32, c->ctrl, pg, nb, pu);
+    auto ku = nt ? (fp16 ? k_cgp<GC_F16, true> : k_cgp<GC_BF16, true>)
+                 : (fp16 ? k_cgp_cached<GC_F16, true> : k_cgp_cached<GC_BF16, true>);
+    ku<<<nb, TBV, 0, c->stream>>>(c->g, t, cgp_r(c, t - 1), cgp_r(c, t + 1), cgp_p(c, t - 1), cgp_p(c, t + 1), c->x32,
+                                  c->gcell, c->hx32, c->hy32, c->ctrl, pg, nb, pu);
     if (prof) prof_stop(c);
     return hipGetLastError();
 }
