@@ -25,8 +25,9 @@
 // (v_mfma_f32_16x16x16_bf16: a wave computes 16 pixels x 16 output channels
 // per instruction, K = 16 input channels of one tap).  The input-gradient of
 // a convolution is the same kernel on the output-gradient with flipped,
-// transposed weights.  Weight gradients are FP32 sums over pixels (per-block
-// partials reduced in fixed order), then Adam on the FP32 master weights.
+// transposed weights.  Weight gradients are FP32 sums over pixels on the matrix
+// cores (per-block partials reduced in fixed order), then Adam on the FP32
+// master weights.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -64,6 +65,13 @@ typedef uint16_t bf16;
 #endif
 #ifndef TL_CONV_WPE2
 #define TL_CONV_WPE2 2
+#endif
+
+// blocks per launch of the weight gradients (chunks of tiles x channel groups).
+// 16 crops of 128^2, 48 -> 16 channels, k_dw + k_dw_reduce: 512 blocks 30 + 8 us,
+// 256 34 + 6, 1024 37 + 12.
+#ifndef TL_DW_BLOCKS
+#define TL_DW_BLOCKS 512
 #endif
 
 constexpr int NL = 11;
@@ -314,87 +322,187 @@ __global__ void k_up_back(TV in, TV out, int C)
 }
 
 // dz = (g [+ pool_back(gp)]) * (y > 0 if relu): the gradient at a conv's
-// pre-activation; gp (H/2) is the gradient of the 2x2 pool that reads y
+// pre-activation, and the zero border around it; gp (H/2) is the gradient of
+// the 2x2 pool that reads y.  8 channels (16 bytes) per item.
 __global__ void k_dz(TV g, TV gp, int has_gp, TV y, int relu, TV dz, int C)
 {
-    const long n = (long)dz.B * dz.H * dz.W * C;
+    typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+    const int C8 = C / 8, H2 = dz.H + 2, W2 = dz.W + 2;
+    const long n = (long)dz.B * H2 * W2 * C8;
     for (long t = (long)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (long)gridDim.x * blockDim.x) {
-    const int c = (int)(t % C);
-    long r = t / C;
-    const int x = (int)(r % dz.W);
-    r /= dz.W;
-    const int yy = (int)(r % dz.H);
-    const int b = (int)(r / dz.H);
-    float v = bf2f(g.p[g.idx(b, yy, x) + c]);
-    if (has_gp) v += 0.25f * bf2f(gp.p[gp.idx(b, yy / 2, x / 2) + c]);
-    if (relu && !(bf2f(y.p[y.idx(b, yy, x) + c]) > 0.f)) v = 0.f;
-    dz.p[dz.idx(b, yy, x) + c] = f2bf(v);
+        const int c = (int)(t % C8) * 8;
+        long r = t / C8;
+        const int x = (int)(r % W2) - 1;
+        r /= W2;
+        const int yy = (int)(r % H2) - 1;
+        const int b = (int)(r / H2);
+        u4 o = {0, 0, 0, 0};
+        if (x >= 0 && x < dz.W && yy >= 0 && yy < dz.H) {
+            const u4 vg = *(const u4 *)(g.p + g.idx(b, yy, x) + c);
+            u4 vp = {0, 0, 0, 0}, vy = {0, 0, 0, 0};
+            if (has_gp) vp = *(const u4 *)(gp.p + gp.idx(b, yy / 2, x / 2) + c);
+            if (relu) vy = *(const u4 *)(y.p + y.idx(b, yy, x) + c);
+            auto one = [&](uint32_t gw, uint32_t pw, uint32_t yw) -> uint32_t {
+                float v = bf2f((bf16)gw);
+                if (has_gp) v += 0.25f * bf2f((bf16)pw);
+                if (relu && !(bf2f((bf16)yw) > 0.f)) v = 0.f;
+                return f2bf(v);
+            };
+#pragma unroll
+            for (int h = 0; h < 4; ++h)
+                o[h] = one(vg[h] & 0xffffu, vp[h] & 0xffffu, vy[h] & 0xffffu) |
+                       one(vg[h] >> 16, vp[h] >> 16, vy[h] >> 16) << 16;
+        }
+        *(u4 *)(dz.p + dz.idx(b, yy, x) + c) = o;
     }
 }
 
-// weight-gradient partials: block (chunk) sums over its pixels, thread = one
-// (co, ci) pair with its 9 taps: part[chunk][tap][co][ci]
-__global__ __launch_bounds__(256) void k_dw(TV x, TV dz, int cinp, int coutp, int px_per_chunk,
+// Weight and bias gradients: dw[tap][co][ci] = sum over pixels of dz[p][co]
+// x[p + tap][ci], a contraction over pixels on the matrix cores (A = dz: 16 co
+// x 16 pixels, B = x: 16 pixels x 16 ci; the bias is B = 1).  A block takes 16
+// output and 16 NCI input channels and, tile by tile (4 RW rows of 32 columns,
+// one quarter of the rows per wave), keeps the 9 taps' sums in registers.
+// A lane's 4 pixels of a product lie 8 columns apart (segments j = 0..3 of a
+// tile's row), so a tile's LDS image is [channel][row][column s of a segment]
+// [j] and a tap's shift by a row or a column moves by whole 8-byte vectors;
+// s = 0 and 9 of x are the columns beside a segment.  The transposition from
+// channels to pixels is that of 4x4 values in a thread's registers.  Rows and
+// columns past the image read the tensors' zero border.  The waves' sums are
+// added in order and stored as the block's partials: part[chunk][9 npair
+// weights, then coutp biases], npair = cinp coutp.
+// Bound by the latency of load, transpose and product within a tile (2 to 4
+// blocks per CU overlap it).  16 crops of 128^2: 16 -> 16 channels 15 us, 48 -> 16
+// 30 us, 64 -> 64 at 32^2 16 us; one thread per (co, ci) walking 1024 pixels took
+// 626, 1299 and 700 us, and a block per co for the bias another 494 us at 128^2.
+// Relative error against FP64 7.5e-8 (was 3.8e-7), of the bias 2.3e-8 (4.1e-8).
+template <int NCI, int RW>
+__global__ __launch_bounds__(256) void k_dw(TV x, TV dz, int cinp, int coutp, int ntx, int nty, int ntile,
                                             float *__restrict__ part)
 {
-    const int pair = blockIdx.x * 256 + threadIdx.x;
-    const int chunk = blockIdx.y;
-    const int npair = cinp * coutp;
-    const long npx = (long)x.B * x.H * x.W;
-    float acc[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-    const int co = pair / cinp, ci = pair % cinp;
-    if (pair < npair) {
-        const long p0 = (long)chunk * px_per_chunk;
-        const long p1 = min(p0 + px_per_chunk, npx);
-        for (long p = p0; p < p1; ++p) {
-            const int xx = (int)(p % x.W);
-            const long r = p / x.W;
-            const int yy = (int)(r % x.H);
-            const int b = (int)(r / x.H);
-            const float g = bf2f(dz.p[dz.idx(b, yy, xx) + co]);
+    constexpr int S = 8, ROWS = 4 * RW;
+    // vectors per channel, 4 modulo 16: a fragment's 16 channels x 4 vectors
+    // then spread over all banks
+    constexpr int XS = (ROWS + 2) * (S + 2), DS = ROWS * S + 4;
+    static_assert(XS % 16 == 4 && DS % 16 == 4, "LDS strides");
+    static_assert((size_t)16 * NCI * XS * sizeof(s4) >= (size_t)9 * NCI * 64 * sizeof(f4), "wave sums fit the x tile");
+    __shared__ __attribute__((aligned(16))) s4 xl[16 * NCI * XS];
+    __shared__ __attribute__((aligned(16))) s4 dl[16 * DS];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int i = lane & 15, kq = lane >> 4;
+    const int ncig = cinp / (16 * NCI);
+    const int co0 = (int)blockIdx.y / ncig * 16, cig = (int)blockIdx.y % ncig, ci0 = cig * 16 * NCI;
+    const s4 ones = {0x3F80, 0x3F80, 0x3F80, 0x3F80};
+    f4 acc[NCI][9], accb = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int tap = 0; tap < 9; ++tap) {
-                const int dy = tap / 3 - 1, dx = tap % 3 - 1;
-                acc[tap] += g * bf2f(x.p[x.idx(b, yy + dy, xx + dx) + ci]);
-            }
+    for (int n = 0; n < NCI; ++n)
+#pragma unroll
+        for (int t = 0; t < 9; ++t) acc[n][t] = f4{0.f, 0.f, 0.f, 0.f};
+    for (int tile = blockIdx.x; tile < ntile; tile += gridDim.x) {
+        const int tx = tile % ntx, q2 = tile / ntx, ty = q2 % nty, b = q2 / nty;
+        const int x0 = tx * 4 * S, y0 = ty * ROWS;
+        for (int v = threadIdx.x; v < 4 * NCI * XS; v += 256) {
+            const int c = v % (4 * NCI) * 4, q = v / (4 * NCI), s = q % (S + 2), r = q / (S + 2);
+            const int y = min(y0 + r - 1, x.H);
+            s4 f[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                f[j] = *(const s4 *)(x.p + x.idx(b, y, min(x0 + j * S + s - 1, x.W)) + ci0 + c);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) xl[(c + k) * XS + q] = s4{f[0][k], f[1][k], f[2][k], f[3][k]};
         }
+        for (int v = threadIdx.x; v < 4 * ROWS * S; v += 256) {
+            const int c = v % 4 * 4, q = v / 4, s = q % S, r = q / S;
+            const int y = min(y0 + r, dz.H);
+            s4 f[4];
 #pragma unroll
-        for (int tap = 0; tap < 9; ++tap)
-            part[((long)chunk * 9 + tap) * npair + (long)co * cinp + ci] = acc[tap];
+            for (int j = 0; j < 4; ++j)
+                f[j] = *(const s4 *)(dz.p + dz.idx(b, y, min(x0 + j * S + s, dz.W)) + co0 + c);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) dl[(c + k) * DS + q] = s4{f[0][k], f[1][k], f[2][k], f[3][k]};
+        }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < S / 4; ++q) {
+            s4 d[RW];
+#pragma unroll
+            for (int r = 0; r < RW; ++r) {
+                d[r] = dl[i * DS + (wave * RW + r) * S + 4 * q + kq];
+                accb = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(d[r], ones, accb, 0, 0, 0);
+            }
+            // each row of x is read once for the (up to) three taps' rows that use it
+#pragma unroll
+            for (int n = 0; n < NCI; ++n)
+#pragma unroll
+                for (int xr = 0; xr < RW + 2; ++xr)
+#pragma unroll
+                    for (int dx = 0; dx < 3; ++dx) {
+                        const s4 fx = xl[(n * 16 + i) * XS + (wave * RW + xr) * (S + 2) + 4 * q + kq + dx];
+#pragma unroll
+                        for (int dy = 0; dy < 3; ++dy)
+                            if (xr - dy >= 0 && xr - dy < RW)
+                                acc[n][3 * dy + dx] =
+                                    __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(d[xr - dy], fx, acc[n][3 * dy + dx], 0, 0, 0);
+                    }
+        }
+        __syncthreads();
     }
+    // the waves' sums, in order; lane (i, kq) holds co = 4 kq .. 4 kq + 3 of ci = i
+    f4 *const sh = (f4 *)xl, *const shb = (f4 *)dl;
+    for (int w = 1; w < 4; ++w) {
+        if (wave == w) {
+#pragma unroll
+            for (int n = 0; n < NCI; ++n)
+#pragma unroll
+                for (int t = 0; t < 9; ++t) sh[(n * 9 + t) * 64 + lane] = acc[n][t];
+            shb[lane] = accb;
+        }
+        __syncthreads();
+        if (wave == 0) {
+#pragma unroll
+            for (int n = 0; n < NCI; ++n)
+#pragma unroll
+                for (int t = 0; t < 9; ++t) acc[n][t] += sh[(n * 9 + t) * 64 + lane];
+            accb += shb[lane];
+        }
+        __syncthreads();
+    }
+    if (wave != 0) return;
+    const long npair = (long)cinp * coutp;
+    float *const out = part + (long)blockIdx.x * (9 * npair + coutp);
+#pragma unroll
+    for (int n = 0; n < NCI; ++n)
+#pragma unroll
+        for (int t = 0; t < 9; ++t)
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                out[t * npair + (long)(co0 + 4 * kq + k) * cinp + ci0 + n * 16 + i] = acc[n][t][k];
+    if (cig == 0 && i == 0)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) out[9 * npair + co0 + 4 * kq + k] = accb[k];
 }
 
-// fixed-order sum of the partials into dw[tap][co][ci]
-__global__ void k_dw_reduce(const float *__restrict__ part, int nchunk, long n, float *__restrict__ dw)
+// fixed-order sum of the chunks' partials into dw[tap][co][ci] and db[co], in
+// FP64: a block sums 16 of them, 16 threads each (every 16th chunk)
+__global__ __launch_bounds__(256) void k_dw_reduce(const float *__restrict__ part, int nchunk, long nw, int coutp,
+                                                   int co_real, float *__restrict__ dw, float *__restrict__ db)
 {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    float s = 0.f;
-    for (int c = 0; c < nchunk; ++c) s += part[(long)c * n + i];
-    dw[i] = s;
-}
-
-// bias gradient: db[co] = sum over pixels of dz[.., co] (one block per co)
-__global__ __launch_bounds__(256) void k_db(TV dz, int co_real, float *__restrict__ db)
-{
-    const int co = blockIdx.x;
-    const long npx = (long)dz.B * dz.H * dz.W;
-    float s = 0.f;
-    for (long p = threadIdx.x; p < npx; p += 256) {
-        const int xx = (int)(p % dz.W);
-        const long r = p / dz.W;
-        const int yy = (int)(r % dz.H);
-        const int b = (int)(r / dz.H);
-        s += bf2f(dz.p[dz.idx(b, yy, xx) + co]);
-    }
-    __shared__ float sh[256];
+    const int e = threadIdx.x & 15, grp = threadIdx.x >> 4;
+    const long i = (long)blockIdx.x * 16 + e, n = nw + coutp;  // both multiples of 16
+    double s = 0.0;
+#pragma unroll 8
+    for (int c = grp; c < nchunk; c += 16) s += (double)part[(long)c * n + i];
+    __shared__ double sh[256];
     sh[threadIdx.x] = s;
     __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
+    for (int o = 128; o >= 16; o >>= 1) {
         if (threadIdx.x < o) sh[threadIdx.x] += sh[threadIdx.x + o];
         __syncthreads();
     }
-    if (threadIdx.x == 0) db[co] = co < co_real ? sh[0] : 0.f;
+    if (threadIdx.x >= 16) return;
+    if (i < nw)
+        dw[i] = (float)sh[e];
+    else
+        db[i - nw] = i - nw < co_real ? (float)sh[e] : 0.f;
 }
 
 // FP32 master weights -> BF16 [tap][co][ci] and flipped/transposed
@@ -963,15 +1071,20 @@ static int back_layer(tl_ctx *c, Unet *u, int l, const TV &g, const TV &gp, int 
     Acts &a = u->acts;
     const LayerDef &L = LAY[l];
     TV dz{a.dz.p, y.B, y.H, y.W, L.coutp, 0};
-    const long npx = (long)y.B * y.H * y.W;
-    // the buffer is shared by all layers: clear it so its border is zero
-    UCHK(c, hipMemsetAsync(a.dz.p, 0, (size_t)y.B * (y.H + 2) * (y.W + 2) * L.coutp * sizeof(bf16), c->stream));
-    k_dz<<<gs_blocks(npx * L.coutp), 256, 0, c->stream>>>(g, gp, has_gp, y, L.relu, dz, L.coutp);
-    // weight gradient: partials over pixel chunks, then a fixed-order sum
-    const int px_chunk = 1024;
-    const int nchunk = (int)((npx + px_chunk - 1) / px_chunk);
-    const long npair = (long)L.cinp * L.coutp;
-    const size_t need = (size_t)nchunk * 9 * npair;
+    k_dz<<<gs_blocks((long)y.B * (y.H + 2) * (y.W + 2) * (L.coutp / 8)), 256, 0, c->stream>>>(g, gp, has_gp, y, L.relu,
+                                                                                            dz, L.coutp);
+    // weight and bias gradients: partials over chunks of tiles, then a fixed-order sum
+    const int nci = L.cinp % 48 == 0 ? 3 : L.cinp % 32 == 0 ? 2 : 1, rows = nci == 3 ? 8 : 16;
+    const int ngrp = L.coutp / 16 * (L.cinp / (16 * nci));
+    const int ntx = (y.W + 31) / 32, nty = (y.H + rows - 1) / rows;
+    const long ntile = (long)ntx * nty * y.B;
+    if (ntile > INT_MAX) {
+        c->err = "unet: batch too large";
+        return TL_E_INVALID;
+    }
+    const int nchunk = (int)std::min<long>(ntile, std::max(1, TL_DW_BLOCKS / ngrp));
+    const long npart = 9L * L.cinp * L.coutp + L.coutp;
+    const size_t need = (size_t)nchunk * npart;
     if (need > u->dw_part_len) {
         if (u->dw_part) (void)hipFree(u->dw_part);
         u->dw_part = nullptr;
@@ -979,9 +1092,15 @@ static int back_layer(tl_ctx *c, Unet *u, int l, const TV &g, const TV &gp, int 
         if (int rc = ualloc(c, (void **)&u->dw_part, need * sizeof(float))) return rc;
         u->dw_part_len = need;
     }
-    k_dw<<<dim3(blocks(npair), nchunk), 256, 0, c->stream>>>(x, dz, L.cinp, L.coutp, px_chunk, u->dw_part);
-    k_dw_reduce<<<blocks(9 * npair), 256, 0, c->stream>>>(u->dw_part, nchunk, 9 * npair, u->gw[l]);
-    k_db<<<L.coutp, 256, 0, c->stream>>>(dz, L.cout, u->gb[l]);
+    const dim3 grid(nchunk, ngrp);
+    if (nci == 3)
+        k_dw<3, 2><<<grid, 256, 0, c->stream>>>(x, dz, L.cinp, L.coutp, ntx, nty, (int)ntile, u->dw_part);
+    else if (nci == 2)
+        k_dw<2, 4><<<grid, 256, 0, c->stream>>>(x, dz, L.cinp, L.coutp, ntx, nty, (int)ntile, u->dw_part);
+    else
+        k_dw<1, 4><<<grid, 256, 0, c->stream>>>(x, dz, L.cinp, L.coutp, ntx, nty, (int)ntile, u->dw_part);
+    k_dw_reduce<<<(unsigned)(npart / 16), 256, 0, c->stream>>>(u->dw_part, nchunk, npart - L.coutp, L.coutp, L.cout,
+                                                              u->gw[l], u->gb[l]);
     if (gx) UCHK(c, conv(c, dz, *gx, u->wt[l], nullptr, L.coutp, L.cinp, 0));
     UCHK(c, hipGetLastError());
     return TL_OK;
