@@ -74,6 +74,8 @@ typedef uint16_t bf16;
 #define TL_DW_BLOCKS 512
 #endif
 
+constexpr int GATHER_BLOCKS = 32;  // blocks per sample of a minibatch's gather
+
 constexpr int NL = 11;
 struct LayerDef {
     int cin, cinp, cout, coutp, relu;
@@ -521,24 +523,116 @@ __global__ void k_cvt_w(const float *__restrict__ w, int cinp, int coutp, bf16 *
     wt[((long)(8 - tap) * cinp + ci) * coutp + co] = h;
 }
 
-// Adam (Kingma & Ba 2015) on FP32 parameters
-__global__ void k_adam(float *__restrict__ w, const float *__restrict__ g, float *__restrict__ m,
-                       float *__restrict__ v, long n, float lr, float b1, float b2, float eps, float c1, float c2)
+// Adam (Kingma & Ba 2015) on the FP32 parameters of every layer, and the new
+// weights' BF16 copies (as k_cvt_w makes them), in one launch: blocks
+// first[l] .. first[l+1]-1 take layer l's weights (a multiple of 256), the
+// last of them its biases.  33 launches of 2 us and the gaps between them took
+// 520 us a step, this 7.
+struct AdamArgs {
+    struct {
+        float *w, *g, *m, *v, *b, *gb, *mb, *vb;
+        bf16 *wb, *wt;
+        int cinp, coutp;
+    } l[NL];
+    unsigned first[NL + 1];
+};
+__global__ __launch_bounds__(256) void k_adam(AdamArgs a, float lr, float b1, float b2, float eps, float c1, float c2)
 {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float gi = g[i];
+    int l = 0;
+    while (blockIdx.x >= a.first[l + 1]) ++l;
+    const auto &q = a.l[l];
+    const bool bias = blockIdx.x + 1 == a.first[l + 1];
+    const int i = bias ? (int)threadIdx.x : (int)(blockIdx.x - a.first[l]) * 256 + (int)threadIdx.x;
+    if (bias && i >= q.coutp) return;
+    float *const w = bias ? q.b : q.w, *const m = bias ? q.mb : q.m, *const v = bias ? q.vb : q.v;
+    const float gi = bias ? q.gb[i] : q.g[i];
     const float mi = b1 * m[i] + (1.f - b1) * gi;
     const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
     m[i] = mi;
     v[i] = vi;
-    w[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+    const float wn = w[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+    w[i] = wn;
+    if (bias) return;
+    const int ci = i % q.cinp, co = (i / q.cinp) % q.coutp, tap = i / (q.cinp * q.coutp);
+    const bf16 h = f2bf(wn);
+    q.wb[i] = h;
+    q.wt[((long)(8 - tap) * q.cinp + ci) * q.coutp + co] = h;
+}
+
+// A minibatch from the recorded samples: sample s[b] of the dataset becomes
+// sample b0 + b of the batch (inputs with their border, target, mask, face
+// coefficients, edge flags); cnt[(b0 + b) gridDim.x + block]: the mask's sum
+// over the block's part.  One launch for up to 64 samples: a copy each of the
+// four arrays took 14 us of host and launch time, 900 us for 16 samples, and
+// the number of scored pixels 300 us on the host.
+struct Pick {
+    int s[64], edges[64];
+};
+__global__ __launch_bounds__(256) void k_gather(Pick pk, int b0, long xs, long px, const bf16 *__restrict__ dx,
+                                                const float *__restrict__ dy, const float *__restrict__ dm,
+                                                const float *__restrict__ dk, bf16 *__restrict__ bx,
+                                                float *__restrict__ by, float *__restrict__ bm, float *__restrict__ bk,
+                                                int *__restrict__ edges, double *__restrict__ cnt)
+{
+    typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+    const long s = pk.s[blockIdx.y], b = b0 + (long)blockIdx.y;
+    const long t0 = (long)blockIdx.x * 256 + threadIdx.x, step = (long)gridDim.x * 256;
+    auto copy = [&](const void *src, void *dst, long bytes) {  // multiples of 16 bytes, aligned
+        for (long i = t0; i < bytes / 16; i += step) ((u4 *)dst)[i] = ((const u4 *)src)[i];
+    };
+    copy(dx + s * xs, bx + b * xs, xs * (long)sizeof(bf16));
+    copy(dy + s * px, by + b * px, px * (long)sizeof(float));
+    copy(dk + s * 2 * px, bk + b * 2 * px, 2 * px * (long)sizeof(float));
+    double n = 0.0;
+    for (long i = t0; i < px / 4; i += step) {
+        const f4 v = ((const f4 *)(dm + s * px))[i];
+        ((f4 *)(bm + b * px))[i] = v;
+        n += (double)v[0] + (double)v[1] + (double)v[2] + (double)v[3];
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) edges[b] = pk.edges[blockIdx.y];
+    __shared__ double sh[256];
+    sh[threadIdx.x] = n;
+    __syncthreads();
+    for (int o = 128; o > 0; o >>= 1) {
+        if (threadIdx.x < o) sh[threadIdx.x] += sh[threadIdx.x + o];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) cnt[b * gridDim.x + blockIdx.x] = sh[0];
+}
+
+// FP64 sum of n values by one block of 256 threads (fixed order), on thread 0
+template <typename T>
+__device__ __forceinline__ double block_sum(const T *__restrict__ v, long n)
+{
+    double s = 0.0;
+    for (long i = threadIdx.x; i < n; i += 256) s += (double)v[i];
+    __shared__ double sh[256];
+    sh[threadIdx.x] = s;
+    __syncthreads();
+    for (int o = 128; o > 0; o >>= 1) {
+        if (threadIdx.x < o) sh[threadIdx.x] += sh[threadIdx.x + o];
+        __syncthreads();
+    }
+    return sh[0];
+}
+
+// 1 / (number of scored pixels): the scale of the loss, and the loss itself
+__global__ __launch_bounds__(256) void k_scale(const double *__restrict__ cnt, long n, float *__restrict__ scale)
+{
+    const double s = block_sum(cnt, n);
+    if (threadIdx.x == 0) *scale = s > 0.0 ? (float)(1.0 / s) : 0.f;
+}
+__global__ __launch_bounds__(256) void k_loss_fin(const float *__restrict__ part, long n,
+                                                  const float *__restrict__ scale, float *__restrict__ loss)
+{
+    const double s = block_sum(part, n);
+    if (threadIdx.x == 0) *loss = (float)(s * (double)*scale);
 }
 
 // output gradient of the MSE loss on channel 0, masked to the scored
 // region; partial sums of the squared error per block
 __global__ __launch_bounds__(256) void k_loss(TV out, const float *__restrict__ tgt, const float *__restrict__ wmask,
-                                              TV gout, float scale, float *__restrict__ part)
+                                              TV gout, const float *__restrict__ scale, float *__restrict__ part)
 {
     const long n = (long)out.B * out.H * out.W;
     const long p = (long)blockIdx.x * 256 + threadIdx.x;
@@ -552,7 +646,7 @@ __global__ __launch_bounds__(256) void k_loss(TV out, const float *__restrict__ 
         const float d = (bf2f(out.p[out.idx(b, yy, xx)]) - tgt[p]) * wgt;
         e2 = d * d;
         const long gi = gout.idx(b, yy, xx);
-        gout.p[gi] = f2bf(2.f * d * scale);
+        gout.p[gi] = f2bf(2.f * d * *scale);
         for (int c = 1; c < gout.C; ++c) gout.p[gi + c] = 0;
     }
     __shared__ float sh[256];
@@ -640,7 +734,7 @@ __global__ __launch_bounds__(256) void k_res_r(const float *__restrict__ e, cons
 
 // step 3: dL/d(out) = 2 scale A r (A symmetric), into channel 0 of gout
 __global__ void k_res_g(const float *__restrict__ r, const float *__restrict__ k, const int *__restrict__ edges,
-                        TV gout, float scale)
+                        TV gout, const float *__restrict__ scale)
 {
     const long n = (long)gout.B * gout.H * gout.W;
     const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -651,7 +745,7 @@ __global__ void k_res_g(const float *__restrict__ r, const float *__restrict__ k
     const int y = (int)(q % H);
     const int b = (int)(q / H);
     const long o = (long)b * H * W;
-    const float g = 2.f * scale * crop_apply(r + o, k + 2 * o, x, y, W, H, edges[b]);
+    const float g = 2.f * *scale * crop_apply(r + o, k + 2 * o, x, y, W, H, edges[b]);
     const long gi = gout.idx(b, y, x);
     gout.p[gi] = f2bf(g);
     for (int c = 1; c < gout.C; ++c) gout.p[gi + c] = 0;
@@ -686,7 +780,8 @@ __global__ __launch_bounds__(256) void k_en_r(const float *__restrict__ e, const
 }
 
 // dL/d(out) = 2 scale mask (A (mask e)) into channel 0 of gout
-__global__ void k_en_g(const float *__restrict__ r, const float *__restrict__ mask, TV gout, float scale)
+__global__ void k_en_g(const float *__restrict__ r, const float *__restrict__ mask, TV gout,
+                       const float *__restrict__ scale)
 {
     const long n = (long)gout.B * gout.H * gout.W;
     const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -697,7 +792,7 @@ __global__ void k_en_g(const float *__restrict__ r, const float *__restrict__ ma
     const int y = (int)(q % H);
     const int b = (int)(q / H);
     const long gi = gout.idx(b, y, x);
-    gout.p[gi] = f2bf(2.f * scale * mask[p] * r[p]);
+    gout.p[gi] = f2bf(2.f * *scale * mask[p] * r[p]);
     for (int c = 1; c < gout.C; ++c) gout.p[gi + c] = 0;
 }
 
@@ -739,14 +834,22 @@ __global__ __launch_bounds__(256) void k_absmax3(Geo g, const double *__restrict
         for (int a = 0; a < 3; ++a) part[3 * blockIdx.x + a] = sh[a][0];
 }
 
-__global__ void k_absmax_fin(const float *__restrict__ part, int nb, float *__restrict__ scale)
+// (one thread for the 1024 partials took 130 us)
+__global__ __launch_bounds__(256) void k_absmax_fin(const float *__restrict__ part, int nb, float *__restrict__ scale)
 {
-    if (threadIdx.x != 0) return;
+    __shared__ float sh[3][256];
     for (int a = 0; a < 3; ++a) {
         float v = 0.f;
-        for (int i = 0; i < nb; ++i) v = fmaxf(v, part[3 * i + a]);
-        scale[a] = v > 0.f ? v : 1.f;
+        for (int i = threadIdx.x; i < nb; i += 256) v = fmaxf(v, part[3 * i + a]);
+        sh[a][threadIdx.x] = v;
     }
+    __syncthreads();
+    for (int o = 128; o > 0; o >>= 1) {
+        if (threadIdx.x < o)
+            for (int a = 0; a < 3; ++a) sh[a][threadIdx.x] = fmaxf(sh[a][threadIdx.x], sh[a][threadIdx.x + o]);
+        __syncthreads();
+    }
+    if (threadIdx.x < 3) scale[threadIdx.x] = sh[threadIdx.x][0] > 0.f ? sh[threadIdx.x][0] : 1.f;
 }
 
 // r0 = b - A x with b = x = u_prev: the residual of the previous-step guess
@@ -831,12 +934,14 @@ struct tl::Unet {
     bool weights_set = false;
     int adam_t = 0;
     Acts acts;
-    float *scale = nullptr;      // [3]: s_u, s_e, s_r
+    float *scale = nullptr;      // [4]: s_u, s_e, s_r, the loss's scale
     float *mx_part = nullptr;    // absmax partials
     float *dw_part = nullptr;
     size_t dw_part_len = 0;
     float *loss_part = nullptr;
     size_t loss_part_len = 0;
+    float *loss_dev = nullptr;  // losses of a call's steps
+    size_t loss_dev_len = 0;
     // dataset of training samples: inputs (bordered, 16 ch), target, loss mask
     bf16 *ds_x = nullptr;
     float *ds_y = nullptr, *ds_m = nullptr, *ds_k = nullptr;
@@ -846,6 +951,7 @@ struct tl::Unet {
     // batch buffers
     float *bt_y = nullptr, *bt_m = nullptr, *bt_k = nullptr, *bt_e = nullptr, *bt_r = nullptr;
     int *bt_edges = nullptr;
+    double *bt_cnt = nullptr;  // sums of the masks, GATHER_BLOCKS per sample
     int bt_cap = 0;
 };
 
@@ -1145,16 +1251,20 @@ static int backward(tl_ctx *c, Unet *u)
     return TL_OK;
 }
 
+// one Adam step; the BF16 weights follow
 static int adam_step(tl_ctx *c, Unet *u, float lr)
 {
     u->adam_t += 1;
     const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
     const float c1 = 1.f - std::pow(b1, (float)u->adam_t), c2 = 1.f - std::pow(b2, (float)u->adam_t);
+    AdamArgs a;
+    a.first[0] = 0;
     for (int l = 0; l < NL; ++l) {
-        const long nw = (long)wcount(l), nb = LAY[l].coutp;
-        k_adam<<<blocks(nw), 256, 0, c->stream>>>(u->w[l], u->gw[l], u->mw[l], u->vw[l], nw, lr, b1, b2, eps, c1, c2);
-        k_adam<<<blocks(nb), 256, 0, c->stream>>>(u->b[l], u->gb[l], u->mb[l], u->vb[l], nb, lr, b1, b2, eps, c1, c2);
+        a.l[l] = {u->w[l],  u->gw[l], u->mw[l], u->vw[l], u->b[l],     u->gb[l],
+                  u->mb[l], u->vb[l], u->wb[l], u->wt[l], LAY[l].cinp, LAY[l].coutp};
+        a.first[l + 1] = a.first[l] + (unsigned)(wcount(l) / 256) + 1;
     }
+    k_adam<<<a.first[NL], 256, 0, c->stream>>>(a, lr, b1, b2, eps, c1, c2);
     UCHK(c, hipGetLastError());
     return TL_OK;
 }
@@ -1185,7 +1295,7 @@ static int grid_scales(tl_ctx *c, Unet *u, const double *uprev, const double *en
     const int nb = 1024;
     k_r0<<<dim3(blocks(c->g.nx), c->g.ny), 256, 0, c->stream>>>(c->g, uprev, c->f[TL_F_KX], c->f[TL_F_KY], r0);
     k_absmax3<<<nb, 256, 0, c->stream>>>(c->g, uprev, energy, r0, u->mx_part);
-    k_absmax_fin<<<1, 64, 0, c->stream>>>(u->mx_part, nb, u->scale);
+    k_absmax_fin<<<1, 256, 0, c->stream>>>(u->mx_part, nb, u->scale);
     UCHK(c, hipGetLastError());
     return TL_OK;
 }
@@ -1229,7 +1339,7 @@ void unet_destroy(tl_ctx *c)
             if (p) (void)hipFree(p);
     }
     void *ps[] = {u->scale, u->mx_part, u->dw_part, u->loss_part, u->ds_x, u->ds_y, u->ds_m, u->ds_k,
-                  u->bt_y, u->bt_m, u->bt_k, u->bt_e, u->bt_r, u->bt_edges};
+                  u->bt_y, u->bt_m, u->bt_k, u->bt_e, u->bt_r, u->bt_edges, u->bt_cnt, u->loss_dev};
     for (void *p : ps)
         if (p) (void)hipFree(p);
     delete u;
@@ -1391,7 +1501,7 @@ extern "C" int tl_unet_train(tl_ctx *c, const tl_train_params *tp, float *loss_o
     if (int rc = acts_ensure(c, u, B, crop, crop, true)) return rc;
     if (u->bt_cap < B) {
         void **old[] = {(void **)&u->bt_y, (void **)&u->bt_m, (void **)&u->bt_k,
-                        (void **)&u->bt_e, (void **)&u->bt_r, (void **)&u->bt_edges};
+                        (void **)&u->bt_e, (void **)&u->bt_r, (void **)&u->bt_edges, (void **)&u->bt_cnt};
         for (void **q : old) {
             if (*q) (void)hipFree(*q);
             *q = nullptr;
@@ -1403,10 +1513,10 @@ extern "C" int tl_unet_train(tl_ctx *c, const tl_train_params *tp, float *loss_o
         if (int rc = ualloc(c, (void **)&u->bt_e, B * px * sizeof(float))) return rc;
         if (int rc = ualloc(c, (void **)&u->bt_r, B * px * sizeof(float))) return rc;
         if (int rc = ualloc(c, (void **)&u->bt_edges, B * sizeof(int))) return rc;
+        if (int rc = ualloc(c, (void **)&u->bt_cnt, (size_t)B * GATHER_BLOCKS * sizeof(double))) return rc;
         u->bt_cap = B;
     }
     const int loss_kind = tp->reserved[0];  // 0 residual, 1 mse, 2 energy norm
-    std::vector<int> edges(B);
     const long npx = (long)B * px;
     const unsigned nlb = blocks(npx);
     if ((size_t)nlb > u->loss_part_len) {
@@ -1416,39 +1526,39 @@ extern "C" int tl_unet_train(tl_ctx *c, const tl_train_params *tp, float *loss_o
         if (int rc = ualloc(c, (void **)&u->loss_part, nlb * sizeof(float))) return rc;
         u->loss_part_len = nlb;
     }
+    if ((size_t)tp->steps > u->loss_dev_len) {
+        if (u->loss_dev) (void)hipFree(u->loss_dev);
+        u->loss_dev = nullptr;
+        u->loss_dev_len = 0;
+        if (int rc = ualloc(c, (void **)&u->loss_dev, tp->steps * sizeof(float))) return rc;
+        u->loss_dev_len = tp->steps;
+    }
+    float *const scale = u->scale + 3;
     std::mt19937_64 g(0x5eed0000ULL + (uint64_t)tp->seed);
     const size_t xs = (size_t)(crop + 2) * (crop + 2) * 16;
-    std::vector<float> lp(nlb), mk(npx);
     for (int step = 0; step < tp->steps; ++step) {
-        // gather a batch
-        for (int b = 0; b < B; ++b) {
-            const int s = (int)(g() % (uint64_t)u->ds_n);
-            edges[b] = u->ds_edges[s];
-            UCHK(c, hipMemcpyAsync(u->bt_k + 2 * b * px, u->ds_k + (size_t)s * 2 * px, 2 * px * sizeof(float),
-                                   hipMemcpyDeviceToDevice, c->stream));
-            UCHK(c, hipMemcpyAsync(u->acts.x0.p + b * xs, u->ds_x + (size_t)s * xs, xs * sizeof(bf16),
-                                   hipMemcpyDeviceToDevice, c->stream));
-            UCHK(c, hipMemcpyAsync(u->bt_y + b * px, u->ds_y + (size_t)s * px, px * sizeof(float),
-                                   hipMemcpyDeviceToDevice, c->stream));
-            UCHK(c, hipMemcpyAsync(u->bt_m + b * px, u->ds_m + (size_t)s * px, px * sizeof(float),
-                                   hipMemcpyDeviceToDevice, c->stream));
+        // gather a batch; scale = 1 / (number of scored pixels)
+        for (int b0 = 0; b0 < B; b0 += 64) {
+            Pick pk;
+            const int n = std::min(64, B - b0);
+            for (int b = 0; b < n; ++b) {
+                pk.s[b] = (int)(g() % (uint64_t)u->ds_n);
+                pk.edges[b] = u->ds_edges[pk.s[b]];
+            }
+            k_gather<<<dim3(GATHER_BLOCKS, n), 256, 0, c->stream>>>(pk, b0, xs, px, u->ds_x, u->ds_y, u->ds_m, u->ds_k,
+                                                                    u->acts.x0.p, u->bt_y, u->bt_m, u->bt_k,
+                                                                    u->bt_edges, u->bt_cnt);
         }
+        k_scale<<<1, 256, 0, c->stream>>>(u->bt_cnt, (long)B * GATHER_BLOCKS, scale);
+        UCHK(c, hipGetLastError());
         if (int rc = forward(c, u, true)) return rc;
-        // scale = 1 / (number of scored pixels) (from the masks of the batch)
-        UCHK(c, hipMemcpyAsync(mk.data(), u->bt_m, npx * sizeof(float), hipMemcpyDeviceToHost, c->stream));
-        UCHK(c, hipStreamSynchronize(c->stream));
-        double nsc = 0;
-        for (long i = 0; i < npx; ++i) nsc += mk[i];
-        const float scale = nsc > 0 ? (float)(1.0 / nsc) : 0.f;
         if (loss_kind == 2) {
             // energy norm of the error: L = scale * e^T A e with e = mask (out - target)
-            UCHK(c, hipMemcpyAsync(u->bt_edges, edges.data(), B * sizeof(int), hipMemcpyHostToDevice, c->stream));
             k_err_m<<<nlb, 256, 0, c->stream>>>(u->acts.out.v(), u->bt_y, u->bt_m, u->bt_e);
             k_en_r<<<nlb, 256, 0, c->stream>>>(u->bt_e, u->bt_k, u->bt_edges, B, crop, crop, u->bt_r, u->loss_part);
             k_en_g<<<nlb, 256, 0, c->stream>>>(u->bt_r, u->bt_m, u->acts.g_out.v(), scale);
         } else if (loss_kind == 0) {
             // minimise the residual of the guess: L = scale * sum_scored (A (out - target))^2
-            UCHK(c, hipMemcpyAsync(u->bt_edges, edges.data(), B * sizeof(int), hipMemcpyHostToDevice, c->stream));
             k_res_e<<<nlb, 256, 0, c->stream>>>(u->acts.out.v(), u->bt_y, u->bt_e);
             k_res_r<<<nlb, 256, 0, c->stream>>>(u->bt_e, u->bt_k, u->bt_m, u->bt_edges, B, crop, crop, u->bt_r,
                                                  u->loss_part);
@@ -1460,15 +1570,11 @@ extern "C" int tl_unet_train(tl_ctx *c, const tl_train_params *tp, float *loss_o
         UCHK(c, hipGetLastError());
         if (int rc = backward(c, u)) return rc;
         if (int rc = adam_step(c, u, tp->lr)) return rc;
-        if (int rc = refresh_weights(c, u)) return rc;
-        if (loss_out) {
-            UCHK(c, hipMemcpyAsync(lp.data(), u->loss_part, nlb * sizeof(float), hipMemcpyDeviceToHost, c->stream));
-            UCHK(c, hipStreamSynchronize(c->stream));
-            double s = 0;
-            for (float v : lp) s += v;
-            loss_out[step] = (float)(s * scale);
-        }
+        k_loss_fin<<<1, 256, 0, c->stream>>>(u->loss_part, nlb, scale, u->loss_dev + step);
+        UCHK(c, hipGetLastError());
     }
+    if (loss_out)
+        UCHK(c, hipMemcpyAsync(loss_out, u->loss_dev, tp->steps * sizeof(float), hipMemcpyDeviceToHost, c->stream));
     UCHK(c, hipStreamSynchronize(c->stream));
     return TL_OK;
 }
@@ -1549,7 +1655,8 @@ extern "C" int tl_unet_eval(tl_ctx *c, const float *x, const float *target, int 
     UCHK(c, hipMemcpyAsync(dy, target, npx * sizeof(float), hipMemcpyHostToDevice, c->stream));
     UCHK(c, hipMemcpyAsync(dm, ones.data(), npx * sizeof(float), hipMemcpyHostToDevice, c->stream));
     const float scale = 1.f / (float)npx;
-    k_loss<<<nlb, 256, 0, c->stream>>>(u->acts.out.v(), dy, dm, u->acts.g_out.v(), scale, lp);
+    UCHK(c, hipMemcpyAsync(u->scale + 3, &scale, sizeof(float), hipMemcpyHostToDevice, c->stream));
+    k_loss<<<nlb, 256, 0, c->stream>>>(u->acts.out.v(), dy, dm, u->acts.g_out.v(), u->scale + 3, lp);
     UCHK(c, hipGetLastError());
     if (int rc = backward(c, u)) return rc;
     UCHK(c, hipMemcpyAsync(lph.data(), lp, nlb * sizeof(float), hipMemcpyDeviceToHost, c->stream));

@@ -84,3 +84,20 @@ def test_gradients_of_a_batch_are_those_of_its_samples(chunk, shape):
     s = sum(unet.evaluate(chunk, x[b:b + 1], target[b:b + 1])[2].astype(np.float64) for b in range(4)) / 4
     for (name, a), (_, b) in zip(_layers(g), _layers(s)):
         assert np.linalg.norm(a - b) <= 2e-5 * np.linalg.norm(b), name
+
+
+def test_batches_of_one_sample():
+    """Minibatches are gathered 64 samples at a time: drawn from a dataset of
+    one sample (the whole grid, with edges on all sides), a batch of any size
+    has that sample's loss.  The 256-pixel sums are the same for each of its
+    copies and are added in FP64, so only the scale's rounding (2^-24) differs."""
+    print("case: minibatches of 1 to 130 copies of one sample", flush=True)
+    s = T.Settings.from_text(decks.random_rect_deck(21, n=128, steps=1))
+    c = T.initialiseapp(s)
+    unet.record(c, capacity=1, crops_per_step=1)
+    T.diffuse(c, s, 1)
+    assert unet.dataset_size(c) == 1
+    for kind in ("energy", "mse", "residual"):
+        loss = [unet.train(c, steps=2, batch=b, lr=0.0, loss=kind) for b in (1, 3, 64, 65, 130)]
+        assert np.all(np.isfinite(loss)) and np.min(loss) > 0.0
+        np.testing.assert_allclose(loss, np.full_like(loss, loss[0][0]), rtol=1e-6)
