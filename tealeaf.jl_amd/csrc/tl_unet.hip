@@ -37,6 +37,7 @@
 #include <cstring>
 #include <random>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "tl_internal.hpp"
@@ -47,19 +48,20 @@ typedef short s4 __attribute__((ext_vector_type(4)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef uint16_t bf16;
 
-// output rows per wave of the convolutions: the band of rows a wave walks
-// (fewer on small tensors, so that a launch still has about TL_CONV_BLOCKS
-// blocks); 16 and 64 measured within 2% of 32 at 8192^2
+// output rows per wave of the convolutions: the band of rows a wave walks, at
+// most TL_CONV_ROWS, fewer on small tensors so that a launch has about
+// TL_CONV_WAVES waves.  2048^2 inference / four training steps of 16 crops of
+// 128^2: 2048 waves 2.03 / 2.69 ms, 1024 2.34 / 2.98 (an earlier build; 2.22 /
+// 2.90 with 2048), 4096 2.11 / 2.75, 3072 2.05 / 2.77; at most 16 rows 2.03 / 2.71.
 #ifndef TL_CONV_ROWS
 #define TL_CONV_ROWS 32
 #endif
-#ifndef TL_CONV_BLOCKS
-#define TL_CONV_BLOCKS 4096
+#ifndef TL_CONV_WAVES
+#define TL_CONV_WAVES 2048
 #endif
 // occupancy targets (waves per SIMD) of the convolutions with 16 and 32
-// output channels per launch; the compiler otherwise spends registers down to
-// 2 and 1 waves.  Measured at 8192^2: 16-channel launches at 2 waves (168
-// VGPRs) make the inference 6% faster than at 3 (a few registers spilled)
+// output channels per wave; the compiler otherwise spends registers down to 2
+// and 1 waves
 #ifndef TL_CONV_WPE1
 #define TL_CONV_WPE1 2
 #endif
@@ -106,57 +108,99 @@ struct TV {
 
 // ------------------------------------------------------------- kernels
 
+// elements from one output channel's weights to the next in k_conv's LDS
+__host__ __device__ constexpr int conv_row(int cinp) { return cinp % 32 ? cinp : cinp + 16; }
+
+// the fragment one pixel to the left (SHIFT row_shr:1, ROT row_ror:1) or right
+// (row_shl:1, row_ror:15): 16 lanes are 16 pixels, the one that enters comes
+// from the fragment beside it (rotated) or, unrotated, from the strip's
+// neighbours
+template <int SHIFT, int ROT>
+__device__ __forceinline__ s4 shift_px(s4 f, s4 beside, bool rotate)
+{
+    union {
+        s4 v;
+        int w[2];
+    } a, e, o;
+    a.v = f;
+    e.v = beside;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int in = rotate ? __builtin_amdgcn_update_dpp(0, e.w[h], ROT, 0xF, 0xF, false) : e.w[h];
+        o.w[h] = __builtin_amdgcn_update_dpp(in, a.w[h], SHIFT, 0xF, 0xF, false);
+    }
+    return o.v;
+}
+
 // Convolution 3x3, zero padding, as implicit GEMM on MFMA with the output
 // channels on the M side.  A wave owns 64 pixels (4 groups of 16) of a column
-// strip and walks a band of R output rows down the strip; a block is 4 waves
-// side by side.  Each input row is loaded once per 16-channel chunk (its 3
-// column shifts x 4 pixel groups: 12 fragments), the next (row, chunk)'s
-// fragments requested before this one's products, and added into the three
-// output rows it borders, kept in three rolling accumulator sets: input row r
-// is row dy = 2 of output r-1's window (complete after it: stored), dy = 1 of
-// output r and dy = 0 of output r+1.  Per chunk and tap: A = W[tap][co][ci]
-// (16 co x 16 ci; lane (i, kq) holds ci 4kq..4kq+3 of co i), B =
-// in[pixel][ci] (16 ci x 16 pixels; lane (j, kq) holds ci 4kq..4kq+3 of pixel
-// j), D[co][pixel]: lane (j, kq) holds output channels 4kq..4kq+3 of pixel j,
-// stored as one 8-byte vector.  A launch computes output channels co0 ..
-// co0 + 16 NT - 1 of coutp on the pixel grid of `out`.
-// Input channels [0, csplit) come from `in`, [csplit, cinp) from `skip`
-// (channel c - csplit): a decoder's concatenation [up | skip] read in place.
-// With upin, `in` has half the resolution and is read at (y/2, x/2), the
-// nearest-neighbour upsample (its zero border lands on the output's border).
-template <int NT>
+// strip and walks a band of R output rows down the strip; a block is 4 waves,
+// wx of them side by side (as many as the width has strips, up to 4) and the
+// others on the bands below.  Each input row is loaded once per 16-channel
+// chunk (4 pixel groups and, in one more fragment, the pixels on both sides of
+// the strip; the column shifts of the taps are lane shifts), two steps of (row,
+// chunk) ahead of its products, and added into the three output rows it
+// borders, kept in three rolling accumulator sets: input row r is row dy = 2 of
+// output r-1's window (complete after it: stored), dy = 1 of output r and dy = 0
+// of output r+1.  Per chunk and tap: A = W[tap][co][ci] (16 co x 16 ci; lane
+// (i, kq) holds ci 4kq..4kq+3 of co i), B = in[pixel][ci] (16 ci x 16 pixels;
+// lane (j, kq) holds ci 4kq..4kq+3 of pixel j), D[co][pixel]: lane (j, kq) holds
+// output channels 4kq..4kq+3 of pixel j, stored as one 8-byte vector.  Grid: x is
+// (strips, group of 16 NT output channels from co_first on, of ncg), z the image.
+// With CAT the first two thirds of the input channels come from `in`, which has
+// half the resolution and is read at (y/2, x/2), the others from `skip`: a
+// decoder's concatenation [nearest-neighbour upsample | skip] read in place
+// (the upsample's zero border lands on the output's border).
+// Columns past the border are read as the border (and never stored).
+// Bound by HBM at full resolution (2048^2, 16 -> 16 channels: 55 us, 4.9 TB/s; 32
+// -> 32 at 1024^2 43 us, 48 -> 16 104 us) and by latency on small tensors (64 ->
+// 64 at 32^2, 16 images: 15 us).  With 12 loads per step (3 column shifts) one
+// step ahead, 64-column strips only and a launch per 32 channels they took 104,
+// 64, 234 and 2 x 33 us.  Unconditional loads matter: under a condition the wait
+// for one step's fragments waits for all of them (106 instead of 55 us).
+template <int NCH, int NT, bool CAT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NT == 1 ? TL_CONV_WPE1 : TL_CONV_WPE2))) void k_conv(
-    TV in, TV skip, int csplit, int upin, TV out, const bf16 *__restrict__ wgt, const float *__restrict__ bias,
-    int cinp, int coutp, int co0, int relu, int R)
+    TV in, TV skip, TV out, const bf16 *__restrict__ wgt, const float *__restrict__ bias,
+    int coutp, int co_first, int ncg, int relu, int R, int wx)
 {
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int j = lane & 15, kq = lane >> 4;
-    const int y0 = blockIdx.y * R, b = blockIdx.z;
-    const int x0 = (blockIdx.x * 4 + wave) * 64;
+    const int b = blockIdx.z, co0 = co_first + (int)(blockIdx.x % ncg) * 16 * NT;
+    const int x0 = ((int)(blockIdx.x / ncg) * wx + wave % wx) * 64;
+    const int y0 = ((int)blockIdx.y * (4 / wx) + wave / wx) * R;
     // this launch's weights, [tap][16 NT output channels][cinp], copied into
     // the LDS once per block: every wave reads all of them for every row, and
-    // from the caches they would be fetched by all CUs from the same lines
+    // from the caches they would be fetched by all CUs from the same lines.
+    // Rows are padded to 32 or 96 bytes modulo 128, so that the 16 channels of a
+    // fragment spread over all banks.
     extern __shared__ __attribute__((aligned(16))) bf16 wl[];
+    constexpr int cinp = 16 * NCH, ws = conv_row(cinp);
     {
         typedef uint32_t u4 __attribute__((ext_vector_type(4)));
         const int per = cinp / 8, nvec = 9 * 16 * NT * per;  // 16-byte vectors
         for (int v = threadIdx.x; v < nvec; v += 256) {
             const int rowi = v / per, c8 = (v % per) * 8;
             const int tap = rowi / (16 * NT), co = rowi % (16 * NT);
-            *(u4 *)(wl + (long)rowi * cinp + c8) = *(const u4 *)(wgt + ((long)tap * coutp + co0 + co) * cinp + c8);
+            *(u4 *)(wl + rowi * ws + c8) = *(const u4 *)(wgt + ((long)tap * coutp + co0 + co) * cinp + c8);
         }
     }
     __syncthreads();
-    if (x0 >= out.W) return;
+    if (x0 >= out.W || y0 >= out.H) return;
     const int yout = min(y0 + R, out.H);  // output rows y0 .. yout-1
-    int xa[4];  // this lane's pixel of each group (clamped: pixels past W are never stored)
-#pragma unroll
-    for (int m = 0; m < 4; ++m) xa[m] = min(x0 + 16 * m + j, out.W - 1);
     float bb[NT][4];  // requested first: their latency overlaps the main loop
 #pragma unroll
     for (int n = 0; n < NT; ++n)
 #pragma unroll
         for (int i = 0; i < 4; ++i) bb[n][i] = bias ? bias[co0 + n * 16 + 4 * kq + i] : 0.f;
+    // byte offsets in a row of this lane's pixels, fragments 0..3 and the
+    // strip's neighbours (lanes j = 0 and 15)
+    unsigned xin[5], xsk[CAT ? 5 : 1];
+#pragma unroll
+    for (int m = 0; m < 5; ++m) {
+        const int x = min(m < 4 ? x0 + 16 * m + j : j == 0 ? x0 - 1 : x0 + 64, out.W);
+        xin[m] = (unsigned)(((CAT ? x >> 1 : x) + 1) * in.C + kq * 4) * (unsigned)sizeof(bf16);
+        if constexpr (CAT) xsk[m] = (unsigned)((x + 1) * skip.C + kq * 4) * (unsigned)sizeof(bf16);
+    }
     f4 a0[4][NT], a1[4][NT], a2[4][NT];
     auto zero = [&](f4 (&a)[4][NT]) {
 #pragma unroll
@@ -168,6 +212,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NT == 1 ? T
     zero(a1);
     zero(a2);
     auto store = [&](const f4 (&a)[4][NT], int y) {
+        bf16 *const ob = out.p + out.idx(b, y, -1);
 #pragma unroll
         for (int n = 0; n < NT; ++n) {
             const int co = co0 + n * 16 + 4 * kq;
@@ -186,72 +231,73 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NT == 1 ? T
                         w2[h] = (uint32_t)f2bf(v0) | ((uint32_t)f2bf(v1) << 16);
                     }
                     typedef uint32_t u2 __attribute__((ext_vector_type(2)));
-                    *(u2 *)(out.p + out.idx(b, y, x) + co) = u2{w2[0], w2[1]};
+                    *(u2 *)((char *)ob + (unsigned)((x + 1) * out.C + co) * (unsigned)sizeof(bf16)) = u2{w2[0], w2[1]};
                 }
             }
         }
     };
-    // the 12 fragments of input row r, chunk kc
-    auto load = [&](s4 (&f)[3][4], int r, int kc) {
-        if (kc < csplit) {
-            const int ry = upin ? r >> 1 : r;
+    // the 5 fragments of input row r (past the last one: that again), chunk kc
+    auto load = [&](s4 (&f)[5], int r, int kc) {
+        r = min(r, yout);
+        if constexpr (CAT)
+            if (kc >= NCH / 3 * 32) {
+                const bf16 *const p = skip.p + (skip.idx(b, r, -1) + kc - NCH / 3 * 32);
 #pragma unroll
-            for (int dx = 0; dx < 3; ++dx)
+                for (int m = 0; m < 5; ++m) f[m] = *(const s4 *)((const char *)p + xsk[m]);
+                return;
+            }
+        const bf16 *const p = in.p + (in.idx(b, CAT ? r >> 1 : r, -1) + kc);
 #pragma unroll
-                for (int m = 0; m < 4; ++m) {
-                    const int x = xa[m] + dx - 1;
-                    f[dx][m] = *(const s4 *)(in.p + in.idx(b, ry, upin ? x >> 1 : x) + kc + kq * 4);
-                }
-        } else {
-#pragma unroll
-            for (int dx = 0; dx < 3; ++dx)
-#pragma unroll
-                for (int m = 0; m < 4; ++m)
-                    f[dx][m] = *(const s4 *)(skip.p + skip.idx(b, r, xa[m] + dx - 1) + kc - csplit + kq * 4);
-        }
+        for (int m = 0; m < 5; ++m) f[m] = *(const s4 *)((const char *)p + xin[m]);
     };
-    s4 fc[3][4], fn[3][4];
-    load(fc, y0 - 1, 0);
-    // input row r into the outputs r-1 (up), r (mid), r+1 (dn); then output
-    // r-1 is complete
-    auto row = [&](int r, f4 (&up)[4][NT], f4 (&mid)[4][NT], f4 (&dn)[4][NT]) {
-        for (int kc = 0; kc < cinp; kc += 16) {
-            // the next step: the next chunk of this row, or the next row's first
-            const bool last = kc + 16 >= cinp;
-            if (!last || r + 1 <= yout) load(fn, last ? r + 1 : r, last ? 0 : kc + 16);
+    // the steps of the walk: input rows y0-1 .. yout (row yout may be the zero
+    // bottom border), the chunks of each; load() runs two steps ahead
+    s4 fb[3][5];  // step s's fragments in fb[s % 3]: every index is a constant
+    load(fb[0], y0 - 1, 0);
+    load(fb[1], y0 - 1 + 1 / NCH, 1 % NCH * 16);
+    // input row r = y0 - 1 + Q (modulo 3) into the outputs r-1 (up), r (mid), r+1
+    // (dn) of the band; then output r-1 is complete
+    auto row = [&](auto Q, int r, f4 (&up)[4][NT], f4 (&mid)[4][NT], f4 (&dn)[4][NT]) {
+#pragma unroll
+        for (int k = 0; k < NCH; ++k) {
+            const int kc = 16 * k, step = decltype(Q)::value * NCH + k;
+            load(fb[(step + 2) % 3], r + (k + 2) / NCH, (k + 2) % NCH * 16);
+            const s4(&fc)[5] = fb[step % 3];
             // keeps the following steps' loads below this step's products
             asm volatile("" ::: "memory");
-            s4 wv[9][NT];
+            s4 fl[4], fr[4];  // the pixels to the left and right
 #pragma unroll
-            for (int tap = 0; tap < 9; ++tap)
+            for (int m = 0; m < 4; ++m) {
+                fl[m] = shift_px<0x111, 0x121>(fc[m], m ? fc[m ? m - 1 : 0] : fc[4], m > 0);
+                fr[m] = shift_px<0x101, 0x12F>(fc[m], m < 3 ? fc[m < 3 ? m + 1 : 3] : fc[4], m < 3);
+            }
+            const bf16 *const wk = wl + j * ws + kc + kq * 4;
+            auto taps = [&](int dy, f4 (&a)[4][NT]) {
 #pragma unroll
-                for (int n = 0; n < NT; ++n) wv[tap][n] = *(const s4 *)(wl + (tap * 16 * NT + n * 16 + j) * cinp + kc + kq * 4);
+                for (int dx = 0; dx < 3; ++dx)
 #pragma unroll
-            for (int dx = 0; dx < 3; ++dx)
+                    for (int n = 0; n < NT; ++n) {
+                        const s4 wv = *(const s4 *)(wk + ((dy * 3 + dx) * 16 * NT + n * 16) * ws);
 #pragma unroll
-                for (int n = 0; n < NT; ++n)
-#pragma unroll
-                    for (int m = 0; m < 4; ++m) {
-                        dn[m][n] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(wv[dx][n], fc[dx][m], dn[m][n], 0, 0, 0);
-                        mid[m][n] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(wv[3 + dx][n], fc[dx][m], mid[m][n], 0, 0, 0);
-                        up[m][n] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(wv[6 + dx][n], fc[dx][m], up[m][n], 0, 0, 0);
+                        for (int m = 0; m < 4; ++m)
+                            a[m][n] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(wv, dx == 0 ? fl[m] : dx == 1 ? fc[m] : fr[m],
+                                                                                a[m][n], 0, 0, 0);
                     }
-#pragma unroll
-            for (int dx = 0; dx < 3; ++dx)
-#pragma unroll
-                for (int m = 0; m < 4; ++m) fc[dx][m] = fn[dx][m];
+            };
+            if (r + 1 < yout) taps(0, dn);
+            if (r >= y0 && r < yout) taps(1, mid);
+            if (r > y0) taps(2, up);
         }
-        if (r - 1 >= y0 && r - 1 < yout) store(up, r - 1);
+        if (r > y0) store(up, r - 1);
         zero(up);
     };
-    // input rows y0-1 .. yout (row yout may be the zero bottom border); the
-    // roles of the three accumulator sets rotate with the row
+    // the roles of the three accumulator sets rotate with the row
     for (int r = y0 - 1; r <= yout; r += 3) {
-        row(r, a0, a1, a2);
+        row(std::integral_constant<int, 0>{}, r, a0, a1, a2);
         if (r + 1 > yout) break;
-        row(r + 1, a1, a2, a0);
+        row(std::integral_constant<int, 1>{}, r + 1, a1, a2, a0);
         if (r + 2 > yout) break;
-        row(r + 2, a2, a0, a1);
+        row(std::integral_constant<int, 2>{}, r + 2, a2, a0, a1);
     }
 }
 
@@ -1082,29 +1128,44 @@ static unsigned blocks(long n, int bs = 256) { return (unsigned)((n + bs - 1) / 
 // so full-grid tensors of 16384^2 x 64 channels need the loop
 static unsigned gs_blocks(long n, int bs = 256) { return (unsigned)std::min<long>((n + bs - 1) / bs, 1L << 20); }
 
-// out = conv(in) (same size); or, with skip, out = conv([up2(in) | skip])
-// with csplit channels from in (upsampled 2x when upin)
+// out = conv(in) (same size); or, with skip, out = conv([up2(in) | skip]) with
+// two thirds of the channels from in
 static hipError_t conv(tl_ctx *c, const TV &in, const TV &out, const bf16 *w, const float *bias, int cinp, int coutp,
-                       int relu, const TV *skip = nullptr, int csplit = 0, int upin = 0)
+                       int relu, const TV *skip = nullptr)
 {
-    if (coutp % 16 || coutp < 16 || cinp % 16 || cinp < 16 || cinp > 96) return hipErrorInvalidValue;
-    if (skip && (csplit % 16 || csplit <= 0 || csplit >= cinp)) return hipErrorInvalidValue;
-    // 32 output channels per launch (16 for the last 16 of 48): the three
-    // rolling accumulator sets stay at 96 registers
-    const int gx = (out.W + 255) / 256;
-    int R = TL_CONV_ROWS;
-    while (R > 4 && (long)gx * ((out.H + R - 1) / R) * out.B < TL_CONV_BLOCKS) R /= 2;
-    const dim3 grid(gx, (out.H + R - 1) / R, out.B);
+    if (coutp % 16 || coutp < 16 || cinp % 16 || cinp < 16 || cinp > 96 || cinp == 80) return hipErrorInvalidValue;
+    if (skip && (cinp % 48 || in.C != cinp / 3 * 2 || skip->C != cinp / 3)) return hipErrorInvalidValue;
+    const int strips = (out.W + 63) / 64, wx = strips >= 3 ? 4 : strips;
+    const int gx = (strips + wx - 1) / wx;
     const TV &sk = skip ? *skip : in;
-    const int cs = skip ? csplit : cinp;
-    for (int co0 = 0; co0 < coutp; co0 += 32) {
-        const int nt = coutp - co0 >= 32 ? 2 : 1;
-        const size_t lds = (size_t)9 * 16 * nt * cinp * sizeof(bf16);  // at most 55 KB (96 -> 32)
-        if (nt == 2)
-            k_conv<2><<<grid, 256, lds, c->stream>>>(in, sk, cs, upin, out, w, bias, cinp, coutp, co0, relu, R);
-        else
-            k_conv<1><<<grid, 256, lds, c->stream>>>(in, sk, cs, upin, out, w, bias, cinp, coutp, co0, relu, R);
-    }
+    // 32 output channels per wave (16 for the last 16 of 48): the three rolling
+    // accumulator sets stay at 96 registers
+    const auto launch = [&](int nt, int co0, int ncg) {
+        int R = TL_CONV_ROWS;
+        while (R > 1 && (long)strips * ((out.H + R - 1) / R) * out.B * ncg < TL_CONV_WAVES) R /= 2;
+        const int rows = 4 / wx * R;
+        const dim3 grid(gx * ncg, (out.H + rows - 1) / rows, out.B);
+        const size_t lds = (size_t)9 * 16 * nt * conv_row(cinp) * sizeof(bf16);  // at most 63 KB (96 -> 32)
+        const auto go = [&](auto nch, auto cat) {
+            constexpr int N = decltype(nch)::value;
+            constexpr bool CAT = decltype(cat)::value;
+            if (nt == 2)
+                k_conv<N, 2, CAT><<<grid, 256, lds, c->stream>>>(in, sk, out, w, bias, coutp, co0, ncg, relu, R, wx);
+            else
+                k_conv<N, 1, CAT><<<grid, 256, lds, c->stream>>>(in, sk, out, w, bias, coutp, co0, ncg, relu, R, wx);
+        };
+        const std::false_type one{};
+        const std::true_type two{};
+        switch (cinp / 16) {
+        case 1: go(std::integral_constant<int, 1>{}, one); break;
+        case 2: go(std::integral_constant<int, 2>{}, one); break;
+        case 3: skip ? go(std::integral_constant<int, 3>{}, two) : go(std::integral_constant<int, 3>{}, one); break;
+        case 4: go(std::integral_constant<int, 4>{}, one); break;
+        default: skip ? go(std::integral_constant<int, 6>{}, two) : go(std::integral_constant<int, 6>{}, one); break;
+        }
+    };
+    if (coutp >= 32) launch(2, 0, coutp / 32);
+    if (coutp % 32) launch(1, coutp / 32 * 32, 1);
     return hipGetLastError();
 }
 
@@ -1154,7 +1215,7 @@ static int forward(tl_ctx *c, Unet *u, bool concat)
         UCHK(c, fwd_layer(c, u, 6, a.c2.v(), a.d2a.v()));
     } else {
         const TV sk = a.e2b.v();
-        UCHK(c, conv(c, a.e3b.v(), a.d2a.v(), u->wb[6], u->b[6], LAY[6].cinp, LAY[6].coutp, LAY[6].relu, &sk, 64, 1));
+        UCHK(c, conv(c, a.e3b.v(), a.d2a.v(), u->wb[6], u->b[6], LAY[6].cinp, LAY[6].coutp, LAY[6].relu, &sk));
     }
     UCHK(c, fwd_layer(c, u, 7, a.d2a.v(), a.d2b.v()));
     if (concat) {
@@ -1162,7 +1223,7 @@ static int forward(tl_ctx *c, Unet *u, bool concat)
         UCHK(c, fwd_layer(c, u, 8, a.c1.v(), a.d1a.v()));
     } else {
         const TV sk = a.e1b.v();
-        UCHK(c, conv(c, a.d2b.v(), a.d1a.v(), u->wb[8], u->b[8], LAY[8].cinp, LAY[8].coutp, LAY[8].relu, &sk, 32, 1));
+        UCHK(c, conv(c, a.d2b.v(), a.d1a.v(), u->wb[8], u->b[8], LAY[8].cinp, LAY[8].coutp, LAY[8].relu, &sk));
     }
     UCHK(c, fwd_layer(c, u, 9, a.d1a.v(), a.d1b.v()));
     UCHK(c, fwd_layer(c, u, 10, a.d1b.v(), a.out.v()));

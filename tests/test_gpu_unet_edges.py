@@ -1,5 +1,6 @@
 """GPU: the U-Net's weight and bias gradients at the edges of their tiles (32
-columns by 8 or 16 rows, at full, half and quarter resolution).
+columns by 8 or 16 rows, at full, half and quarter resolution), its forward
+pass at the edges of strips, its minibatches.
 
 The loss is made of few pixels: the target is the network's own output except
 at the corners and on both sides of tile edges, 100 away, so that a pixel left
@@ -74,6 +75,23 @@ def test_gradients_at_tile_edges(chunk, bf16_oracle, shape):
     assert abs(loss - L) / L < 2e-2
     for (name, a), (_, b) in zip(_layers(g), _layers(gref)):
         assert np.linalg.norm(a - b) <= 8e-2 * np.linalg.norm(b) + 1e-6, name
+
+
+@pytest.mark.parametrize("shape", [(1, 4, 4), (2, 36, 64), (1, 12, 516), (1, 100, 260)])
+def test_forward_at_strip_edges(chunk, bf16_oracle, shape):
+    """Strips of 64 columns (1, 2 or 4 of them to a block, at each of the three
+    resolutions) and bands of 1 to 32 rows; test_gpu_unet.py's tolerance, on the
+    whole output and on the columns and rows beside the edges."""
+    print(f"case: unet forward {shape}", flush=True)
+    p, x, _ = _case(chunk, *shape)
+    out = np.asarray(unet.evaluate(chunk, x))
+    x16 = np.zeros(shape + (16,))
+    x16[..., :6] = bf16(x)
+    ref, _ = U.forward(bf16(p), x16)
+    cols = sorted({c for c in (0, 63, 64, 127, 128, 255, 256, shape[2] - 1) if c < shape[2]})
+    rows = sorted({r for r in (0, 1, 2, 3, 31, 32, shape[1] - 1) if r < shape[1]})
+    for a, b in ((out, ref), (out[:, :, cols], ref[:, :, cols]), (out[:, rows], ref[:, rows])):
+        assert np.linalg.norm(a - b) < 2e-2 * np.linalg.norm(b)
 
 
 @pytest.mark.parametrize("shape", [(4, 20, 36), (4, 64, 72)])
