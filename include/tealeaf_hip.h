@@ -56,7 +56,9 @@ extern "C" {
 
 /* tl_solve_params.launch: how the CG iterations of TL_CG solves (FP64 and
  * TL_FP32_IR) reach the GPU.  Both give bit-identical results.  Other solvers
- * always use stream launches. */
+ * always use stream launches.  FP64 CG on up to about 983040 cells (2048 tiles of
+ * 120 x 4) runs up to 256 iterations per launch with either, unless its kernels
+ * are being timed (tl_profile_begin with TL_K_CG_W64 or TL_K_CG_UR64). */
 #define TL_LAUNCH_STREAM 0  /* kernels enqueued in batches of up to 64 iterations */
 #define TL_LAUNCH_GRAPH 1   /* after a first stream batch, replays of one hipGraph of 64 iterations
                                (captured on first use, kept with the context, re-captured when

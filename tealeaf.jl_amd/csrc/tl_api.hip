@@ -160,7 +160,7 @@ extern "C" void tl_destroy(tl_ctx *c)
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     unet_destroy(c);
     void *bufs[] = {c->u_alt, c->sd_alt, c->r_alt1, c->r_alt2, c->p_alt, c->p32b, c->guess, c->gcell, c->gc_range, c->p32, c->r32, c->x32,
-                    c->r32b, c->part_f, c->part_j, c->g64, c->partials, c->ctrl, c->hist_a, c->hist_b, c->states_d};
+                    c->r32b, c->part_f, c->part_j, c->g64, c->slots, c->partials, c->ctrl, c->hist_a, c->hist_b, c->states_d};
     for (int i = 0; i < TL_NFIELDS; ++i)
         if (c->f[i]) (void)hipFree(c->f[i]);
     for (void *b : bufs)
@@ -572,7 +572,32 @@ static int ensure_cgs(tl_ctx *c)
     if (!c->r_alt1) RETIF(alloc_d(c, &c->r_alt1, c->g.elems));
     if (!c->g64) RETIF(alloc_d(c, &c->g64, c->g.elems));
     if (!c->part_f) RETIF(alloc_d(c, &c->part_f, (size_t)9 * c->g.nbmax));
+    if (c->coop_cus < 0) {
+        int coop = 0, cus = 0;
+        HIPCHK(c, hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, c->device));
+        HIPCHK(c, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device));
+        c->coop_cus = coop ? cus : 0;
+    }
     return TL_OK;
+}
+
+// FP64 CG with the grid held in registers (k_cgr): on every grid that fits (up
+// to 2048 tiles of 120 columns by 4 rows, 983040 cells), where it is faster than
+// the sweeps at every size measured (k_cgr's comment), with stream launches and
+// hipGraph batches alike: a launch is a batch of iterations already.  Not where
+// the launches of the sweeps are timed one by one (tl_profile_begin).
+static bool resident_pays(tl_ctx *c)
+{
+    const int nb = c->g.r64.blocks;
+    if (c->prof_mask & ((1u << TL_K_CG_W64) | (1u << TL_K_CG_UR64))) return false;  // timed launch by launch
+    if (nb < 1 || nb > c->coop_cus) return false;
+    // without memory for the exchange the sweeps run, as on larger grids
+    if (!c->slots && hipMalloc((void **)&c->slots, 3 * 4 * CGR_MAXB * sizeof(*c->slots)) != hipSuccess) {
+        c->slots = nullptr;
+        (void)hipGetLastError();
+        return false;
+    }
+    return true;
 }
 
 static bool fused_fits(const tl_ctx *c) { return c->g.nx % 4 == 0; }
@@ -809,11 +834,29 @@ static int solve_cg64(tl_ctx *c, const tl_solve_params *p, double rx, double ry,
     HIPCHK(c, launch_cgs_dots(c, 0));
     Ctrl k;
     int t = 0;
+    const bool resident = resident_pays(c);
     for (;;) {
-        RETIF(run_until_stop(c, 64, (long)p->max_iters + 16, [&]() { return launch_cgs64(c, ++t); }, &k,
-                             p->launch == TL_LAUNCH_GRAPH ? GRAPH_CG64 : -1, &t));
+        if (resident) {
+            hipError_t e;
+            do {
+                e = launch_cgr64(c, t + 1, CGR_BATCH);
+                t += CGR_BATCH;
+                RETIF(read_ctrl(c, &k));
+            } while (e == hipSuccess && k.stop_iter == INT_MAX);
+            if (e != hipSuccess || k.status == TL_E_HIP) {
+                // no cooperative launch to be had, or a block of one did not
+                // arrive: from the start in sweeps, as every later solve
+                (void)hipGetLastError();
+                c->coop_cus = 0;
+                c->cg_u = nullptr;
+                return solve_cg64(c, p, rx, ry, st);
+            }
+        } else {
+            RETIF(run_until_stop(c, 64, (long)p->max_iters + 16, [&]() { return launch_cgs64(c, ++t); }, &k,
+                                 p->launch == TL_LAUNCH_GRAPH ? GRAPH_CG64 : -1, &t));
+        }
         t = k.stop_iter;
-        if (t >= 1) HIPCHK(c, launch_cgs_pending(c, t));
+        if (!resident && t >= 1) HIPCHK(c, launch_cgs_pending(c, t));
         if (mode != MODE_CG_REL || k.why != WHY_CONVERGED) break;
         // the relative rule is met by the recursive residual: confirm it on the
         // true one, and if rounding has let the two drift apart, continue CG

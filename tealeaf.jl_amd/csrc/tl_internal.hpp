@@ -124,6 +124,9 @@ constexpr int TBV = TL_TBV;
 #define TL_S32_COLS 240
 #define TL_S32_WAVES 3072
 #define TL_S32_ROWS 4
+// k_cgr: threads per block, blocks (one per CU) and iterations per launch (the
+// host reads the state once per launch, 15 us)
+constexpr int CGR_NT = 512, CGR_MAXB = 256, CGR_BATCH = 256;
 // sweeps over more bytes than this (the Infinity Cache) use streaming access.
 // Measured with the FP64 CG sweep: 453 MB of arrays (3072^2) 92.6 us per
 // iteration streaming, 102.2 cached; 83 MB (1501x1103) 25.1 and 21.9.
@@ -241,6 +244,7 @@ struct Geo {
     int gyq, tyq;              // two-step PPCG kernel: gx2*gyq blocks of 2*TB columns x tyq rows
     Tiles s64;                 // single-sweep FP64 CG
     Tiles s32;                 // pairs of FP32 CG iterations
+    Tiles r64;                 // FP64 CG held in registers (blocks 0: the grid is too large)
     int nbmax;                 // stride of the partial-sum arrays (max block count)
     size_t elems;              // elements per allocation
 };
@@ -300,6 +304,8 @@ struct tl_ctx {
     double *f[TL_NFIELDS] = {};
     double *u_alt = nullptr, *sd_alt = nullptr, *guess = nullptr;
     double *r_alt1 = nullptr, *r_alt2 = nullptr;  // r's second buffer (CG sweeps) / between PPCG's two-step sweeps
+    unsigned long long *slots = nullptr;  // k_cgr: the blocks' sums of three iterations
+    int coop_cus = -1;        // compute units for cooperative launches (-1: not asked yet)
     double *g64 = nullptr;    // FP64 cell coefficient 1/w of the CG sweeps (see k_init_coef)
     double hx64 = 0, hy64 = 0;  // its face scales rx/2, ry/2
     // FP32 fields of the mixed-precision solve
@@ -394,6 +400,7 @@ hipError_t launch_resid_norm_slot(tl_ctx *c, const double *b, const double *x, i
 // iteration is tref (t only selects the buffers; the kernel takes its
 // iteration number from Ctrl::tg)
 hipError_t launch_cgs64(tl_ctx *c, int t, int tref = 0);
+hipError_t launch_cgr64(tl_ctx *c, int t0, int n);
 hipError_t launch_cgs_dots(tl_ctx *c, int T);
 hipError_t launch_cgs_pending(tl_ctx *c, int T);
 hipError_t launch_cgs_final(tl_ctx *c, int T);
