@@ -572,12 +572,6 @@ static int ensure_cgs(tl_ctx *c)
     if (!c->r_alt1) RETIF(alloc_d(c, &c->r_alt1, c->g.elems));
     if (!c->g64) RETIF(alloc_d(c, &c->g64, c->g.elems));
     if (!c->part_f) RETIF(alloc_d(c, &c->part_f, (size_t)9 * c->g.nbmax));
-    if (c->coop_cus < 0) {
-        int coop = 0, cus = 0;
-        HIPCHK(c, hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, c->device));
-        HIPCHK(c, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device));
-        c->coop_cus = coop ? cus : 0;
-    }
     return TL_OK;
 }
 
@@ -586,11 +580,15 @@ static int ensure_cgs(tl_ctx *c)
 // the sweeps at every size measured (k_cgr's comment), with stream launches and
 // hipGraph batches alike: a launch is a batch of iterations already.  Not where
 // the launches of the sweeps are timed one by one (tl_profile_begin).
-static bool resident_pays(tl_ctx *c)
+static bool resident_fits(tl_ctx *c, const Tiles &o)
 {
-    const int nb = c->g.r64.blocks;
-    if (c->prof_mask & ((1u << TL_K_CG_W64) | (1u << TL_K_CG_UR64))) return false;  // timed launch by launch
-    if (nb < 1 || nb > c->coop_cus) return false;
+    if (c->coop_cus < 0) {
+        int coop = 0, cus = 0;
+        (void)hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, c->device);
+        (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device);
+        c->coop_cus = coop ? cus : 0;
+    }
+    if (o.blocks < 1 || o.blocks > c->coop_cus) return false;
     // without memory for the exchange the sweeps run, as on larger grids
     if (!c->slots && hipMalloc((void **)&c->slots, 3 * 4 * CGR_MAXB * sizeof(*c->slots)) != hipSuccess) {
         c->slots = nullptr;
@@ -598,6 +596,19 @@ static bool resident_pays(tl_ctx *c)
         return false;
     }
     return true;
+}
+static bool resident_pays(tl_ctx *c)
+{
+    return !(c->prof_mask & ((1u << TL_K_CG_W64) | (1u << TL_K_CG_UR64))) && resident_fits(c, c->g.r64);
+}
+
+// The same in FP32, TL_FP32_KERNELS_AUTO with stream launches: faster than the
+// pairs on every grid that fits (2048 tiles of 240 x 4, 1966080 cells; k_cgr's
+// comment).  Below 32768 cells the choice is as before (a solve takes a few ms).
+static bool resident32_pays(tl_ctx *c)
+{
+    return !(c->prof_mask & ((1u << TL_K_CGP_G32) | (1u << TL_K_CGP_U32))) && (long)c->g.nx * c->g.ny >= 32768 &&
+           resident_fits(c, c->g.r32);
 }
 
 static bool fused_fits(const tl_ctx *c) { return c->g.nx % 4 == 0; }
@@ -1202,12 +1213,13 @@ static int solve_cg_ir(tl_ctx *c, const tl_solve_params *p, double rx, double ry
     HIPCHK(c, launch_init_ctrl(c, MODE_IR, p->max_iters, p->eps, p->rel_tol, delta, 0, 0, p->epslim));
     // pairs of iterations (k_cgp) run as stream launches; with TL_LAUNCH_GRAPH
     // the automatic choice takes the fused kernel
+    const bool resident = p->fp32_kernels == TL_FP32_KERNELS_AUTO && p->launch != TL_LAUNCH_GRAPH && resident32_pays(c);
     const bool pairs = p->fp32_kernels == TL_FP32_KERNELS_PAIRS ||
-                       (p->fp32_kernels == TL_FP32_KERNELS_AUTO && TL_CGP_AUTO && pairs_pay(c) &&
+                       (p->fp32_kernels == TL_FP32_KERNELS_AUTO && !resident && TL_CGP_AUTO && pairs_pay(c) &&
                         p->launch != TL_LAUNCH_GRAPH);
-    const bool fused = !pairs && (p->fp32_kernels == TL_FP32_KERNELS_FUSED ||
+    const bool fused = !pairs && !resident && (p->fp32_kernels == TL_FP32_KERNELS_FUSED ||
                                   (p->fp32_kernels == TL_FP32_KERNELS_AUTO && fused_fits(c)));
-    if (fused || pairs) RETIF(ensure_fused(c));
+    if (fused || pairs || resident) RETIF(ensure_fused(c));
     const double *guess = nullptr;
     RETIF(choose_guess(c, p, rx, ry, &guess, st));
     // u0 = b = energy*density; u = guess or b; bb, tol_abs
@@ -1217,7 +1229,7 @@ static int solve_cg_ir(tl_ctx *c, const tl_solve_params *p, double rx, double ry
     // r = u0 - A u (FP64, stored in FP32) and p = r; fused: the four sums of
     // iteration 1 (r and p in the buffers of iteration 0)
     HIPCHK(c, launch_ir_residual(c, 1, t + 1));
-    if (fused) HIPCHK(c, launch_cgf_dots(c, 0));
+    if (fused || resident) HIPCHK(c, launch_cgf_dots(c, 0));
     int tfirst = 1;  // pairs: the first pair after a start or a refresh
     Ctrl k;
     RETIF(read_ctrl(c, &k));
@@ -1226,7 +1238,13 @@ static int solve_cg_ir(tl_ctx *c, const tl_solve_params *p, double rx, double ry
     while (k.stop_iter == INT_MAX || k.why == WHY_REFRESH) {
         if (k.stop_iter != INT_MAX && k.why == WHY_REFRESH) {
             t = k.stop_iter;
-            if (pairs) {
+            if (resident) {
+                // u += x (complete after every launch), the FP64 residual into
+                // r(t)'s buffer, p(t) kept, and the four sums
+                HIPCHK(c, launch_ir_accumulate(c, 0, nullptr));
+                HIPCHK(c, launch_ir_residual(c, 0, t + 1, cgf_r(c, t)));
+                HIPCHK(c, launch_cgf_dots(c, t));
+            } else if (pairs) {
                 // u += x (complete after every pair), the FP64 residual into
                 // r(t)'s buffer, p(t) kept
                 HIPCHK(c, launch_ir_accumulate(c, t, nullptr));
@@ -1246,7 +1264,20 @@ static int solve_cg_ir(tl_ctx *c, const tl_solve_params *p, double rx, double ry
             RETIF(read_ctrl(c, &k));
             continue;
         }
-        if (pairs)
+        if (resident) {
+            hipError_t e;
+            const int from = t + 1;
+            do {
+                e = launch_cgr32(c, t + 1, CGR_BATCH, t + 1 == from);
+                t += CGR_BATCH;
+                RETIF(read_ctrl(c, &k));
+            } while (e == hipSuccess && k.stop_iter == INT_MAX);
+            if (e != hipSuccess || k.status == TL_E_HIP) {  // as in solve_cg64
+                (void)hipGetLastError();
+                c->coop_cus = 0;
+                return solve_cg_ir(c, p, rx, ry, st);
+            }
+        } else if (pairs)
             RETIF(run_until_stop(c, 32, (long)p->max_iters / 2 + 16,
                                  [&]() {
                                      const hipError_t e = launch_cgp(c, t + 1, t + 1 == tfirst);
@@ -1262,7 +1293,7 @@ static int solve_cg_ir(tl_ctx *c, const tl_solve_params *p, double rx, double ry
                                  p->launch == TL_LAUNCH_GRAPH ? GRAPH_CG32 : -1, &t));
     }
     if (k.why == WHY_MAXITERS)  // keep the partial correction
-        HIPCHK(c, launch_ir_accumulate(c, k.stop_iter, fused ? cgf_p(c, k.stop_iter) : nullptr));
+        HIPCHK(c, launch_ir_accumulate(c, resident ? 0 : k.stop_iter, fused ? cgf_p(c, k.stop_iter) : nullptr));
     st->inner_iters = k.iters;
     st->iterations = k.iters;
     st->cg_iters = k.iters;

@@ -244,7 +244,7 @@ struct Geo {
     int gyq, tyq;              // two-step PPCG kernel: gx2*gyq blocks of 2*TB columns x tyq rows
     Tiles s64;                 // single-sweep FP64 CG
     Tiles s32;                 // pairs of FP32 CG iterations
-    Tiles r64;                 // FP64 CG held in registers (blocks 0: the grid is too large)
+    Tiles r64, r32;            // CG held in registers (blocks 0: the grid is too large)
     int nbmax;                 // stride of the partial-sum arrays (max block count)
     size_t elems;              // elements per allocation
 };
@@ -401,6 +401,7 @@ hipError_t launch_resid_norm_slot(tl_ctx *c, const double *b, const double *x, i
 // iteration number from Ctrl::tg)
 hipError_t launch_cgs64(tl_ctx *c, int t, int tref = 0);
 hipError_t launch_cgr64(tl_ctx *c, int t0, int n);
+hipError_t launch_cgr32(tl_ctx *c, int t0, int n, bool first);
 hipError_t launch_cgs_dots(tl_ctx *c, int T);
 hipError_t launch_cgs_pending(tl_ctx *c, int T);
 hipError_t launch_cgs_final(tl_ctx *c, int T);

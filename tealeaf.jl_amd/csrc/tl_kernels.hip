@@ -134,17 +134,22 @@ Geo make_geo(int nx, int ny, int hd)
     // k_cgr: 2 rows per wave, or 4 where 2048 waves of 2 do not hold the grid
     // (us per iteration, 2 / 4 rows: 64^2 5.6 / 6.4, 256^2 5.8 / 6.4, 512^2 6.9 /
     // 7.0, 700x500 7.4 / 7.1)
-    g.r64 = Tiles{};
-    for (int rw = 2; rw <= 4 && !g.r64.blocks; rw *= 2) {
-        Tiles o;
-        o.strips = (nx + TL_S64_COLS - 1) / TL_S64_COLS;
-        o.bands = (ny + rw - 1) / rw;
-        o.ty = rw;
-        const long blocks = ((long)o.strips * o.bands + CGR_NT / 64 - 1) / (CGR_NT / 64);
-        o.blocks = (int)blocks;
-        if (blocks <= CGR_MAXB) g.r64 = o;
-    }
-    g.nbmax = std::max(g.nbmax, g.r64.blocks);
+    const auto resident = [&](int cols) {
+        Tiles o{};
+        for (o.ty = 2; o.ty <= 4; o.ty *= 2) {
+            o.strips = (nx + cols - 1) / cols;
+            o.bands = (ny + o.ty - 1) / o.ty;
+            const long blocks = ((long)o.strips * o.bands + CGR_NT / 64 - 1) / (CGR_NT / 64);
+            if (blocks <= CGR_MAXB) {
+                o.blocks = (int)blocks;
+                return o;
+            }
+        }
+        return Tiles{};
+    };
+    g.r64 = resident(120);
+    g.r32 = resident(240);
+    g.nbmax = std::max(g.nbmax, std::max(g.r64.blocks, g.r32.blocks));
     g.s32 = make_tiles(nx, ny, TL_S32_COLS, TL_S32_WAVES, TL_S32_ROWS);
     g.nbmax = std::max(g.nbmax, std::max(g.s64.blocks, g.s32.blocks));
     int gxs;
@@ -1370,333 +1375,6 @@ __global__ __launch_bounds__(TBV) __attribute__((amdgpu_waves_per_eu(2))) void k
     write_block_sums<4, TBV>(acc, sout);
 }
 
-// Many iterations of k_cgs in one launch, for grids whose r, p, g and u fit the
-// register files: a wave keeps its tile (120 columns as in k_cgs, RW rows) and
-// the two cells around it in registers from the first iteration to the last.
-// The arithmetic is k_cgs's, cell by cell.  Per iteration a wave publishes the
-// cells of r(t) that its neighbours need, the second row and column from each
-// edge (r(t) of the cells next to a tile, and p(t) of both, they compute
-// themselves), a block its four sums; and every block waits until it has all
-// blocks' sums, which tells it that the neighbours' cells have arrived as well.
-//
-// Published values bypass the caches that the 8 XCDs do not share (agent scope);
-// a wave's cells are complete (vmcnt(0)) before its block's sums appear.  A sum's
-// place holds EMPTY, a signalling NaN that no arithmetic yields, until it is
-// written; the places of iteration t are emptied by their block at t + 1, when
-// all blocks have published again and so have read them, and are used again at
-// t + 3 (three sets).  Cells go to the two arrays of r in turn: whoever
-// overwrites r(t) has seen all sums of t + 1, published after r(t) was read.
-// All blocks run at once (cooperative launch) and a wait ends after CGR_SPIN
-// polls: a block that gives up records TL_E_HIP and leaves, and so do the others;
-// the host then solves again in sweeps.
-// Bound by the latency of one exchange per iteration: store, sums, poll, load
-// across the XCDs, 4 to 5 us.  Microseconds per iteration, sweeps / this: 64^2 10.4
-// / 5.6, 256^2 8.8 / 5.8, 512^2 9.0 / 6.9, 700x500 9.3 / 7.4, 900^2 12.6 / 8.5.
-// Measured and left: the neighbours' cells with EMPTY places of their own, polled
-// with the sums, spilled registers (512^2 9.6); so did 8 rows per wave, which
-// would reach 1.9 million cells (1501x1103 24.0 against 18.9 in sweeps).
-constexpr unsigned long long EMPTY = 0x7ff4dead00000000ull;
-constexpr int CGR_SPIN = 1 << 20;  // about a second
-
-__device__ __forceinline__ unsigned long long agent_load(const unsigned long long *p)
-{
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void agent_store(unsigned long long *p, unsigned long long v)
-{
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-__device__ __forceinline__ double cell_load(const double *p)
-{
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void cell_store(double *p, double v)
-{
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-__global__ __launch_bounds__(256) void k_cgr_clear(unsigned long long *__restrict__ places, size_t n)
-{
-    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) places[i] = EMPTY;
-}
-
-template <typename T>
-__device__ __forceinline__ T *bytes_on(T *p, unsigned n)
-{
-    return (T *)((char *)const_cast<std::remove_const_t<T> *>(p) + n);
-}
-
-template <int RW>
-__global__ __launch_bounds__(CGR_NT) __attribute__((amdgpu_waves_per_eu(2))) void k_cgr(
-    Geo g, int t0, int n, double *__restrict__ r_even, double *__restrict__ r_odd, double *__restrict__ p_even,
-    double *__restrict__ p_odd, double *__restrict__ u, const double *__restrict__ gc, double hx, double hy,
-    Ctrl *__restrict__ ctrl, const double *__restrict__ sin, unsigned nbin, double *__restrict__ sout,
-    unsigned long long *__restrict__ slots, double *__restrict__ hist_a, double *__restrict__ hist_b)
-{
-    typedef unsigned long long u64;
-    constexpr int V = 2, NR = RW + 4, NW = CGR_NT / 64;  // rows held: y0 - 2 .. y0 + RW + 1
-    if (t0 > ctrl->stop_iter) return;
-    __shared__ double sh[NW][4], sh2[NW][4];
-    __shared__ int gone;
-    __shared__ Ctrl rules;  // what the stop test reads, which does not change
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int nb = (int)gridDim.x, tidx = (int)blockIdx.x * NW + wave;
-    const int strip = tidx % g.r64.strips, band = tidx / g.r64.strips;
-    const bool tile = band < g.r64.bands;
-    const int y0 = band * RW, x = strip * TL_S64_COLS + (lane - 1) * V;
-    const bool act = tile && lane >= 1 && lane <= TL_S64_COLS / V && x < g.nx;
-    // lanes past the ring's column nx + 1 and rows past ny + 1 read those again;
-    // r and p of cells outside the domain are held as zeros, which the iterations
-    // leave as they are (the domain faces' coefficients are zero)
-    bool in[V];
-#pragma unroll
-    for (int j = 0; j < V; ++j) in[j] = tile && x + j >= 0 && x + j < g.nx;
-    auto inside = [&](int i) { return y0 - 2 + i >= 0 && y0 - 2 + i < g.ny; };
-    unsigned xb = (unsigned)(min(x, (g.nx + 1) / V * V) + XCOL) * (unsigned)sizeof(double);
-    auto row = [&](auto *q, int i) {
-        return bytes_on(q + (g.off - XCOL + (long)min(y0 - 2 + i, g.ny + 1) * g.pitch), xb);
-    };
-    double R[NR][V], P[NR][V], G[NR][V], U[RW][V];
-    if (threadIdx.x == 0) {
-        gone = 0;
-        rules = *ctrl;
-    }
-    {
-        const double *const r = (t0 & 1) ? r_even : r_odd, *const p = (t0 & 1) ? p_even : p_odd;
-#pragma unroll
-        for (int i = 0; i < NR; ++i) {
-#pragma unroll
-            for (int j = 0; j < V; ++j) R[i][j] = P[i][j] = G[i][j] = 0.0;
-            if (tile) {
-#pragma unroll
-                for (int j = 0; j < V; ++j) R[i][j] = cell_load(row(r, i) + j);
-                vload<double, V, false>(P[i], row(p, i));
-                vload<double, V, false>(G[i], row(gc, i));
-#pragma unroll
-                for (int j = 0; j < V; ++j)
-                    if (!in[j] || !inside(i)) R[i][j] = P[i][j] = 0.0;
-            }
-            if (i >= 2 && i < RW + 2) {
-#pragma unroll
-                for (int j = 0; j < V; ++j) U[i - 2][j] = 0.0;
-                if (tile) vload<double, V, false>(U[i - 2], row(u, i));
-            }
-        }
-    }
-    double s4[4];
-    sum_block_sums<4, CGR_NT>(sin, nbin, s4);
-    double gam_prev = t0 >= 2 ? ctrl->rrs[(t0 - 2) & 1] : 1.0;
-    int t = t0;
-    for (;;) {
-        const double gam = s4[0];
-        const int why = t >= 2 ? decide_why(&rules, t - 1, gam) : (int)WHY_NONE;
-        const double bd = t >= 2 ? gam / gam_prev : 0.0;
-        const double pap = s4[1] + bd * (2.0 * s4[2] + bd * s4[3]);
-        const double alpha = gam / pap;
-        const bool ok = pap > 0.0 && isfinite(alpha);
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
-            ctrl->rrs[(t - 1) & 1] = gam;
-            ctrl->rro = gam;
-            if (t >= 2) {
-                ctrl->err = gam;
-                ctrl->beta = bd;
-                ctrl->iters = t - 1;
-                hist_b[t - 2] = bd;
-                record_stop(ctrl, t - 1, why);
-            }
-            if (why == WHY_NONE) {
-                ctrl->pw = pap;
-                ctrl->alpha = alpha;
-                ctrl->alphas[t & 1] = alpha;
-                hist_a[t - 1] = alpha;
-                if (!ok) {  // non-positive curvature: stop before this iteration's update
-                    ctrl->status = TL_E_BREAKDOWN;
-                    ctrl->why = WHY_BREAKDOWN;
-                    ctrl->stop_iter = t - 1;
-                }
-            }
-        }
-        if (why != WHY_NONE || !ok) break;  // every block derives the same decision
-        gam_prev = gam;
-        // the face coefficients are formed anew in every iteration: kept over the
-        // loop they would not fit the registers
-#pragma unroll
-        for (int i = 0; i < NR; ++i)
-#pragma unroll
-            for (int j = 0; j < V; ++j) asm volatile("" : "+v"(G[i][j]));
-        double acc[4] = {0.0, 0.0, 0.0, 0.0};
-        // A applied to row i of c
-        auto apply = [&](double (&q)[V], const double (&c)[NR][V], int i) {
-            double D[V + 1], KX[V + 1];
-            KX[0] = hx * (lane_up1<true>(G[i][V - 1]) + G[i][0]);
-            D[0] = c[i][0] - lane_up1<true>(c[i][V - 1]);
-#pragma unroll
-            for (int j = 1; j < V; ++j) {
-                KX[j] = hx * (G[i][j - 1] + G[i][j]);
-                D[j] = c[i][j] - c[i][j - 1];
-            }
-            KX[V] = lane_down1<true>(KX[0]);
-            D[V] = lane_down1<true>(D[0]);
-#pragma unroll
-            for (int j = 0; j < V; ++j) {
-                double s = KX[j] * D[j];
-                s = __builtin_fma(-KX[j + 1], D[j + 1], s);
-                s = __builtin_fma(hy * (G[i - 1][j] + G[i][j]), c[i][j] - c[i - 1][j], s);
-                s = __builtin_fma(hy * (G[i][j] + G[i + 1][j]), c[i][j] - c[i + 1][j], s);
-                q[j] = c[i][j] + s;
-            }
-        };
-#pragma unroll
-        for (int i = 0; i < NR; ++i)
-#pragma unroll
-            for (int j = 0; j < V; ++j) P[i][j] = __builtin_fma(bd, P[i][j], R[i][j]);
-#pragma unroll
-        for (int i = 1; i < NR - 1; ++i) {
-            double q[V];
-            apply(q, P, i);
-#pragma unroll
-            for (int j = 0; j < V; ++j) R[i][j] = __builtin_fma(-alpha, q[j], R[i][j]);
-            if (i >= 2 && i < RW + 2) {
-#pragma unroll
-                for (int j = 0; j < V; ++j) {
-                    U[i - 2][j] = __builtin_fma(alpha, P[i][j], U[i - 2][j]);
-                    if (act) {
-                        acc[2] = __builtin_fma(R[i][j], q[j], acc[2]);
-                        acc[3] = __builtin_fma(P[i][j], q[j], acc[3]);
-                    }
-                }
-            }
-        }
-        const bool last = t == t0 + n - 1;
-        double *const rt = (t & 1) ? r_odd : r_even;
-        if (!last) {
-            // the cells that neighbours need: rows 1 and RW - 2, columns 1 and W - 2
-#pragma unroll
-            for (int i = 2; i < RW + 2; ++i) {
-                if (!inside(i)) continue;
-                double *const q = row(rt, i);
-                if (i == 3 || i == RW) {
-                    if (act) {
-                        cell_store(q, R[i][0]);
-                        cell_store(q + 1, R[i][1]);
-                    }
-                } else if (act && (lane == 1 || lane == TL_S64_COLS / V)) {
-                    cell_store(q + (lane == 1 ? 1 : 0), lane == 1 ? R[i][1] : R[i][0]);
-                }
-            }
-        }
-#pragma unroll
-        for (int i = 2; i < RW + 2; ++i) {
-            double ar[V];
-            apply(ar, R, i);
-            if (act) {
-#pragma unroll
-                for (int j = 0; j < V; ++j) {
-                    acc[0] = __builtin_fma(R[i][j], R[i][j], acc[0]);
-                    acc[1] = __builtin_fma(R[i][j], ar[j], acc[1]);
-                }
-            }
-        }
-        if (last) {
-            write_block_sums<4, CGR_NT>(acc, sout);
-            ++t;
-            break;
-        }
-        // the sums of iteration t + 1
-        const int e = (t - t0) % 3, pe = (t - t0 + 2) % 3;
-        {
-            const double ws = wave_sums<4>(acc);
-            if ((lane & 15) == 0) sh[wave][lane >> 4] = ws;
-        }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the published cells have arrived
-        __syncthreads();
-        if (nb > 1) {
-            u64 *const se = slots + (size_t)e * 4 * CGR_MAXB;
-            if (threadIdx.x < 4) {
-                double b = sh[0][threadIdx.x];
-#pragma unroll
-                for (int w = 1; w < NW; ++w) b += sh[w][threadIdx.x];
-                agent_store(&se[threadIdx.x * CGR_MAXB + blockIdx.x], (u64)__double_as_longlong(b));
-            }
-            double v[4] = {0.0, 0.0, 0.0, 0.0};
-            if ((int)threadIdx.x < nb) {
-                u64 q[4];
-                for (int spin = 0;; ++spin) {
-                    bool full = true;
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) {
-                        q[k] = agent_load(&se[k * CGR_MAXB + threadIdx.x]);
-                        full = full && q[k] != EMPTY;
-                    }
-                    if (full) break;
-                    if (spin > CGR_SPIN) {
-                        gone = 1;
-                        break;
-                    }
-                }
-#pragma unroll
-                for (int k = 0; k < 4; ++k) v[k] = __longlong_as_double((long long)q[k]);
-            }
-            const double ws = wave_sums<4>(v);
-            if ((lane & 15) == 0) sh2[wave][lane >> 4] = ws;
-        } else if ((lane & 15) == 0) {
-            sh2[wave][lane >> 4] = sh[wave][lane >> 4];
-        }
-        __syncthreads();
-        if (gone) {
-            if (threadIdx.x == 0) {
-                ctrl->status = TL_E_HIP;
-                ctrl->why = WHY_BREAKDOWN;
-                ctrl->stop_iter = t;
-            }
-            return;
-        }
-        // the neighbours' cells two away: rows -2 and RW + 1, columns -2 and W + 1
-        if (tile) {
-#pragma unroll
-            for (int j = 0; j < V; ++j) {
-                const double a = cell_load(row(rt, 0) + j), b = cell_load(row(rt, NR - 1) + j);
-                R[0][j] = in[j] && inside(0) ? a : 0.0;
-                R[NR - 1][j] = in[j] && inside(NR - 1) ? b : 0.0;
-            }
-            if (lane == 0 || lane == TL_S64_COLS / V + 1) {
-                double h[NR];
-#pragma unroll
-                for (int i = 1; i < NR - 1; ++i) {
-                    const double a = cell_load(row(rt, i) + (lane == 0 ? 0 : 1));
-                    h[i] = (lane == 0 ? in[0] : in[1]) && inside(i) ? a : 0.0;
-                }
-#pragma unroll
-                for (int i = 1; i < NR - 1; ++i) {
-                    R[i][0] = lane == 0 ? h[i] : R[i][0];
-                    R[i][1] = lane == 0 ? R[i][1] : h[i];
-                }
-            }
-        }
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            double b = sh2[0][k];
-#pragma unroll
-            for (int w = 1; w < NW; ++w) b += sh2[w][k];
-            s4[k] = b;
-        }
-        if (nb > 1 && threadIdx.x < 4 && t > t0)  // empty the places of iteration t - 1
-            agent_store(&slots[((size_t)pe * 4 + threadIdx.x) * CGR_MAXB + blockIdx.x], EMPTY);
-        ++t;
-    }
-    // r, p and u of the last iteration, T = t - 1
-    if (t == t0 || !tile) return;
-    double *const rT = (t & 1) ? r_even : r_odd, *const pT = (t & 1) ? p_even : p_odd;
-#pragma unroll
-    for (int i = 2; i < RW + 2; ++i)
-        if (act && y0 - 2 + i < g.ny) {
-            vstore<double, V, false>(row(rT, i), R[i]);
-            vstore<double, V, false>(row(pT, i), P[i]);
-            vstore<double, V, false>(row(u, i), U[i - 2]);
-        }
-}
-
 // The four sums k_cgs needs at its first iteration and after a new true
 // residual, for r and the kept direction p, with its operator.  One thread per
 // cell of a column band; runs once per start or new residual.
@@ -2867,6 +2545,384 @@ template <int FMT, bool UPD>
 __global__ __launch_bounds__(TBV) __attribute__((amdgpu_waves_per_eu(3))) void k_cgp_cached(TL_CGP_ARGS)
 {
     cgp_sweep<FMT, UPD, false>(g, t, rin, rout, pin, pout, x, gc, hx, hy, ctrl, sin, nbin, sout);
+}
+
+// Many iterations of single-reduction CG (k_cgs) in one launch, in FP64 or, as
+// inner CG of the mixed-precision solver, in FP32, for grids whose r, p,
+// coefficients and u (FP32: the correction x) fit the register files: a wave keeps
+// its tile (60 lanes of 16 bytes, 120 or 240 columns, by RW rows) and the cells
+// around it in registers from the first iteration to the last.  The arithmetic is
+// k_cgs's, cell by cell, and in FP32 that with FP64 sums and the operator of the
+// pairs (k_cgp).  FMT: the FP32 form's 16-bit coefficients.  Per iteration a wave publishes the
+// cells of r(t) that its neighbours need, the second row and column from each
+// edge (r(t) of the cells next to a tile, and p(t) of both, they compute
+// themselves), a block its four sums; and every block waits until it has all
+// blocks' sums, which tells it that the neighbours' cells have arrived as well.
+//
+// Published values bypass the caches that the 8 XCDs do not share (agent scope);
+// a wave's cells are complete (vmcnt(0)) before its block's sums appear.  A sum's
+// place holds EMPTY, a signalling NaN that no arithmetic yields, until it is
+// written; the places of iteration t are emptied by their block at t + 1, when
+// all blocks have published again and so have read them, and are used again at
+// t + 3 (three sets).  Cells go to the two arrays of r in turn: whoever
+// overwrites r(t) has seen all sums of t + 1, published after r(t) was read.
+// All blocks run at once (cooperative launch) and a wait ends after CGR_SPIN
+// polls: a block that gives up records TL_E_HIP and leaves, and so do the others;
+// the host then solves again in sweeps.
+// Bound by the latency of one exchange per iteration: store, sums, poll, load
+// across the XCDs, 4 to 5 us.  Microseconds per iteration, sweeps / this: 64^2 10.4
+// / 5.6, 256^2 8.8 / 5.8, 512^2 9.0 / 6.9, 700x500 9.3 / 7.4, 900^2 12.6 / 8.2;
+// FP32, pairs / this: 182^2 13.2 / 7.8, 256^2 11.4 / 7.5, 512x400 10.5 / 7.5, 1024^2
+// 11.0 / 9.3.
+// Measured and left: the neighbours' cells with EMPTY places of their own, polled
+// with the sums, spilled registers (512^2 9.6); so did 8 rows per wave, which
+// would hold twice the cells (FP64 1501x1103 24.0 against 18.9 in sweeps, FP32
+// 2047x1533 20.2 against 17.4 in pairs).
+constexpr unsigned long long EMPTY = 0x7ff4dead00000000ull;
+constexpr int CGR_SPIN = 1 << 20;  // about a second
+
+__device__ __forceinline__ unsigned long long agent_load(const unsigned long long *p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void agent_store(unsigned long long *p, unsigned long long v)
+{
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+template <typename T>
+__device__ __forceinline__ T cell_load(const T *p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T>
+__device__ __forceinline__ void cell_store(T *p, T v)
+{
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__global__ __launch_bounds__(256) void k_cgr_clear(unsigned long long *__restrict__ places, size_t n)
+{
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) places[i] = EMPTY;
+}
+
+template <typename T>
+__device__ __forceinline__ T *bytes_on(T *p, unsigned n)
+{
+    return (T *)((char *)const_cast<std::remove_const_t<T> *>(p) + n);
+}
+
+__device__ __forceinline__ double fma_(double a, double b, double c) { return __builtin_fma(a, b, c); }
+__device__ __forceinline__ float fma_(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double next_up1(double v) { return lane_up1<true>(v); }
+__device__ __forceinline__ float next_up1(float v) { return dpp_up1f(v); }
+__device__ __forceinline__ double next_down1(double v) { return lane_down1<true>(v); }
+__device__ __forceinline__ float next_down1(float v) { return dpp_down1f(v); }
+
+template <typename T, int FMT, int RW>
+__global__ __launch_bounds__(CGR_NT) __attribute__((amdgpu_waves_per_eu(2))) void k_cgr(
+    Geo g, Tiles o, int t0, int n, T *__restrict__ r_even, T *__restrict__ r_odd, T *__restrict__ p_even,
+    T *__restrict__ p_odd, T *__restrict__ u, const std::conditional_t<sizeof(T) == 8, double, tl_gc_t> *__restrict__ gc,
+    T hx, T hy, Ctrl *__restrict__ ctrl, const double *__restrict__ sin, unsigned nbin, int side, double *__restrict__ sout,
+    unsigned long long *__restrict__ slots, double *__restrict__ hist_a, double *__restrict__ hist_b)
+{
+    typedef unsigned long long u64;
+    constexpr bool F64 = sizeof(T) == 8;
+    constexpr int V = 16 / sizeof(T), COLS = 60 * V, NR = RW + 4, NW = CGR_NT / 64;  // rows held: y0 - 2 .. y0 + RW + 1
+    if (t0 > ctrl->stop_iter) return;
+    __shared__ double sh[NW][4], sh2[NW][4];
+    __shared__ int gone;
+    __shared__ Ctrl rules;  // what the stop test reads, which does not change
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nb = (int)gridDim.x, tidx = (int)blockIdx.x * NW + wave;
+    const int strip = tidx % o.strips, band = tidx / o.strips;
+    const bool tile = band < o.bands;
+    const int y0 = band * RW, x = strip * COLS + (lane - 1) * V;
+    const bool act = tile && lane >= 1 && lane <= 60 && x < g.nx;
+    // lanes past the one beside the last owner and rows past ny + 1 read those again;
+    // r and p of cells outside the domain are held as zeros, which the iterations
+    // leave as they are (the domain faces' coefficients are zero)
+    bool in[V];
+#pragma unroll
+    for (int j = 0; j < V; ++j) in[j] = tile && x + j >= 0 && x + j < g.nx;
+    auto inside = [&](int i) { return y0 - 2 + i >= 0 && y0 - 2 + i < g.ny; };
+    unsigned xb = (unsigned)(min(x, (g.nx - 1) / V * V + V) + XCOL) * (unsigned)sizeof(T);
+    auto row = [&](auto *q, int i) {
+        return bytes_on(q + (g.off - XCOL + (long)min(y0 - 2 + i, g.ny + 1) * g.pitch), xb);
+    };
+    T R[NR][V], P[NR][V], U[RW][V];
+    struct Coef {
+        double d[F64 ? V : 1];
+        GcRaw<4> h;
+    } G[NR];
+    auto coef = [&](T (&c)[V], int i) {
+        if constexpr (F64) {
+#pragma unroll
+            for (int j = 0; j < V; ++j) c[j] = G[i].d[j];
+        } else {
+            gc_unpack<V, FMT>(c, G[i].h);
+        }
+    };
+    if (threadIdx.x == 0) {
+        gone = 0;
+        rules = *ctrl;
+    }
+    {
+        const T *const r = (t0 & 1) ? r_even : r_odd, *const p = (t0 & 1) ? p_even : p_odd;
+#pragma unroll
+        for (int i = 0; i < NR; ++i) {
+#pragma unroll
+            for (int j = 0; j < V; ++j) R[i][j] = P[i][j] = 0;
+            G[i] = Coef{};
+            if (tile) {
+#pragma unroll
+                for (int j = 0; j < V; ++j) R[i][j] = cell_load(row(r, i) + j);
+                vload<T, V, false>(P[i], row(p, i));
+                if constexpr (F64)
+                    vload<double, V, false>(G[i].d, row(gc, i));
+                else  // half the bytes of a field's
+                    gc_load_raw<V>(G[i].h, gc + (row(r, i) - r));
+#pragma unroll
+                for (int j = 0; j < V; ++j)
+                    if (!in[j] || !inside(i)) R[i][j] = P[i][j] = 0;
+            }
+            if (i >= 2 && i < RW + 2) {
+#pragma unroll
+                for (int j = 0; j < V; ++j) U[i - 2][j] = 0;
+                if (tile) vload<T, V, false>(U[i - 2], row(u, i));
+            }
+        }
+    }
+    double s4[4];
+    if (side)
+        sum_block_sums<4, CGR_NT>(sin, nbin, s4);
+    else  // k_cgf_dots: one sum after the other
+        sum_partials<4, CGR_NT>(sin, nbin, g.nbmax, s4);
+    double gam_prev = t0 >= 2 ? ctrl->rrs[(t0 - 2) & 1] : 1.0;
+    int t = t0;
+    for (;;) {
+        const double gam = s4[0];
+        const int why = !F64 || t >= 2 ? decide_why(&rules, t - 1, gam) : (int)WHY_NONE;
+        const double bd = t >= 2 ? gam / gam_prev : 0.0;
+        const double pap = s4[1] + bd * (2.0 * s4[2] + bd * s4[3]);
+        const double alpha = gam / pap;
+        const bool ok = pap > 0.0 && isfinite(alpha);
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            ctrl->rrs[(t - 1) & 1] = gam;
+            ctrl->rro = gam;
+            if (!F64 || t >= 2) {
+                ctrl->err = gam;
+                ctrl->beta = bd;
+                ctrl->iters = t - 1;
+                if (F64) hist_b[t - 2] = bd;
+                record_stop(ctrl, t - 1, why);
+            }
+            if (why == WHY_NONE) {
+                ctrl->pw = pap;
+                ctrl->alpha = alpha;
+                ctrl->alphas[t & 1] = alpha;
+                if (F64) hist_a[t - 1] = alpha;
+                if (!ok) {  // non-positive curvature: stop before this iteration's update
+                    ctrl->status = TL_E_BREAKDOWN;
+                    ctrl->why = WHY_BREAKDOWN;
+                    ctrl->stop_iter = t - 1;
+                }
+            }
+        }
+        if (why != WHY_NONE || !ok) break;  // every block derives the same decision
+        gam_prev = gam;
+        const T beta = (T)bd, al = (T)alpha;
+        // the face coefficients are formed anew in every iteration, with many rows
+        // for each operator: kept they would not fit the registers
+        auto anew = [&]() {
+#pragma unroll
+            for (int i = 0; i < NR; ++i) {
+                if constexpr (F64) {
+#pragma unroll
+                    for (int j = 0; j < V; ++j) asm volatile("" : "+v"(G[i].d[j]));
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) asm volatile("" : "+v"(G[i].h.w[j]));
+                }
+            }
+        };
+        anew();
+        double acc[4] = {0.0, 0.0, 0.0, 0.0};
+        // A applied to row i of c
+        auto apply = [&](T (&q)[V], const T (&c)[NR][V], int i) {
+            T D[V + 1], KX[V + 1], gd[V], gm[V], gu[V];
+            coef(gd, i - 1);
+            coef(gm, i);
+            coef(gu, i + 1);
+            KX[0] = hx * (next_up1(gm[V - 1]) + gm[0]);
+            D[0] = c[i][0] - next_up1(c[i][V - 1]);
+#pragma unroll
+            for (int j = 1; j < V; ++j) {
+                KX[j] = hx * (gm[j - 1] + gm[j]);
+                D[j] = c[i][j] - c[i][j - 1];
+            }
+            KX[V] = next_down1(KX[0]);
+            D[V] = next_down1(D[0]);
+#pragma unroll
+            for (int j = 0; j < V; ++j) {
+                T s = KX[j] * D[j];
+                s = fma_(-KX[j + 1], D[j + 1], s);
+                s = fma_(hy * (gd[j] + gm[j]), c[i][j] - c[i - 1][j], s);
+                s = fma_(hy * (gm[j] + gu[j]), c[i][j] - c[i + 1][j], s);
+                q[j] = c[i][j] + s;
+            }
+        };
+#pragma unroll
+        for (int i = 0; i < NR; ++i)
+#pragma unroll
+            for (int j = 0; j < V; ++j) P[i][j] = fma_(beta, P[i][j], R[i][j]);
+#pragma unroll
+        for (int i = 1; i < NR - 1; ++i) {
+            T q[V];
+            apply(q, P, i);
+#pragma unroll
+            for (int j = 0; j < V; ++j) R[i][j] = fma_(-al, q[j], R[i][j]);
+            if (i >= 2 && i < RW + 2) {
+#pragma unroll
+                for (int j = 0; j < V; ++j) {
+                    U[i - 2][j] = fma_(al, P[i][j], U[i - 2][j]);
+                    if (act) {
+                        acc[2] = __builtin_fma((double)R[i][j], (double)q[j], acc[2]);
+                        acc[3] = __builtin_fma((double)P[i][j], (double)q[j], acc[3]);
+                    }
+                }
+            }
+        }
+        const bool last = t == t0 + n - 1;
+        T *const rt = (t & 1) ? r_odd : r_even;
+        if (!last) {
+            // the cells that neighbours need: rows 1 and RW - 2, columns 1 and W - 2
+#pragma unroll
+            for (int i = 2; i < RW + 2; ++i) {
+                if (!inside(i)) continue;
+                T *const q = row(rt, i);
+                if (i == 3 || i == RW) {
+                    if (act) {
+#pragma unroll
+                        for (int j = 0; j < V; ++j) cell_store(q + j, R[i][j]);
+                    }
+                } else if (act && (lane == 1 || lane == 60)) {
+                    cell_store(q + (lane == 1 ? 1 : V - 2), lane == 1 ? R[i][1] : R[i][V - 2]);
+                }
+            }
+        }
+        if constexpr (RW >= 4) anew();
+#pragma unroll
+        for (int i = 2; i < RW + 2; ++i) {
+            T ar[V];
+            apply(ar, R, i);
+            if (act) {
+#pragma unroll
+                for (int j = 0; j < V; ++j) {
+                    acc[0] = __builtin_fma((double)R[i][j], (double)R[i][j], acc[0]);
+                    acc[1] = __builtin_fma((double)R[i][j], (double)ar[j], acc[1]);
+                }
+            }
+        }
+        if (last) {
+            write_block_sums<4, CGR_NT>(acc, sout);
+            ++t;
+            break;
+        }
+        // the sums of iteration t + 1
+        const int e = (t - t0) % 3, pe = (t - t0 + 2) % 3;
+        {
+            const double ws = wave_sums<4>(acc);
+            if ((lane & 15) == 0) sh[wave][lane >> 4] = ws;
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the published cells have arrived
+        __syncthreads();
+        if (nb > 1) {
+            u64 *const se = slots + (size_t)e * 4 * CGR_MAXB;
+            if (threadIdx.x < 4) {
+                double b = sh[0][threadIdx.x];
+#pragma unroll
+                for (int w = 1; w < NW; ++w) b += sh[w][threadIdx.x];
+                agent_store(&se[threadIdx.x * CGR_MAXB + blockIdx.x], (u64)__double_as_longlong(b));
+            }
+            double v[4] = {0.0, 0.0, 0.0, 0.0};
+            if ((int)threadIdx.x < nb) {
+                u64 q[4];
+                for (int spin = 0;; ++spin) {
+                    bool full = true;
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        q[k] = agent_load(&se[k * CGR_MAXB + threadIdx.x]);
+                        full = full && q[k] != EMPTY;
+                    }
+                    if (full) break;
+                    if (spin > CGR_SPIN) {
+                        gone = 1;
+                        break;
+                    }
+                }
+#pragma unroll
+                for (int k = 0; k < 4; ++k) v[k] = __longlong_as_double((long long)q[k]);
+            }
+            const double ws = wave_sums<4>(v);
+            if ((lane & 15) == 0) sh2[wave][lane >> 4] = ws;
+        } else if ((lane & 15) == 0) {
+            sh2[wave][lane >> 4] = sh[wave][lane >> 4];
+        }
+        __syncthreads();
+        if (gone) {
+            if (threadIdx.x == 0) {
+                ctrl->status = TL_E_HIP;
+                ctrl->why = WHY_BREAKDOWN;
+                ctrl->stop_iter = t;
+            }
+            return;
+        }
+        // the neighbours' cells two away: rows -2 and RW + 1, columns -2 and W + 1
+        if (tile) {
+#pragma unroll
+            for (int j = 0; j < V; ++j) {
+                const T a = cell_load(row(rt, 0) + j), b = cell_load(row(rt, NR - 1) + j);
+                R[0][j] = in[j] && inside(0) ? a : (T)0;
+                R[NR - 1][j] = in[j] && inside(NR - 1) ? b : (T)0;
+            }
+            if (lane == 0 || lane == 60 + 1) {
+                const int j = lane == 0 ? V - 2 : 1;
+                T h[NR];
+#pragma unroll
+                for (int i = 1; i < NR - 1; ++i) {
+                    const T a = cell_load(row(rt, i) + j);
+                    h[i] = (lane == 0 ? in[V - 2] : in[1]) && inside(i) ? a : (T)0;
+                }
+                // V = 2: columns 0 and 1 of the lane, V = 4: 2 and 1
+#pragma unroll
+                for (int i = 1; i < NR - 1; ++i) {
+                    R[i][V - 2] = lane == 0 ? h[i] : R[i][V - 2];
+                    R[i][1] = lane == 0 ? R[i][1] : h[i];
+                }
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            double b = sh2[0][k];
+#pragma unroll
+            for (int w = 1; w < NW; ++w) b += sh2[w][k];
+            s4[k] = b;
+        }
+        if (nb > 1 && threadIdx.x < 4 && t > t0)  // empty the places of iteration t - 1
+            agent_store(&slots[((size_t)pe * 4 + threadIdx.x) * CGR_MAXB + blockIdx.x], EMPTY);
+        ++t;
+    }
+    // r, p and u of the last iteration, T = t - 1
+    if (t == t0 || !tile) return;
+    T *const rT = (t & 1) ? r_even : r_odd, *const pT = (t & 1) ? p_even : p_odd;
+#pragma unroll
+    for (int i = 2; i < RW + 2; ++i)
+        if (act && y0 - 2 + i < g.ny) {
+            vstore<T, V, false>(row(rT, i), R[i]);
+            vstore<T, V, false>(row(pT, i), P[i]);
+            vstore<T, V, false>(row(u, i), U[i - 2]);
+        }
 }
 
 // The four sums k_cgf needs at its first iteration and after an FP64 refresh,
@@ -4170,23 +4226,27 @@ hipError_t launch_cgs64(tl_ctx *c, int t, int tref)
 }
 
 // iterations t0 .. t0 + n - 1 in one launch (k_cgr); u has every update after it
+static hipError_t launch_resident(tl_ctx *c, const void *kern, const Tiles &o, void **args)
+{
+    if (o.blocks == 1) return hipLaunchKernel(kern, dim3(1), dim3(CGR_NT), args, 0, c->stream);
+    k_cgr_clear<<<12, 256, 0, c->stream>>>(c->slots, 3 * 4 * CGR_MAXB);
+    return hipLaunchCooperativeKernel(kern, dim3(o.blocks), dim3(CGR_NT), args, 0, c->stream);
+}
+
 hipError_t launch_cgr64(tl_ctx *c, int t0, int n)
 {
-    const bool one = c->g.r64.blocks == 1;
-    if (!one) k_cgr_clear<<<12, 256, 0, c->stream>>>(c->slots, 3 * 4 * CGR_MAXB);
     Geo g = c->g;
+    Tiles o = g.r64;
     double *re = cgs_r(c, 0), *ro = cgs_r(c, 1), *pe = cgs_p(c, 0), *po = cgs_p(c, 1), *u = cgs_u(c);
     const double *gc = c->g64, *sin = part_f(c, t0 - 1);
     double hx = c->hx64, hy = c->hy64, *sout = part_f(c, t0 + n - 1);
-    Ctrl *ctrl = c->ctrl;
-    unsigned nbin = c->nb_f[(t0 - 1) & 1];
-    unsigned long long *slots = c->slots;
-    double *ha = c->hist_a, *hb = c->hist_b;
-    void *args[] = {&g, &t0, &n, &re, &ro, &pe, &po, &u, &gc, &hx, &hy, &ctrl, &sin, &nbin, &sout, &slots, &ha, &hb};
-    const void *kern = g.r64.ty == 2 ? (const void *)k_cgr<2> : (const void *)k_cgr<4>;
-    c->nb_f[(t0 + n - 1) & 1] = (unsigned)g.r64.blocks;
-    return one ? hipLaunchKernel(kern, dim3(1), dim3(CGR_NT), args, 0, c->stream)
-               : hipLaunchCooperativeKernel(kern, dim3(g.r64.blocks), dim3(CGR_NT), args, 0, c->stream);
+    int side = 1;
+    void *args[] = {&g, &o, &t0, &n, &re, &ro, &pe, &po, &u, &gc, &hx, &hy, &c->ctrl, &sin, &c->nb_f[(t0 - 1) & 1], &side,
+                    &sout, &c->slots, &c->hist_a, &c->hist_b};
+    const void *kern = o.ty == 2 ? (const void *)k_cgr<double, 0, 2> : (const void *)k_cgr<double, 0, 4>;
+    const hipError_t e = launch_resident(c, kern, o, args);
+    c->nb_f[(t0 + n - 1) & 1] = (unsigned)o.blocks;
+    return e;
 }
 
 // the four sums of r(T) and p(T) for iteration T+1 (after a start or a new
@@ -4613,6 +4673,26 @@ hipError_t launch_cgf_dots(tl_ctx *c, int T)
                                             part_f(c, T));
     c->nb_f[T & 1] = nbh(c);
     return hipGetLastError();
+}
+
+// FP32 inner iterations t0 .. t0 + n - 1 in one launch (k_cgr), x complete after
+// it; first: after k_cgf_dots (a start or a refresh)
+hipError_t launch_cgr32(tl_ctx *c, int t0, int n, bool first)
+{
+    Geo g = c->g;
+    Tiles o = g.r32;
+    float *re = cgf_r(c, 0), *ro = cgf_r(c, 1), *pe = cgf_p(c, 0), *po = cgf_p(c, 1);
+    const double *sin = part_f(c, t0 - 1);
+    double *sout = part_f(c, t0 + n - 1), *none = nullptr;
+    int side = !first;
+    void *args[] = {&g,       &o,        &t0,   &n,    &re,  &ro,   &pe,       &po,   &c->x32, &c->gcell, &c->hx32,
+                    &c->hy32, &c->ctrl, &sin,  &c->nb_f[(t0 - 1) & 1], &side, &sout, &c->slots, &none, &none};
+    const bool h = c->gc_fmt == GC_F16;
+    const void *kern = o.ty == 2 ? (h ? (const void *)k_cgr<float, GC_F16, 2> : (const void *)k_cgr<float, GC_BF16, 2>)
+                                 : (h ? (const void *)k_cgr<float, GC_F16, 4> : (const void *)k_cgr<float, GC_BF16, 4>);
+    const hipError_t e = launch_resident(c, kern, o, args);
+    c->nb_f[(t0 + n - 1) & 1] = (unsigned)o.blocks;
+    return e;
 }
 
 }  // namespace tl
