@@ -1061,6 +1061,7 @@ static int unet_alloc(tl_ctx *c, Unet *u)
         if (int rc = ualloc(c, (void **)&u->wt[l], nw * sizeof(bf16))) return rc;
     }
     if (int rc = ualloc(c, (void **)&u->scale, 4 * sizeof(float))) return rc;
+    if (int rc = ualloc(c, (void **)&u->flat, (size_t)tl_unet_param_count() * sizeof(float))) return rc;
     return ualloc(c, (void **)&u->mx_part, 3 * 1024 * sizeof(float));
 }
 
@@ -1355,8 +1356,6 @@ static int get_flat(tl_ctx *c, Unet *u, float *const *w, float *const *b, float 
 {
     UCHK(c, hipSetDevice(c->device));
     const size_t n = (size_t)tl_unet_param_count();
-    if (!u->flat)
-        if (int rc = ualloc(c, (void **)&u->flat, n * sizeof(float))) return rc;
     FlatArgs a;
     int first = 0;
     for (int l = 0; l < NL; ++l) {
