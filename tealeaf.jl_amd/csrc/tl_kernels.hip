@@ -153,7 +153,8 @@ Geo make_geo(int nx, int ny, int hd)
     g.s32 = make_tiles(nx, ny, TL_S32_COLS, TL_S32_WAVES, TL_S32_ROWS);
     g.nbmax = std::max(g.nbmax, std::max(g.s64.blocks, g.s32.blocks));
     int gxs;
-    g.nbmax = std::max(g.nbmax, (int)steps_blocks(steps_tiles(nx, ny, 64, 32, gxs)));  // its smallest tiles
+    g.nbmax = std::max(g.nbmax, (int)steps_blocks(steps_tiles(nx, ny, 64, 32, gxs)));  // its smallest tiles but one
+    g.nbmax = std::max(g.nbmax, (int)steps_blocks(256));                               // at most that many of 64 x 24
     return g;
 }
 
@@ -4479,11 +4480,15 @@ hipError_t launch_ppcg_inner2(tl_ctx *c, double a1, double b1, double a2, double
 // CUs, else 64 x 32.  Measured, PPCG iterations with 10 inner steps, 128x64 /
 // 64x32 / 128x32 tiles: 500x600 (65 tiles of 128x64) 36.6 / 33.3 / 33.1 us,
 // 800x700 (120) 43.4 / 42.2 / 44.9; 1000x900 (171) 48.8 and 128x32 55.1,
-// 1000x1300 (252) 62.7 and 70.3, 1600x1500 (480) 110.7 and 124.3.
-template <class F>
+// 1000x1300 (252) 62.7 and 70.3, 1600x1500 (480) 110.7 and 124.3.  Jacobi takes
+// 64 x 24 where that is one tile per CU at most (3000 iterations at 200x300, 190
+// such tiles: 6.7 ms, 95 of 64x32 7.3 ms; Chebyshev and PPCG within 2%).
+template <bool JACOBI = false, class F>
 static hipError_t with_steps_tile(const Geo &g, F &&f)
 {
     int gx;
+    if (JACOBI && steps_tiles(g.nx, g.ny, 64, 24, gx) <= 256)
+        return f(std::integral_constant<int, 1>{}, std::integral_constant<int, 8>{}, std::integral_constant<int, 3>{});
     if (steps_tiles(g.nx, g.ny, 128, 64, gx) >= 128)
         return f(std::integral_constant<int, 2>{}, std::integral_constant<int, 8>{}, std::integral_constant<int, 8>{});
     return f(std::integral_constant<int, 1>{}, std::integral_constant<int, 8>{}, std::integral_constant<int, 4>{});
@@ -4525,7 +4530,7 @@ hipError_t launch_jacobi_steps(tl_ctx *c, int n, const double *u_in, double *u_o
 {
     c->jset ^= 1;
     const bool prof = prof_start(c, TL_K_JACOBI64);
-    const hipError_t e = with_steps_tile(c->g, [&](auto v, auto nw, auto rw) {
+    const hipError_t e = with_steps_tile<true>(c->g, [&](auto v, auto nw, auto rw) {
         constexpr int V = decltype(v)::value, NW = decltype(nw)::value, RW = decltype(rw)::value;
         int gx;
         const unsigned nb = steps_blocks(steps_tiles(c->g.nx, c->g.ny, 64 * V, NW * RW, gx));
@@ -4541,7 +4546,7 @@ hipError_t launch_jacobi_steps(tl_ctx *c, int n, const double *u_in, double *u_o
 // the stop test of the last launch's steps, which ended before iteration t
 hipError_t launch_jacobi_end(tl_ctx *c, int nprev, int residp, int t)
 {
-    return with_steps_tile(c->g, [&](auto v, auto nw, auto rw) {
+    return with_steps_tile<true>(c->g, [&](auto v, auto nw, auto rw) {
         constexpr int V = decltype(v)::value, NW = decltype(nw)::value, RW = decltype(rw)::value;
         int gx;
         const unsigned nb = steps_blocks(steps_tiles(c->g.nx, c->g.ny, 64 * V, NW * RW, gx));

@@ -6,7 +6,8 @@ Chebyshev and PPCG: every field and statistic bit-identical to one step per
 sweep, as there.  1003x500 takes many tiles of 64x32 cells, 1803x771 tiles of
 128x64, both with an odd width and a last row of tiles that is cut.
 
-Jacobi: the iteration limit is not a multiple of the steps per launch, so the
+Jacobi (760x128 has the 256 tiles of 64x24 cells that it takes at most, 760x129
+more): the iteration limit is not a multiple of the steps per launch, so the
 solve stops inside one and the remaining steps are repeated; u is compared with
 the oracle's Jacobi after the same number of iterations, and r, which the
 reference also uses as scratch, where the last iteration forms the residual
@@ -50,7 +51,7 @@ def test_large_tiles_bit_identical_to_single_steps(nx, ny, solver, key, inner):
         assert np.array_equal(fa[f], fb[f]), f
 
 
-@pytest.mark.parametrize("nx,ny", [(3, 2), (47, 20), (131, 77), (1003, 500), (1803, 771)])
+@pytest.mark.parametrize("nx,ny", [(3, 2), (47, 20), (131, 77), (760, 128), (760, 129), (1003, 500), (1803, 771)])
 def test_jacobi_iteration_limits_match_oracle(nx, ny):
     for limit in (1, 8, 21, 49, 50, 57, 107):
         print(f"case: Jacobi {nx}x{ny}, {limit} iterations", flush=True)
