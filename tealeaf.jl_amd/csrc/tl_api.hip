@@ -1292,8 +1292,8 @@ static int solve_cg_ir(tl_ctx *c, const tl_solve_params *p, double rx, double ry
             RETIF(run_until_stop(c, 64, (long)p->max_iters + 16, [&]() { return cg32_iteration(c, ++t); }, &k,
                                  p->launch == TL_LAUNCH_GRAPH ? GRAPH_CG32 : -1, &t));
     }
-    if (k.why == WHY_MAXITERS)  // keep the partial correction
-        HIPCHK(c, launch_ir_accumulate(c, resident ? 0 : k.stop_iter, fused ? cgf_p(c, k.stop_iter) : nullptr));
+    if (k.why == WHY_MAXITERS)  // keep the partial correction (complete in x, or with an odd iteration's update pending)
+        HIPCHK(c, launch_ir_accumulate(c, resident || pairs ? 0 : k.stop_iter, fused ? cgf_p(c, k.stop_iter) : nullptr));
     st->inner_iters = k.iters;
     st->iterations = k.iters;
     st->cg_iters = k.iters;

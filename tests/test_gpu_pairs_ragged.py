@@ -42,3 +42,26 @@ def test_ragged_pairs_match_oracle(nx, ny, coefficient):
     a, b = iters[_lib.TL_FP32_KERNELS_AUTO], iters[_lib.TL_FP32_KERNELS_TWO]
     assert a % 2 == 0  # the pairs ran
     assert abs(a - b) <= max(6, 0.05 * b) + refreshes[_lib.TL_FP32_KERNELS_AUTO], (iters, refreshes)
+
+
+@pytest.mark.parametrize("nx,ny,form", [(130, 127, "AUTO"), (128, 96, "PAIRS")])
+def test_iteration_limit_adds_every_update_once(nx, ny, form):
+    """A limit ends the solve inside a pair (9) or after one (10) with the partial
+    correction kept.  Without a refresh (ir_delta far below what ten iterations
+    reach) the pairs and the two-kernel form take the same CG steps up to FP32
+    rounding, about 1e-6 of the correction; an update missing or added twice
+    changes it by percents."""
+    text = (decks.random_rect_deck(17, n=nx, steps=1, nrect=8, precision="fp32_ir")
+            .replace(f"y_cells={nx}", f"y_cells={ny}"))
+    for limit in (9, 10):
+        print(f"case: FP32 CG pairs {nx}x{ny} stopped after {limit} iterations", flush=True)
+        u = {}
+        for f in (form, "TWO"):
+            s = T.Settings.from_text(text).set(fp32_kernels=getattr(_lib, f"TL_FP32_KERNELS_{f}"), max_iters=limit,
+                                               ir_delta=1e-6)
+            c = T.initialiseapp(s)
+            st = T.step(c, s)
+            assert st["iterations"] == limit and st["refreshes"] == 0, st
+            u[f], u0 = c.interior("u"), c.interior("u0")
+            c.close()
+        assert np.linalg.norm(u[form] - u["TWO"]) <= 1e-4 * np.linalg.norm(u["TWO"] - u0)

@@ -62,3 +62,25 @@ def test_iteration_limit():
         c.close()
         assert st[0]["iterations"] == lim and st[0]["converged"] == 0, st[0]
         assert st[0]["rel_resid"] < st[0]["init_rel_resid"], st[0]
+
+
+def test_bfloat16_coefficients():
+    """A density range beyond a scaled half's: the coefficients are held as
+    bfloat16 (the formats and decks of test_gpu_parity.py, on a grid that is held
+    in registers)."""
+    print("case: FP32 CG in registers 200x180, bfloat16 coefficients", flush=True)
+    text = decks.reference_deck(200, 2, extra="stop_rule=relative\nrel_tol=1e-10\nprecision=fp32_ir\n")
+    text = text.replace("y_cells=200", "y_cells=180").replace("density=100.0", "density=1e5").replace("density=0.1",
+                                                                                                      "density=1e-5")
+    d = O.parse_deck(text)
+    d.stop_rule, d.rel_tol, d.maxiters = O.STOP_RELATIVE, 1e-12, 200000
+    o = O.Oracle(d, threads=8)
+    o.initialise()
+    osum = o.run(2)[0]
+    c = T.initialiseapp(T.Settings.from_text(text))
+    summ, st = T.diffuse(c, T.Settings.from_text(text), 2)
+    c.close()
+    for t in range(2):
+        assert st[t]["coef_format"] == _lib.TL_COEF_BF16, st[t]
+        assert st[t]["converged"] == 1 and st[t]["rel_resid"] <= 1e-10, (t, st[t])
+        assert np.max(np.abs(summ[t] - osum[t]) / np.abs(osum[t])) < 1e-9, (t, summ[t], osum[t])
