@@ -56,8 +56,8 @@ extern "C" {
 
 /* tl_solve_params.launch: how the CG iterations of TL_CG solves (FP64 and
  * TL_FP32_IR) reach the GPU.  Both give bit-identical results.  Other solvers
- * always use stream launches.  FP64 CG on up to about 983040 cells (2048 tiles of
- * 120 x 4) runs up to 256 iterations per launch with either, unless its kernels
+ * always use stream launches.  FP64 CG on up to about 1966080 cells (1024 tiles
+ * of 120 x 16) runs up to 256 iterations per launch with either, unless its kernels
  * are being timed (tl_profile_begin with TL_K_CG_W64 or TL_K_CG_UR64). */
 #define TL_LAUNCH_STREAM 0  /* kernels enqueued in batches of up to 64 iterations */
 #define TL_LAUNCH_GRAPH 1   /* after a first stream batch, replays of one hipGraph of 64 iterations
@@ -136,8 +136,8 @@ typedef struct {
 
 /* tl_solve_params.fp32_kernels: how a TL_FP32_IR iteration is split into kernels.
  * Both reach the same FP64 tolerance; their FP32 roundings differ. */
-#define TL_FP32_KERNELS_AUTO 0   /* stream launches: from 32768 up to about 1966080 cells (2048 tiles
-                                   of 240 x 4) up to 256 iterations per launch, unless the pairs'
+#define TL_FP32_KERNELS_AUTO 0   /* stream launches: from 32768 up to about 3932160 cells (1024 tiles
+                                   of 240 x 16) up to 256 iterations per launch, unless the pairs'
                                    kernels are being timed; else pairs when nx is a multiple of 4 or
                                    the grid has 16384 cells or more; TL_LAUNCH_GRAPH: fused when nx
                                    is a multiple of 4; else two kernels */

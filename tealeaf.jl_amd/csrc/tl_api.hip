@@ -576,7 +576,7 @@ static int ensure_cgs(tl_ctx *c)
 }
 
 // FP64 CG with the grid held in registers (k_cgr): on every grid that fits (up
-// to 2048 tiles of 120 columns by 4 rows, 983040 cells), where it is faster than
+// to 1024 tiles of 120 columns by 16 rows, 1966080 cells), where it is faster than
 // the sweeps at every size measured (k_cgr's comment), with stream launches and
 // hipGraph batches alike: a launch is a batch of iterations already.  Not where
 // the launches of the sweeps are timed one by one (tl_profile_begin).
@@ -602,8 +602,8 @@ static bool resident_pays(tl_ctx *c)
     return !(c->prof_mask & ((1u << TL_K_CG_W64) | (1u << TL_K_CG_UR64))) && resident_fits(c, c->g.r64);
 }
 
-// The same in FP32, TL_FP32_KERNELS_AUTO with stream launches: faster than the
-// pairs on every grid that fits (2048 tiles of 240 x 4, 1966080 cells; k_cgr's
+// The same in FP32, TL_FP32_KERNELS_AUTO with stream launches: no slower than the
+// pairs on any grid that fits (1024 tiles of 240 x 16, 3932160 cells; k_cgr's
 // comment).  Below 32768 cells the choice is as before (a solve takes a few ms).
 static bool resident32_pays(tl_ctx *c)
 {

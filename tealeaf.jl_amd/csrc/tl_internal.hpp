@@ -124,9 +124,9 @@ constexpr int TBV = TL_TBV;
 #define TL_S32_COLS 240
 #define TL_S32_WAVES 3072
 #define TL_S32_ROWS 4
-// k_cgr: threads per block, blocks (one per CU) and iterations per launch (the
+// k_cgr: blocks at most (one per CU) and iterations per launch (the
 // host reads the state once per launch, 15 us)
-constexpr int CGR_NT = 512, CGR_MAXB = 256, CGR_BATCH = 256;
+constexpr int CGR_MAXB = 256, CGR_BATCH = 256;
 // sweeps over more bytes than this (the Infinity Cache) use streaming access.
 // Measured with the FP64 CG sweep: 453 MB of arrays (3072^2) 92.6 us per
 // iteration streaming, 102.2 cached; 83 MB (1501x1103) 25.1 and 21.9.

@@ -43,6 +43,9 @@ namespace tl {
 
 // Tiles of `cols` columns for at most about `waves` waves (one round of them on
 // the chip), bands of at least `min_rows` rows.
+// threads per block of k_cgr by rows per wave
+static int cgr_threads(const Tiles &o) { return o.ty <= 4 ? 512 : 256; }
+
 static Tiles make_tiles(int nx, int ny, int cols, int waves, int min_rows)
 {
     Tiles t{};
@@ -131,15 +134,18 @@ Geo make_geo(int nx, int ny, int hd)
     g.nbmax = std::max(std::max(g.gx * g.gy, g.gx4 * g.gyp4), std::max(g.gx4 * g.gy4, g.gx2 * g.gy2));
     g.nbmax = std::max(g.nbmax, g.gx4 * g.gyf);
     g.s64 = make_tiles(nx, ny, TL_S64_COLS, TL_S64_WAVES, TL_S64_ROWS);
-    // k_cgr: 2 rows per wave, or 4 where 2048 waves of 2 do not hold the grid
-    // (us per iteration, 2 / 4 rows: 64^2 5.6 / 6.4, 256^2 5.8 / 6.4, 512^2 6.9 /
-    // 7.0, 700x500 7.4 / 7.1)
+    // k_cgr: the fewest rows per wave, 2 or 4 (2048 waves), 12 or 16 (1024), that
+    // hold the grid (us per iteration, 2 / 4 rows: 64^2 5.6 / 6.4, 256^2 5.8 / 6.4,
+    // 512^2 6.9 / 7.0, 700x500 7.4 / 7.1; 4 / 16: 900^2 8.2 / 13.7, FP32 1024^2 9.4 /
+    // 13.8; 12 / 16: 1100x1000 11.0 / 14.6)
     const auto resident = [&](int cols) {
         Tiles o{};
-        for (o.ty = 2; o.ty <= 4; o.ty *= 2) {
+        for (const int rows : {2, 4, 12, 16}) {
+            o.ty = rows;
             o.strips = (nx + cols - 1) / cols;
             o.bands = (ny + o.ty - 1) / o.ty;
-            const long blocks = ((long)o.strips * o.bands + CGR_NT / 64 - 1) / (CGR_NT / 64);
+            const int waves = cgr_threads(o) / 64;
+            const long blocks = ((long)o.strips * o.bands + waves - 1) / waves;
             if (blocks <= CGR_MAXB) {
                 o.blocks = (int)blocks;
                 return o;
@@ -2574,11 +2580,13 @@ __global__ __launch_bounds__(TBV) __attribute__((amdgpu_waves_per_eu(3))) void k
 // across the XCDs, 4 to 5 us.  Microseconds per iteration, sweeps / this: 64^2 10.4
 // / 5.6, 256^2 8.8 / 5.8, 512^2 9.0 / 6.9, 700x500 9.3 / 7.4, 900^2 12.6 / 8.2;
 // FP32, pairs / this: 182^2 13.2 / 7.8, 256^2 11.4 / 7.5, 512x400 10.5 / 7.5, 1024^2
-// 11.0 / 9.3.
+// 11.0 / 9.3.  Larger grids take 12 or 16 rows per wave and one wave per SIMD (NT
+// 256: 512 registers a lane), bound by arithmetic: FP64 1000^2 14.5 / 10.8,
+// 1200x1150 17.5 / 11.0, 1501x1103 18.8 / 14.9; FP32 1300x1400 13.7 / 13.6, 1700x1600
+// 16.3 / 15.3, 2047x1533 17.5 / 15.0.
 // Measured and left: the neighbours' cells with EMPTY places of their own, polled
-// with the sums, spilled registers (512^2 9.6); so did 8 rows per wave, which
-// would hold twice the cells (FP64 1501x1103 24.0 against 18.9 in sweeps, FP32
-// 2047x1533 20.2 against 17.4 in pairs).
+// with the sums, spilled registers (512^2 9.6); so did 8 rows with two waves per
+// SIMD (FP64 1501x1103 24.0, FP32 2047x1533 20.2).
 constexpr unsigned long long EMPTY = 0x7ff4dead00000000ull;
 constexpr int CGR_SPIN = 1 << 20;  // about a second
 
@@ -2620,8 +2628,8 @@ __device__ __forceinline__ float next_up1(float v) { return dpp_up1f(v); }
 __device__ __forceinline__ double next_down1(double v) { return lane_down1<true>(v); }
 __device__ __forceinline__ float next_down1(float v) { return dpp_down1f(v); }
 
-template <typename T, int FMT, int RW>
-__global__ __launch_bounds__(CGR_NT) __attribute__((amdgpu_waves_per_eu(2))) void k_cgr(
+template <typename T, int FMT, int RW, int NT>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT / 256, NT / 256))) void k_cgr(
     Geo g, Tiles o, int t0, int n, T *__restrict__ r_even, T *__restrict__ r_odd, T *__restrict__ p_even,
     T *__restrict__ p_odd, T *__restrict__ u, const std::conditional_t<sizeof(T) == 8, double, tl_gc_t> *__restrict__ gc,
     T hx, T hy, Ctrl *__restrict__ ctrl, const double *__restrict__ sin, unsigned nbin, int side, double *__restrict__ sout,
@@ -2629,7 +2637,7 @@ __global__ __launch_bounds__(CGR_NT) __attribute__((amdgpu_waves_per_eu(2))) voi
 {
     typedef unsigned long long u64;
     constexpr bool F64 = sizeof(T) == 8;
-    constexpr int V = 16 / sizeof(T), COLS = 60 * V, NR = RW + 4, NW = CGR_NT / 64;  // rows held: y0 - 2 .. y0 + RW + 1
+    constexpr int V = 16 / sizeof(T), COLS = 60 * V, NR = RW + 4, NW = NT / 64;  // rows held: y0 - 2 .. y0 + RW + 1
     if (t0 > ctrl->stop_iter) return;
     __shared__ double sh[NW][4], sh2[NW][4];
     __shared__ int gone;
@@ -2696,9 +2704,9 @@ __global__ __launch_bounds__(CGR_NT) __attribute__((amdgpu_waves_per_eu(2))) voi
     }
     double s4[4];
     if (side)
-        sum_block_sums<4, CGR_NT>(sin, nbin, s4);
+        sum_block_sums<4, NT>(sin, nbin, s4);
     else  // k_cgf_dots: one sum after the other
-        sum_partials<4, CGR_NT>(sin, nbin, g.nbmax, s4);
+        sum_partials<4, NT>(sin, nbin, g.nbmax, s4);
     double gam_prev = t0 >= 2 ? ctrl->rrs[(t0 - 2) & 1] : 1.0;
     int t = t0;
     for (;;) {
@@ -2826,7 +2834,7 @@ __global__ __launch_bounds__(CGR_NT) __attribute__((amdgpu_waves_per_eu(2))) voi
             }
         }
         if (last) {
-            write_block_sums<4, CGR_NT>(acc, sout);
+            write_block_sums<4, NT>(acc, sout);
             ++t;
             break;
         }
@@ -4229,9 +4237,17 @@ hipError_t launch_cgs64(tl_ctx *c, int t, int tref)
 // iterations t0 .. t0 + n - 1 in one launch (k_cgr); u has every update after it
 static hipError_t launch_resident(tl_ctx *c, const void *kern, const Tiles &o, void **args)
 {
-    if (o.blocks == 1) return hipLaunchKernel(kern, dim3(1), dim3(CGR_NT), args, 0, c->stream);
+    if (o.blocks == 1) return hipLaunchKernel(kern, dim3(1), dim3(cgr_threads(o)), args, 0, c->stream);
     k_cgr_clear<<<12, 256, 0, c->stream>>>(c->slots, 3 * 4 * CGR_MAXB);
-    return hipLaunchCooperativeKernel(kern, dim3(o.blocks), dim3(CGR_NT), args, 0, c->stream);
+    return hipLaunchCooperativeKernel(kern, dim3(o.blocks), dim3(cgr_threads(o)), args, 0, c->stream);
+}
+template <typename T, int FMT>
+static const void *cgr_kernel(const Tiles &o)
+{
+    return o.ty == 2    ? (const void *)k_cgr<T, FMT, 2, 512>
+           : o.ty == 4  ? (const void *)k_cgr<T, FMT, 4, 512>
+           : o.ty == 12 ? (const void *)k_cgr<T, FMT, 12, 256>
+                        : (const void *)k_cgr<T, FMT, 16, 256>;
 }
 
 hipError_t launch_cgr64(tl_ctx *c, int t0, int n)
@@ -4244,7 +4260,7 @@ hipError_t launch_cgr64(tl_ctx *c, int t0, int n)
     int side = 1;
     void *args[] = {&g, &o, &t0, &n, &re, &ro, &pe, &po, &u, &gc, &hx, &hy, &c->ctrl, &sin, &c->nb_f[(t0 - 1) & 1], &side,
                     &sout, &c->slots, &c->hist_a, &c->hist_b};
-    const void *kern = o.ty == 2 ? (const void *)k_cgr<double, 0, 2> : (const void *)k_cgr<double, 0, 4>;
+    const void *kern = cgr_kernel<double, 0>(o);
     const hipError_t e = launch_resident(c, kern, o, args);
     c->nb_f[(t0 + n - 1) & 1] = (unsigned)o.blocks;
     return e;
@@ -4692,9 +4708,7 @@ hipError_t launch_cgr32(tl_ctx *c, int t0, int n, bool first)
     int side = !first;
     void *args[] = {&g,       &o,        &t0,   &n,    &re,  &ro,   &pe,       &po,   &c->x32, &c->gcell, &c->hx32,
                     &c->hy32, &c->ctrl, &sin,  &c->nb_f[(t0 - 1) & 1], &side, &sout, &c->slots, &none, &none};
-    const bool h = c->gc_fmt == GC_F16;
-    const void *kern = o.ty == 2 ? (h ? (const void *)k_cgr<float, GC_F16, 2> : (const void *)k_cgr<float, GC_BF16, 2>)
-                                 : (h ? (const void *)k_cgr<float, GC_F16, 4> : (const void *)k_cgr<float, GC_BF16, 4>);
+    const void *kern = c->gc_fmt == GC_F16 ? cgr_kernel<float, GC_F16>(o) : cgr_kernel<float, GC_BF16>(o);
     const hipError_t e = launch_resident(c, kern, o, args);
     c->nb_f[(t0 + n - 1) & 1] = (unsigned)o.blocks;
     return e;

@@ -1,11 +1,11 @@
 """GPU: the FP32 inner CG held in registers over many iterations (the automatic
-choice from 32768 cells up to 2048 tiles of 240 columns by 4 rows), in the
+choice from 32768 cells up to 1024 tiles of 240 columns by 16 rows), in the
 conventions of test_gpu_pairs.py: every step meets the FP64 true residual of
 1e-10, agrees with the oracle's FP64 solution within 1e-9 in every field-summary
 quantity, and takes as many iterations as the two-kernel form within 5%.  Widths
 lie around one and two tiles and leave 1, 2 and 3 columns of a last vector;
-heights leave a remainder of the 2 or 4 rows of a tile.  The long grids lie at the
-edges of the rule (2048 tiles of 2 rows, of 4, and beyond, where the pairs run,
+heights leave a remainder of the rows of a tile.  The long grids lie at the edges of
+the rule (2048 tiles of 2 rows, of 4, 1024 of 12, of 16, and beyond, where the pairs run,
 whose refreshes may add a counted null step each, as in test_gpu_pairs_ragged.py),
 with a short timestep that keeps their solves to some tens of iterations."""
 import numpy as np
@@ -19,7 +19,8 @@ pytestmark = pytest.mark.gpu
 
 GRIDS = [(240, 137, 0.004), (241, 140, 0.004), (242, 137, 0.004), (243, 139, 0.004), (479, 71, 0.004),
          (482, 69, 0.004), (1100, 31, 0.004),
-         (241, 2047, 4e-6), (241, 2050, 4e-6), (241, 4095, 1e-6), (241, 4098, 1e-6)]
+         (241, 2047, 4e-6), (241, 2050, 4e-6), (241, 4095, 1e-6), (241, 4098, 1e-6),
+         (241, 6144, 4e-7), (241, 6147, 4e-7), (241, 8192, 2e-7), (241, 8195, 2e-7), (2047, 1533, 4e-6)]
 
 
 @pytest.mark.parametrize("coefficient", [1, 2])
@@ -35,7 +36,7 @@ def test_resident_matches_oracle(nx, ny, dt, coefficient):
     o.initialise()
     osum = o.run(2)[0]
     iters = {}
-    pairs = -(-nx // 240) * -(-ny // 4) > 2048
+    pairs = -(-nx // 240) * -(-ny // 16) > 1024
     for form in (_lib.TL_FP32_KERNELS_TWO, _lib.TL_FP32_KERNELS_AUTO):
         s = T.Settings.from_text(text).set(fp32_kernels=form)
         c = T.initialiseapp(s)

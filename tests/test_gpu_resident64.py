@@ -2,8 +2,8 @@
 CG in the conventions of test_gpu_sweep64.py: every field-summary quantity within
 1e-10, u and p within 1e-9 of u's scale, iterations within max(3, 2%).  The grids
 lie at the edges of its tiles (120 columns by 2 or 4 rows, one or several waves
-and blocks) and of the rule that takes it: 2048 tiles of 2 rows, then of 4, then
-one sweep per iteration, which is also run at each of these sizes (it is the form
+and blocks) and of the rule that takes it: 2048 tiles of 2 rows, then of 4, 1024
+of 12, then of 16, then one sweep per iteration, which is also run at each of these sizes (it is the form
 that launches timed one by one take).  A launch holds up to 256 iterations; one
 grid needs several."""
 import numpy as np
@@ -18,7 +18,8 @@ pytestmark = pytest.mark.gpu
 SWEEPS = (1 << 0) | (1 << 1)  # TL_K_CG_W64, TL_K_CG_UR64
 
 SMALL = [(2, 2), (119, 15), (120, 16), (121, 17), (122, 35), (241, 34), (700, 3)]
-EDGES = [(121, 2047), (121, 2050), (1081, 410), (121, 4095), (121, 4098)]
+EDGES = [(121, 2047), (121, 2050), (1081, 410), (121, 4095), (121, 4098), (121, 6144), (121, 6147), (121, 8192),
+         (121, 8195), (1500, 1100)]
 
 
 def _check(nx, ny, coefficient, max_iters, sweeps):
