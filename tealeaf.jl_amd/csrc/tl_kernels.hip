@@ -1384,13 +1384,16 @@ __global__ __launch_bounds__(TBV) __attribute__((amdgpu_waves_per_eu(2))) void k
 
 // The four sums k_cgs needs at its first iteration and after a new true
 // residual, for r and the kept direction p, with its operator.  One thread per
-// cell of a column band; runs once per start or new residual.
+// cell of a column band; runs once per start or new residual.  (r, r) is rr, the
+// finalizer's, and not summed again: the stop test has just let the iterations
+// run on that value, and another rounding of it could fail the test that the
+// next sweep repeats, whereupon the host would refresh the same residual for ever.
 __global__ __launch_bounds__(TB) void k_cgs_dots(Geo g, const double *__restrict__ r, const double *__restrict__ p,
                                                  const double *__restrict__ gc, double hx, double hy,
-                                                 double *__restrict__ part)
+                                                 const double *__restrict__ rr, double *__restrict__ part)
 {
     const Col c = column(g);
-    double acc[4] = {0.0, 0.0, 0.0, 0.0};
+    double acc[4] = {block_id() == 0 && threadIdx.x == 0 ? *rr : 0.0, 0.0, 0.0, 0.0};
     if (c.active) {
         for (int y = c.y0; y < c.y1; ++y) {
             const long i = at(g, c.x, y);
@@ -1406,7 +1409,6 @@ __global__ __launch_bounds__(TB) void k_cgs_dots(Geo g, const double *__restrict
                 return vc + s;
             };
             const double rc = r[i], ar = apply(r), ap = apply(p);
-            acc[0] += rc * rc;
             acc[1] += rc * ar;
             acc[2] += rc * ap;
             acc[3] += p[i] * ap;
@@ -2937,14 +2939,17 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT / 256, NT
 // The four sums k_cgf needs at its first iteration and after an FP64 refresh,
 // for the residual r and the kept direction p: (r, r), (r, A r), (r, A p),
 // (p, A p), with the same FP32 operator (flux form, clamped neighbours).  One
-// thread per cell of a column band; runs once per start or refresh.
+// thread per cell of a column band; runs once per start or refresh.  (r, r) is the
+// finalizer's rr of the FP64 residual, as in k_cgs_dots: the sum over the FP32
+// residual can lie on the other side of the tolerance (always, where small fields
+// underflow in FP32).
 template <int FMT>
 __global__ __launch_bounds__(TB) void k_cgf_dots(Geo g, const float *__restrict__ r, const float *__restrict__ p,
                                                  const tl_gc_t *__restrict__ gc, float hx, float hy,
-                                                 double *__restrict__ part)
+                                                 const double *__restrict__ rr, double *__restrict__ part)
 {
     const Col c = column(g);
-    double acc[4] = {0.0, 0.0, 0.0, 0.0};
+    double acc[4] = {block_id() == 0 && threadIdx.x == 0 ? *rr : 0.0, 0.0, 0.0, 0.0};
     if (c.active) {
         const int x = c.x;
         const int xl = max(x - 1, 0), xr = min(x + 1, g.nx - 1);
@@ -2960,7 +2965,6 @@ __global__ __launch_bounds__(TB) void k_cgf_dots(Geo g, const float *__restrict_
             const float ap = smvp5f(pc, p[at(g, xl, y)], p[at(g, xr, y)], p[at(g, x, yd)], p[at(g, x, yu)], kxl,
                                     kxr, kyd, kyu);
             const double rd = (double)rc;
-            acc[0] += rd * rd;
             acc[1] += rd * (double)ar;
             acc[2] += rd * (double)ap;
             acc[3] += (double)pc * (double)ap;
@@ -4271,7 +4275,7 @@ hipError_t launch_cgr64(tl_ctx *c, int t0, int n)
 hipError_t launch_cgs_dots(tl_ctx *c, int T)
 {
     k_cgs_dots<<<sgrid(c->g), TB, 0, c->stream>>>(c->g, cgs_r(c, T), cgs_p(c, T), c->g64, c->hx64, c->hy64,
-                                                  part_f(c, T));
+                                                  &c->ctrl->rrs[T & 1], part_f(c, T));
     c->nb_f[T & 1] = nbh(c);
     return hipGetLastError();
 }
@@ -4691,7 +4695,7 @@ hipError_t launch_cgf_dots(tl_ctx *c, int T)
 {
     auto kern = c->gc_fmt == GC_F16 ? k_cgf_dots<GC_F16> : k_cgf_dots<GC_BF16>;
     kern<<<sgrid(c->g), TB, 0, c->stream>>>(c->g, cgf_r(c, T), cgf_p(c, T), c->gcell, c->hx32, c->hy32,
-                                            part_f(c, T));
+                                            &c->ctrl->rrs[T & 1], part_f(c, T));
     c->nb_f[T & 1] = nbh(c);
     return hipGetLastError();
 }
