@@ -500,6 +500,20 @@ __device__ void record_stop(Ctrl *c, int t, int why)
     c->stop_iter = t;
 }
 
+// Is iteration t past the stop?  The same answer for every wave of a block: where
+// block 0 of the same launch records a stop, a block that starts late may read
+// stop_iter before or after that, and if each wave read it for itself some of them
+// could leave while the others go on, into sums over LDS entries that nobody wrote.
+// One answer either way is right: the blocks that go on derive the same stop from
+// the sums.  A barrier, 0.1 us or less of a launch.
+__device__ __forceinline__ bool past_stop(const Ctrl *c, int t)
+{
+    __shared__ int stop;
+    if (threadIdx.x == 0) stop = c->stop_iter;
+    __syncthreads();
+    return t > stop;
+}
+
 // Iteration number of a CG iteration kernel.  Stream launches pass t >= 1.
 // The launches of a hipGraph batch pass -i for the i-th iteration of the
 // batch and take t = Ctrl::tg + i, tg being set by the batch's first node
@@ -891,7 +905,7 @@ __global__ __launch_bounds__(TB) void k_cg_ur(Geo g, int t, T *__restrict__ u, c
                                               const double *__restrict__ prprev, unsigned nbp,
                                               double *__restrict__ prcur, double *__restrict__ hist_a)
 {
-    if (t > ctrl->stop_iter) return;
+    if (past_stop(ctrl, t)) return;
     double ad;
     if (!cg_alpha(g, t, ctrl, pw, nbw, prprev, nbp, hist_a, &ad)) return;
     const T alpha = (T)ad;
@@ -1227,7 +1241,7 @@ __global__ __launch_bounds__(TBV) __attribute__((amdgpu_waves_per_eu(2))) void k
         double r[V], p[V], g[V], u[V];
     };
     t = iter_of(t, ctrl);
-    if (t > ctrl->stop_iter) return;
+    if (past_stop(ctrl, t)) return;
     int strip, band;
     const bool tile = wave_tile(g.s64, strip, band);
     const int lane = threadIdx.x & 63;
@@ -1552,7 +1566,7 @@ __global__ __launch_bounds__(TBV) TL_CGG_ATTR void k_cgg(Geo g, int ty, int t, c
                                             double *__restrict__ part_out, const float *__restrict__ pprev)
 {
     t = iter_of(t, ctrl);
-    if (t > ctrl->stop_iter) return;
+    if (past_stop(ctrl, t)) return;
     float beta = 0.0f, alpha = 0.0f;
     const bool fuse = !UR && t >= 2;
     // UR at even t also applies the x update of iteration t-1, whose p is
@@ -1905,7 +1919,7 @@ __global__ __launch_bounds__(TBV) TL_CGF_ATTR void k_cgf(Geo g, int ty, int t, c
                                                          unsigned nbin, double *__restrict__ sout)
 {
     t = iter_of(t, ctrl);
-    if (t > ctrl->stop_iter) return;
+    if (past_stop(ctrl, t)) return;
     const bool xupd = (t & 1) == 0;
     const VCol<4> cl = vcolumn<4>(g, ty);
     const int x0 = cl.x0, lane = cl.lane;
@@ -2300,7 +2314,7 @@ __device__ __forceinline__ void cgp_sweep(const Geo &g, int t, const float *__re
         float r[V], p[V], x[V];
         GcRaw<V> g;
     };
-    if (t > ctrl->stop_iter) return;
+    if (past_stop(ctrl, t)) return;
     int strip, band;
     const Tiles &o = g.s32;
     const bool tile = wave_tile(o, strip, band);
@@ -2640,7 +2654,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT / 256, NT
     typedef unsigned long long u64;
     constexpr bool F64 = sizeof(T) == 8;
     constexpr int V = 16 / sizeof(T), COLS = 60 * V, NR = RW + 4, NW = NT / 64;  // rows held: y0 - 2 .. y0 + RW + 1
-    if (t0 > ctrl->stop_iter) return;
+    if (past_stop(ctrl, t0)) return;
     __shared__ double sh[NW][4], sh2[NW][4];
     __shared__ int gone;
     __shared__ Ctrl rules;  // what the stop test reads, which does not change
@@ -3202,7 +3216,7 @@ __global__ __launch_bounds__(TB) void k_ppcg_ur_sd(Geo g, int t, double *__restr
                                                    const double *__restrict__ pw, unsigned nbw,
                                                    const double *__restrict__ prprev, unsigned nbp)
 {
-    if (t > ctrl->stop_iter) return;
+    if (past_stop(ctrl, t)) return;
     double alpha;
     if (!cg_alpha(g, t, ctrl, pw, nbw, prprev, nbp, nullptr, &alpha)) return;
     const Col c = column(g);
@@ -3776,7 +3790,7 @@ __global__ __launch_bounds__(NW * 64) void k_steps(Geo g, int gx, int t, int n, 
     struct vec {
         double e[V];
     };
-    if (t > ctrl->stop_iter) return;
+    if (past_stop(ctrl, t)) return;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // tiles dealt to the XCDs in runs, as in wave_tile
     const int xb = (int)(blockIdx.x >> 3);
