@@ -1225,6 +1225,7 @@ static int solve_cg_ir(tl_ctx *c, const tl_solve_params *p, double rx, double ry
     // u0 = b = energy*density; u = guess or b; bb, tol_abs
     HIPCHK(c, launch_cg_init_resid(c, guess));
     HIPCHK(c, hipMemsetAsync(c->x32, 0, c->g.elems * sizeof(float), c->stream));
+    if (pairs || resident) HIPCHK(c, launch_ir_clear_tail(c));
     int t = 0;  // last iteration enqueued
     // r = u0 - A u (FP64, stored in FP32) and p = r; fused: the four sums of
     // iteration 1 (r and p in the buffers of iteration 0)

@@ -447,6 +447,7 @@ hipError_t launch_jacobi_steps(tl_ctx *c, int n, const double *u_in, double *u_o
                                int nprev, int residp, int t);
 hipError_t launch_jacobi_end(tl_ctx *c, int nprev, int residp, int t);
 hipError_t launch_ir_prepare(tl_ctx *c, double rx, double ry, int coefficient);
+hipError_t launch_ir_clear_tail(tl_ctx *c);
 hipError_t launch_ir_accumulate(tl_ctx *c, int T, const float *pT = nullptr);
 hipError_t launch_acc64(tl_ctx *c, double *u, double *d);
 

@@ -4006,6 +4006,21 @@ __global__ __launch_bounds__(TB) void k_gcell(Geo g, const double *__restrict__ 
     gc[(long)j * g.pitch + col] = gc_store<FMT>(f);
 }
 
+// The columns from nx to the end of the last 4 of every row, of four arrays: the
+// forms of the FP32 CG that store whole vectors store there too, zeros, or NaN
+// after an overflow at the last column (0 times infinity), which the pairs would
+// read in a later solve.  A solve therefore starts with zeros there.
+__global__ __launch_bounds__(TB) void k_clear_tail(Geo g, float *__restrict__ a, float *__restrict__ b,
+                                                   float *__restrict__ c, float *__restrict__ d)
+{
+    const int y = blockIdx.x * TB + threadIdx.x;
+    if (y >= g.ny) return;
+    for (int x = g.nx; x % 4 != 0; ++x) {
+        const long i = at(g, x, y);
+        a[i] = b[i] = c[i] = d[i] = 0.0f;
+    }
+}
+
 // per-block minimum and maximum of gc over the cells with a density (grid-
 // stride over the allocation; TL_RANGE_BLOCKS blocks): out[2b], out[2b + 1]
 __global__ __launch_bounds__(TB) void k_gc_range(const double *__restrict__ rho, size_t n, int coefficient,
@@ -4644,6 +4659,13 @@ hipError_t launch_ir_prepare(tl_ctx *c, double rx, double ry, int coefficient)
     // kx = hx (gc(x-1) + gc(x)): the scale of the stored gc is divided out of hx, hy
     c->hx32 = (float)(0.5 * rx / scale);
     c->hy32 = (float)(0.5 * ry / scale);
+    return hipGetLastError();
+}
+
+hipError_t launch_ir_clear_tail(tl_ctx *c)
+{
+    if (c->g.nx % 4 == 0) return hipSuccess;
+    k_clear_tail<<<(c->g.ny + TB - 1) / TB, TB, 0, c->stream>>>(c->g, c->r32, c->r32b, c->p32, c->p32b);
     return hipGetLastError();
 }
 
