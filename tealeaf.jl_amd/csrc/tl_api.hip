@@ -73,6 +73,7 @@ extern "C" void tl_default_params(tl_solve_params *p)
 static int alloc_d(tl_ctx *c, double **p, size_t n)
 {
     if (hipMalloc((void **)p, n * sizeof(double)) != hipSuccess) {
+        (void)hipGetLastError();  // or the next launch would report it
         c->err = "device allocation failed";
         *p = nullptr;
         return TL_E_NOMEM;
@@ -84,6 +85,7 @@ static int alloc_d(tl_ctx *c, double **p, size_t n)
 static int alloc_f(tl_ctx *c, float **p, size_t n)
 {
     if (hipMalloc((void **)p, n * sizeof(float)) != hipSuccess) {
+        (void)hipGetLastError();
         c->err = "device allocation failed";
         *p = nullptr;
         return TL_E_NOMEM;
@@ -385,7 +387,7 @@ static std::vector<uintptr_t> graph_key(const tl_ctx *c, int kind, int k)
                                 c->nb_r[0], c->nb_r[1], c->nb_w, (uintptr_t)c->gc_fmt};
     if (kind == GRAPH_CG64) {
         for (const void *q : {(const void *)c->f[TL_F_P], (const void *)c->p_alt, (const void *)c->f[TL_F_R],
-                              (const void *)c->r_alt1, (const void *)c->g64, (const void *)c->part_f,
+                              (const void *)c->sd_alt, (const void *)cgs_g(c), (const void *)c->part_f,
                               (const void *)(c->cg_u ? c->cg_u : c->f[TL_F_U]), (const void *)c->hist_a,
                               (const void *)c->hist_b})
             v.push_back((uintptr_t)q);
@@ -566,12 +568,17 @@ static int ensure_fused(tl_ctx *c)
     return TL_OK;
 }
 
-// the FP64 CG sweeps' second residual buffer, cell coefficient and sums
+// The FP64 CG sweeps' cell coefficient and sums.  The second buffers of r and p
+// are those of sd and p, which every context has; where there is no room for a
+// field more, the coefficient is kept in w, which is free until the last iteration
+// is done (cgs_g).
 static int ensure_cgs(tl_ctx *c)
 {
-    if (!c->r_alt1) RETIF(alloc_d(c, &c->r_alt1, c->g.elems));
-    if (!c->g64) RETIF(alloc_d(c, &c->g64, c->g.elems));
     if (!c->part_f) RETIF(alloc_d(c, &c->part_f, (size_t)9 * c->g.nbmax));
+    if (!c->g64) {
+        const int rc = alloc_d(c, &c->g64, c->g.elems);
+        if (rc != TL_OK && rc != TL_E_NOMEM) return rc;
+    }
     return TL_OK;
 }
 
@@ -831,7 +838,7 @@ static int solve_cg64(tl_ctx *c, const tl_solve_params *p, double rx, double ry,
                                p->epslim));
     const double *guess = nullptr;
     RETIF(choose_guess(c, p, rx, ry, &guess, st));
-    HIPCHK(c, launch_cg_init_resid(c, guess));
+    HIPCHK(c, launch_cg_init_resid(c, guess, !c->g64));
     // Under the relative rule the iterations add alpha p to a correction d
     // (u_alt, free during CG) instead of to u, and d is added to u at every
     // true-residual check ("reliable updates" with group-wise solution
@@ -882,6 +889,10 @@ static int solve_cg64(tl_ctx *c, const tl_solve_params *p, double rx, double ry,
     if (group) HIPCHK(c, launch_acc64(c, c->f[TL_F_U], c->u_alt));  // pending updates (max_iters, breakdown)
     c->cg_u = nullptr;  // other callers of the CG sweeps update u
     const int T = k.stop_iter;
+    if (!c->g64) {  // w held the coefficient: as CG.init! leaves it, for T = 0
+        HIPCHK(c, hipMemsetAsync(c->f[TL_F_W], 0, c->g.elems * sizeof(double), c->stream));
+        HIPCHK(c, launch_apply(c, c->f[TL_F_U], c->f[TL_F_W]));
+    }
     if (T >= 1) {
         HIPCHK(c, launch_cgs_final(c, T));
         RETIF(read_ctrl(c, &k));
@@ -1132,13 +1143,13 @@ static int solve_ppcg(tl_ctx *c, const tl_solve_params *p, double rx, double ry,
 static int solve_jacobi(tl_ctx *c, const tl_solve_params *p, double rx, double ry, tl_solve_stats *st)
 {
     if (!c->part_j) RETIF(alloc_d(c, &c->part_j, (size_t)2 * STEPS_HALO * c->g.nbmax));
-    if (!c->r_alt1) RETIF(alloc_d(c, &c->r_alt1, c->g.elems));
     HIPCHK(c, launch_init_coef(c, rx, ry, p->coefficient, INIT_JACOBI));
     HIPCHK(c, launch_init_ctrl(c, MODE_JACOBI, p->max_iters, p->eps, p->rel_tol, 0.0, 0, 0, p->epslim));
     // Several iterations per launch; the iterations 50, 100, ... end a launch,
     // which also forms the residual that joins their error (Jacobi.jl:21-24).
-    // Its r goes to two buffers in turn: a launch may have run past the stop.
-    HIPCHK(c, launch_copy_full(c, c->f[TL_F_R], c->r_alt1));
+    // Its r goes to two buffers in turn, its own and p's second one: a launch may
+    // have run past the stop.
+    HIPCHK(c, launch_copy_full(c, c->f[TL_F_R], c->p_alt));
     double *ucur = c->f[TL_F_U], *unext = c->u_alt;
     struct Launch {
         int t0, n;  // iterations t0 .. t0+n-1
@@ -1160,7 +1171,7 @@ static int solve_jacobi(tl_ctx *c, const tl_solve_params *p, double rx, double r
                              if (n == to50 && n == STEPS_HALO) n = STEPS_HALO / 2;
                              const int resid = (tt + n) % 50 == 0;
                              const hipError_t e = launch_jacobi_steps(
-                                 c, n, ucur, unext, ((tt + n) / 50) & 1 ? c->r_alt1 : c->f[TL_F_R], resid, nprev,
+                                 c, n, ucur, unext, ((tt + n) / 50) & 1 ? c->p_alt : c->f[TL_F_R], resid, nprev,
                                  residp, tt + 1);
                              if (made.size() >= 256) made.erase(made.begin(), made.begin() + 128);
                              made.push_back({tt + 1, n, ucur, unext});
@@ -1184,7 +1195,7 @@ static int solve_jacobi(tl_ctx *c, const tl_solve_params *p, double rx, double r
         break;
     }
     if (ucur != c->f[TL_F_U]) std::swap(c->f[TL_F_U], c->u_alt);
-    if ((T / 50) & 1) std::swap(c->f[TL_F_R], c->r_alt1);
+    if ((T / 50) & 1) std::swap(c->f[TL_F_R], c->p_alt);
     st->iterations = T;
     fill_stats(k, st);
     HIPCHK(c, launch_halo(c, TL_X_U, 1, nullptr, 0));
@@ -1213,13 +1224,17 @@ static int solve_cg_ir(tl_ctx *c, const tl_solve_params *p, double rx, double ry
     HIPCHK(c, launch_init_ctrl(c, MODE_IR, p->max_iters, p->eps, p->rel_tol, delta, 0, 0, p->epslim));
     // pairs of iterations (k_cgp) run as stream launches; with TL_LAUNCH_GRAPH
     // the automatic choice takes the fused kernel
-    const bool resident = p->fp32_kernels == TL_FP32_KERNELS_AUTO && p->launch != TL_LAUNCH_GRAPH && resident32_pays(c);
-    const bool pairs = p->fp32_kernels == TL_FP32_KERNELS_PAIRS ||
+    bool resident = p->fp32_kernels == TL_FP32_KERNELS_AUTO && p->launch != TL_LAUNCH_GRAPH && resident32_pays(c);
+    bool pairs = p->fp32_kernels == TL_FP32_KERNELS_PAIRS ||
                        (p->fp32_kernels == TL_FP32_KERNELS_AUTO && !resident && TL_CGP_AUTO && pairs_pay(c) &&
                         p->launch != TL_LAUNCH_GRAPH);
-    const bool fused = !pairs && !resident && (p->fp32_kernels == TL_FP32_KERNELS_FUSED ||
+    bool fused = !pairs && !resident && (p->fp32_kernels == TL_FP32_KERNELS_FUSED ||
                                   (p->fp32_kernels == TL_FP32_KERNELS_AUTO && fused_fits(c)));
-    if (fused || pairs || resident) RETIF(ensure_fused(c));
+    if (fused || pairs || resident) {
+        const int rc = ensure_fused(c);
+        if (rc != TL_OK && (rc != TL_E_NOMEM || p->fp32_kernels != TL_FP32_KERNELS_AUTO)) return rc;
+        if (rc != TL_OK) fused = pairs = resident = false;  // the two kernels need no second r
+    }
     const double *guess = nullptr;
     RETIF(choose_guess(c, p, rx, ry, &guess, st));
     // u0 = b = energy*density; u = guess or b; bb, tol_abs
@@ -1366,7 +1381,7 @@ extern "C" int tl_kernel_repeat(tl_ctx *c, int kernel_id, int reps)
     RETIF(ensure_cgs(c));
     HIPCHK(c, launch_init_coef(c, 1.0, 1.0, 1, INIT_CG64));
     HIPCHK(c, launch_init_ctrl(c, MODE_CG_REF, 1 << 30, 0.0, 0.0, 0.1, 0, 0, 0.0));
-    HIPCHK(c, launch_cg_init_resid(c, nullptr));
+    HIPCHK(c, launch_cg_init_resid(c, nullptr, !c->g64));
     if (kernel_id == TL_K_CGF32) {
         // `reps` iterations of the fused FP32 CG (after three warm-up ones)
         if (!fused_fits(c)) return TL_E_INVALID;
@@ -1396,6 +1411,7 @@ extern "C" int tl_kernel_repeat(tl_ctx *c, int kernel_id, int reps)
         // (u, u0, p, r, kx, ky) with fixed coefficients; never stopped
         HIPCHK(c, launch_set_mode(c, MODE_JACOBI, 1 << 30));
         if (!c->part_j) RETIF(alloc_d(c, &c->part_j, (size_t)2 * STEPS_HALO * c->g.nbmax));
+        if (kernel_id == TL_K_PPCG2_64 && !c->r_alt1) RETIF(alloc_d(c, &c->r_alt1, c->g.elems));
         double *a = c->f[TL_F_U], *b = c->u_alt, *s0 = c->f[TL_F_SD], *s1 = c->sd_alt;
         double *r0 = c->f[TL_F_R], *r1 = c->r_alt1, *q0 = c->f[TL_F_P], *q1 = c->p_alt;
         for (int i = 0; i < reps; ++i) {

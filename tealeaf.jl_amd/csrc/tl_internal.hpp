@@ -303,10 +303,10 @@ struct tl_ctx {
     // FP64 fields (reference Chunk fields; u and sd have ping-pong twins)
     double *f[TL_NFIELDS] = {};
     double *u_alt = nullptr, *sd_alt = nullptr, *guess = nullptr;
-    double *r_alt1 = nullptr, *r_alt2 = nullptr;  // r's second buffer (CG sweeps) / between PPCG's two-step sweeps
+    double *r_alt1 = nullptr, *r_alt2 = nullptr;  // PPCG: r between the sweeps of an outer iteration
     unsigned long long *slots = nullptr;  // k_cgr: the blocks' sums of three iterations
     int coop_cus = -1;        // compute units for cooperative launches (-1: not asked yet)
-    double *g64 = nullptr;    // FP64 cell coefficient 1/w of the CG sweeps (see k_init_coef)
+    double *g64 = nullptr;    // FP64 cell coefficient 1/w of the CG sweeps (see k_init_coef, cgs_g)
     double hx64 = 0, hy64 = 0;  // its face scales rx/2, ry/2
     // FP32 fields of the mixed-precision solve
     // FP32 inner CG: cell coefficient gc = 1/w (tl_gc_t) and its face scale
@@ -389,12 +389,15 @@ hipError_t launch_copy_energy(tl_ctx *c);
 // rows j0 .. j0+rows-1 of a field to / from packed rows of X doubles
 hipError_t launch_pack_rows(tl_ctx *c, const double *field, double *packed, int j0, int rows);
 hipError_t launch_unpack_rows(tl_ctx *c, double *field, const double *packed, int j0, int rows);
+// the array of the FP64 CG sweeps' cell coefficient: its own, or w's
+inline double *cgs_g(tl_ctx *c) { return c->g64 ? c->g64 : c->f[TL_F_W]; }
+inline const double *cgs_g(const tl_ctx *c) { return c->g64 ? c->g64 : c->f[TL_F_W]; }
 // what k_init_coef writes besides kx, ky (INIT_CG64: also what the single-sweep
 // FP64 CG needs, the cell coefficient and cleared second buffers)
 enum { INIT_CG = 0, INIT_JACOBI = 1, INIT_COEF_ONLY = 2, INIT_CG64 = 3 };
 hipError_t launch_init_coef(tl_ctx *c, double rx, double ry, int coefficient, int what);
 hipError_t launch_halo(tl_ctx *c, unsigned mask, int depth, double *const *extra, int nextra);
-hipError_t launch_cg_init_resid(tl_ctx *c, const double *guess);
+hipError_t launch_cg_init_resid(tl_ctx *c, const double *guess, bool keep_w = false);
 hipError_t launch_resid_norm_slot(tl_ctx *c, const double *b, const double *x, int slot);
 // tref > 0: the launch is being captured into a hipGraph batch whose first
 // iteration is tref (t only selects the buffers; the kernel takes its

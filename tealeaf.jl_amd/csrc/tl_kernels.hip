@@ -4190,18 +4190,20 @@ hipError_t launch_init_coef(tl_ctx *c, double rx, double ry, int coefficient, in
 {
     k_init_coef<<<fgrid(c->g), TB, 0, c->stream>>>(c->g, c->f[TL_F_DENSITY], c->f[TL_F_ENERGY], c->f[TL_F_U],
                                                    c->f[TL_F_P], c->f[TL_F_R], c->f[TL_F_U0], c->f[TL_F_KX],
-                                                   c->f[TL_F_KY], c->p_alt, c->r_alt1, c->g64, rx, ry,
+                                                   c->f[TL_F_KY], c->p_alt, c->sd_alt, cgs_g(c), rx, ry,
                                                    coefficient == 2 ? 1 : 0, what);
     c->hx64 = 0.5 * rx;
     c->hy64 = 0.5 * ry;
     return hipGetLastError();
 }
 
-hipError_t launch_cg_init_resid(tl_ctx *c, const double *guess)
+// (w goes to the scratch behind r where the FP64 sweeps keep their coefficient in w)
+hipError_t launch_cg_init_resid(tl_ctx *c, const double *guess, bool keep_w)
 {
+    double *w = keep_w ? c->sd_alt : c->f[TL_F_W];
     k_cg_init_resid<<<sgrid(c->g), TB, 0, c->stream>>>(c->g, c->f[TL_F_U], guess, c->f[TL_F_U0], c->f[TL_F_P],
-                                                       c->f[TL_F_R], c->f[TL_F_W], c->f[TL_F_KX], c->f[TL_F_KY],
-                                                       part_r(c, 0), part_m(c));
+                                                       c->f[TL_F_R], w, c->f[TL_F_KX], c->f[TL_F_KY], part_r(c, 0),
+                                                       part_m(c));
     nbr(c, 0) = nbh(c);
     c->nb_m = nbh(c);
     hipError_t e = hipGetLastError();
@@ -4246,7 +4248,7 @@ hipError_t launch_cg_p64(tl_ctx *c, int t)
 
 // FP64 CG sweeps: r(t) and p(t) in buffer t & 1, the four per-block sums for
 // iteration t+1 in set t & 1
-static inline double *cgs_r(tl_ctx *c, int t) { return (t & 1) ? c->r_alt1 : c->f[TL_F_R]; }
+static inline double *cgs_r(tl_ctx *c, int t) { return (t & 1) ? c->sd_alt : c->f[TL_F_R]; }
 static inline double *cgs_p(tl_ctx *c, int t) { return (t & 1) ? c->p_alt : c->f[TL_F_P]; }
 static inline double *cgs_u(tl_ctx *c) { return c->cg_u ? c->cg_u : c->f[TL_F_U]; }
 static inline double *part_f(tl_ctx *c, int t) { return c->part_f + (size_t)4 * (t & 1) * stride(c); }
@@ -4259,7 +4261,7 @@ hipError_t launch_cgs64(tl_ctx *c, int t, int tref)
     const bool nt = (size_t)6 * c->g.elems * sizeof(double) > TL_CACHE_BYTES;
     auto kern = even ? (nt ? k_cgs<true, true> : k_cgs<true, false>) : (nt ? k_cgs<false, true> : k_cgs<false, false>);
     kern<<<c->g.s64.blocks, TBV, 0, c->stream>>>(c->g, targ(t, tref), cgs_r(c, t - 1), cgs_r(c, t), cgs_p(c, t - 1),
-                                                cgs_p(c, t), cgs_u(c), c->g64, c->hx64, c->hy64, c->ctrl,
+                                                cgs_p(c, t), cgs_u(c), cgs_g(c), c->hx64, c->hy64, c->ctrl,
                                                 part_f(c, t - 1), c->nb_f[(t - 1) & 1], part_f(c, t), c->hist_a,
                                                 c->hist_b);
     c->nb_f[t & 1] = (unsigned)c->g.s64.blocks;
@@ -4288,7 +4290,7 @@ hipError_t launch_cgr64(tl_ctx *c, int t0, int n)
     Geo g = c->g;
     Tiles o = g.r64;
     double *re = cgs_r(c, 0), *ro = cgs_r(c, 1), *pe = cgs_p(c, 0), *po = cgs_p(c, 1), *u = cgs_u(c);
-    const double *gc = c->g64, *sin = part_f(c, t0 - 1);
+    const double *gc = cgs_g(c), *sin = part_f(c, t0 - 1);
     double hx = c->hx64, hy = c->hy64, *sout = part_f(c, t0 + n - 1);
     int side = 1;
     void *args[] = {&g, &o, &t0, &n, &re, &ro, &pe, &po, &u, &gc, &hx, &hy, &c->ctrl, &sin, &c->nb_f[(t0 - 1) & 1], &side,
@@ -4303,7 +4305,7 @@ hipError_t launch_cgr64(tl_ctx *c, int t0, int n)
 // true residual)
 hipError_t launch_cgs_dots(tl_ctx *c, int T)
 {
-    k_cgs_dots<<<sgrid(c->g), TB, 0, c->stream>>>(c->g, cgs_r(c, T), cgs_p(c, T), c->g64, c->hx64, c->hy64,
+    k_cgs_dots<<<sgrid(c->g), TB, 0, c->stream>>>(c->g, cgs_r(c, T), cgs_p(c, T), cgs_g(c), c->hx64, c->hy64,
                                                   &c->ctrl->rrs[T & 1], part_f(c, T));
     c->nb_f[T & 1] = nbh(c);
     return hipGetLastError();
@@ -4324,7 +4326,7 @@ hipError_t launch_cgs_final(tl_ctx *c, int T)
 {
     if (T & 1) {
         std::swap(c->f[TL_F_P], c->p_alt);
-        std::swap(c->f[TL_F_R], c->r_alt1);
+        std::swap(c->f[TL_F_R], c->sd_alt);
     }
     hipError_t e = launch_apply(c, c->f[TL_F_P], c->f[TL_F_W]);
     if (e != hipSuccess) return e;
