@@ -1156,6 +1156,7 @@ static int solve_jacobi(tl_ctx *c, const tl_solve_params *p, double rx, double r
         double *in, *out;
     };
     std::vector<Launch> made;  // the last ones enqueued
+    const bool self = jacobi_self(c->g);
     int tt = 0, nprev = 0, residp = 0;
     Ctrl k;
     RETIF(run_until_stop(c, 16, (long)p->max_iters + 16,
@@ -1170,15 +1171,16 @@ static int solve_jacobi(tl_ctx *c, const tl_solve_params *p, double rx, double r
                              // leave the residual's launch at most STEPS_HALO - 1 steps, and one at least
                              if (n == to50 && n == STEPS_HALO) n = STEPS_HALO / 2;
                              const int resid = (tt + n) % 50 == 0;
-                             const hipError_t e = launch_jacobi_steps(
+                             hipError_t e = launch_jacobi_steps(
                                  c, n, ucur, unext, ((tt + n) / 50) & 1 ? c->p_alt : c->f[TL_F_R], resid, nprev,
                                  residp, tt + 1);
                              if (made.size() >= 256) made.erase(made.begin(), made.begin() + 128);
                              made.push_back({tt + 1, n, ucur, unext});
                              std::swap(ucur, unext);
                              tt += n;
-                             nprev = n;
+                             nprev = self ? n : 0;
                              residp = resid;
+                             if (!self && e == hipSuccess) e = launch_jacobi_end(c, n, resid, tt + 1);
                              return e;
                          },
                          &k));
@@ -1432,10 +1434,15 @@ extern "C" int tl_kernel_repeat(tl_ctx *c, int kernel_id, int reps)
                 std::swap(s0, s1);
                 std::swap(r0, r1);
                 break;
-            case TL_K_JACOBI64:
-                HIPCHK(c, launch_jacobi_steps(c, STEPS_HALO, a, b, nullptr, 0, 0, 0, t));
+            case TL_K_JACOBI64: {
+                // with their stop tests, as a solve makes them
+                const bool self = jacobi_self(c->g);
+                const int t8 = t * STEPS_HALO;
+                HIPCHK(c, launch_jacobi_steps(c, STEPS_HALO, a, b, nullptr, 0, self && i > 0 ? STEPS_HALO : 0, 0, t8));
+                if (!self) HIPCHK(c, launch_jacobi_end(c, STEPS_HALO, 0, t8 + STEPS_HALO));
                 std::swap(a, b);
                 break;
+            }
             default: HIPCHK(c, launch_residual(c)); break;
             }
         }

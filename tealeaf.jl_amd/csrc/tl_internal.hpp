@@ -222,6 +222,14 @@ struct Tiles {
 // STEPS_HALO cells on every side shared with the neighbouring tiles; tiles are
 // dealt to the XCDs in runs of STEPS_CHUNK
 constexpr int STEPS_HALO = 8;
+// Jacobi: blocks up to which the next launch makes a launch's stop test itself.  Its
+// every block then reads the sums of all, 64 bytes each, which grows with the square
+// of the grid; a block of its own costs a launch and 40 us.  Us per iteration, itself /
+// one block: 1000^2 (192 blocks) 6.5 / 12.5, 2048^2 (832) 23.9 / 28.0, 3072^2 (1792)
+// 46.0 / 48.1, 4096^2 (3200) 86.3 / 79.9, 8192^2 403 / 275, 16384^2 2834 / 1044.
+#ifndef TL_JACOBI_SELF
+#define TL_JACOBI_SELF 2048u
+#endif
 constexpr int STEPS_CHUNK = 4;
 struct StepCoef {
     double a[STEPS_HALO], b[STEPS_HALO];
@@ -449,6 +457,7 @@ hipError_t launch_ppcg_steps(tl_ctx *c, int n, const StepCoef &co, const double 
 hipError_t launch_jacobi_steps(tl_ctx *c, int n, const double *u_in, double *u_out, double *r_out, int resid,
                                int nprev, int residp, int t);
 hipError_t launch_jacobi_end(tl_ctx *c, int nprev, int residp, int t);
+bool jacobi_self(const Geo &g);
 hipError_t launch_ir_prepare(tl_ctx *c, double rx, double ry, int coefficient);
 hipError_t launch_ir_clear_tail(tl_ctx *c);
 hipError_t launch_ir_accumulate(tl_ctx *c, int T, const float *pT = nullptr);

@@ -58,16 +58,30 @@ static Tiles make_tiles(int nx, int ny, int cols, int waves, int min_rows)
     return t;
 }
 
-// tiles of k_steps of w columns x h rows, and its blocks (a multiple of 8 runs)
-static inline int steps_tiles(int nx, int ny, int w, int h, int &gx)
+// Tiles of k_steps: 8 waves of 64 v columns x rw rows each, the tiles of a row, all
+// of them, and the blocks (a multiple of 8 runs)
+struct StepsTile {
+    int v, rw, gx, tiles;
+    unsigned blocks;
+};
+static StepsTile steps_shape(int nx, int ny, int v, int rw)
 {
-    const int uw = w - 2 * STEPS_HALO, uh = h - 2 * STEPS_HALO;
-    gx = (nx + uw - 1) / uw;
-    return gx * ((ny + uh - 1) / uh);
+    const int uw = 64 * v - 2 * STEPS_HALO, uh = 8 * rw - 2 * STEPS_HALO, gx = (nx + uw - 1) / uw;
+    const int tiles = gx * ((ny + uh - 1) / uh);
+    return {v, rw, gx, tiles, (unsigned)((tiles + 8 * STEPS_CHUNK - 1) / (8 * STEPS_CHUNK) * 8 * STEPS_CHUNK)};
 }
-static inline unsigned steps_blocks(int tiles)
+// 128 x 64 cells (one block per CU: 246 registers) from 128 such tiles on, half the
+// CUs, else 64 x 32.  Measured, PPCG iterations with 10 inner steps, 128x64 /
+// 64x32 / 128x32 tiles: 500x600 (65 tiles of 128x64) 36.6 / 33.3 / 33.1 us,
+// 800x700 (120) 43.4 / 42.2 / 44.9; 1000x900 (171) 48.8 and 128x32 55.1,
+// 1000x1300 (252) 62.7 and 70.3, 1600x1500 (480) 110.7 and 124.3.  Jacobi takes
+// 64 x 24 where that is one tile per CU at most (3000 iterations at 200x300, 190
+// such tiles: 6.7 ms, 95 of 64x32 7.3 ms; Chebyshev and PPCG within 2%).
+static StepsTile steps_tile(int nx, int ny, bool jacobi)
 {
-    return (unsigned)((tiles + 8 * STEPS_CHUNK - 1) / (8 * STEPS_CHUNK) * 8 * STEPS_CHUNK);
+    const StepsTile narrow = steps_shape(nx, ny, 1, 3), wide = steps_shape(nx, ny, 2, 8);
+    if (jacobi && narrow.tiles <= 256) return narrow;
+    return wide.tiles >= 128 ? wide : steps_shape(nx, ny, 1, 4);
 }
 
 Geo make_geo(int nx, int ny, int hd)
@@ -158,9 +172,7 @@ Geo make_geo(int nx, int ny, int hd)
     g.nbmax = std::max(g.nbmax, std::max(g.r64.blocks, g.r32.blocks));
     g.s32 = make_tiles(nx, ny, TL_S32_COLS, TL_S32_WAVES, TL_S32_ROWS);
     g.nbmax = std::max(g.nbmax, std::max(g.s64.blocks, g.s32.blocks));
-    int gxs;
-    g.nbmax = std::max(g.nbmax, (int)steps_blocks(steps_tiles(nx, ny, 64, 32, gxs)));  // its smallest tiles but one
-    g.nbmax = std::max(g.nbmax, (int)steps_blocks(256));                               // at most that many of 64 x 24
+    for (const bool jacobi : {false, true}) g.nbmax = std::max(g.nbmax, (int)steps_tile(nx, ny, jacobi).blocks);
     return g;
 }
 
@@ -3733,10 +3745,10 @@ __global__ __launch_bounds__(TBV) void k_cheby2(Geo g, int ty, int t, const doub
 //   VS_PPCG   a: sd, d: r, b: u (own cells).  64 for up to 8 steps (64 for each)
 //   VS_JACOBI a: u, d: u0 (const).            40 for up to 8 steps (40 for each)
 // times the rim's re-reads (most of them cache hits).  Jacobi's error sum
-// |u' - u| of every step is one of eight sums per block; the next launch sums
-// them over the blocks, in order, and stops the solve at the first step that met
-// the rule (the host then repeats the steps up to that one from the launch's
-// input).  With resid a last stage forms r = u0 - A u and its sum of squares,
+// |u' - u| of every step is one of eight sums per block; the next launch, or on large
+// grids a launch of one block, sums them over the blocks, in order, and stops the
+// solve at the first step that met the rule (the host then repeats the steps up to
+// that one from the launch's input).  With resid a last stage forms r = u0 - A u and its sum of squares,
 // which Jacobi adds to the error of every 50th iteration (Jacobi.jl:21-24).
 // Bound by latency, a block per CU loading, stepping and storing in turn: eight
 // PPCG steps take 53 us at 1300x1700 (two rounds of 432 tiles; two steps as one
@@ -3770,11 +3782,14 @@ __device__ __forceinline__ bool jacobi_stopped(Ctrl *__restrict__ ctrl, const do
     return stop;
 }
 
-__global__ __launch_bounds__(TB) void k_jacobi_end(Ctrl *__restrict__ ctrl, const double *__restrict__ part,
-                                                   unsigned nb, int n, int resid, int t0)
+// the same by one block: after the last launch, and after every launch of more than
+// TL_JACOBI_SELF blocks, where every block of the next one would read all sums
+constexpr int JACOBI_END = 1024;
+__global__ __launch_bounds__(JACOBI_END) void k_jacobi_end(Ctrl *__restrict__ ctrl, const double *__restrict__ part,
+                                                           unsigned nb, int n, int resid, int t0)
 {
     if (t0 > ctrl->stop_iter) return;
-    (void)jacobi_stopped<TB>(ctrl, part, nb, n, resid, t0);
+    (void)jacobi_stopped<JACOBI_END>(ctrl, part, nb, n, resid, t0);
 }
 
 template <int OP, int V, int NW, int RW>
@@ -4526,33 +4541,25 @@ hipError_t launch_ppcg_inner2(tl_ctx *c, double a1, double b1, double a2, double
     return hipGetLastError();
 }
 
-// calls f(columns per lane, waves per block, rows per wave) for the tile: 128 x
-// 64 cells (one block per CU: 246 registers) from 128 such tiles on, half the
-// CUs, else 64 x 32.  Measured, PPCG iterations with 10 inner steps, 128x64 /
-// 64x32 / 128x32 tiles: 500x600 (65 tiles of 128x64) 36.6 / 33.3 / 33.1 us,
-// 800x700 (120) 43.4 / 42.2 / 44.9; 1000x900 (171) 48.8 and 128x32 55.1,
-// 1000x1300 (252) 62.7 and 70.3, 1600x1500 (480) 110.7 and 124.3.  Jacobi takes
-// 64 x 24 where that is one tile per CU at most (3000 iterations at 200x300, 190
-// such tiles: 6.7 ms, 95 of 64x32 7.3 ms; Chebyshev and PPCG within 2%).
-template <bool JACOBI = false, class F>
-static hipError_t with_steps_tile(const Geo &g, F &&f)
+// calls f(columns per lane, waves per block, rows per wave) for the tile
+template <class F>
+static hipError_t with_steps_tile(const StepsTile &s, F &&f)
 {
-    int gx;
-    if (JACOBI && steps_tiles(g.nx, g.ny, 64, 24, gx) <= 256)
-        return f(std::integral_constant<int, 1>{}, std::integral_constant<int, 8>{}, std::integral_constant<int, 3>{});
-    if (steps_tiles(g.nx, g.ny, 128, 64, gx) >= 128)
-        return f(std::integral_constant<int, 2>{}, std::integral_constant<int, 8>{}, std::integral_constant<int, 8>{});
-    return f(std::integral_constant<int, 1>{}, std::integral_constant<int, 8>{}, std::integral_constant<int, 4>{});
+    const std::integral_constant<int, 1> one{};
+    const std::integral_constant<int, 2> two{};
+    const std::integral_constant<int, 8> eight{};
+    return s.rw == 3   ? f(one, eight, std::integral_constant<int, 3>{})
+           : s.rw == 4 ? f(one, eight, std::integral_constant<int, 4>{})
+                       : f(two, eight, eight);
 }
 
 hipError_t launch_cheby_steps(tl_ctx *c, int n, const StepCoef &co, const double *u_in, double *u_out,
                               const double *p_in, double *p_out, int t)
 {
-    return with_steps_tile(c->g, [&](auto v, auto nw, auto rw) {
+    const StepsTile o = steps_tile(c->g.nx, c->g.ny, false);
+    return with_steps_tile(o, [&](auto v, auto nw, auto rw) {
         constexpr int V = decltype(v)::value, NW = decltype(nw)::value, RW = decltype(rw)::value;
-        int gx;
-        const unsigned nb = steps_blocks(steps_tiles(c->g.nx, c->g.ny, 64 * V, NW * RW, gx));
-        k_steps<VS_CHEBY, V, NW, RW><<<nb, NW * 64, 0, c->stream>>>(c->g, gx, t, n, u_in, u_out, c->f[TL_F_U0], nullptr, p_in,
+        k_steps<VS_CHEBY, V, NW, RW><<<o.blocks, NW * 64, 0, c->stream>>>(c->g, o.gx, t, n, u_in, u_out, c->f[TL_F_U0], nullptr, p_in,
                                                             p_out, c->f[TL_F_KX], c->f[TL_F_KY], co, c->ctrl, nullptr,
                                                             nullptr, 0, 0, 0);
         return hipGetLastError();
@@ -4562,11 +4569,10 @@ hipError_t launch_cheby_steps(tl_ctx *c, int n, const StepCoef &co, const double
 hipError_t launch_ppcg_steps(tl_ctx *c, int n, const StepCoef &co, const double *sd_in, double *sd_out,
                              const double *r_in, double *r_out, int t)
 {
-    return with_steps_tile(c->g, [&](auto v, auto nw, auto rw) {
+    const StepsTile o = steps_tile(c->g.nx, c->g.ny, false);
+    return with_steps_tile(o, [&](auto v, auto nw, auto rw) {
         constexpr int V = decltype(v)::value, NW = decltype(nw)::value, RW = decltype(rw)::value;
-        int gx;
-        const unsigned nb = steps_blocks(steps_tiles(c->g.nx, c->g.ny, 64 * V, NW * RW, gx));
-        k_steps<VS_PPCG, V, NW, RW><<<nb, NW * 64, 0, c->stream>>>(c->g, gx, t, n, sd_in, sd_out, r_in, r_out, c->f[TL_F_U],
+        k_steps<VS_PPCG, V, NW, RW><<<o.blocks, NW * 64, 0, c->stream>>>(c->g, o.gx, t, n, sd_in, sd_out, r_in, r_out, c->f[TL_F_U],
                                                            c->f[TL_F_U], c->f[TL_F_KX], c->f[TL_F_KY], co, c->ctrl,
                                                            nullptr, nullptr, 0, 0, 0);
         return hipGetLastError();
@@ -4576,17 +4582,19 @@ hipError_t launch_ppcg_steps(tl_ctx *c, int n, const StepCoef &co, const double 
 // the error sums of a launch at iterations t .. alternate between two sets
 static inline double *part_j(tl_ctx *c, int set) { return c->part_j + (size_t)set * STEPS_HALO * stride(c); }
 
+// does the next launch make the stop test of a launch itself (else k_jacobi_end)?
+bool jacobi_self(const Geo &g) { return steps_tile(g.nx, g.ny, true).blocks <= TL_JACOBI_SELF; }
+
 hipError_t launch_jacobi_steps(tl_ctx *c, int n, const double *u_in, double *u_out, double *r_out, int resid,
                                int nprev, int residp, int t)
 {
     c->jset ^= 1;
     const bool prof = prof_start(c, TL_K_JACOBI64);
-    const hipError_t e = with_steps_tile<true>(c->g, [&](auto v, auto nw, auto rw) {
+    const StepsTile o = steps_tile(c->g.nx, c->g.ny, true);
+    const hipError_t e = with_steps_tile(o, [&](auto v, auto nw, auto rw) {
         constexpr int V = decltype(v)::value, NW = decltype(nw)::value, RW = decltype(rw)::value;
-        int gx;
-        const unsigned nb = steps_blocks(steps_tiles(c->g.nx, c->g.ny, 64 * V, NW * RW, gx));
-        k_steps<VS_JACOBI, V, NW, RW><<<nb, NW * 64, 0, c->stream>>>(
-            c->g, gx, t, n, u_in, u_out, c->f[TL_F_U0], r_out, nullptr, nullptr, c->f[TL_F_KX], c->f[TL_F_KY],
+        k_steps<VS_JACOBI, V, NW, RW><<<o.blocks, NW * 64, 0, c->stream>>>(
+            c->g, o.gx, t, n, u_in, u_out, c->f[TL_F_U0], r_out, nullptr, nullptr, c->f[TL_F_KX], c->f[TL_F_KY],
             StepCoef{}, c->ctrl, part_j(c, c->jset ^ 1), part_j(c, c->jset), nprev, residp, resid);
         return hipGetLastError();
     });
@@ -4597,13 +4605,9 @@ hipError_t launch_jacobi_steps(tl_ctx *c, int n, const double *u_in, double *u_o
 // the stop test of the last launch's steps, which ended before iteration t
 hipError_t launch_jacobi_end(tl_ctx *c, int nprev, int residp, int t)
 {
-    return with_steps_tile<true>(c->g, [&](auto v, auto nw, auto rw) {
-        constexpr int V = decltype(v)::value, NW = decltype(nw)::value, RW = decltype(rw)::value;
-        int gx;
-        const unsigned nb = steps_blocks(steps_tiles(c->g.nx, c->g.ny, 64 * V, NW * RW, gx));
-        k_jacobi_end<<<1, TB, 0, c->stream>>>(c->ctrl, part_j(c, c->jset), nb, nprev, residp, t - nprev);
-        return hipGetLastError();
-    });
+    k_jacobi_end<<<1, JACOBI_END, 0, c->stream>>>(c->ctrl, part_j(c, c->jset), steps_tile(c->g.nx, c->g.ny, true).blocks,
+                                                  nprev, residp, t - nprev);
+    return hipGetLastError();
 }
 
 // u += d; d = 0 over the whole allocation (d is zero outside the interior)
