@@ -55,8 +55,10 @@ extern "C" {
 #define TL_WARM_GUESS 2     /* caller-provided guess set with tl_set_guess, same fallback */
 
 /* tl_solve_params.launch: how the CG iterations of TL_CG solves (FP64 and
- * TL_FP32_IR) reach the GPU.  Both give bit-identical results.  Other solvers
- * always use stream launches.  FP64 CG on up to about 1966080 cells (1024 tiles
+ * TL_FP32_IR) reach the GPU.  Both give bit-identical results for the same form of
+ * the iteration: always in FP64; in FP32 for an explicit fp32_kernels, and for
+ * TL_FP32_KERNELS_AUTO when nx is not a multiple of 4 (when it is, AUTO takes another
+ * form with TL_LAUNCH_GRAPH).  Other solvers always use stream launches.  FP64 CG on up to about 1966080 cells (1024 tiles
  * of 120 x 16) runs up to 256 iterations per launch with either, unless its kernels
  * are being timed (tl_profile_begin with TL_K_CG_W64 or TL_K_CG_UR64). */
 #define TL_LAUNCH_STREAM 0  /* kernels enqueued in batches of up to 64 iterations */
@@ -136,11 +138,11 @@ typedef struct {
 
 /* tl_solve_params.fp32_kernels: how a TL_FP32_IR iteration is split into kernels.
  * Both reach the same FP64 tolerance; their FP32 roundings differ. */
-#define TL_FP32_KERNELS_AUTO 0   /* stream launches: from 32768 up to about 3932160 cells (1024 tiles
-                                   of 240 x 16) up to 256 iterations per launch, unless the pairs'
-                                   kernels are being timed; else pairs when nx is a multiple of 4 or
-                                   the grid has 16384 cells or more; TL_LAUNCH_GRAPH: fused when nx
-                                   is a multiple of 4; else two kernels */
+#define TL_FP32_KERNELS_AUTO 0   /* TL_LAUNCH_GRAPH and nx a multiple of 4: fused.  Else from 32768 up
+                                   to about 3932160 cells (1024 tiles of 240 x 16) up to 256
+                                   iterations per launch, unless the pairs' kernels are being timed;
+                                   else pairs when nx is a multiple of 4 or the grid has 16384 cells
+                                   or more; else two kernels */
 #define TL_FP32_KERNELS_TWO 1    /* two kernels and two reductions per iteration (34 B/cell) */
 #define TL_FP32_KERNELS_FUSED 2  /* one kernel and one reduction per iteration (22 B/cell); needs nx % 4 == 0 */
 #define TL_FP32_KERNELS_PAIRS 3  /* two iterations per two kernels and two reductions (s-step CG, s = 2;

@@ -609,9 +609,11 @@ static bool resident_pays(tl_ctx *c)
     return !(c->prof_mask & ((1u << TL_K_CG_W64) | (1u << TL_K_CG_UR64))) && resident_fits(c, c->g.r64);
 }
 
-// The same in FP32, TL_FP32_KERNELS_AUTO with stream launches: no slower than the
-// pairs on any grid that fits (1024 tiles of 240 x 16, 3932160 cells; k_cgr's
-// comment).  Below 32768 cells the choice is as before (a solve takes a few ms).
+// The same in FP32, TL_FP32_KERNELS_AUTO: no slower than the pairs on any grid that
+// fits (1024 tiles of 240 x 16, 3932160 cells; k_cgr's comment).  Below 32768 cells,
+// where a solve takes a few ms either way, the forms that these grids have had, with
+// their iteration counts and bits (182^2, just above: 13.2 us per iteration in pairs,
+// 7.8 in registers).
 static bool resident32_pays(tl_ctx *c)
 {
     return !(c->prof_mask & ((1u << TL_K_CGP_G32) | (1u << TL_K_CGP_U32))) && (long)c->g.nx * c->g.ny >= 32768 &&
@@ -620,12 +622,11 @@ static bool resident32_pays(tl_ctx *c)
 
 static bool fused_fits(const tl_ctx *c) { return c->g.nx % 4 == 0; }
 
-// TL_FP32_KERNELS_AUTO with stream launches: pairs of iterations, which take
-// any nx.  They are the faster form on ragged grids of every size measured
-// (milliseconds of a solve, two kernels / pairs: 63x61 2.9 / 1.9, 131x77 5.9 /
-// 3.2, 151x153 5.9 / 3.4, 201x203 10.0 / 5.6), but on small ones the two kernels
-// stay: there stream launches and hipGraph batches are held to give the same
-// bits (the pairs have no batch form), and a solve takes a few ms.
+// TL_FP32_KERNELS_AUTO: pairs of iterations, which take any nx.  They were the
+// faster form on ragged grids of every size measured (milliseconds of a solve, two
+// kernels / pairs: 63x61 2.9 / 1.9, 131x77 5.9 / 3.2, 151x153 5.9 / 3.4, 201x203
+// 10.0 / 5.6).  Below 16384 cells, where a solve takes a few ms either way, ragged
+// grids keep the two kernels with the iteration counts and bits they have had.
 static bool pairs_pay(const tl_ctx *c) { return fused_fits(c) || (long)c->g.nx * c->g.ny >= 16384; }
 
 static int status_of(tl_ctx *c, const Ctrl &k)
@@ -1224,17 +1225,19 @@ static int solve_cg_ir(tl_ctx *c, const tl_solve_params *p, double rx, double ry
     HIPCHK(c, launch_ir_prepare(c, rx, ry, p->coefficient));
     const double delta = p->ir_delta > 0 && p->ir_delta < 1 ? p->ir_delta : 0.1;
     HIPCHK(c, launch_init_ctrl(c, MODE_IR, p->max_iters, p->eps, p->rel_tol, delta, 0, 0, p->epslim));
-    // pairs of iterations (k_cgp) run as stream launches; with TL_LAUNCH_GRAPH
-    // the automatic choice takes the fused kernel
-    bool resident = p->fp32_kernels == TL_FP32_KERNELS_AUTO && p->launch != TL_LAUNCH_GRAPH && resident32_pays(c);
+    // The automatic choice: many iterations per launch or pairs of iterations
+    // (k_cgp), which run as stream launches; with TL_LAUNCH_GRAPH the fused kernel
+    // where it fits, else the same as with stream launches, so that both modes give
+    // the same bits there
+    const bool choose = p->fp32_kernels == TL_FP32_KERNELS_AUTO;
+    const bool stream = p->launch != TL_LAUNCH_GRAPH || !fused_fits(c);
+    bool resident = choose && stream && resident32_pays(c);
     bool pairs = p->fp32_kernels == TL_FP32_KERNELS_PAIRS ||
-                       (p->fp32_kernels == TL_FP32_KERNELS_AUTO && !resident && TL_CGP_AUTO && pairs_pay(c) &&
-                        p->launch != TL_LAUNCH_GRAPH);
-    bool fused = !pairs && !resident && (p->fp32_kernels == TL_FP32_KERNELS_FUSED ||
-                                  (p->fp32_kernels == TL_FP32_KERNELS_AUTO && fused_fits(c)));
+                 (choose && !resident && TL_CGP_AUTO && pairs_pay(c) && stream);
+    bool fused = !pairs && !resident && (p->fp32_kernels == TL_FP32_KERNELS_FUSED || (choose && fused_fits(c)));
     if (fused || pairs || resident) {
         const int rc = ensure_fused(c);
-        if (rc != TL_OK && (rc != TL_E_NOMEM || p->fp32_kernels != TL_FP32_KERNELS_AUTO)) return rc;
+        if (rc != TL_OK && (rc != TL_E_NOMEM || !choose)) return rc;
         if (rc != TL_OK) fused = pairs = resident = false;  // the two kernels need no second r
     }
     const double *guess = nullptr;
