@@ -1047,6 +1047,8 @@ template <int V>
 struct VCol {
     int x0;        // first column owned (may be >= nx: inactive)
     int xl;        // first column loaded (clamped into the grid)
+    int xk;        // the same for kx, whose last face is nx: it is the right one of column nx - 1,
+                   // which takes it from the lane beside it
     int y0, y1;
     bool active;
     int lane;
@@ -1090,6 +1092,7 @@ __device__ __forceinline__ VCol<V> vcolumn(const Geo &g, int ty)
     vtile<V>(g, bx, by);
     c.x0 = (bx * TBV + threadIdx.x) * V;
     c.xl = min(c.x0, ((g.nx - 1) / V) * V);
+    c.xk = min(c.x0, g.nx / V * V);
     c.y0 = by * ty;
     c.y1 = min(c.y0 + ty, g.ny);
     c.active = c.x0 < g.nx;
@@ -3305,7 +3308,7 @@ __global__ __launch_bounds__(TBV) void k_vs64(Geo g, int ty, int t, const double
                 const int y = yb + q;
                 const long ic = atc(g, cl.xl, y), iu = atc(g, cl.xl, y + 1);
                 vload<T, V>(B.up[q], a_in + iu);
-                vload<T, V>(B.kxv[q], kx + ic);
+                vload<T, V>(B.kxv[q], kx + atc(g, cl.xk, y));
                 vload<T, V>(B.kyu[q], ky + at(g, cl.xl, min(y + 1, g.ny)));
                 vload<T, V>(B.e1[q], f1 + ic);
                 vload<T, V>(B.e2[q], f2 + ic);
@@ -3422,7 +3425,7 @@ __global__ __launch_bounds__(TBV) void k_ppcg2(Geo g, int ty, int t, const doubl
             const int yk = min(max(L, 0), g.ny), yu = min(max(L - 2, 0), g.ny - 1);
             vload<T, V, TL_NT_2STEP_LD != 0>(B.s, sdin + at(g, xl, ys));
             vload<T, V, TL_NT_2STEP_LD != 0>(B.r, rin + at(g, xl, yr));
-            vload<T, V, TL_NT_2STEP_LD != 0>(B.kx, kx + at(g, xl, yr));
+            vload<T, V, TL_NT_2STEP_LD != 0>(B.kx, kx + at(g, cl.xk, yr));
             vload<T, V, TL_NT_2STEP_LD != 0>(B.ky, ky + at(g, xl, yk));
             vload<T, V, TL_NT_2STEP_LD != 0>(B.u, u + at(g, xl, yu));
             B.es = B.ef = B.er = B.ekx1 = B.eky = (T)0;
@@ -3594,7 +3597,7 @@ __global__ __launch_bounds__(TBV) void k_cheby2(Geo g, int ty, int t, const doub
             vload<T, V, TL_NT_2STEP_LD != 0>(B.u, uin + at(g, xl, ys));
             vload<T, V, TL_NT_2STEP_LD != 0>(B.u0, u0 + at(g, xl, yr));
             vload<T, V, TL_NT_2STEP_LD != 0>(B.p, pin + at(g, xl, yr));
-            vload<T, V, TL_NT_2STEP_LD != 0>(B.kx, kx + at(g, xl, yr));
+            vload<T, V, TL_NT_2STEP_LD != 0>(B.kx, kx + at(g, cl.xk, yr));
             vload<T, V, TL_NT_2STEP_LD != 0>(B.ky, ky + at(g, xl, yk));
             B.eu = B.ef = B.eu0 = B.ep = B.ekx1 = B.eky = (T)0;
             // lane 63's right face of its last column, as the single step loads it
@@ -3813,11 +3816,9 @@ __global__ __launch_bounds__(NW * 64) void k_steps(Geo g, int gx, int t, int n, 
     const int bx = tile % gx, by = tile / gx;
     const int x = bx * UW - HALO + lane * V;
     const int yw = by * UH - HALO + wave * RW;  // the wave's first row
-    // left of column 0: halo and padding columns (valid memory).  Right of the
-    // grid Jacobi needs the domain face's coefficient kx(nx), which stays in its
-    // denominator; in the residual forms it cancels with the reflected neighbour
-    // and its rounding is the single step's, which reads the last vector again.
-    const int xc = min(x, (OP == VS_JACOBI ? g.nx : g.nx - 1) / V * V);
+    // left of column 0: halo and padding columns (valid memory); right of the grid the
+    // column of the domain face's coefficient kx(nx)
+    const int xc = min(x, g.nx / V * V);
     const bool own_x = lane >= HALO / V && lane < 64 - HALO / V && x < g.nx;
     // element of row y's storage: a uniform row start and a 32-bit lane offset
     const unsigned xo = (unsigned)(xc + XCOL);
