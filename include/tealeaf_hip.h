@@ -309,9 +309,11 @@ int tl_get_cg_history(tl_ctx *ctx, double *alpha, double *beta, int n);
  * grid.  An FP32 CG iteration in its two-kernel form:
  * PW = end of the previous iteration (beta, stop test, p = r + beta p) fused
  * with w = A p and <p, w>; UR = x += alpha p, r -= alpha w and <r, r>. */
-#define TL_K_CG_W64 0  /* FP64 CG sweep at odd iterations (also the w = A p of PPCG's outer iterations) */
-#define TL_K_CG_UR64 1 /* FP64 CG sweep at even iterations, which also updates u */
-#define TL_K_CG_P64 2  /* FP64 p = r + beta p of PPCG's outer iterations */
+#define TL_K_CG_W64 0  /* FP64 CG sweep at odd iterations (also the w = A p of the CG phase of Chebyshev and
+                          PPCG and of PPCG's outer iterations) */
+#define TL_K_CG_UR64 1 /* FP64 CG sweep at even iterations, which also updates u (also the u and r updates
+                          of that CG phase) */
+#define TL_K_CG_P64 2  /* FP64 p = r + beta p of that CG phase and of PPCG's outer iterations */
 #define TL_K_CG_W32 3  /* FP32 PW of the inner CG (w = A p only reduced, not stored) */
 #define TL_K_CG_UR32 4 /* FP32 UR of the inner CG (recomputes A p) */
 #define TL_K_CG_P32 5  /* unused: folded into TL_K_CG_W32 */

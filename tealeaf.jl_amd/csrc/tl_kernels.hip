@@ -4245,10 +4245,12 @@ hipError_t launch_cg_w64(tl_ctx *c, int t)
 
 hipError_t launch_cg_ur64(tl_ctx *c, int t)
 {
+    const bool prof = prof_start(c, TL_K_CG_UR64);
     k_cg_ur<double><<<sgrid(c->g), TB, 0, c->stream>>>(c->g, t, c->f[TL_F_U], c->f[TL_F_P], c->f[TL_F_R],
                                                         c->f[TL_F_W], c->ctrl, part_w(c), c->nb_w, part_r(c, t - 1),
                                                         nbr(c, t - 1), part_r(c, t), c->hist_a);
     nbr(c, t) = nbh(c);
+    if (prof) prof_stop(c);
     return hipGetLastError();
 }
 
