@@ -60,7 +60,8 @@ extern "C" {
  * TL_FP32_KERNELS_AUTO when nx is not a multiple of 4 (when it is, AUTO takes another
  * form with TL_LAUNCH_GRAPH).  Other solvers always use stream launches.  FP64 CG on up to about 1966080 cells (1024 tiles
  * of 120 x 16) runs up to 256 iterations per launch with either, unless its kernels
- * are being timed (tl_profile_begin with TL_K_CG_W64 or TL_K_CG_UR64). */
+ * are being timed (tl_profile_begin with TL_K_CG_W64 or TL_K_CG_UR64) or resident_polls
+ * is negative. */
 #define TL_LAUNCH_STREAM 0  /* kernels enqueued in batches of up to 64 iterations */
 #define TL_LAUNCH_GRAPH 1   /* after a first stream batch, replays of one hipGraph of 64 iterations
                                (captured on first use, kept with the context, re-captured when
@@ -115,7 +116,13 @@ typedef struct {
     int warm_policy;      /* TL_WARM_LEARNED: TL_WARM_POLICY_* */
     int ppcg_pairs;       /* TL_PPCG: TL_PPCG_PAIRS_* */
     int cheby_pairs;      /* TL_CHEBY: TL_CHEBY_PAIRS_* */
-    int reserved[3];
+    int resident_polls;   /* TL_CG held in registers (TL_FORM_RESIDENT), whose blocks wait for one another
+                             in every iteration: how often a block looks before it gives up and the
+                             solve starts again in another form, as every later solve of the context
+                             does.  0: about a second's worth; < 0: never held in registers (several
+                             threads that solve at once on one GPU: the runtime runs such launches one
+                             after the other) */
+    int reserved[2];
 } tl_solve_params;
 
 /* tl_solve_params.warm_policy: when a TL_WARM_LEARNED solve runs the network.
@@ -140,8 +147,8 @@ typedef struct {
  * Both reach the same FP64 tolerance; their FP32 roundings differ. */
 #define TL_FP32_KERNELS_AUTO 0   /* TL_LAUNCH_GRAPH and nx a multiple of 4: fused.  Else from 32768 up
                                    to about 3932160 cells (1024 tiles of 240 x 16) up to 256
-                                   iterations per launch, unless the pairs' kernels are being timed;
-                                   else pairs when nx is a multiple of 4 or the grid has 16384 cells
+                                   iterations per launch, unless the pairs' kernels are being timed
+                                   or resident_polls is negative; else pairs when nx is a multiple of 4 or the grid has 16384 cells
                                    or more; else two kernels */
 #define TL_FP32_KERNELS_TWO 1    /* two kernels and two reductions per iteration (34 B/cell) */
 #define TL_FP32_KERNELS_FUSED 2  /* one kernel and one reduction per iteration (22 B/cell); needs nx % 4 == 0 */
@@ -169,7 +176,7 @@ typedef struct {
     int start;            /* initial guess used: TL_START_* */
     int coef_format;      /* TL_FP32_IR: storage of the inner CG's cell coefficient, TL_COEF_*; 0 otherwise */
     int warm_attempted;   /* a warm start was evaluated in this solve (network run or guess tested) */
-    int reserved_i;
+    int cg_form;          /* TL_CG: how the iterations ran, TL_FORM_* */
     double warm_ms;       /* wall time of that evaluation (prediction and residual test) */
     double reserved[1];
 } tl_solve_stats;
@@ -179,6 +186,15 @@ typedef struct {
 #define TL_COEF_FP16 1
 #define TL_COEF_BF16 2
 #define TL_COEF_FP32 3
+
+/* tl_solve_stats.cg_form (0: another solver) */
+#define TL_FORM_SWEEP 1     /* FP64: one sweep over the grid per iteration */
+#define TL_FORM_RESIDENT 2  /* up to 256 iterations per launch, the grid held in registers */
+#define TL_FORM_TWO 3       /* TL_FP32_KERNELS_TWO */
+#define TL_FORM_FUSED 4     /* TL_FP32_KERNELS_FUSED */
+#define TL_FORM_PAIRS 5     /* TL_FP32_KERNELS_PAIRS */
+#define TL_FORM_RESTARTED 16 /* added to the form: a launch of TL_FORM_RESIDENT was refused or gave up
+                                before, and the solve started again */
 
 /* tl_solve_stats.start */
 #define TL_START_PREVIOUS 0 /* u = energy*density (the reference's start) */

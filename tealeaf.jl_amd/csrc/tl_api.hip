@@ -586,9 +586,11 @@ static int ensure_cgs(tl_ctx *c)
 // to 1024 tiles of 120 columns by 16 rows, 1966080 cells), where it is faster than
 // the sweeps at every size measured (k_cgr's comment), with stream launches and
 // hipGraph batches alike: a launch is a batch of iterations already.  Not where
-// the launches of the sweeps are timed one by one (tl_profile_begin).
-static bool resident_fits(tl_ctx *c, const Tiles &o)
+// the launches of the sweeps are timed one by one (tl_profile_begin), nor where the
+// caller declines it (tl_solve_params.resident_polls).
+static bool resident_fits(tl_ctx *c, const tl_solve_params *p, const Tiles &o)
 {
+    if (p->resident_polls < 0) return false;
     if (c->coop_cus < 0) {
         int coop = 0, cus = 0;
         (void)hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, c->device);
@@ -604,9 +606,9 @@ static bool resident_fits(tl_ctx *c, const Tiles &o)
     }
     return true;
 }
-static bool resident_pays(tl_ctx *c)
+static bool resident_pays(tl_ctx *c, const tl_solve_params *p)
 {
-    return !(c->prof_mask & ((1u << TL_K_CG_W64) | (1u << TL_K_CG_UR64))) && resident_fits(c, c->g.r64);
+    return !(c->prof_mask & ((1u << TL_K_CG_W64) | (1u << TL_K_CG_UR64))) && resident_fits(c, p, c->g.r64);
 }
 
 // The same in FP32, TL_FP32_KERNELS_AUTO: no slower than the pairs on any grid that
@@ -614,11 +616,12 @@ static bool resident_pays(tl_ctx *c)
 // where a solve takes a few ms either way, the forms that these grids have had, with
 // their iteration counts and bits (182^2, just above: 13.2 us per iteration in pairs,
 // 7.8 in registers).
-static bool resident32_pays(tl_ctx *c)
+static bool resident32_pays(tl_ctx *c, const tl_solve_params *p)
 {
     return !(c->prof_mask & ((1u << TL_K_CGP_G32) | (1u << TL_K_CGP_U32))) && (long)c->g.nx * c->g.ny >= 32768 &&
-           resident_fits(c, c->g.r32);
+           resident_fits(c, p, c->g.r32);
 }
+static int polls_of(const tl_solve_params *p) { return p->resident_polls > 0 ? p->resident_polls : CGR_POLLS; }
 
 static bool fused_fits(const tl_ctx *c) { return c->g.nx % 4 == 0; }
 
@@ -828,18 +831,46 @@ static void fill_stats(const Ctrl &k, tl_solve_stats *st)
     st->converged = k.why == WHY_CONVERGED;
 }
 
+// the iterations of solve_cg64 from CG.init! on; *lost: no cooperative launch was to
+// be had, or a block of one did not arrive
+static int cg64_iterate(tl_ctx *c, const tl_solve_params *p, bool rel, bool resident, Ctrl *k, int *refreshes,
+                        bool *lost)
+{
+    int t = 0;
+    for (;;) {
+        if (resident) {
+            hipError_t e;
+            do {
+                e = launch_cgr64(c, t + 1, CGR_BATCH, polls_of(p));
+                t += CGR_BATCH;
+                RETIF(read_ctrl(c, k));
+            } while (e == hipSuccess && k->stop_iter == INT_MAX);
+            *lost = e != hipSuccess || k->status == TL_E_HIP;
+            if (*lost) return TL_OK;
+        } else {
+            RETIF(run_until_stop(c, 64, (long)p->max_iters + 16, [&]() { return launch_cgs64(c, ++t); }, k,
+                                 p->launch == TL_LAUNCH_GRAPH ? GRAPH_CG64 : -1, &t));
+        }
+        t = k->stop_iter;
+        if (!resident && t >= 1) HIPCHK(c, launch_cgs_pending(c, t));
+        if (!rel || k->why != WHY_CONVERGED) return TL_OK;
+        // the relative rule is met by the recursive residual: confirm it on the
+        // true one, and if rounding has let the two drift apart, continue CG
+        // from the true residual (keeping the search direction)
+        HIPCHK(c, launch_acc64(c, c->f[TL_F_U], c->u_alt));
+        HIPCHK(c, launch_cg64_true_residual(c, t));
+        RETIF(read_ctrl(c, k));
+        if (k->stop_iter != INT_MAX) return TL_OK;
+        HIPCHK(c, launch_cgs_dots(c, t));
+        ++*refreshes;
+    }
+}
+
 // CG.solve!, CG.jl:7-29 (FP64)
 static int solve_cg64(tl_ctx *c, const tl_solve_params *p, double rx, double ry, tl_solve_stats *st)
 {
     RETIF(ensure_history(c, p->max_iters));
     RETIF(ensure_cgs(c));
-    HIPCHK(c, launch_init_coef(c, rx, ry, p->coefficient, INIT_CG64));
-    const int mode = p->stop_rule == TL_STOP_RELATIVE ? MODE_CG_REL : MODE_CG_REF;
-    HIPCHK(c, launch_init_ctrl(c, mode, p->max_iters, p->eps, p->rel_tol, 0.0, p->presteps, p->error_switch,
-                               p->epslim));
-    const double *guess = nullptr;
-    RETIF(choose_guess(c, p, rx, ry, &guess, st));
-    HIPCHK(c, launch_cg_init_resid(c, guess, !c->g64));
     // Under the relative rule the iterations add alpha p to a correction d
     // (u_alt, free during CG) instead of to u, and d is added to u at every
     // true-residual check ("reliable updates" with group-wise solution
@@ -847,47 +878,30 @@ static int solve_cg64(tl_ctx *c, const tl_solve_params *p, double rx, double ry,
     // correction, not to u, so the true residual can reach tolerances that
     // CG updating u directly stalls above (measured at 8192^2 from the 69th
     // timestep of a random-rectangle problem: 2-3e-9 against 1e-10).
-    const bool group = mode == MODE_CG_REL;
-    if (group) HIPCHK(c, hipMemsetAsync(c->u_alt, 0, c->g.elems * sizeof(double), c->stream));
-    c->cg_u = group ? c->u_alt : nullptr;
-    HIPCHK(c, launch_cgs_dots(c, 0));
+    const bool rel = p->stop_rule == TL_STOP_RELATIVE;
+    const double *guess = nullptr;
+    bool resident = resident_pays(c, p), lost = false;
+    st->cg_form = resident ? TL_FORM_RESIDENT : TL_FORM_SWEEP;
     Ctrl k;
-    int t = 0;
-    const bool resident = resident_pays(c);
-    for (;;) {
-        if (resident) {
-            hipError_t e;
-            do {
-                e = launch_cgr64(c, t + 1, CGR_BATCH);
-                t += CGR_BATCH;
-                RETIF(read_ctrl(c, &k));
-            } while (e == hipSuccess && k.stop_iter == INT_MAX);
-            if (e != hipSuccess || k.status == TL_E_HIP) {
-                // no cooperative launch to be had, or a block of one did not
-                // arrive: from the start in sweeps, as every later solve
-                (void)hipGetLastError();
-                c->coop_cus = 0;
-                c->cg_u = nullptr;
-                return solve_cg64(c, p, rx, ry, st);
-            }
-        } else {
-            RETIF(run_until_stop(c, 64, (long)p->max_iters + 16, [&]() { return launch_cgs64(c, ++t); }, &k,
-                                 p->launch == TL_LAUNCH_GRAPH ? GRAPH_CG64 : -1, &t));
+    do {
+        if (lost) {  // from the start in sweeps, as every later solve
+            (void)hipGetLastError();
+            c->coop_cus = 0;
+            resident = lost = false;
+            st->cg_form = TL_FORM_SWEEP | TL_FORM_RESTARTED;
         }
-        t = k.stop_iter;
-        if (!resident && t >= 1) HIPCHK(c, launch_cgs_pending(c, t));
-        if (mode != MODE_CG_REL || k.why != WHY_CONVERGED) break;
-        // the relative rule is met by the recursive residual: confirm it on the
-        // true one, and if rounding has let the two drift apart, continue CG
-        // from the true residual (keeping the search direction)
-        HIPCHK(c, launch_acc64(c, c->f[TL_F_U], c->u_alt));
-        HIPCHK(c, launch_cg64_true_residual(c, t));
-        RETIF(read_ctrl(c, &k));
-        if (k.stop_iter != INT_MAX) break;
-        HIPCHK(c, launch_cgs_dots(c, t));
-        ++st->refreshes;
-    }
-    if (group) HIPCHK(c, launch_acc64(c, c->f[TL_F_U], c->u_alt));  // pending updates (max_iters, breakdown)
+        HIPCHK(c, launch_init_coef(c, rx, ry, p->coefficient, INIT_CG64));
+        HIPCHK(c, launch_init_ctrl(c, rel ? MODE_CG_REL : MODE_CG_REF, p->max_iters, p->eps, p->rel_tol, 0.0,
+                                   p->presteps, p->error_switch, p->epslim));
+        if (!(st->cg_form & TL_FORM_RESTARTED)) RETIF(choose_guess(c, p, rx, ry, &guess, st));
+        HIPCHK(c, launch_cg_init_resid(c, guess, !c->g64));
+        if (rel) HIPCHK(c, hipMemsetAsync(c->u_alt, 0, c->g.elems * sizeof(double), c->stream));
+        c->cg_u = rel ? c->u_alt : nullptr;
+        HIPCHK(c, launch_cgs_dots(c, 0));
+        st->refreshes = 0;
+        RETIF(cg64_iterate(c, p, rel, resident, &k, &st->refreshes, &lost));
+    } while (lost);
+    if (rel) HIPCHK(c, launch_acc64(c, c->f[TL_F_U], c->u_alt));  // pending updates (max_iters, breakdown)
     c->cg_u = nullptr;  // other callers of the CG sweeps update u
     const int T = k.stop_iter;
     if (!c->g64) {  // w held the coefficient: as CG.init! leaves it, for T = 0
@@ -1213,52 +1227,23 @@ static hipError_t cg32_iteration(tl_ctx *c, int t)
     return e;
 }
 
-// FP32 inner CG with FP64 residual replacement ("reliable updates"): the
-// FP32 recurrence runs on the correction x; when its residual has fallen by
-// ir_delta (or reaches the tolerance) the FP64 solution is accumulated,
-// u += x, and the FP64 residual r = u0 - A u replaces the FP32 one, keeping
-// the search direction.  Converged when the FP64 residual meets rel_tol.
-static int solve_cg_ir(tl_ctx *c, const tl_solve_params *p, double rx, double ry, tl_solve_stats *st)
+// the iterations of solve_cg_ir from its first FP64 residual on, in one of the forms
+// TL_FORM_*; *lost as in cg64_iterate
+static int ir_iterate(tl_ctx *c, const tl_solve_params *p, int form, Ctrl *k, tl_solve_stats *st, bool *lost)
 {
-    RETIF(ensure_fp32(c));
-    HIPCHK(c, launch_init_coef(c, rx, ry, p->coefficient, INIT_CG));
-    HIPCHK(c, launch_ir_prepare(c, rx, ry, p->coefficient));
-    const double delta = p->ir_delta > 0 && p->ir_delta < 1 ? p->ir_delta : 0.1;
-    HIPCHK(c, launch_init_ctrl(c, MODE_IR, p->max_iters, p->eps, p->rel_tol, delta, 0, 0, p->epslim));
-    // The automatic choice: many iterations per launch or pairs of iterations
-    // (k_cgp), which run as stream launches; with TL_LAUNCH_GRAPH the fused kernel
-    // where it fits, else the same as with stream launches, so that both modes give
-    // the same bits there
-    const bool choose = p->fp32_kernels == TL_FP32_KERNELS_AUTO;
-    const bool stream = p->launch != TL_LAUNCH_GRAPH || !fused_fits(c);
-    bool resident = choose && stream && resident32_pays(c);
-    bool pairs = p->fp32_kernels == TL_FP32_KERNELS_PAIRS ||
-                 (choose && !resident && TL_CGP_AUTO && pairs_pay(c) && stream);
-    bool fused = !pairs && !resident && (p->fp32_kernels == TL_FP32_KERNELS_FUSED || (choose && fused_fits(c)));
-    if (fused || pairs || resident) {
-        const int rc = ensure_fused(c);
-        if (rc != TL_OK && (rc != TL_E_NOMEM || !choose)) return rc;
-        if (rc != TL_OK) fused = pairs = resident = false;  // the two kernels need no second r
-    }
-    const double *guess = nullptr;
-    RETIF(choose_guess(c, p, rx, ry, &guess, st));
-    // u0 = b = energy*density; u = guess or b; bb, tol_abs
-    HIPCHK(c, launch_cg_init_resid(c, guess));
-    HIPCHK(c, hipMemsetAsync(c->x32, 0, c->g.elems * sizeof(float), c->stream));
-    if (pairs || resident) HIPCHK(c, launch_ir_clear_tail(c));
+    const bool resident = form == TL_FORM_RESIDENT, pairs = form == TL_FORM_PAIRS, fused = form == TL_FORM_FUSED;
     int t = 0;  // last iteration enqueued
     // r = u0 - A u (FP64, stored in FP32) and p = r; fused: the four sums of
     // iteration 1 (r and p in the buffers of iteration 0)
     HIPCHK(c, launch_ir_residual(c, 1, t + 1));
     if (fused || resident) HIPCHK(c, launch_cgf_dots(c, 0));
     int tfirst = 1;  // pairs: the first pair after a start or a refresh
-    Ctrl k;
-    RETIF(read_ctrl(c, &k));
-    st->init_rel_resid = k.bb > 0 ? std::sqrt(k.sums[0] / k.bb) : 0.0;
-    int refreshes = 0;
-    while (k.stop_iter == INT_MAX || k.why == WHY_REFRESH) {
-        if (k.stop_iter != INT_MAX && k.why == WHY_REFRESH) {
-            t = k.stop_iter;
+    RETIF(read_ctrl(c, k));
+    st->init_rel_resid = k->bb > 0 ? std::sqrt(k->sums[0] / k->bb) : 0.0;
+    st->refreshes = 0;
+    while (k->stop_iter == INT_MAX || k->why == WHY_REFRESH) {
+        if (k->stop_iter != INT_MAX && k->why == WHY_REFRESH) {
+            t = k->stop_iter;
             if (resident) {
                 // u += x (complete after every launch), the FP64 residual into
                 // r(t)'s buffer, p(t) kept, and the four sums
@@ -1281,23 +1266,20 @@ static int solve_cg_ir(tl_ctx *c, const tl_solve_params *p, double rx, double ry
                 HIPCHK(c, launch_ir_accumulate(c, t));
                 HIPCHK(c, launch_ir_residual(c, 0, t + 1));
             }
-            ++refreshes;
-            RETIF(read_ctrl(c, &k));
+            ++st->refreshes;
+            RETIF(read_ctrl(c, k));
             continue;
         }
         if (resident) {
             hipError_t e;
             const int from = t + 1;
             do {
-                e = launch_cgr32(c, t + 1, CGR_BATCH, t + 1 == from);
+                e = launch_cgr32(c, t + 1, CGR_BATCH, t + 1 == from, polls_of(p));
                 t += CGR_BATCH;
-                RETIF(read_ctrl(c, &k));
-            } while (e == hipSuccess && k.stop_iter == INT_MAX);
-            if (e != hipSuccess || k.status == TL_E_HIP) {  // as in solve_cg64
-                (void)hipGetLastError();
-                c->coop_cus = 0;
-                return solve_cg_ir(c, p, rx, ry, st);
-            }
+                RETIF(read_ctrl(c, k));
+            } while (e == hipSuccess && k->stop_iter == INT_MAX);
+            *lost = e != hipSuccess || k->status == TL_E_HIP;
+            if (*lost) return TL_OK;
         } else if (pairs)
             RETIF(run_until_stop(c, 32, (long)p->max_iters / 2 + 16,
                                  [&]() {
@@ -1305,20 +1287,74 @@ static int solve_cg_ir(tl_ctx *c, const tl_solve_params *p, double rx, double ry
                                      t += 2;
                                      return e;
                                  },
-                                 &k));
+                                 k));
         else if (fused)
-            RETIF(run_until_stop(c, 64, (long)p->max_iters + 16, [&]() { return launch_cgf(c, ++t); }, &k,
+            RETIF(run_until_stop(c, 64, (long)p->max_iters + 16, [&]() { return launch_cgf(c, ++t); }, k,
                                  p->launch == TL_LAUNCH_GRAPH ? GRAPH_CGF : -1, &t));
         else
-            RETIF(run_until_stop(c, 64, (long)p->max_iters + 16, [&]() { return cg32_iteration(c, ++t); }, &k,
+            RETIF(run_until_stop(c, 64, (long)p->max_iters + 16, [&]() { return cg32_iteration(c, ++t); }, k,
                                  p->launch == TL_LAUNCH_GRAPH ? GRAPH_CG32 : -1, &t));
     }
-    if (k.why == WHY_MAXITERS)  // keep the partial correction (complete in x, or with an odd iteration's update pending)
-        HIPCHK(c, launch_ir_accumulate(c, resident || pairs ? 0 : k.stop_iter, fused ? cgf_p(c, k.stop_iter) : nullptr));
+    if (k->why == WHY_MAXITERS)  // keep the partial correction (complete in x, or with an odd iteration's update pending)
+        HIPCHK(c, launch_ir_accumulate(c, resident || pairs ? 0 : k->stop_iter, fused ? cgf_p(c, k->stop_iter) : nullptr));
+    return TL_OK;
+}
+
+// FP32 inner CG with FP64 residual replacement ("reliable updates"): the
+// FP32 recurrence runs on the correction x; when its residual has fallen by
+// ir_delta (or reaches the tolerance) the FP64 solution is accumulated,
+// u += x, and the FP64 residual r = u0 - A u replaces the FP32 one, keeping
+// the search direction.  Converged when the FP64 residual meets rel_tol.
+static int solve_cg_ir(tl_ctx *c, const tl_solve_params *p, double rx, double ry, tl_solve_stats *st)
+{
+    RETIF(ensure_fp32(c));
+    const double delta = p->ir_delta > 0 && p->ir_delta < 1 ? p->ir_delta : 0.1;
+    // The automatic choice: many iterations per launch or pairs of iterations
+    // (k_cgp), which run as stream launches; with TL_LAUNCH_GRAPH the fused kernel
+    // where it fits, else the same as with stream launches, so that both modes give
+    // the same bits there
+    const bool choose = p->fp32_kernels == TL_FP32_KERNELS_AUTO;
+    const bool stream = p->launch != TL_LAUNCH_GRAPH || !fused_fits(c);
+    const auto automatic = [&]() {
+        return stream && resident32_pays(c, p)               ? TL_FORM_RESIDENT
+               : stream && TL_CGP_AUTO && pairs_pay(c) ? TL_FORM_PAIRS
+               : fused_fits(c)                           ? TL_FORM_FUSED
+                                                         : TL_FORM_TWO;
+    };
+    int form = p->fp32_kernels == TL_FP32_KERNELS_TWO     ? TL_FORM_TWO
+               : p->fp32_kernels == TL_FP32_KERNELS_FUSED ? TL_FORM_FUSED
+               : p->fp32_kernels == TL_FP32_KERNELS_PAIRS ? TL_FORM_PAIRS
+                                                          : automatic();
+    if (form != TL_FORM_TWO) {
+        const int rc = ensure_fused(c);
+        if (rc != TL_OK && (rc != TL_E_NOMEM || !choose)) return rc;
+        if (rc != TL_OK) form = TL_FORM_TWO;  // needs no second r
+    }
+    const double *guess = nullptr;
+    bool lost = false;
+    st->cg_form = form;
+    Ctrl k;
+    do {
+        if (lost) {  // from the start in another form, as every later solve
+            (void)hipGetLastError();
+            c->coop_cus = 0;
+            lost = false;
+            form = automatic();
+            st->cg_form = form | TL_FORM_RESTARTED;
+        }
+        HIPCHK(c, launch_init_coef(c, rx, ry, p->coefficient, INIT_CG));
+        HIPCHK(c, launch_ir_prepare(c, rx, ry, p->coefficient));
+        HIPCHK(c, launch_init_ctrl(c, MODE_IR, p->max_iters, p->eps, p->rel_tol, delta, 0, 0, p->epslim));
+        if (!(st->cg_form & TL_FORM_RESTARTED)) RETIF(choose_guess(c, p, rx, ry, &guess, st));
+        // u0 = b = energy*density; u = guess or b; bb, tol_abs
+        HIPCHK(c, launch_cg_init_resid(c, guess));
+        HIPCHK(c, hipMemsetAsync(c->x32, 0, c->g.elems * sizeof(float), c->stream));
+        if (form == TL_FORM_PAIRS || form == TL_FORM_RESIDENT) HIPCHK(c, launch_ir_clear_tail(c));
+        RETIF(ir_iterate(c, p, form, &k, st, &lost));
+    } while (lost);
     st->inner_iters = k.iters;
     st->iterations = k.iters;
     st->cg_iters = k.iters;
-    st->refreshes = refreshes;
     st->coef_format = !TL_GC16 ? TL_COEF_FP32 : c->gc_fmt == GC_F16 ? TL_COEF_FP16 : TL_COEF_BF16;
     fill_stats(k, st);
     HIPCHK(c, launch_halo(c, TL_X_U, 1, nullptr, 0));

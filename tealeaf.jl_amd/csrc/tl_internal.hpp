@@ -124,9 +124,9 @@ constexpr int TBV = TL_TBV;
 #define TL_S32_COLS 240
 #define TL_S32_WAVES 3072
 #define TL_S32_ROWS 4
-// k_cgr: blocks at most (one per CU) and iterations per launch (the
-// host reads the state once per launch, 15 us)
-constexpr int CGR_MAXB = 256, CGR_BATCH = 256;
+// k_cgr: blocks at most (one per CU), iterations per launch (the host reads the
+// state once per launch, 15 us) and polls of a wait, about a second's
+constexpr int CGR_MAXB = 256, CGR_BATCH = 256, CGR_POLLS = 1 << 20;
 // sweeps over more bytes than this (the Infinity Cache) use streaming access.
 // Measured with the FP64 CG sweep: 453 MB of arrays (3072^2) 92.6 us per
 // iteration streaming, 102.2 cached; 83 MB (1501x1103) 25.1 and 21.9.
@@ -411,8 +411,8 @@ hipError_t launch_resid_norm_slot(tl_ctx *c, const double *b, const double *x, i
 // iteration is tref (t only selects the buffers; the kernel takes its
 // iteration number from Ctrl::tg)
 hipError_t launch_cgs64(tl_ctx *c, int t, int tref = 0);
-hipError_t launch_cgr64(tl_ctx *c, int t0, int n);
-hipError_t launch_cgr32(tl_ctx *c, int t0, int n, bool first);
+hipError_t launch_cgr64(tl_ctx *c, int t0, int n, int polls);
+hipError_t launch_cgr32(tl_ctx *c, int t0, int n, bool first, int polls);
 hipError_t launch_cgs_dots(tl_ctx *c, int T);
 hipError_t launch_cgs_pending(tl_ctx *c, int T);
 hipError_t launch_cgs_final(tl_ctx *c, int T);

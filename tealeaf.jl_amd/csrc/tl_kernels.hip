@@ -2604,7 +2604,7 @@ __global__ __launch_bounds__(TBV) __attribute__((amdgpu_waves_per_eu(3))) void k
 // all blocks have published again and so have read them, and are used again at
 // t + 3 (three sets).  Cells go to the two arrays of r in turn: whoever
 // overwrites r(t) has seen all sums of t + 1, published after r(t) was read.
-// All blocks run at once (cooperative launch) and a wait ends after CGR_SPIN
+// All blocks run at once (cooperative launch) and a wait ends after `polls`
 // polls: a block that gives up records TL_E_HIP and leaves, and so do the others;
 // the host then solves again in sweeps.
 // Bound by the latency of one exchange per iteration: store, sums, poll, load
@@ -2619,7 +2619,6 @@ __global__ __launch_bounds__(TBV) __attribute__((amdgpu_waves_per_eu(3))) void k
 // with the sums, spilled registers (512^2 9.6); so did 8 rows with two waves per
 // SIMD (FP64 1501x1103 24.0, FP32 2047x1533 20.2).
 constexpr unsigned long long EMPTY = 0x7ff4dead00000000ull;
-constexpr int CGR_SPIN = 1 << 20;  // about a second
 
 __device__ __forceinline__ unsigned long long agent_load(const unsigned long long *p)
 {
@@ -2664,7 +2663,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT / 256, NT
     Geo g, Tiles o, int t0, int n, T *__restrict__ r_even, T *__restrict__ r_odd, T *__restrict__ p_even,
     T *__restrict__ p_odd, T *__restrict__ u, const std::conditional_t<sizeof(T) == 8, double, tl_gc_t> *__restrict__ gc,
     T hx, T hy, Ctrl *__restrict__ ctrl, const double *__restrict__ sin, unsigned nbin, int side, double *__restrict__ sout,
-    unsigned long long *__restrict__ slots, double *__restrict__ hist_a, double *__restrict__ hist_b)
+    unsigned long long *__restrict__ slots, int polls, double *__restrict__ hist_a, double *__restrict__ hist_b)
 {
     typedef unsigned long long u64;
     constexpr bool F64 = sizeof(T) == 8;
@@ -2896,7 +2895,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT / 256, NT
                         full = full && q[k] != EMPTY;
                     }
                     if (full) break;
-                    if (spin > CGR_SPIN) {
+                    if (spin > polls) {
                         gone = 1;
                         break;
                     }
@@ -4303,7 +4302,7 @@ static const void *cgr_kernel(const Tiles &o)
                         : (const void *)k_cgr<T, FMT, 16, 256>;
 }
 
-hipError_t launch_cgr64(tl_ctx *c, int t0, int n)
+hipError_t launch_cgr64(tl_ctx *c, int t0, int n, int polls)
 {
     Geo g = c->g;
     Tiles o = g.r64;
@@ -4312,7 +4311,7 @@ hipError_t launch_cgr64(tl_ctx *c, int t0, int n)
     double hx = c->hx64, hy = c->hy64, *sout = part_f(c, t0 + n - 1);
     int side = 1;
     void *args[] = {&g, &o, &t0, &n, &re, &ro, &pe, &po, &u, &gc, &hx, &hy, &c->ctrl, &sin, &c->nb_f[(t0 - 1) & 1], &side,
-                    &sout, &c->slots, &c->hist_a, &c->hist_b};
+                    &sout, &c->slots, &polls, &c->hist_a, &c->hist_b};
     const void *kern = cgr_kernel<double, 0>(o);
     const hipError_t e = launch_resident(c, kern, o, args);
     c->nb_f[(t0 + n - 1) & 1] = (unsigned)o.blocks;
@@ -4747,7 +4746,7 @@ hipError_t launch_cgf_dots(tl_ctx *c, int T)
 
 // FP32 inner iterations t0 .. t0 + n - 1 in one launch (k_cgr), x complete after
 // it; first: after k_cgf_dots (a start or a refresh)
-hipError_t launch_cgr32(tl_ctx *c, int t0, int n, bool first)
+hipError_t launch_cgr32(tl_ctx *c, int t0, int n, bool first, int polls)
 {
     Geo g = c->g;
     Tiles o = g.r32;
@@ -4756,7 +4755,7 @@ hipError_t launch_cgr32(tl_ctx *c, int t0, int n, bool first)
     double *sout = part_f(c, t0 + n - 1), *none = nullptr;
     int side = !first;
     void *args[] = {&g,       &o,        &t0,   &n,    &re,  &ro,   &pe,       &po,   &c->x32, &c->gcell, &c->hx32,
-                    &c->hy32, &c->ctrl, &sin,  &c->nb_f[(t0 - 1) & 1], &side, &sout, &c->slots, &none, &none};
+                    &c->hy32, &c->ctrl, &sin,  &c->nb_f[(t0 - 1) & 1], &side, &sout, &c->slots, &polls, &none, &none};
     const void *kern = c->gc_fmt == GC_F16 ? cgr_kernel<float, GC_F16>(o) : cgr_kernel<float, GC_BF16>(o);
     const hipError_t e = launch_resident(c, kern, o, args);
     c->nb_f[(t0 + n - 1) & 1] = (unsigned)o.blocks;

@@ -42,6 +42,7 @@ TL_START_PREVIOUS, TL_START_WARM = 0, 1
  TL_K_JACOBI64, TL_K_RESID64, TL_K_CGF32, TL_K_PPCG2_64, TL_K_CHEBY2_64, TL_K_CGP_G32, TL_K_CGP_U32) = range(15)
 TL_K_COUNT = 15
 TL_FP32_KERNELS_AUTO, TL_FP32_KERNELS_TWO, TL_FP32_KERNELS_FUSED, TL_FP32_KERNELS_PAIRS = 0, 1, 2, 3
+(TL_FORM_SWEEP, TL_FORM_RESIDENT, TL_FORM_TWO, TL_FORM_FUSED, TL_FORM_PAIRS), TL_FORM_RESTARTED = range(1, 6), 16
 TL_WARM_POLICY_BACKOFF, TL_WARM_POLICY_EVERY = 0, 1
 TL_PPCG_PAIRS_AUTO, TL_PPCG_PAIRS_OFF = 0, 1
 TL_CHEBY_PAIRS_AUTO, TL_CHEBY_PAIRS_OFF = 0, 1
@@ -76,7 +77,8 @@ class SolveParams(C.Structure):
         ("ppcg_inner_steps", C.c_int), ("error_switch", C.c_int), ("eps", C.c_double), ("epslim", C.c_double),
         ("precision", C.c_int), ("stop_rule", C.c_int), ("rel_tol", C.c_double), ("warm_start", C.c_int),
         ("check_result", C.c_int), ("ir_delta", C.c_double), ("launch", C.c_int), ("fp32_kernels", C.c_int),
-        ("warm_policy", C.c_int), ("ppcg_pairs", C.c_int), ("cheby_pairs", C.c_int), ("reserved", C.c_int * 3),
+        ("warm_policy", C.c_int), ("ppcg_pairs", C.c_int), ("cheby_pairs", C.c_int),
+        ("resident_polls", C.c_int), ("reserved", C.c_int * 2),
     ]
 
 
@@ -86,7 +88,7 @@ class SolveStats(C.Structure):
         ("inner_iters", C.c_int), ("refreshes", C.c_int), ("converged", C.c_int), ("fallback", C.c_int),
         ("error", C.c_double), ("eigmin", C.c_double), ("eigmax", C.c_double), ("rel_resid", C.c_double),
         ("init_rel_resid", C.c_double), ("solve_ms", C.c_double), ("start", C.c_int), ("coef_format", C.c_int),
-        ("warm_attempted", C.c_int), ("reserved_i", C.c_int), ("warm_ms", C.c_double), ("reserved", C.c_double * 1),
+        ("warm_attempted", C.c_int), ("cg_form", C.c_int), ("warm_ms", C.c_double), ("reserved", C.c_double * 1),
     ]
 
     def as_dict(self):
