@@ -1019,9 +1019,10 @@ static int solve_cheby(tl_ctx *c, const tl_solve_params *p, double rx, double ry
     while (k.stop_iter == INT_MAX && tt < maxiters) {
         made.clear();
         for (int norms = 0; norms < ahead && tt < maxiters;) {
-            // iterations up to the next one with a norm (Cheby.jl:47-50)
+            // iterations up to the next one with a norm (Cheby.jl:47-50), as far as they
+            // decide how many this launch takes: far from it, STEPS_HALO
             int d = 1;
-            while (tt + d < maxiters && !(chebyiters + d >= estiter && (tt + d + 1) % 10 == 0)) ++d;
+            while (d < STEPS_HALO + 2 && tt + d < maxiters && !(chebyiters + d >= estiter && (tt + d + 1) % 10 == 0)) ++d;
             const int norm = chebyiters + d >= estiter && (tt + d + 1) % 10 == 0;
             const int n = !pairs || d == 1 ? 1 : d == 2 ? 2 : std::min(STEPS_HALO, norm ? d - 2 : d);
             const int last = norm && n == d;
