@@ -59,7 +59,7 @@ extern "C" {
  * the iteration: always in FP64; in FP32 for an explicit fp32_kernels, and for
  * TL_FP32_KERNELS_AUTO when nx is not a multiple of 4 (when it is, AUTO takes another
  * form with TL_LAUNCH_GRAPH).  Other solvers always use stream launches.  FP64 CG on up to about 1966080 cells (1024 tiles
- * of 120 x 16) runs up to 256 iterations per launch with either, unless its kernels
+ * of 120 x 16) runs up to 255 iterations per launch with either, unless its kernels
  * are being timed (tl_profile_begin with TL_K_CG_W64 or TL_K_CG_UR64) or resident_polls
  * is negative. */
 #define TL_LAUNCH_STREAM 0  /* kernels enqueued in batches of up to 64 iterations */
@@ -146,7 +146,7 @@ typedef struct {
 /* tl_solve_params.fp32_kernels: how a TL_FP32_IR iteration is split into kernels.
  * Both reach the same FP64 tolerance; their FP32 roundings differ. */
 #define TL_FP32_KERNELS_AUTO 0   /* TL_LAUNCH_GRAPH and nx a multiple of 4: fused.  Else from 32768 up
-                                   to about 3932160 cells (1024 tiles of 240 x 16) up to 256
+                                   to about 3932160 cells (1024 tiles of 240 x 16) up to 255
                                    iterations per launch, unless the pairs' kernels are being timed
                                    or resident_polls is negative; else pairs when nx is a multiple of 4 or the grid has 16384 cells
                                    or more; else two kernels */
@@ -189,7 +189,7 @@ typedef struct {
 
 /* tl_solve_stats.cg_form (0: another solver) */
 #define TL_FORM_SWEEP 1     /* FP64: one sweep over the grid per iteration */
-#define TL_FORM_RESIDENT 2  /* up to 256 iterations per launch, the grid held in registers */
+#define TL_FORM_RESIDENT 2  /* up to 255 iterations per launch, the grid held in registers */
 #define TL_FORM_TWO 3       /* TL_FP32_KERNELS_TWO */
 #define TL_FORM_FUSED 4     /* TL_FP32_KERNELS_FUSED */
 #define TL_FORM_PAIRS 5     /* TL_FP32_KERNELS_PAIRS */

@@ -125,8 +125,9 @@ constexpr int TBV = TL_TBV;
 #define TL_S32_WAVES 3072
 #define TL_S32_ROWS 4
 // k_cgr: blocks at most (one per CU), iterations per launch (the host reads the
-// state once per launch, 15 us) and polls of a wait, about a second's
-constexpr int CGR_MAXB = 256, CGR_BATCH = 256, CGR_POLLS = 1 << 20;
+// state once per launch, 15 us; odd, so that the sums a launch reads and those it
+// writes lie in different sets) and polls of a wait, about a second's
+constexpr int CGR_MAXB = 256, CGR_BATCH = 255, CGR_POLLS = 1 << 20;
 // sweeps over more bytes than this (the Infinity Cache) use streaming access.
 // Measured with the FP64 CG sweep: 453 MB of arrays (3072^2) 92.6 us per
 // iteration streaming, 102.2 cached; 83 MB (1501x1103) 25.1 and 21.9.

@@ -3745,7 +3745,7 @@ __global__ __launch_bounds__(TBV) void k_cheby2(Geo g, int ty, int t, const doub
 // The operations and their association are the single step's (k_vs64), so each
 // step is bit-identical to a launch of it.
 //   VS_CHEBY  a: u, b: p, d: u0 (const).      Bytes per cell: 56 for up to 8 steps (56 for each)
-//   VS_PPCG   a: sd, d: r, b: u (own cells).  64 for up to 8 steps (64 for each)
+//   VS_PPCG   a: sd, d: r, b: u (own cells, in place).  64 for up to 8 steps (64 for each)
 //   VS_JACOBI a: u, d: u0 (const).            40 for up to 8 steps (40 for each)
 // times the rim's re-reads (most of them cache hits).  Jacobi's error sum
 // |u' - u| of every step is one of eight sums per block; the next launch, or on large
@@ -3798,8 +3798,8 @@ __global__ __launch_bounds__(JACOBI_END) void k_jacobi_end(Ctrl *__restrict__ ct
 template <int OP, int V, int NW, int RW>
 __global__ __launch_bounds__(NW * 64) void k_steps(Geo g, int gx, int t, int n, const double *__restrict__ a_in,
                                                    double *__restrict__ a_out, const double *__restrict__ d_in,
-                                                   double *__restrict__ d_out, const double *__restrict__ b_in,
-                                                   double *__restrict__ b_out, const double *__restrict__ kx,
+                                                   double *__restrict__ d_out, const double *b_in,
+                                                   double *b_out, const double *__restrict__ kx,
                                                    const double *__restrict__ ky, StepCoef co,
                                                    Ctrl *__restrict__ ctrl, const double *__restrict__ part_in,
                                                    double *__restrict__ part_out, int nprev, int residp, int resid)
