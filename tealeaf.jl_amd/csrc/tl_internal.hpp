@@ -98,9 +98,13 @@ constexpr int TBV = TL_TBV;
 // iteration against 0.311 ms for register loads; depth 2 (5 waves per SIMD)
 // and 4 (2 waves) 2-5% slower.  A band-walking copy with the same arrays and
 // geometry streams at 5.0 TB/s, so more rows in flight have little to win.
-// blocks of the two-step PPCG kernel on large grids (its launches that do
-// not form the residual sum; the one that does keeps the FP64 kernels'
-// bands, so that the sum is the single step's bit for bit)
+#ifndef TL_CGF_DEPTH
+#define TL_CGF_DEPTH 0
+#endif
+// blocks of the two-step PPCG kernel on large grids in launches that do not form
+// the residual sum (with 4 or more inner steps only the last two of an outer iteration
+// run in it, which do: those keep the FP64 kernels' bands, so that the sum is the
+// single step's bit for bit; with inner steps that leave a remainder of two others do)
 #ifndef TL_VEC_BLOCKS_PPCG2
 #define TL_VEC_BLOCKS_PPCG2 768
 #endif
@@ -132,9 +136,6 @@ constexpr int CGR_MAXB = 256, CGR_BATCH = 255, CGR_POLLS = 1 << 20;
 // Measured with the FP64 CG sweep: 453 MB of arrays (3072^2) 92.6 us per
 // iteration streaming, 102.2 cached; 83 MB (1501x1103) 25.1 and 21.9.
 constexpr size_t TL_CACHE_BYTES = (size_t)256 << 20;
-#ifndef TL_CGF_DEPTH
-#define TL_CGF_DEPTH 0
-#endif
 // TL_FP32_KERNELS_AUTO takes the pairs of iterations (k_cgp) with stream launches
 // (1), or the fused kernel where it fits (0).  Measured at 8192^2: 0.240 ms per
 // iteration (first sweep 0.118, second 0.361 per pair) against 0.287 for the

@@ -41,11 +41,11 @@
 
 namespace tl {
 
-// Tiles of `cols` columns for at most about `waves` waves (one round of them on
-// the chip), bands of at least `min_rows` rows.
 // threads per block of k_cgr by rows per wave
 static int cgr_threads(const Tiles &o) { return o.ty <= 4 ? 512 : 256; }
 
+// Tiles of `cols` columns for at most about `waves` waves (one round of them on
+// the chip), bands of at least `min_rows` rows.
 static Tiles make_tiles(int nx, int ny, int cols, int waves, int min_rows)
 {
     Tiles t{};
@@ -75,8 +75,10 @@ static StepsTile steps_shape(int nx, int ny, int v, int rw)
 // 64x32 / 128x32 tiles: 500x600 (65 tiles of 128x64) 36.6 / 33.3 / 33.1 us,
 // 800x700 (120) 43.4 / 42.2 / 44.9; 1000x900 (171) 48.8 and 128x32 55.1,
 // 1000x1300 (252) 62.7 and 70.3, 1600x1500 (480) 110.7 and 124.3.  Jacobi takes
-// 64 x 24 where that is one tile per CU at most (3000 iterations at 200x300, 190
-// such tiles: 6.7 ms, 95 of 64x32 7.3 ms; Chebyshev and PPCG within 2%).
+// 64 x 24 where that is one tile per CU at most; us per iteration, 64x24 / 64x32:
+// 64^2 2.64 / 2.93, 100^2 2.33 / 2.58, 200x300 2.23 / 2.44, 288x336 (252 tiles) 2.28 /
+// 2.46; 760x129 (272) 3.77 / 2.47, 600x300 (494) 4.19 /
+// 2.57; Chebyshev and PPCG within 2%.
 static StepsTile steps_tile(int nx, int ny, bool jacobi)
 {
     const StepsTile narrow = steps_shape(nx, ny, 1, 3), wide = steps_shape(nx, ny, 2, 8);
@@ -2612,10 +2614,10 @@ __global__ __launch_bounds__(TBV) __attribute__((amdgpu_waves_per_eu(3))) void k
 // across the XCDs, 4 to 5 us.  Microseconds per iteration, sweeps / this: 64^2 10.4
 // / 5.6, 256^2 8.8 / 5.8, 512^2 9.0 / 6.9, 700x500 9.3 / 7.4, 900^2 12.6 / 8.2;
 // FP32, pairs / this: 182^2 13.2 / 7.8, 256^2 11.4 / 7.5, 512x400 10.5 / 7.5, 1024^2
-// 11.0 / 9.3.  Larger grids take 12 or 16 rows per wave and one wave per SIMD (NT
+// 11.0 / 9.4.  Larger grids take 12 or 16 rows per wave and one wave per SIMD (NT
 // 256: 512 registers a lane), bound by arithmetic: FP64 1000^2 14.5 / 10.8,
-// 1200x1150 17.5 / 11.0, 1501x1103 18.8 / 14.9; FP32 1300x1400 13.7 / 13.6, 1700x1600
-// 16.3 / 15.3, 2047x1533 17.5 / 15.0.
+// 1200x1150 17.5 / 11.0, 1501x1103 18.8 / 14.0; FP32 1300x1400 13.7 / 13.6, 1700x1600
+// 16.3 / 15.3, 2047x1533 17.5 / 15.3.
 // Measured and left: the neighbours' cells with EMPTY places of their own, polled
 // with the sums, spilled registers (512^2 9.6); so did 8 rows with two waves per
 // SIMD (FP64 1501x1103 24.0, FP32 2047x1533 20.2).
@@ -4287,7 +4289,7 @@ hipError_t launch_cgs64(tl_ctx *c, int t, int tref)
     return hipGetLastError();
 }
 
-// iterations t0 .. t0 + n - 1 in one launch (k_cgr); u has every update after it
+// a launch of k_cgr; one block needs no other
 static hipError_t launch_resident(tl_ctx *c, const void *kern, const Tiles &o, void **args)
 {
     if (o.blocks == 1) return hipLaunchKernel(kern, dim3(1), dim3(cgr_threads(o)), args, 0, c->stream);
@@ -4303,6 +4305,7 @@ static const void *cgr_kernel(const Tiles &o)
                         : (const void *)k_cgr<T, FMT, 16, 256>;
 }
 
+// iterations t0 .. t0 + n - 1 in one launch (k_cgr); u has every update after it
 hipError_t launch_cgr64(tl_ctx *c, int t0, int n, int polls)
 {
     Geo g = c->g;
