@@ -119,9 +119,7 @@ typedef struct {
     int resident_polls;   /* TL_CG held in registers (TL_FORM_RESIDENT), whose blocks wait for one another
                              in every iteration: how often a block looks before it gives up and the
                              solve starts again in another form, as every later solve of the context
-                             does.  0: about a second's worth; < 0: never held in registers (several
-                             threads that solve at once on one GPU: the runtime runs such launches one
-                             after the other) */
+                             does.  0: about a second's worth; < 0: never held in registers */
     int reserved[2];
 } tl_solve_params;
 

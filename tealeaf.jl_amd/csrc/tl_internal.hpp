@@ -226,7 +226,7 @@ struct Tiles {
 constexpr int STEPS_HALO = 8;
 // Jacobi: blocks up to which the next launch makes a launch's stop test itself.  Its
 // every block then reads the sums of all, 64 bytes each, which grows with the square
-// of the grid; a block of its own costs a launch and 40 us.  Us per iteration, itself /
+// of the grid; a block of its own costs a launch and 45 to 80 us.  Us per iteration, itself /
 // one block: 1000^2 (192 blocks) 6.5 / 12.5, 2048^2 (832) 23.9 / 28.0, 3072^2 (1792)
 // 46.0 / 48.1, 4096^2 (3200) 86.3 / 79.9, 8192^2 403 / 275, 16384^2 2834 / 1044.
 #ifndef TL_JACOBI_SELF
