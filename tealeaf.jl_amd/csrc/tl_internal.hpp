@@ -196,9 +196,8 @@ enum GcFmt : int { GC_BF16 = 0, GC_F16 = 1 };
 // kernels: each sweep reads and writes fields far larger than the caches.
 // Measured at 8192^2 (A/B in one box, loads and stores together against
 // neither): fused FP32 CG 4.68 / 4.78 -> 5.14 / 5.04 TB/s (odd / even t), FP32
-// PW 4.65 -> 5.37, FP32 UR 5.03 / 5.09 -> 6.08 / 5.98, FP64 PW 5.23 -> 5.33,
-// Chebyshev / PPCG steps +6-7%; loads alone
-// made the fused kernel 4% slower.  The two-step solver kernels have their
+// PW 4.65 -> 5.37, FP32 UR 5.03 / 5.09 -> 6.08 / 5.98, Chebyshev / PPCG
+// steps +6-7%; loads alone made the fused kernel 4% slower.  The two-step solver kernels have their
 // own switches: with both they ran 2-4% slower, with loads alone 6-8% slower,
 // with stores alone within +-2%.
 #ifndef TL_NT_LOAD

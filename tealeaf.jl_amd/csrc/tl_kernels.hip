@@ -8,21 +8,25 @@
 // fetched from HBM once per sweep.  Left/right neighbours are re-read through
 // L1/L2.
 //
-// The iteration kernels are vectorised: a
-// thread owns V = 4 (FP32) or 2 (FP64) consecutive columns loaded as one
-// 16-byte vector, left/right neighbours come from the adjacent lanes (lanes
-// 0 and 63 load the column outside the wave together with the row loads),
-// and the rows of a band are loaded in batches that are software-pipelined
-// (row_batches): the next batch's loads are issued before the current batch
-// is computed, so a wave keeps loads in flight while it computes.
+// The iteration kernels are vectorised: a thread owns V = 4 (FP32) or 2 (FP64)
+// consecutive columns loaded as one 16-byte vector, left/right neighbours come
+// from the adjacent lanes (lanes 0 and 63 load the column outside the wave
+// together with the row loads), and the rows of a band are loaded in batches that
+// are software-pipelined (row_batches): the next batch's loads are issued before
+// the current batch is computed, so a wave keeps loads in flight while it
+// computes.  The CG sweeps (k_cgs, k_cgp) and the CG held in registers (k_cgr) use
+// overlapped wave tiles instead, whose outer lanes hold the neighbours' columns.
 //
 // Halo.  The depth-1 reflective halo of kernels.jl:191-210 (with the index
 // correction of the intended algorithm) is applied by clamping neighbour
 // indices to the interior: a reflected ghost cell holds exactly the value of
 // the interior cell it mirrors, so the arithmetic is bit-identical to reading
-// an updated halo and no halo exchange is needed inside a solve.
+// an updated halo and no halo exchange is needed inside a solve.  In the CG kernels
+// with overlapped tiles the domain faces' coefficients are zero instead (k_init_coef,
+// k_gcell).
 //
-// Reductions need no atomics and no fences.  A producing kernel writes one
+// Reductions need no atomics and no fences (but k_cgr's, whose blocks exchange
+// within a launch).  A producing kernel writes one
 // partial sum per block (wave64 butterfly, then a fixed-order block sum).
 // The consuming kernel -- the next one on the stream, so the kernel boundary
 // makes the partials visible -- has every block sum the ~2k partials in the
